@@ -228,7 +228,7 @@ struct vamx_batch {
   struct Layout {
     std::vector<int> sig;          // per problem: kernel path chosen for the buffers' alignment
     std::vector<char> devs;        // the plans' ParDev bytes (work order set by vamx_par_set_tuning)
-    std::vector<int> single;       // forward: problems projected by their own single-problem launch
+    std::vector<int> single;       // problems projected by their own single-problem launch
     std::vector<Chunk> chunks;
   };
   std::vector<Layout> layouts[2];  // [0] backward, [1] forward
@@ -293,8 +293,11 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
 }
 
 // kernel path of problem i for these buffers: wave z width (1, 2, 4; 3 = z
-// and z + 64), or -1 / -4 for the per-lane kernels with 1 / 4 z per thread
+// and z + 64), -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
+// kOwnLaunch for plans whose kernels the persistent launch does not hold
+constexpr int kOwnLaunch = 0;
 int problem_path(vamx_plan* p, const float* in, float* out, bool forward) {
+  if (incl_wave_ok(p)) return kOwnLaunch;
   int wz = forward ? par_fp_wave_zv(p, in, out) : par_wave_zv(p, in, out, p->par.bp_zv);
   if (par_wave_split(p, wz)) return 3;
   if (wz) return wz;
@@ -326,6 +329,10 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
     it.minmax = p->d_minmax;
     it.clip = forward ? !(p->flags & VAMX_PAR_NO_WARP_CLIP) : !(p->flags & VAMX_PAR_NO_CIRCLE_CLIP);
     const int path = sig[(size_t)i];
+    if (path == kOwnLaunch) {
+      L.single.push_back(i);
+      continue;
+    }
     if (path > 0) {
       const int wz = path == 3 ? 2 : path;
       it.wave = 1;
@@ -422,7 +429,7 @@ int run_batch(vamx_batch* b, const float* const* ins, float* const* outs, hipStr
     int rc = build_layout(b, sig, devs, forward, s, &L);
     if (rc) return rc;
   }
-  // single-problem forward launches round-robin on the caller's stream and
+  // single-problem launches round-robin on the caller's stream and
   // two side streams forked from and joined back to it with events (so the
   // call stays graph-capturable): one launch's tail overlaps the next one's
   // start
@@ -438,7 +445,8 @@ int run_batch(vamx_batch* b, const float* const* ins, float* const* outs, hipStr
       const int i = L->single[k];
       vamx_plan* p = b->plans[(size_t)i];
       hipStream_t st = (k % ns == 0) ? s : b->side[k % ns - 1];
-      rc = par_forward_launch(p, ins[i], outs[i], st, !(p->flags & VAMX_PAR_NO_WARP_CLIP));
+      rc = forward ? par_forward_launch(p, ins[i], outs[i], st, !(p->flags & VAMX_PAR_NO_WARP_CLIP))
+                   : par_backward_launch(p, ins[i], outs[i], st, !(p->flags & VAMX_PAR_NO_CIRCLE_CLIP));
     }
     if (ns > 1) {
       // joined also after a failed launch, so a capture on s is never left

@@ -12,6 +12,7 @@
 //   C  forward projection of the operand (or the exact transpose of the back
 //      projection) fused with g <- clip(g - lr * scale * grad, glb, gub).
 // The per-voxel epilogue runs in float64, as the reference does in NumPy.
+#include <algorithm>
 #include <mutex>
 
 #include "bclp_core.h"
@@ -96,6 +97,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void b
   }
   const double s = block_sum_256(part, sh);
   if (threadIdx.x == 0) partials[lb] = s;
+}
+
+// A, second half, after a back projection into `dose` by the plain kernels:
+// response, band, Lp weighting and loss partials of a whole dose, grid-stride
+// (bound by its 12 bytes per voxel)
+__global__ __launch_bounds__(256) void bclp_epilogue_kernel(RespDev r, BclpDev b, const float* __restrict__ dose,
+                                                            const float* __restrict__ target,
+                                                            float* __restrict__ operand,
+                                                            double* __restrict__ partials, long long nv) {
+  __shared__ double sh[256];
+  double part = 0.0;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += 256ll * gridDim.x) {
+    float o;
+    part += bclp_voxel(r, b, dose[i], target[i], (size_t)i, o);
+    operand[i] = o;
+  }
+  const double s = block_sum_256(part, sh);
+  if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
 // C (wavefront-uniform variant)
@@ -351,6 +370,19 @@ WsLayout ws_layout(const vamx_plan* p) {
   return w;
 }
 
+// Kernel A as two launches: the plain back projection into `dose`, then the
+// element-wise epilogue, whose at most 2048 partials replace the count in nparts
+int split_epilogue(vamx_plan* p, const RespDev& r, const BclpDev& b, const float* g, const float* target, float* dose,
+                   float* operand, double* partials, int clipc, int& nparts, hipStream_t s) {
+  const int rc = par_backward_launch(p, g, dose, s, clipc != 0);
+  if (rc) return rc;
+  const long long nv = (long long)p->par.n * p->par.n * p->par.nz;
+  nparts = std::min(nparts, 2048);
+  hipLaunchKernelGGL(bclp_epilogue_kernel, dim3(nparts), dim3(256), 0, s, r, b, dose, target, operand, partials, nv);
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
 // Launches kernel A; its per-block loss partials go to partials[0, nparts).
 // Fails before launching when nparts would exceed max_parts.
 int launch_epilogue(vamx_plan* p, const RespDev& r, const BclpDev& b, const float* g, const float* target,
@@ -390,6 +422,7 @@ int launch_epilogue(vamx_plan* p, const RespDev& r, const BclpDev& b, const floa
   if (nparts > max_parts)
     return set_error(VAMX_ERR_ARG, "bclp: " + std::to_string(nparts) + " loss partials exceed the " +
                                         std::to_string(max_parts) + " slots of the scratch");
+  if (incl_wave_ok(p)) return split_epilogue(p, r, b, g, target, dose, operand, partials, clipc, nparts, s);
   const dim3 grid(nparts), block(256);
   if (gd.incl)
     hipLaunchKernelGGL((bclp_bp_epilogue<1, true>), grid, block, 0, s, gd, clipc, r, b, g, target, dose, operand,
@@ -441,6 +474,7 @@ int bclp_update_impl(vamx_plan* plan, const vamx_bclp_params* prm, float* g, con
       rc = par_slice_minmax(plan, operand, s);
       if (rc) return rc;
     }
+    if (incl_wave_ok(plan)) return incl_forward_update(plan, operand, UpdateOut{g, scale, lr, glb, gub}, s);
     const int wz = par_fp_wave_zv(plan, operand, g);
     if (wz && gd.fp_pair && gd.pair_ok) {
       const long long threads = fp_pair_tiled(gd) * wave_zchunks(gd.nz, wz) * 64;

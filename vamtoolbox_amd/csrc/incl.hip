@@ -1,0 +1,358 @@
+// Inclined projections (rays tilted by phi against the detector's rows) on
+// wavefronts: forward of one ray, back projection of one voxel column, with z
+// across the lanes.
+//
+// At inclination phi a sample at along-ray coordinate s lies s tan(phi)
+// slices above the ray's detector row: floor q and fraction w of that shift
+// are the same for every row, so a sample's in-plane taps, its absorption
+// weight, q and w are wave-uniform.  Lane l evaluates the geometry of sample
+// r0 + l (or angle i0 + l) once, in float64, into a per-wavefront LDS table;
+// the wavefront then walks the table.  Lane l loads slice j + q of its
+// detector row j and adds it, weighted 1 - w, to row j's sum and, weighted w,
+// to a second sum that belongs to row j - 1 (whose upper slice it is): each
+// in-plane tap is one load, not two.  The second sum moves down one lane
+// after the walk, so the last lane's row is not complete and a wavefront
+// covers 64 NS - 1 rows (L - 1 in the grouped form).  Slices outside the
+// volume get an offset past the buffer descriptor's range and read 0.
+//
+// Below 64 rows (nz <= 31) the lanes form 64 / L groups of L; group g takes
+// every (64 / L)-th table entry, and the groups' sums are added at the end.
+//
+// Bound by vector instruction issue: per sample and 64 rows four dword loads
+// (5 cycles of the texture path each) and six multiply-adds.  The per-lane
+// kernels this replaces evaluated the float64 geometry in every lane and
+// loaded eight taps per sample.
+#include <type_traits>
+
+#include "par_core.h"
+
+namespace vamx {
+
+namespace {
+
+constexpr int kU = 4;                 // table entries per step (loads in flight)
+constexpr int kTab = 64 + kU * 8;     // entries past 64 are empty
+constexpr int kNone = 1 << 29;        // shift of an empty entry: every slice is out of range, so it reads 0
+constexpr int kOne = 1 << 28;         // cell flags: one column (kOne) or row (2 kOne) only -- the weightless
+                                      // second one is not read (its voxels may lie outside, or hold no number)
+
+struct InclSlot {
+  float4* w;   // forward: bilinear tap weights; back: row weights for the two sums
+  float4* a;   // forward: weights of the two sums, cell, shift; back: -, second row, row, shift
+};
+__device__ __forceinline__ InclSlot incl_slot() {
+  __shared__ float4 w[4][kTab];
+  __shared__ float4 a[4][kTab];
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 3;
+  return {w[wv], a[wv]};
+}
+
+__device__ __forceinline__ void incl_pad(const InclSlot& sl, int lane) {
+  if (lane < kTab - 64) {
+    sl.w[64 + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+    sl.a[64 + lane] = make_float4(0.f, 0.f, 0.f, __int_as_float(kNone));
+  }
+}
+
+// the taps of one axis: first one b with weight s0, and b + 1 with s1 (0: no second tap)
+__device__ __forceinline__ void axis_taps(double coord, int n, int& b, double& s0, double& s1) {
+  const double f = floor(coord), d = coord - f;
+  const int fi = (int)f;
+  b = fi < 0 ? 0 : fi;
+  s0 = fi < 0 ? d : 1.0 - d;
+  s1 = fi < 0 || fi >= n - 1 ? 0.0 : d;
+}
+
+// byte offset of slice zz, or one that the descriptor's range rejects (reads 0)
+__device__ __forceinline__ uint32_t slice_off(int zz, int nz) {
+  return (unsigned)zz < (unsigned)nz ? 4u * (uint32_t)zz : 0x80000000u;
+}
+
+// completes the two sums of every row: out[s] is the row j0 + l + 64 s (valid
+// below the wavefront's row count, in group 0)
+template <int NS, int L>
+__device__ __forceinline__ void incl_combine(float (&lo)[NS], float (&hi)[NS], int lane) {
+  if constexpr (L < 64) {
+#pragma unroll
+    for (int o = L; o < 64; o <<= 1) {
+      lo[0] += __shfl_xor(lo[0], o);
+      hi[0] += __shfl_xor(hi[0], o);
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    float up = __shfl_down(hi[s], 1);
+    if (s + 1 < NS) {
+      const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hi[s + 1]), 0));
+      if (lane == 63) up = first;
+    }
+    lo[s] += up;
+  }
+}
+
+// rows of one wavefront
+template <int NS, int L> constexpr int incl_rows() { return (L < 64 ? L : 64 * NS) - 1; }
+
+template <int NS, int L, class Out>
+__global__ __launch_bounds__(256) void incl_fp_kernel(ParDev g, const float* __restrict__ vol, Out out) {
+  constexpr int G = 64 / L, S = incl_rows<NS, L>();
+  const int lane = threadIdx.x & 63, l = lane & (L - 1), grp = lane / L;
+  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long rays = (long long)g.n * g.na;
+  const int nch = (g.nz + S - 1) / S;
+  if (wave >= rays * nch) return;   // whole wavefronts
+  const int j0 = (int)(wave / rays) * S;
+  const int i = (int)((wave % rays) / g.n), k = (int)((wave % rays) % g.n);
+  const int n = g.n, nz = g.nz;
+  const double* M = g.mats + 6 * i;
+  const double kp = (double)k - g.det_offset;
+  const double a0 = M[0] * kp, a1 = M[3] * kp;
+  const double t = (double)(k - g.c) - g.det_offset;
+  const uint32_t oc = 4u * (uint32_t)nz, orr = (uint32_t)n * oc, span = orr + 2 * oc;
+  const InclSlot sl = incl_slot();
+  incl_pad(sl, lane);
+  float lo[NS] = {}, hi[NS] = {};
+  for (int r0 = 0; r0 < n; r0 += 64) {
+    const int r = r0 + lane;
+    float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+    float aw0 = 0.f, aw1 = 0.f;
+    int base = 0, q = kNone;
+    bool valid = false;
+    if (r < n) {
+      const double rr = (double)r;
+      const double col = (a0 + M[1] * rr) + M[2];
+      const double row = (a1 + M[4] * rr) + M[5];
+      if (row > -1.0 && row < (double)n && col > -1.0 && col < (double)n) {
+        int br, bc;
+        double r0w, r1w, c0w, c1w;
+        axis_taps(row, n, br, r0w, r1w);
+        axis_taps(col, n, bc, c0w, c1w);
+        const double s = (double)(r - g.c), dz = s * g.tan_phi, fz = floor(dz);
+        const float aw = abs_weight(g, t, s);
+        base = (br * n + bc) | (c1w == 0.0 ? kOne : 0) | (r1w == 0.0 ? 2 * kOne : 0);
+        if (aw != 0.0f) q = (int)fz;
+        aw0 = aw * (float)(1.0 - (dz - fz));
+        aw1 = aw * (float)(dz - fz);
+        w = make_float4((float)(r0w * c0w), (float)(r0w * c1w), (float)(r1w * c0w), (float)(r1w * c1w));
+        valid = aw != 0.0f;
+      }
+    }
+    const unsigned long long m = __ballot(valid);
+    __builtin_amdgcn_wave_barrier();
+    sl.w[lane] = w;
+    sl.a[lane] = make_float4(aw0, aw1, __int_as_float(base), __int_as_float(q));
+    __builtin_amdgcn_wave_barrier();
+    if (!m) continue;
+    const int first = __builtin_ctzll(m) & ~(G - 1), last = 63 - __builtin_clzll(m);
+    for (int e0 = first; e0 <= last; e0 += kU * G) {
+      float v[kU][NS][4];
+      float4 ww[kU];
+      float2 aa[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const int e = e0 + u * G + grp;
+        ww[u] = sl.w[e];
+        const float4 A = sl.a[e];
+        aa[u] = make_float2(A.x, A.y);
+        const int b = __float_as_int(A.z), qs = __float_as_int(A.w);
+        if constexpr (G == 1) {
+          const int bu = __builtin_amdgcn_readfirstlane(b);
+          const __amdgpu_buffer_rsrc_t rs = buf_rsrc(vol + (size_t)(bu & (kOne - 1)) * nz, span);
+          const uint32_t o1 = bu & kOne ? 0u : oc, o2 = bu & (2 * kOne) ? 0u : orr;
+          const int z = j0 + lane + __builtin_amdgcn_readfirstlane(qs);
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            const uint32_t vo = slice_off(z + 64 * s, nz);
+            v[u][s][0] = bload<1>(rs, vo, 0);
+            v[u][s][1] = bload<1>(rs, vo, o1);
+            v[u][s][2] = bload<1>(rs, vo, o2);
+            v[u][s][3] = bload<1>(rs, vo, o1 + o2);
+          }
+        } else {
+          const int z = j0 + l + qs;
+          const bool in = (unsigned)z < (unsigned)nz;
+          const float* p = vol + (size_t)(b & (kOne - 1)) * nz + (in ? z : 0);
+          const int o1 = b & kOne ? 0 : nz, o2 = b & (2 * kOne) ? 0 : n * nz;
+          const float x0 = p[0], x1 = p[o1], x2 = p[o2], x3 = p[o1 + o2];
+          v[u][0][0] = in ? x0 : 0.0f;
+          v[u][0][1] = in ? x1 : 0.0f;
+          v[u][0][2] = in ? x2 : 0.0f;
+          v[u][0][3] = in ? x3 : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const float x = vfma(ww[u].w, v[u][s][3],
+                               vfma(ww[u].z, v[u][s][2], vfma(ww[u].y, v[u][s][1], ww[u].x * v[u][s][0])));
+          lo[s] = vfma(aa[u].x, x, lo[s]);
+          hi[s] = vfma(aa[u].y, x, hi[s]);
+        }
+    }
+  }
+  incl_combine<NS, L>(lo, hi, lane);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int so = l + 64 * s;
+    if (grp == 0 && so < S && j0 + so < nz) out.put(((size_t)k * g.na + i) * nz + j0 + so, lo[s]);
+  }
+}
+
+template <int NS, int L>
+__global__ __launch_bounds__(256) void incl_bp_kernel(ParDev g, const float* __restrict__ sino,
+                                                      float* __restrict__ vol, int clipc) {
+  constexpr int G = 64 / L, S = incl_rows<NS, L>();
+  const int lane = threadIdx.x & 63, l = lane & (L - 1), grp = lane / L;
+  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  // consecutive wavefronts walk 8 x 8 patches of voxel columns (neighbouring
+  // columns read the same detector rows)
+  const int n = g.n, nz = g.nz, nt = (n + 7) / 8;
+  const long long cols = 64ll * nt * nt;
+  const int nch = (nz + S - 1) / S;
+  if (wave >= cols * nch) return;   // whole wavefronts
+  const int j0 = (int)(wave / cols) * S;
+  const int patch = (int)((wave % cols) >> 6), in = (int)(wave & 63);
+  const int row = (patch / nt) * 8 + (in >> 3), col = (patch % nt) * 8 + (in & 7);
+  if (row >= n || col >= n) return;
+  float lo[NS] = {}, hi[NS] = {};
+  if (!(clipc && g.outside[row * n + col])) {
+    const double x = (double)(col - g.c), y = (double)(row - g.c);
+    const uint32_t row_b = 4u * (uint32_t)g.na * (uint32_t)nz, span = row_b + 4u * (uint32_t)nz;
+    const InclSlot sl = incl_slot();
+    incl_pad(sl, lane);
+    for (int i0 = 0; i0 < g.na; i0 += 64) {
+      const int i = i0 + lane;
+      float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+      int at = 0, q = kNone, step = 0;
+      if (i < g.na) {
+        const double co = g.cs[2 * i], sn = g.cs[2 * i + 1];
+        const double t = x * co - y * sn;
+        int j, j1;
+        float f;
+        if (interp_node(g, t, j, j1, f)) {
+          const double s = x * sn + y * co, dz = -(s * g.tan_phi), fz = floor(dz);
+          const float aw = abs_weight(g, t, s);
+          const float b0 = aw * (float)(1.0 - (dz - fz)), b1 = aw * (float)(dz - fz);
+          at = j * g.na + i;
+          step = j1 > j;   // 0 exactly at the last node: fp[n - 1]
+          if (aw != 0.0f) q = (int)fz;
+          w = make_float4((1.0f - f) * b0, f * b0, (1.0f - f) * b1, f * b1);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      sl.w[lane] = w;
+      sl.a[lane] = make_float4(0.f, __int_as_float(step), __int_as_float(at), __int_as_float(q));
+      __builtin_amdgcn_wave_barrier();
+      const int rows = g.na - i0 < 64 ? g.na - i0 : 64;
+      for (int e0 = 0; e0 < rows; e0 += kU * G) {
+        float v[kU][NS][2];
+        float4 ww[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int e = e0 + u * G + grp;
+          ww[u] = sl.w[e];
+          const float4 A = sl.a[e];
+          const int st = __float_as_int(A.y), b = __float_as_int(A.z), qs = __float_as_int(A.w);
+          if constexpr (G == 1) {
+            const uint32_t o1 = __builtin_amdgcn_readfirstlane(st) ? row_b : 0u;
+            const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sino + (size_t)__builtin_amdgcn_readfirstlane(b) * nz, span);
+            const int z = j0 + lane + __builtin_amdgcn_readfirstlane(qs);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+              const uint32_t vo = slice_off(z + 64 * s, nz);
+              v[u][s][0] = bload<1>(rs, vo, 0);
+              v[u][s][1] = bload<1>(rs, vo, o1);
+            }
+          } else {
+            const int z = j0 + l + qs;
+            const bool in_z = (unsigned)z < (unsigned)nz;
+            const float* p = sino + (size_t)b * nz + (in_z ? z : 0);
+            const float x0 = p[0], x1 = p[st ? (size_t)g.na * nz : 0];
+            v[u][0][0] = in_z ? x0 : 0.0f;
+            v[u][0][1] = in_z ? x1 : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            lo[s] = vfma(ww[u].y, v[u][s][1], vfma(ww[u].x, v[u][s][0], lo[s]));
+            hi[s] = vfma(ww[u].w, v[u][s][1], vfma(ww[u].z, v[u][s][0], hi[s]));
+          }
+      }
+    }
+    incl_combine<NS, L>(lo, hi, lane);
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int so = l + 64 * s;
+    if (grp == 0 && so < S && j0 + so < nz) vol[((size_t)row * n + col) * nz + j0 + so] = lo[s];
+  }
+}
+
+// slabs of 64 rows per wavefront: a wavefront's geometry costs about 0.7 of a
+// slab's walk, so NS minimises chunks (NS + 0.7)
+int incl_slabs(int nz) {
+  int best = 1;
+  double cost = 1e30;
+  for (int ns = 1; ns <= 3; ++ns) {
+    const double c = (double)((nz + 64 * ns - 2) / (64 * ns - 1)) * (ns + 0.7);
+    if (c < cost) {
+      cost = c;
+      best = ns;
+    }
+  }
+  return best;
+}
+
+template <class F>
+void incl_dispatch(int nz, F&& f) {
+  using std::integral_constant;
+  if (nz <= 7) f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+  else if (nz <= 15) f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+  else if (nz <= 31) f(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+  else if (incl_slabs(nz) == 1) f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
+  else if (incl_slabs(nz) == 2) f(integral_constant<int, 2>{}, integral_constant<int, 64>{});
+  else f(integral_constant<int, 3>{}, integral_constant<int, 64>{});
+}
+
+template <class Out>
+int incl_forward(vamx_plan* p, const float* vol, Out out, hipStream_t s) {
+  const ParDev& g = p->par;
+  incl_dispatch(g.nz, [&](auto ns, auto l) {
+    constexpr int NS = decltype(ns)::value, L = decltype(l)::value, S = incl_rows<NS, L>();
+    const long long waves = (long long)g.n * g.na * ((g.nz + S - 1) / S);
+    hipLaunchKernelGGL((incl_fp_kernel<NS, L, Out>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, vol, out);
+  });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+}  // namespace
+
+bool incl_wave_ok(const vamx_plan* p) {
+  return p->par.incl && p->par.n >= 2 && !(p->flags & VAMX_PAR_PER_LANE_GEOMETRY);
+}
+
+int incl_forward_store(vamx_plan* p, const float* vol, float* sino, hipStream_t s) {
+  return incl_forward(p, vol, StoreOut{sino}, s);
+}
+
+int incl_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, hipStream_t s) {
+  return incl_forward(p, vol, out, s);
+}
+
+int incl_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s) {
+  const ParDev& g = p->par;
+  incl_dispatch(g.nz, [&](auto ns, auto l) {
+    constexpr int NS = decltype(ns)::value, L = decltype(l)::value, S = incl_rows<NS, L>();
+    const long long nt = (g.n + 7) / 8, waves = 64 * nt * nt * ((g.nz + S - 1) / S);
+    hipLaunchKernelGGL((incl_bp_kernel<NS, L>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, sino, vol,
+                       clipc ? 1 : 0);
+  });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+}  // namespace vamx

@@ -1474,9 +1474,25 @@ __device__ __forceinline__ void fpT_quad_wave(const ParDev& g, const float* __re
   }
 }
 
+// what a forward kernel does with a ray's value: store it in the sinogram, or
+// the BCLP update g <- clip(g - lr * scale * value) (BCLP.py:486-487, 532)
+struct StoreOut {
+  float* sino;
+  __device__ __forceinline__ void put(size_t at, float v) const { sino[at] = v; }
+};
+struct UpdateOut {
+  float* gsino;
+  const double* scale_p;
+  float lr, glb, gub;
+  __device__ __forceinline__ void put(size_t at, float v) const {
+    gsino[at] = clampf(gsino[at] - lr * ((float)(*scale_p) * v), glb, gub);
+  }
+};
+
 // host helpers implemented in parallel.hip
 int par_slice_minmax(vamx_plan* p, const float* vol, hipStream_t s);
 int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t s, bool warp_clip);
+int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t s, bool clipc);
 bool par_use_vec4(const vamx_plan* p, const void* a, const void* b);
 bool par_use_vec2(const vamx_plan* p, const void* a, const void* b);
 int par_wave_zv(const vamx_plan* p, const void* a, const void* b, int requested);
@@ -1485,5 +1501,10 @@ bool par_wave_split(const vamx_plan* p, int zv);
 int wave_zv_choice(int nz, uintptr_t align_bits, int requested);
 void par_pair_units(const std::vector<double>& cs, int na, int n, int c, double D, std::vector<int>& units,
                     int& npaired_rays, int& first2);
+// inclined projections on wavefronts (incl.hip)
+bool incl_wave_ok(const vamx_plan* p);
+int incl_forward_store(vamx_plan* p, const float* vol, float* sino, hipStream_t s);
+int incl_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, hipStream_t s);
+int incl_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s);
 
 }  // namespace vamx

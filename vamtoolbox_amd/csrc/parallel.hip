@@ -660,6 +660,7 @@ int par_slice_minmax(vamx_plan* p, const float* vol, hipStream_t s) {
 
 int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t s, bool warp_clip) {
   const ParDev& g = p->par;
+  if (incl_wave_ok(p)) return incl_forward_store(p, vol, sino, s);
   if (g.incl) {
     const long long total = (long long)g.na * g.n * g.nz;
     hipLaunchKernelGGL(par_fp_incl_kernel, dim3(blocks_for(total, 256)), dim3(256), 0, s, g, vol, sino);
@@ -742,6 +743,7 @@ int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t 
 
 int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t s, bool clipc) {
   const ParDev& g = p->par;
+  if (incl_wave_ok(p)) return incl_backward(p, sino, vol, clipc, s);
   if (g.incl) {
     const long long total = (long long)g.n * g.n * g.nz;
     hipLaunchKernelGGL(par_bp_incl_kernel, dim3(blocks_for(total, 256)), dim3(256), 0, s, g, sino, vol,
