@@ -297,7 +297,7 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
 // kOwnLaunch for plans whose kernels the persistent launch does not hold
 constexpr int kOwnLaunch = 0;
 int problem_path(vamx_plan* p, const float* in, float* out, bool forward) {
-  if (incl_wave_ok(p)) return kOwnLaunch;
+  if (incl_wave_ok(p) || thin_ok(p)) return kOwnLaunch;
   int wz = forward ? par_fp_wave_zv(p, in, out) : par_wave_zv(p, in, out, p->par.bp_zv);
   if (par_wave_split(p, wz)) return 3;
   if (wz) return wz;

@@ -422,7 +422,7 @@ int launch_epilogue(vamx_plan* p, const RespDev& r, const BclpDev& b, const floa
   if (nparts > max_parts)
     return set_error(VAMX_ERR_ARG, "bclp: " + std::to_string(nparts) + " loss partials exceed the " +
                                         std::to_string(max_parts) + " slots of the scratch");
-  if (incl_wave_ok(p)) return split_epilogue(p, r, b, g, target, dose, operand, partials, clipc, nparts, s);
+  if (incl_wave_ok(p) || thin_ok(p)) return split_epilogue(p, r, b, g, target, dose, operand, partials, clipc, nparts, s);
   const dim3 grid(nparts), block(256);
   if (gd.incl)
     hipLaunchKernelGGL((bclp_bp_epilogue<1, true>), grid, block, 0, s, gd, clipc, r, b, g, target, dose, operand,
@@ -475,6 +475,7 @@ int bclp_update_impl(vamx_plan* plan, const vamx_bclp_params* prm, float* g, con
       if (rc) return rc;
     }
     if (incl_wave_ok(plan)) return incl_forward_update(plan, operand, UpdateOut{g, scale, lr, glb, gub}, s);
+    if (thin_ok(plan)) return thin_forward_update(plan, operand, UpdateOut{g, scale, lr, glb, gub}, clip, s);
     const int wz = par_fp_wave_zv(plan, operand, g);
     if (wz && gd.fp_pair && gd.pair_ok) {
       const long long threads = fp_pair_tiled(gd) * wave_zchunks(gd.nz, wz) * 64;

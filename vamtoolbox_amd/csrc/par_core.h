@@ -1506,5 +1506,11 @@ bool incl_wave_ok(const vamx_plan* p);
 int incl_forward_store(vamx_plan* p, const float* vol, float* sino, hipStream_t s);
 int incl_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, hipStream_t s);
 int incl_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s);
+// thin problems at zero inclination (thin.hip); the forward reads the plan's
+// slice min / max when clip is set
+bool thin_ok(const vamx_plan* p);
+int thin_forward_store(vamx_plan* p, const float* vol, float* sino, bool clip, hipStream_t s);
+int thin_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, bool clip, hipStream_t s);
+int thin_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s);
 
 }  // namespace vamx

@@ -16,7 +16,9 @@ namespace vamx {
 // Per-slice min / max of a volume (the warp clip range), pass 1: block b
 // reduces pixels [b*chunk, (b+1)*chunk) for every z.  Threads form groups of
 // min(nz, 1024) consecutive z values; the groups split the block's pixels and
-// are combined through LDS.
+// are combined through LDS, half of them at a time (one thread walking the
+// 1024 groups of a single slice took 12 us).  A block takes at least 16 values
+// per thread, so a small volume is one block, which writes the result itself.
 __global__ __launch_bounds__(1024) void slice_minmax_part(const float* __restrict__ vol, int npix, int nz,
                                                           int parts, float* __restrict__ part) {
   __shared__ float slo[1024], shi[1024];
@@ -40,13 +42,18 @@ __global__ __launch_bounds__(1024) void slice_minmax_part(const float* __restric
     slo[t] = lo;
     shi[t] = hi;
     __syncthreads();
-    if (grp == 0 && z < nz) {
-      for (int q = 1; q < groups; ++q) {
-        lo = fminf(lo, slo[q * zs + zt]);
-        hi = fmaxf(hi, shi[q * zs + zt]);
+    for (int live = groups; live > 1;) {   // uniform over the block
+      const int half = (live + 1) / 2;
+      if (grp + half < live) {
+        slo[t] = fminf(slo[t], slo[t + half * zs]);
+        shi[t] = fmaxf(shi[t], shi[t + half * zs]);
       }
-      part[(size_t)blockIdx.x * 2 * nz + z] = lo;
-      part[(size_t)blockIdx.x * 2 * nz + nz + z] = hi;
+      live = half;
+      __syncthreads();
+    }
+    if (grp == 0 && z < nz) {
+      part[(size_t)blockIdx.x * 2 * nz + z] = slo[t];
+      part[(size_t)blockIdx.x * 2 * nz + nz + z] = shi[t];
     }
     __syncthreads();
   }
@@ -650,10 +657,13 @@ extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) 
 namespace vamx {
 int par_slice_minmax(vamx_plan* p, const float* vol, hipStream_t s) {
   const ParDev& g = p->par;
-  hipLaunchKernelGGL(slice_minmax_part, dim3(p->minmax_parts), dim3(1024), 0, s, vol, g.n * g.n, g.nz,
-                     p->minmax_parts, p->d_minmax_part);
-  hipLaunchKernelGGL(slice_minmax_final, dim3((g.nz + 63) / 64), dim3(1024), 0, s, p->d_minmax_part, g.nz,
-                     p->minmax_parts, p->d_minmax);
+  const long long values = (long long)g.n * g.n * g.nz;
+  const int parts = (int)std::max(1ll, std::min((long long)p->minmax_parts, values / 16384));
+  hipLaunchKernelGGL(slice_minmax_part, dim3(parts), dim3(1024), 0, s, vol, g.n * g.n, g.nz, parts,
+                     parts == 1 ? p->d_minmax : p->d_minmax_part);
+  if (parts > 1)
+    hipLaunchKernelGGL(slice_minmax_final, dim3((g.nz + 63) / 64), dim3(1024), 0, s, p->d_minmax_part, g.nz, parts,
+                       p->d_minmax);
   VAMX_HIP(hipGetLastError());
   return VAMX_OK;
 }
@@ -671,6 +681,7 @@ int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t 
     int rc = par_slice_minmax(p, vol, s);
     if (rc) return rc;
   }
+  if (thin_ok(p)) return thin_forward_store(p, vol, sino, warp_clip, s);
   int wz = par_fp_wave_zv(p, vol, sino);
   const bool split = par_wave_split(p, wz);
   if (split) wz = 2;
@@ -744,6 +755,7 @@ int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t 
 int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t s, bool clipc) {
   const ParDev& g = p->par;
   if (incl_wave_ok(p)) return incl_backward(p, sino, vol, clipc, s);
+  if (thin_ok(p)) return thin_backward(p, sino, vol, clipc, s);
   if (g.incl) {
     const long long total = (long long)g.n * g.n * g.nz;
     hipLaunchKernelGGL(par_bp_incl_kernel, dim3(blocks_for(total, 256)), dim3(256), 0, s, g, sino, vol,

@@ -1,0 +1,412 @@
+// Thin problems (few slices, down to one) at zero inclination on wavefronts.
+//
+// With fewer than 32 slices one ray (voxel column) leaves most lanes of a
+// wavefront idle, so the lanes form G = 64 / L groups of L, and a lane holds
+// ZV slices (L ZV >= nz).
+//   forward: a wavefront owns a ray -- and its opposite ray, from the same
+//     taps -- and group g takes every G-th sample; the groups' sums are added
+//     at the end.  Lane l evaluates sample r0 + l's float64 geometry once for
+//     all slices, into a per-wavefront LDS table (one slice: a lane uses its
+//     own sample directly).
+//   back: group g owns a voxel column of an 8 x 8 patch; its lanes evaluate L
+//     angles at a time into the table.  Where the columns alone would leave
+//     the GPU short of wavefronts, the wavefronts of a block split the angles
+//     and add their sums through LDS.
+// The per-lane kernels evaluate every sample's geometry in every lane and
+// walk a whole ray (all angles) serially per thread, which leaves a small
+// problem waiting on one chain of loads per thread.
+#include <type_traits>
+
+#include "par_core.h"
+
+namespace vamx {
+
+namespace {
+
+// table entries per step: eight tap loads in flight, and registers for 6 or
+// more wavefronts per SIMD (four steps of 16-byte taps held 152 registers)
+template <int ZV> constexpr int steps() { return ZV == 4 ? 2 : 4; }
+constexpr int kTab = 64 + 4 * 32;      // entries past 64 are empty
+constexpr int kOne = 1 << 28;          // cell flags: one column (kOne) or row (2 kOne) only
+
+// the taps of one axis: first one b with weight s0, and b + 1 with s1 (0: no
+// second tap -- it is not read, its voxels may lie outside or hold no number)
+__device__ __forceinline__ void axis_taps(double coord, int n, int& b, double& s0, double& s1) {
+  const double f = floor(coord), d = coord - f;
+  const int fi = (int)f;
+  b = fi < 0 ? 0 : fi;
+  s0 = fi < 0 ? d : 1.0 - d;
+  s1 = fi < 0 || fi >= n - 1 ? 0.0 : d;
+}
+
+// abs_weight (par_core.h) with the half chord of a ray taken once
+struct Chord {
+  bool in;
+  double half;
+};
+__device__ __forceinline__ Chord chord_of(const ParDev& g, double t) {
+  if (g.mu == 0.0) return {true, 0.0};
+  return {fabs(t) < g.radius, sqrt(fmax(0.0, g.radius * g.radius - t * t))};
+}
+__device__ __forceinline__ float chord_weight(const ParDev& g, const Chord& c, double s) {
+  if (g.mu == 0.0) return 1.0f;
+  return c.in ? expf((float)(-g.mu * (fmax(0.0, c.half - s) * g.inv_cos))) : 0.0f;
+}
+
+// one sample of a ray: cell (with its flags), the axes' weights, the rays' absorption
+struct Sample {
+  int base;
+  float r0, r1, c0, c1, a, a2;
+  bool valid;
+};
+template <bool PAIR>
+__device__ __forceinline__ Sample ray_sample(const ParDev& g, const double* M, double a0, double a1, const Chord& ch,
+                                             int r, int r2_lo) {
+  Sample s{0, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, false};
+  const int n = g.n;
+  const double rr = (double)r;
+  const double col = (a0 + M[1] * rr) + M[2];
+  const double row = (a1 + M[4] * rr) + M[5];
+  if (!(row > -1.0 && row < (double)n && col > -1.0 && col < (double)n)) return s;
+  int br, bc;
+  double r0w, r1w, c0w, c1w;
+  axis_taps(row, n, br, r0w, r1w);
+  axis_taps(col, n, bc, c0w, c1w);
+  if (!PAIR || r < n) s.a = chord_weight(g, ch, (double)(r - g.c));
+  if constexpr (PAIR)
+    if (r >= r2_lo) s.a2 = chord_weight(g, ch, (double)(g.c - r));
+  s.valid = s.a != 0.0f || s.a2 != 0.0f;
+  s.base = (br * n + bc) | (c1w == 0.0 ? kOne : 0) | (r1w == 0.0 ? 2 * kOne : 0);
+  s.r0 = (float)r0w;
+  s.r1 = (float)r1w;
+  s.c0 = (float)c0w;
+  s.c1 = (float)c1w;
+  return s;
+}
+
+struct FpThinSlot {
+  float4* w;   // the axes' weights r0 r1 c0 c1
+  float4* a;   // absorption (ray, partner ray), cell, whether it is a sample
+};
+__device__ __forceinline__ FpThinSlot fp_thin_slot() {
+  __shared__ float4 w[4][kTab];
+  __shared__ float4 a[4][kTab];
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 3;
+  return {w[wv], a[wv]};
+}
+
+// a sample from its taps, clipped to the slice range
+template <int ZV, bool CLIP>
+__device__ __forceinline__ typename VecT<ZV>::T thin_value(const typename VecT<ZV>::T (&t)[4], float r0, float r1,
+                                                           float c0, float c1, const typename VecT<ZV>::T& lo,
+                                                           const typename VecT<ZV>::T& hi) {
+  using V = typename VecT<ZV>::T;
+  V v = vfma(r1 * c1, t[3], vfma(r1 * c0, t[2], vfma(r0 * c1, t[1], vmul(r0 * c0, t[0]))));
+  if constexpr (CLIP) v = vclamp(v, lo, hi);
+  return v;
+}
+
+template <int ZV>
+__device__ __forceinline__ void thin_load(const float* __restrict__ vol, int base, int n, int nz, int z,
+                                          typename VecT<ZV>::T (&t)[4]) {
+  const float* p = vol + (size_t)(base & (kOne - 1)) * nz + z;
+  const int o1 = base & kOne ? 0 : nz, o2 = base & (2 * kOne) ? 0 : n * nz;
+  t[0] = vload<ZV>(p);
+  t[1] = vload<ZV>(p + o1);
+  t[2] = vload<ZV>(p + o2);
+  t[3] = vload<ZV>(p + o1 + o2);
+}
+
+template <int ZV, int L, bool CLIP, bool PAIR>
+__device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restrict__ vol,
+                                         const float* __restrict__ minmax, int k, int i, int z, int lane,
+                                         typename VecT<ZV>::T& acc, typename VecT<ZV>::T& acc2) {
+  using V = typename VecT<ZV>::T;
+  static_assert(!(PAIR && CLIP), "the clipped sample is discontinuous at the border: no pairing");
+  constexpr int G = 64 / L, kU = steps<ZV>();
+  const int n = g.n, nz = g.nz, grp = lane / L;
+  const double* M = g.mats + 6 * i;
+  const double kp = (double)k - g.det_offset;
+  const double a0 = M[0] * kp, a1 = M[3] * kp;
+  const Chord ch = chord_of(g, (double)(k - g.c) - g.det_offset);
+  V lo = vzero<ZV>(), hi = vzero<ZV>();
+  if constexpr (CLIP) {
+    lo = vload<ZV>(minmax + z);
+    hi = vload<ZV>(minmax + nz + z);
+  }
+  acc = vzero<ZV>();
+  acc2 = vzero<ZV>();
+  // samples of the ray and of its opposite ray (fp_ray_wave)
+  const int r_end = PAIR ? (2 * g.c + 1 > n ? 2 * g.c + 1 : n) : n;
+  const int r2_lo = 2 * g.c - n + 1;
+  if constexpr (L == 1) {
+    for (int r0 = 0; r0 < r_end; r0 += 64) {
+      if (r0 + lane >= r_end) continue;
+      const Sample s = ray_sample<PAIR>(g, M, a0, a1, ch, r0 + lane, r2_lo);
+      if (!s.valid) continue;
+      V t[4];
+      thin_load<ZV>(vol, s.base, n, nz, z, t);
+      const V v = thin_value<ZV, CLIP>(t, s.r0, s.r1, s.c0, s.c1, lo, hi);
+      acc = vfma(s.a, v, acc);
+      if constexpr (PAIR) acc2 = vfma(s.a2, v, acc2);
+    }
+  } else {
+    const FpThinSlot sl = fp_thin_slot();
+    for (int p = lane; p < kTab - 64; p += 64) sl.a[64 + p] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int r0 = 0; r0 < r_end; r0 += 64) {
+      Sample s{0, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, false};
+      if (r0 + lane < r_end) s = ray_sample<PAIR>(g, M, a0, a1, ch, r0 + lane, r2_lo);
+      const unsigned long long m = __ballot(s.valid);
+      __builtin_amdgcn_wave_barrier();
+      sl.w[lane] = make_float4(s.r0, s.r1, s.c0, s.c1);
+      sl.a[lane] = make_float4(s.a, s.a2, __int_as_float(s.base), s.valid ? 1.0f : 0.0f);
+      __builtin_amdgcn_wave_barrier();
+      if (!m) continue;
+      const int first = __builtin_ctzll(m) & ~(G - 1), last = 63 - __builtin_clzll(m);
+      for (int e0 = first; e0 <= last; e0 += kU * G) {
+        V t[kU][4];
+        float4 w[kU], a[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int e = e0 + u * G + grp;
+          a[u] = sl.a[e];
+          w[u] = sl.w[e];
+          if (a[u].w != 0.0f) thin_load<ZV>(vol, __float_as_int(a[u].z), n, nz, z, t[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          if (a[u].w == 0.0f) continue;
+          const V v = thin_value<ZV, CLIP>(t[u], w[u].x, w[u].y, w[u].z, w[u].w, lo, hi);
+          acc = vfma(a[u].x, v, acc);
+          if constexpr (PAIR) acc2 = vfma(a[u].y, v, acc2);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int o = L; o < 64; o <<= 1) {
+#pragma unroll
+    for (int q = 0; q < ZV; ++q) {
+      vset(acc, q, vget(acc, q) + __shfl_xor(vget(acc, q), o));
+      if constexpr (PAIR) vset(acc2, q, vget(acc2, q) + __shfl_xor(vget(acc2, q), o));
+    }
+  }
+}
+
+template <int ZV, int L, class Out>
+__global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __restrict__ vol,
+                                                      const float* __restrict__ minmax, int clip, int pair, Out out) {
+  using V = typename VecT<ZV>::T;
+  const int lane = threadIdx.x & 63, z = (lane & (L - 1)) * ZV;
+  const int zl = z < g.nz ? z : g.nz - ZV;   // lanes past nz read a copy and store nothing
+  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  int k, i, k2 = -1, i2 = -1;
+  if (pair) {
+    const PairItem it = fp_pair_item<1>(wave, g, 0);
+    if (!it.ok) return;
+    k = it.k;
+    i = it.i;
+    k2 = it.k2;
+    i2 = it.i2;
+  } else {
+    if (wave >= fp_tiled_rays(g) || !fp_tile_ray(wave, g, k, i)) return;   // whole wavefronts
+  }
+  const bool clip_on = clip && wave_clip_active<ZV>(minmax, g.nz, zl);
+  auto put = [&](int kh, int ih, const V& v) {
+    if (lane < L && z < g.nz) {
+#pragma unroll
+      for (int q = 0; q < ZV; ++q) out.put(((size_t)kh * g.na + ih) * g.nz + z + q, vget(v, q));
+    }
+  };
+  V acc, acc2;
+  if (clip_on) {
+    for (int h = 0; h < (k2 >= 0 ? 2 : 1); ++h) {
+      const int kh = h ? k2 : k, ih = h ? i2 : i;
+      thin_ray<ZV, L, true, false>(g, vol, minmax, kh, ih, zl, lane, acc, acc2);
+      put(kh, ih, acc);
+    }
+  } else if (k2 >= 0) {
+    thin_ray<ZV, L, false, true>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+    put(k, i, acc);
+    put(k2, i2, acc2);
+  } else {
+    thin_ray<ZV, L, false, false>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+    put(k, i, acc);
+  }
+}
+
+template <int ZV, int L>
+__global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __restrict__ sino,
+                                                       float* __restrict__ vol, int clipc) {
+  using V = typename VecT<ZV>::T;
+  constexpr int G = 64 / L, kAng = 4;
+  __shared__ float4 tab[L == 1 ? 1 : 1024];
+  __shared__ float sums[1024 * ZV];
+  const int lane = threadIdx.x & 63, l = lane & (L - 1), grp = lane / L;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), split = blockDim.x >> 6;
+  const int n = g.n, nz = g.nz, nt = (n + 7) / 8;
+  const int z = l * ZV, zl = z < nz ? z : nz - ZV;
+  // block -> G columns of an 8 x 8 patch
+  const unsigned lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int patch = (int)(lb / (64 / G)), in = (int)(lb % (64 / G)) * G + grp;
+  const int row = (patch / nt) * 8 + (in >> 3), col = (patch % nt) * 8 + (in & 7);
+  const bool inside = row < n && col < n;
+  const bool active = inside && !(clipc && g.outside[row * n + col]);
+  const double x = (double)(col - g.c), y = (double)(row - g.c);
+  const int i_end = (int)((long long)g.na * (wv + 1) / split);
+  V acc = vzero<ZV>();
+  // row weights and the first row of angle i; no weight where the column is
+  // not computed (its rows are not read either)
+  auto geom = [&](int i, float& w0, float& w1, int& at, int& step) {
+    w0 = w1 = 0.0f;
+    at = step = 0;
+    if (!active || i >= i_end) return false;
+    const double co = g.cs[2 * i], sn = g.cs[2 * i + 1];
+    const double t = x * co - y * sn;
+    int j, j1;
+    float w;
+    if (!interp_node(g, t, j, j1, w)) return false;
+    const float aw = g.mu != 0.0 ? abs_weight(g, t, x * sn + y * co) : 1.0f;
+    w0 = aw * (1.0f - w);
+    w1 = aw * w;
+    at = j * g.na + i;
+    step = j1 > j ? g.na * nz : 0;
+    return aw != 0.0f;
+  };
+  int i = (int)((long long)g.na * wv / split);
+  if constexpr (L == 1) {
+    for (; i < i_end; i += kAng) {
+      V b0[kAng], b1[kAng];
+      float w0[kAng], w1[kAng];
+      bool ok[kAng];
+#pragma unroll
+      for (int u = 0; u < kAng; ++u) {
+        int at, step;
+        ok[u] = geom(i + u, w0[u], w1[u], at, step);
+        b0[u] = b1[u] = vzero<ZV>();
+        if (ok[u]) {
+          const float* p = sino + (size_t)at * nz + zl;
+          b0[u] = vload<ZV>(p);
+          b1[u] = vload<ZV>(p + step);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kAng; ++u)
+        if (ok[u]) acc = vfma(w1[u], b1[u], vfma(w0[u], b0[u], acc));
+    }
+  } else {
+    float4* const tb = tab + wv * 64;
+    for (; i < i_end; i += L) {
+      float w0, w1;
+      int at, step;
+      const bool ok = geom(i + l, w0, w1, at, step);
+      __builtin_amdgcn_wave_barrier();
+      tb[lane] = make_float4(w0, w1, __int_as_float(ok ? at : -1), __int_as_float(step));
+      __builtin_amdgcn_wave_barrier();
+      constexpr int K = L < kAng ? L : kAng;
+#pragma unroll
+      for (int u0 = 0; u0 < L; u0 += K) {
+        if (u0 > 0 && i + u0 >= i_end) break;
+        V b0[K], b1[K];
+        float4 e[K];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+          e[u] = tb[grp * L + u0 + u];
+          b0[u] = b1[u] = vzero<ZV>();
+          const int a = __float_as_int(e[u].z);
+          if (a >= 0) {
+            const float* p = sino + (size_t)a * nz + zl;
+            b0[u] = vload<ZV>(p);
+            b1[u] = vload<ZV>(p + __float_as_int(e[u].w));
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < K; ++u) acc = vfma(e[u].y, b1[u], vfma(e[u].x, b0[u], acc));
+      }
+    }
+  }
+  if (split > 1) {
+#pragma unroll
+    for (int q = 0; q < ZV; ++q) sums[q * 1024 + threadIdx.x] = vget(acc, q);
+    __syncthreads();
+    if (wv == 0) {
+      for (int s = 1; s < split; ++s)
+#pragma unroll
+        for (int q = 0; q < ZV; ++q) vset(acc, q, vget(acc, q) + sums[q * 1024 + s * 64 + lane]);
+    }
+  }
+  if (wv == 0 && inside && z < nz) vstore<ZV>(vol + ((size_t)row * n + col) * nz + z, acc);
+}
+
+// z layout: four slices per lane where nz is a multiple of 4 and the buffers
+// are 16-byte aligned (a 16-byte load costs the texture path 16 cycles for 64
+// lanes, a dword load 5: 4 slices per 16 against 4 per 20), else one
+bool thin_v4(int nz, const void* a, const void* b) {
+  return nz % 4 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0;
+}
+
+template <class F>
+void thin_dispatch(int nz, bool v4, F&& f) {
+  using std::integral_constant;
+  const int lanes = v4 ? nz / 4 : nz;
+  auto with = [&](auto zv) {
+    if (lanes <= 1) f(zv, integral_constant<int, 1>{});
+    else if (lanes <= 2) f(zv, integral_constant<int, 2>{});
+    else if (lanes <= 4) f(zv, integral_constant<int, 4>{});
+    else if (lanes <= 8) f(zv, integral_constant<int, 8>{});
+    else if (lanes <= 16) f(zv, integral_constant<int, 16>{});
+    else f(zv, integral_constant<int, 32>{});
+  };
+  if (v4) with(integral_constant<int, 4>{});
+  else with(integral_constant<int, 1>{});
+}
+
+template <class Out>
+int thin_forward(vamx_plan* p, const float* vol, const void* sino, Out out, bool clip, hipStream_t s) {
+  const ParDev& g = p->par;
+  // opposite rays share their taps' loads, but below about 4 wavefronts per
+  // SIMD the GPU has room to project them side by side instead
+  const int pair = g.fp_pair && g.pair_ok && fp_pair_tiled(g) >= 4096;
+  const long long waves = pair ? fp_pair_tiled(g) : fp_tiled_rays(g);
+  thin_dispatch(g.nz, thin_v4(g.nz, vol, sino), [&](auto zv, auto l) {
+    constexpr int ZV = decltype(zv)::value, L = decltype(l)::value;
+    hipLaunchKernelGGL((thin_fp_kernel<ZV, L, Out>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, vol,
+                       p->d_minmax, clip ? 1 : 0, pair, out);
+  });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+}  // namespace
+
+bool thin_ok(const vamx_plan* p) {
+  const ParDev& g = p->par;
+  return !g.incl && !g.occ && g.n >= 2 && g.nz < 32 && !(p->flags & VAMX_PAR_PER_LANE_GEOMETRY);
+}
+
+int thin_forward_store(vamx_plan* p, const float* vol, float* sino, bool clip, hipStream_t s) {
+  return thin_forward(p, vol, sino, StoreOut{sino}, clip, s);
+}
+
+int thin_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, bool clip, hipStream_t s) {
+  return thin_forward(p, vol, out.gsino, out, clip, s);
+}
+
+int thin_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s) {
+  const ParDev& g = p->par;
+  const long long nt = (g.n + 7) / 8;
+  thin_dispatch(g.nz, thin_v4(g.nz, sino, vol), [&](auto zv, auto l) {
+    constexpr int ZV = decltype(zv)::value, L = decltype(l)::value;
+    const long long blocks = nt * nt * L;
+    // wavefronts per block: the angles are split until about 8 wavefronts per
+    // SIMD are in flight, at most 16 ways and into no fewer than 8 angles
+    int split = 1;
+    while (split < 16 && blocks * split < 8192 && g.na >= 16 * split) split *= 2;
+    hipLaunchKernelGGL((thin_bp_kernel<ZV, L>), dim3((unsigned)blocks), dim3(64 * split), 0, s, g, sino, vol,
+                       clipc ? 1 : 0);
+  });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+}  // namespace vamx
