@@ -28,6 +28,7 @@ namespace {
 template <int ZV> constexpr int steps() { return ZV == 4 ? 2 : 4; }
 constexpr int kTab = 64 + 4 * 32;      // entries past 64 are empty
 constexpr int kOne = 1 << 28;          // cell flags: one column (kOne) or row (2 kOne) only
+constexpr uint32_t kOut = 0x80000000u; // offset past every buffer: the load returns 0
 
 // the taps of one axis: first one b with weight s0, and b + 1 with s1 (0: no
 // second tap -- it is not read, its voxels may lie outside or hold no number)
@@ -106,18 +107,23 @@ __device__ __forceinline__ typename VecT<ZV>::T thin_value(const typename VecT<Z
   return v;
 }
 
+// its taps at byte offset zb into the columns; a buffer descriptor over the
+// whole volume keeps the addresses to 32-bit offsets (thin_ok)
 template <int ZV>
-__device__ __forceinline__ void thin_load(const float* __restrict__ vol, int base, int n, int nz, int z,
-                                          typename VecT<ZV>::T (&t)[4]) {
-  const float* p = vol + (size_t)(base & (kOne - 1)) * nz + z;
-  const int o1 = base & kOne ? 0 : nz, o2 = base & (2 * kOne) ? 0 : n * nz;
-  t[0] = vload<ZV>(p);
-  t[1] = vload<ZV>(p + o1);
-  t[2] = vload<ZV>(p + o2);
-  t[3] = vload<ZV>(p + o1 + o2);
+__device__ __forceinline__ void thin_load(__amdgpu_buffer_rsrc_t vol, int base, uint32_t row_b, uint32_t col_b,
+                                          uint32_t zb, typename VecT<ZV>::T (&t)[4]) {
+  const uint32_t p = (uint32_t)(base & (kOne - 1)) * col_b + zb;
+  const uint32_t o1 = base & kOne ? kOut : p + col_b, o2 = base & (2 * kOne) ? kOut : p + row_b;
+  const uint32_t o3 = base & (3 * kOne) ? kOut : p + row_b + col_b;
+  t[0] = bload<ZV>(vol, p, 0);
+  t[1] = bload<ZV>(vol, o1, 0);
+  t[2] = bload<ZV>(vol, o2, 0);
+  t[3] = bload<ZV>(vol, o3, 0);
 }
 
-template <int ZV, int L, bool CLIP, bool PAIR>
+// R > 1 (L = 1): the wavefront's lanes are R neighbouring rays (k, per lane)
+// x 64 / R samples
+template <int ZV, int L, int R, bool CLIP, bool PAIR>
 __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restrict__ vol,
                                          const float* __restrict__ minmax, int k, int i, int z, int lane,
                                          typename VecT<ZV>::T& acc, typename VecT<ZV>::T& acc2) {
@@ -125,6 +131,8 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
   static_assert(!(PAIR && CLIP), "the clipped sample is discontinuous at the border: no pairing");
   constexpr int G = 64 / L, kU = steps<ZV>();
   const int n = g.n, nz = g.nz, grp = lane / L;
+  const __amdgpu_buffer_rsrc_t vr = buf_rsrc(vol, (uint32_t)n * (uint32_t)n * (uint32_t)nz * 4u);
+  const uint32_t col_b = 4u * (uint32_t)nz, row_b = (uint32_t)n * col_b, zb = 4u * (uint32_t)z;
   const double* M = g.mats + 6 * i;
   const double kp = (double)k - g.det_offset;
   const double a0 = M[0] * kp, a1 = M[3] * kp;
@@ -140,12 +148,11 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
   const int r_end = PAIR ? (2 * g.c + 1 > n ? 2 * g.c + 1 : n) : n;
   const int r2_lo = 2 * g.c - n + 1;
   if constexpr (L == 1) {
-    for (int r0 = 0; r0 < r_end; r0 += 64) {
-      if (r0 + lane >= r_end) continue;
-      const Sample s = ray_sample<PAIR>(g, M, a0, a1, ch, r0 + lane, r2_lo);
+    for (int r = lane / R; r < r_end; r += 64 / R) {
+      const Sample s = ray_sample<PAIR>(g, M, a0, a1, ch, r, r2_lo);
       if (!s.valid) continue;
       V t[4];
-      thin_load<ZV>(vol, s.base, n, nz, z, t);
+      thin_load<ZV>(vr, s.base, row_b, col_b, zb, t);
       const V v = thin_value<ZV, CLIP>(t, s.r0, s.r1, s.c0, s.c1, lo, hi);
       acc = vfma(s.a, v, acc);
       if constexpr (PAIR) acc2 = vfma(s.a2, v, acc2);
@@ -171,7 +178,7 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
           const int e = e0 + u * G + grp;
           a[u] = sl.a[e];
           w[u] = sl.w[e];
-          if (a[u].w != 0.0f) thin_load<ZV>(vol, __float_as_int(a[u].z), n, nz, z, t[u]);
+          if (a[u].w != 0.0f) thin_load<ZV>(vr, __float_as_int(a[u].z), row_b, col_b, zb, t[u]);
         }
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
@@ -184,7 +191,7 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
     }
   }
 #pragma unroll
-  for (int o = L; o < 64; o <<= 1) {
+  for (int o = L * R; o < 64; o <<= 1) {
 #pragma unroll
     for (int q = 0; q < ZV; ++q) {
       vset(acc, q, vget(acc, q) + __shfl_xor(vget(acc, q), o));
@@ -193,14 +200,53 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
   }
 }
 
-template <int ZV, int L, class Out>
+template <int ZV, int L, int R, class Out>
 __global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __restrict__ vol,
                                                       const float* __restrict__ minmax, int clip, int pair, Out out) {
   using V = typename VecT<ZV>::T;
+  static_assert(R == 1 || L == 1, "several rays per wavefront: one lane per ray and sample");
   const int lane = threadIdx.x & 63, z = (lane & (L - 1)) * ZV;
   const int zl = z < g.nz ? z : g.nz - ZV;   // lanes past nz read a copy and store nothing
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
   int k, i, k2 = -1, i2 = -1;
+  if constexpr (R > 1) {
+    // wavefronts in ray order; a lane without a ray of its own walks the last
+    // one again and stores nothing.  e, k2: extended rays as in fp_pair_item
+    const int ne = pair ? fp_pair_next(g) : g.n, nu = pair ? g.n_units : g.na, nw = (ne + R - 1) / R;
+    if (wave >= (long long)nw * nu) return;   // whole wavefronts
+    const int u = (int)(wave / nw), e = (int)(wave % nw) * R + lane % R;
+    int store = e < ne ? 1 : 0;
+    const int ee = e < ne ? e : ne - 1;
+    k = ee;
+    i = u;
+    if (pair) {
+      const int u1 = g.units[2 * u], u2 = g.units[2 * u + 1], kk = 2 * g.c + g.pair_D - ee;
+      const bool extra = ee >= g.n;            // a partner-angle ray without a primary
+      if (extra && u2 < 0) store = 0;
+      k = extra ? g.pair_first2 + (ee - g.n) : ee;
+      i = extra && u2 >= 0 ? u2 : u1;
+      if (extra && u2 < 0) k = g.n - 1;
+      k2 = !extra && u2 >= 0 && kk >= 0 && kk < g.n ? kk : -1;
+      i2 = u2;
+    }
+    const bool clip_on = clip && wave_clip_active<ZV>(minmax, g.nz, zl);
+    const bool first = lane < R && store;
+    V acc, acc2;
+    if (clip_on) {
+      thin_ray<ZV, L, R, true, false>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+      if (first) out.put(((size_t)k * g.na + i) * g.nz, vget(acc, 0));
+      if (__ballot(k2 >= 0)) {
+        const int kh = k2 >= 0 ? k2 : k, ih = k2 >= 0 ? i2 : i;
+        thin_ray<ZV, L, R, true, false>(g, vol, minmax, kh, ih, zl, lane, acc, acc2);
+        if (first && k2 >= 0) out.put(((size_t)k2 * g.na + i2) * g.nz, vget(acc, 0));
+      }
+    } else {
+      thin_ray<ZV, L, R, false, true>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+      if (first) out.put(((size_t)k * g.na + i) * g.nz, vget(acc, 0));
+      if (first && k2 >= 0) out.put(((size_t)k2 * g.na + i2) * g.nz, vget(acc2, 0));
+    }
+    return;
+  }
   if (pair) {
     const PairItem it = fp_pair_item<1>(wave, g, 0);
     if (!it.ok) return;
@@ -222,15 +268,15 @@ __global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __r
   if (clip_on) {
     for (int h = 0; h < (k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? k2 : k, ih = h ? i2 : i;
-      thin_ray<ZV, L, true, false>(g, vol, minmax, kh, ih, zl, lane, acc, acc2);
+      thin_ray<ZV, L, 1, true, false>(g, vol, minmax, kh, ih, zl, lane, acc, acc2);
       put(kh, ih, acc);
     }
   } else if (k2 >= 0) {
-    thin_ray<ZV, L, false, true>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+    thin_ray<ZV, L, 1, false, true>(g, vol, minmax, k, i, zl, lane, acc, acc2);
     put(k, i, acc);
     put(k2, i2, acc2);
   } else {
-    thin_ray<ZV, L, false, false>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+    thin_ray<ZV, L, 1, false, false>(g, vol, minmax, k, i, zl, lane, acc, acc2);
     put(k, i, acc);
   }
 }
@@ -240,8 +286,8 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
                                                        float* __restrict__ vol, int clipc) {
   using V = typename VecT<ZV>::T;
   constexpr int G = 64 / L, kAng = 4;
-  __shared__ float4 tab[L == 1 ? 1 : 1024];
-  __shared__ float sums[1024 * ZV];
+  // per wavefront: its table of 64 entries (L > 1) and its lanes' sums
+  extern __shared__ float4 thin_bp_lds[];
   const int lane = threadIdx.x & 63, l = lane & (L - 1), grp = lane / L;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), split = blockDim.x >> 6;
   const int n = g.n, nz = g.nz, nt = (n + 7) / 8;
@@ -255,53 +301,57 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
   const double x = (double)(col - g.c), y = (double)(row - g.c);
   const int i_end = (int)((long long)g.na * (wv + 1) / split);
   V acc = vzero<ZV>();
-  // row weights and the first row of angle i; no weight where the column is
-  // not computed (its rows are not read either)
-  auto geom = [&](int i, float& w0, float& w1, int& at, int& step) {
+  const __amdgpu_buffer_rsrc_t sr = buf_rsrc(sino, (uint32_t)n * (uint32_t)g.na * (uint32_t)nz * 4u);
+  const uint32_t bin_b = 4u * (uint32_t)nz, row_b = (uint32_t)g.na * bin_b;
+  // row weights and the byte offsets of the two rows of angle i (np.interp as
+  // in interp_node; the fraction is taken from the distance to the first
+  // node): kOut where a row is not read -- no ray, a column that is not
+  // computed, no absorption weight, past the last node
+  auto geom = [&](int i, float& w0, float& w1, uint32_t& p0, uint32_t& p1) {
     w0 = w1 = 0.0f;
-    at = step = 0;
-    if (!active || i >= i_end) return false;
-    const double co = g.cs[2 * i], sn = g.cs[2 * i + 1];
+    p0 = p1 = kOut;
+    const int ic = i < i_end ? i : i_end - 1;
+    const double co = g.cs[2 * ic], sn = g.cs[2 * ic + 1];
     const double t = x * co - y * sn;
-    int j, j1;
-    float w;
-    if (!interp_node(g, t, j, j1, w)) return false;
-    const float aw = g.mu != 0.0 ? abs_weight(g, t, x * sn + y * co) : 1.0f;
+    if (!active || i >= i_end || !(t >= g.xp0 && t <= g.xp_last)) return;
+    const double u = t - g.xp0, fl = floor(u);
+    const int j = min((int)fl, n - 1);
+    const float w = (float)(u - fl);
+    float aw = 1.0f;
+    if (g.mu != 0.0) {
+      aw = abs_weight(g, t, x * sn + y * co);
+      if (aw == 0.0f) return;
+    }
     w0 = aw * (1.0f - w);
     w1 = aw * w;
-    at = j * g.na + i;
-    step = j1 > j ? g.na * nz : 0;
-    return aw != 0.0f;
+    p0 = ((uint32_t)j * (uint32_t)g.na + (uint32_t)i) * bin_b;
+    p1 = j < n - 1 ? p0 + row_b : kOut;
   };
   int i = (int)((long long)g.na * wv / split);
   if constexpr (L == 1) {
+    const uint32_t zb = 4u * (uint32_t)zl;
     for (; i < i_end; i += kAng) {
       V b0[kAng], b1[kAng];
       float w0[kAng], w1[kAng];
-      bool ok[kAng];
 #pragma unroll
       for (int u = 0; u < kAng; ++u) {
-        int at, step;
-        ok[u] = geom(i + u, w0[u], w1[u], at, step);
-        b0[u] = b1[u] = vzero<ZV>();
-        if (ok[u]) {
-          const float* p = sino + (size_t)at * nz + zl;
-          b0[u] = vload<ZV>(p);
-          b1[u] = vload<ZV>(p + step);
-        }
+        uint32_t p0, p1;
+        geom(i + u, w0[u], w1[u], p0, p1);
+        b0[u] = bload<ZV>(sr, p0 + zb, 0);
+        b1[u] = bload<ZV>(sr, p1 + zb, 0);
       }
 #pragma unroll
-      for (int u = 0; u < kAng; ++u)
-        if (ok[u]) acc = vfma(w1[u], b1[u], vfma(w0[u], b0[u], acc));
+      for (int u = 0; u < kAng; ++u) acc = vfma(w1[u], b1[u], vfma(w0[u], b0[u], acc));
     }
   } else {
-    float4* const tb = tab + wv * 64;
+    float4* const tb = thin_bp_lds + wv * 64;
+    const uint32_t zb = 4u * (uint32_t)zl;
     for (; i < i_end; i += L) {
       float w0, w1;
-      int at, step;
-      const bool ok = geom(i + l, w0, w1, at, step);
+      uint32_t p0, p1;
+      geom(i + l, w0, w1, p0, p1);
       __builtin_amdgcn_wave_barrier();
-      tb[lane] = make_float4(w0, w1, __int_as_float(ok ? at : -1), __int_as_float(step));
+      tb[lane] = make_float4(w0, w1, __uint_as_float(p0), __uint_as_float(p1));
       __builtin_amdgcn_wave_barrier();
       constexpr int K = L < kAng ? L : kAng;
 #pragma unroll
@@ -312,13 +362,8 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
 #pragma unroll
         for (int u = 0; u < K; ++u) {
           e[u] = tb[grp * L + u0 + u];
-          b0[u] = b1[u] = vzero<ZV>();
-          const int a = __float_as_int(e[u].z);
-          if (a >= 0) {
-            const float* p = sino + (size_t)a * nz + zl;
-            b0[u] = vload<ZV>(p);
-            b1[u] = vload<ZV>(p + __float_as_int(e[u].w));
-          }
+          b0[u] = bload<ZV>(sr, __float_as_uint(e[u].z) + zb, 0);
+          b1[u] = bload<ZV>(sr, __float_as_uint(e[u].w) + zb, 0);
         }
 #pragma unroll
         for (int u = 0; u < K; ++u) acc = vfma(e[u].y, b1[u], vfma(e[u].x, b0[u], acc));
@@ -326,13 +371,14 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
     }
   }
   if (split > 1) {
+    float* const sums = reinterpret_cast<float*>(thin_bp_lds + (L == 1 ? 0 : blockDim.x));
 #pragma unroll
-    for (int q = 0; q < ZV; ++q) sums[q * 1024 + threadIdx.x] = vget(acc, q);
+    for (int q = 0; q < ZV; ++q) sums[q * blockDim.x + threadIdx.x] = vget(acc, q);
     __syncthreads();
     if (wv == 0) {
       for (int s = 1; s < split; ++s)
 #pragma unroll
-        for (int q = 0; q < ZV; ++q) vset(acc, q, vget(acc, q) + sums[q * 1024 + s * 64 + lane]);
+        for (int q = 0; q < ZV; ++q) vset(acc, q, vget(acc, q) + sums[q * blockDim.x + s * 64 + lane]);
     }
   }
   if (wv == 0 && inside && z < nz) vstore<ZV>(vol + ((size_t)row * n + col) * nz + z, acc);
@@ -368,9 +414,20 @@ int thin_forward(vamx_plan* p, const float* vol, const void* sino, Out out, bool
   // SIMD the GPU has room to project them side by side instead
   const int pair = g.fp_pair && g.pair_ok && fp_pair_tiled(g) >= 4096;
   const long long waves = pair ? fp_pair_tiled(g) : fp_tiled_rays(g);
+  // one slice: 8 neighbouring rays x 8 samples per wavefront, whose taps lie in
+  // a patch of about 11 x 11 voxels (64 samples of one ray can touch 64 cache
+  // lines), where that still leaves 4 wavefronts per SIMD
+  const int nu = pair ? g.n_units : g.na, ne = pair ? fp_pair_next(g) : g.n;
+  const long long waves8 = (long long)nu * ((ne + 7) / 8);
+  if (g.nz == 1 && waves8 >= 4096) {
+    hipLaunchKernelGGL((thin_fp_kernel<1, 1, 8, Out>), dim3(blocks_for(waves8 * 64, 256)), dim3(256), 0, s, g, vol,
+                       p->d_minmax, clip ? 1 : 0, pair, out);
+    VAMX_HIP(hipGetLastError());
+    return VAMX_OK;
+  }
   thin_dispatch(g.nz, thin_v4(g.nz, vol, sino), [&](auto zv, auto l) {
     constexpr int ZV = decltype(zv)::value, L = decltype(l)::value;
-    hipLaunchKernelGGL((thin_fp_kernel<ZV, L, Out>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, vol,
+    hipLaunchKernelGGL((thin_fp_kernel<ZV, L, 1, Out>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, vol,
                        p->d_minmax, clip ? 1 : 0, pair, out);
   });
   VAMX_HIP(hipGetLastError());
@@ -381,7 +438,9 @@ int thin_forward(vamx_plan* p, const float* vol, const void* sino, Out out, bool
 
 bool thin_ok(const vamx_plan* p) {
   const ParDev& g = p->par;
-  return !g.incl && !g.occ && g.n >= 2 && g.nz < 32 && !(p->flags & VAMX_PAR_PER_LANE_GEOMETRY);
+  // 32-bit byte offsets into the volume and the sinogram
+  const double most = 4.0 * g.n * (double)(g.n > g.na ? g.n : g.na) * g.nz;
+  return !g.incl && !g.occ && g.n >= 2 && g.nz < 32 && most < 2147483648.0 && !(p->flags & VAMX_PAR_PER_LANE_GEOMETRY);
 }
 
 int thin_forward_store(vamx_plan* p, const float* vol, float* sino, bool clip, hipStream_t s) {
@@ -402,8 +461,9 @@ int thin_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipSt
     // SIMD are in flight, at most 16 ways and into no fewer than 8 angles
     int split = 1;
     while (split < 16 && blocks * split < 8192 && g.na >= 16 * split) split *= 2;
-    hipLaunchKernelGGL((thin_bp_kernel<ZV, L>), dim3((unsigned)blocks), dim3(64 * split), 0, s, g, sino, vol,
-                       clipc ? 1 : 0);
+    hipLaunchKernelGGL((thin_bp_kernel<ZV, L>), dim3((unsigned)blocks), dim3(64 * split),
+                       (L == 1 ? 0 : 64 * split * sizeof(float4)) + (split > 1 ? 64 * split * ZV * sizeof(float) : 0), s, g,
+                       sino, vol, clipc ? 1 : 0);
   });
   VAMX_HIP(hipGetLastError());
   return VAMX_OK;
