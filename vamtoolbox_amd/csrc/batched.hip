@@ -35,7 +35,8 @@ struct BatchItem {
   int clip;              // forward: warp clip; backward: circle clip
   int wave;              // 1: wavefront-uniform kernels
   int pair;              // forward, wave mode: opposite-angle pairs (the plan's paired work order)
-  int split;             // wave mode, zv 2: lanes hold z and z + 64
+  int split;             // forward, wave mode, zv 2: lanes hold z and z + 64
+  int contig, comb, chunks;   // backward, wave mode: BpLayout
 };
 
 // Buffers of the problems of one launch, passed by value as a kernel
@@ -94,23 +95,18 @@ __device__ __forceinline__ void batch_fp_pair(const BatchItem& it, const float* 
   if (pi.k2 >= 0) wave_zstore<ZV, SPLIT>(out + ((size_t)pi.k2 * g.na + pi.i2) * g.nz, z, g.nz, acc2);
 }
 
-template <int ZV, bool SPLIT>
-__device__ __forceinline__ void batch_bp_wave(const BatchItem& it, const float* in, float* out, long long w,
-                                              int lane) {
+template <int ZV, bool CONTIG, bool COMB>
+__device__ __forceinline__ void batch_bp_patch(const BatchItem& it, const float* in, float* out, long long w,
+                                               int lane) {
   const ParDev& g = it.g;
-  int r0, c0, z, zl, zl2;
-  if (!bp_wave_quad<ZV, SPLIT>(w, g, lane, r0, c0, z)) return;
-  wave_zload<ZV, SPLIT>(z, g.nz, zl, zl2);
+  int r0, c0, chunk;
+  if (!bp_wave_patch<2>(w, it.chunks, g, r0, c0, chunk)) return;
+  const ZLane<ZV, CONTIG> ln(chunk, lane, g.nz);
   unsigned inrange, active;
-  bp_quad_masks(g, r0, c0, it.clip, inrange, active);
-  typename VecT<ZV>::T acc[4];
-  bp_quad_wave<ZV, SPLIT>(g, in, r0, c0, active, zl, lane, acc, zl2);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if (!((inrange >> q) & 1u)) continue;
-    float* outp = out + ((size_t)(r0 + (q >> 1)) * g.n + c0 + (q & 1)) * g.nz;
-    wave_zstore<ZV, SPLIT>(outp, z, g.nz, ((active >> q) & 1u) ? acc[q] : vzero<ZV>());
-  }
+  bp_patch_masks<2>(g, r0, c0, it.clip, inrange, active);
+  mf4 acc[2][ZV];
+  bp_patch<2, ZV, CONTIG, COMB>(g, in, r0, c0, active, ln, lane, acc);
+  bp_patch_store<2, ZV, CONTIG>(g, in, out, r0, c0, inrange, active, ln, acc);
 }
 
 template <bool FORWARD>
@@ -146,7 +142,7 @@ __device__ __forceinline__ void batch_lane_item(const BatchItem& it, const float
 }
 
 template <bool FORWARD>
-__global__ __launch_bounds__(256) void batch_kernel(const BatchItem* __restrict__ items, int nitems,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void batch_kernel(const BatchItem* __restrict__ items, int nitems,
                                                     long long ntiles, unsigned long long* counter,
                                                     BatchPtrs ptrs) {
   __shared__ long long tile_sh;
@@ -188,10 +184,19 @@ __global__ __launch_bounds__(256) void batch_kernel(const BatchItem* __restrict_
           else if (it.zv == 2) batch_fp_wave<2, false>(it, in, out, w, lane);
           else batch_fp_wave<1, false>(it, in, out, w, lane);
         } else {
-          if (it.split) batch_bp_wave<2, true>(it, in, out, w, lane);
-          else if (it.zv == 4) batch_bp_wave<4, false>(it, in, out, w, lane);
-          else if (it.zv == 2) batch_bp_wave<2, false>(it, in, out, w, lane);
-          else batch_bp_wave<1, false>(it, in, out, w, lane);
+          if (it.comb) {
+            if (it.contig) batch_bp_patch<4, true, true>(it, in, out, w, lane);
+            else if (it.zv == 4) batch_bp_patch<4, false, true>(it, in, out, w, lane);
+            else if (it.zv == 3) batch_bp_patch<3, false, true>(it, in, out, w, lane);
+            else if (it.zv == 2) batch_bp_patch<2, false, true>(it, in, out, w, lane);
+            else batch_bp_patch<1, false, true>(it, in, out, w, lane);
+          } else {
+            if (it.contig) batch_bp_patch<4, true, false>(it, in, out, w, lane);
+            else if (it.zv == 4) batch_bp_patch<4, false, false>(it, in, out, w, lane);
+            else if (it.zv == 3) batch_bp_patch<3, false, false>(it, in, out, w, lane);
+            else if (it.zv == 2) batch_bp_patch<2, false, false>(it, in, out, w, lane);
+            else batch_bp_patch<1, false, false>(it, in, out, w, lane);
+          }
         }
       }
     } else {
@@ -292,15 +297,21 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
   return VAMX_OK;
 }
 
-// kernel path of problem i for these buffers: wave z width (1, 2, 4; 3 = z
-// and z + 64), -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
+// kernel path of problem i for these buffers: forward, wave z width (1, 2, 4;
+// 3 = z and z + 64); backward, slices per lane (+ 8: contiguous, + 16: opposite
+// angles combined); -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
 // kOwnLaunch for plans whose kernels the persistent launch does not hold
 constexpr int kOwnLaunch = 0;
 int problem_path(vamx_plan* p, const float* in, float* out, bool forward) {
   if (incl_wave_ok(p) || thin_ok(p)) return kOwnLaunch;
-  int wz = forward ? par_fp_wave_zv(p, in, out) : par_wave_zv(p, in, out, p->par.bp_zv);
-  if (par_wave_split(p, wz)) return 3;
-  if (wz) return wz;
+  if (forward) {
+    const int wz = par_fp_wave_zv(p, in, out);
+    if (par_wave_split(p, wz)) return 3;
+    if (wz) return wz;
+  } else {
+    const BpLayout l = bp_layout(p, (uintptr_t)in | (uintptr_t)out);
+    if (l.zv) return l.zv | (l.contig ? 8 : 0) | (l.comb ? 16 : 0);
+  }
   return par_use_vec4(p, in, out) ? -4 : -1;
 }
 
@@ -333,15 +344,21 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
       L.single.push_back(i);
       continue;
     }
-    if (path > 0) {
+    if (path > 0 && !forward) {
+      it.wave = 1;
+      it.zv = path & 7;
+      it.contig = (path >> 3) & 1;
+      it.comb = (path >> 4) & 1;
+      it.chunks = wave_zchunks(it.g.nz, it.zv);
+      it.items = bp_patches(it.g, 2) * it.chunks;
+    } else if (path > 0) {
       const int wz = path == 3 ? 2 : path;
       it.wave = 1;
       it.zv = wz;
       it.split = path == 3 ? 1 : 0;
-      it.pair = forward && it.g.fp_pair && it.g.pair_ok ? 1 : 0;
-      const long long units = it.pair ? fp_pair_tiled(it.g) : forward ? fp_tiled_rays(it.g) : bp_tiled_quads(it.g);
-      it.items = units * wave_zchunks(it.g.nz, wz);
-      if (forward && !it.g.incl && it.items >= 16ll * cus) {
+      it.pair = it.g.fp_pair && it.g.pair_ok ? 1 : 0;
+      it.items = (it.pair ? fp_pair_tiled(it.g) : fp_tiled_rays(it.g)) * wave_zchunks(it.g.nz, wz);
+      if (!it.g.incl && it.items >= 16ll * cus) {
         L.single.push_back(i);
         continue;
       }

@@ -57,48 +57,6 @@ __global__ __launch_bounds__(256) void bclp_bp_epilogue(ParDev g, int clipc, Res
   if (threadIdx.x == 0) partials[lb] = s;
 }
 
-// A (wavefront-uniform variant): one wavefront = one 2x2 quad of voxel
-// columns x 64*ZV z
-template <int ZV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void bclp_bp_epilogue_wave(ParDev g, int clipc, RespDev r, BclpDev b,
-                                                             const float* __restrict__ gsino,
-                                                             const float* __restrict__ target,
-                                                             float* __restrict__ dose, float* __restrict__ operand,
-                                                             double* __restrict__ partials) {
-  __shared__ double sh[256];
-  const int lane = threadIdx.x & 63;
-  const unsigned lb = xcd_remap(blockIdx.x, gridDim.x);
-  const long long wave = wave_index(lb);
-  double part = 0.0;
-  int r0 = 0, c0 = 0, z = 0;
-  if (bp_wave_quad<ZV>(wave, g, lane, r0, c0, z)) {
-    const int zl = z < g.nz - ZV ? z : g.nz - ZV;
-    unsigned inrange, active;
-    bp_quad_masks(g, r0, c0, clipc, inrange, active);
-    typename VecT<ZV>::T acc[4];
-    bp_quad_wave<ZV>(g, gsino, r0, c0, active, zl, lane, acc);
-    if (z >= g.nz) inrange = 0u;   // lanes past nz: no store, no loss term
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (!((inrange >> q) & 1u)) continue;
-      const size_t base = ((size_t)(r0 + (q >> 1)) * g.n + c0 + (q & 1)) * g.nz + z;
-      const typename VecT<ZV>::T d = ((active >> q) & 1u) ? acc[q] : vzero<ZV>();
-      vstore<ZV>(dose + base, d);
-      typename VecT<ZV>::T op = vzero<ZV>();
-      const typename VecT<ZV>::T tg = vload<ZV>(target + base);
-#pragma unroll
-      for (int e = 0; e < ZV; ++e) {
-        float o;
-        part += bclp_voxel(r, b, vget(d, e), vget(tg, e), base + e, o);
-        vset(op, e, o);
-      }
-      vstore<ZV>(operand + base, op);
-    }
-  }
-  const double s = block_sum_256(part, sh);
-  if (threadIdx.x == 0) partials[lb] = s;
-}
-
 // A, second half, after a back projection into `dose` by the plain kernels:
 // response, band, Lp weighting and loss partials of a whole dose, grid-stride
 // (bound by its 12 bytes per voxel)
@@ -398,31 +356,19 @@ int launch_epilogue(vamx_plan* p, const RespDev& r, const BclpDev& b, const floa
                          (uintptr_t)b.eps_arr | (uintptr_t)b.w_arr;
     wz = wave_zv_choice(gd.nz, al, gd.bp_zv);
   }
-  if (wz) {
-    const long long threads = bp_tiled_quads(gd) * wave_zchunks(gd.nz, wz) * 64;
-    nparts = (int)blocks_for(threads, 256);
-    if (nparts > max_parts)
-      return set_error(VAMX_ERR_ARG, "bclp: " + std::to_string(nparts) + " loss partials exceed the " +
-                                          std::to_string(max_parts) + " slots of the scratch");
-    const dim3 grid(nparts), block(256);
-    if (wz == 4)
-      hipLaunchKernelGGL(bclp_bp_epilogue_wave<4>, grid, block, 0, s, gd, clipc, r, b, g, target, dose, operand,
-                         partials);
-    else if (wz == 2)
-      hipLaunchKernelGGL(bclp_bp_epilogue_wave<2>, grid, block, 0, s, gd, clipc, r, b, g, target, dose, operand,
-                         partials);
-    else
-      hipLaunchKernelGGL(bclp_bp_epilogue_wave<1>, grid, block, 0, s, gd, clipc, r, b, g, target, dose, operand,
-                         partials);
-    VAMX_HIP(hipGetLastError());
-    return VAMX_OK;
-  }
-  const long long total = (long long)gd.n * gd.n * (gd.nz / (v4 ? 4 : 1));
-  nparts = (int)blocks_for(total, 256);
+  // a scratch of max_parts slots takes problems of at most that many blocks: of
+  // four 2 x 2 quads of columns x 64 wz slices, or of 256 voxels (x 4 slices)
+  nparts = (int)(wz ? blocks_for(bp_tiled_quads(gd) * wave_zchunks(gd.nz, wz) * 64, 256)
+                    : blocks_for((long long)gd.n * gd.n * (gd.nz / (v4 ? 4 : 1)), 256));
   if (nparts > max_parts)
     return set_error(VAMX_ERR_ARG, "bclp: " + std::to_string(nparts) + " loss partials exceed the " +
                                         std::to_string(max_parts) + " slots of the scratch");
-  if (incl_wave_ok(p) || thin_ok(p)) return split_epilogue(p, r, b, g, target, dose, operand, partials, clipc, nparts, s);
+  // the back projections on wavefronts and the element-wise epilogue as two
+  // launches: with the epilogue in the patch kernel, whose accumulators fill
+  // its registers, 824 us at 256^3 x 360, apart 718 + 41; 160 x 120 x 180
+  // angles 155 and 138 + 14
+  if (incl_wave_ok(p) || thin_ok(p) || bp_layout(p, 0).zv)
+    return split_epilogue(p, r, b, g, target, dose, operand, partials, clipc, nparts, s);
   const dim3 grid(nparts), block(256);
   if (gd.incl)
     hipLaunchKernelGGL((bclp_bp_epilogue<1, true>), grid, block, 0, s, gd, clipc, r, b, g, target, dose, operand,

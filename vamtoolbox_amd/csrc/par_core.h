@@ -16,6 +16,8 @@
 // multiply-adds.  No core uses atomics.
 #pragma once
 
+#include <type_traits>
+
 #include "vamx_internal.h"
 
 namespace vamx {
@@ -918,10 +920,6 @@ __device__ __forceinline__ FpSlot fp_lds_slot() {
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 3;
   return {w[wv], a[wv]};
 }
-__device__ __forceinline__ float4* bp_lds_slot() {
-  __shared__ float4 w[4][2][16];   // weights of the lower / upper row, 16 angles x 4 pixels
-  return w[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 3][0];
-}
 
 template <int ZV, bool CLIP, bool REUSE, bool PAIR = false, bool SPLIT = false>
 __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, const float* __restrict__ vol,
@@ -1086,126 +1084,299 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
   return acc;
 }
 
-// Back projection of a 2x2 quad of voxel columns, lanes = z.  Pixel p
-// (0..3) is at row r0 + (p >> 1), column c0 + (p & 1); bit p of `active`
-// says whether it is computed (in range and not circle-clipped).  Within one
-// angle the four pixels' detector coordinates t differ by at most
-// |cos| + |sin| <= sqrt(2), so their lower np.interp nodes span at most two
-// detector rows and the quad needs at most four distinct rows (usually
-// three) where four separate columns would load eight.  Lanes first evaluate
-// the float64 geometry of 16 angles x 4 pixels; the per-angle loop then
-// loads the rows [bmin, bmax + 1] once and every pixel accumulates
-// fma(w1, b[j+1], fma(w0, b[j], acc)) in angle order -- the same operations,
-// in the same order, as one column at a time.  The 16 angles' weights pass
-// through a per-wavefront LDS buffer and come back as one broadcast 16-byte
-// read per row weight, and each angle's row offsets, span and first row are
-// packed into one value: the per-angle loop moves one value from a lane.
-// Requires n >= 2, all 64 lanes of the wavefront (cross-lane swizzles) and
-// blocks of at most 4 wavefronts (the LDS buffer's size).
-template <int ZV, bool SPLIT = false>
-__device__ __forceinline__ void bp_quad_wave(const ParDev& g, const float* __restrict__ sino, int r0, int c0,
-                                             unsigned active, int z, int lane, typename VecT<ZV>::T acc[4],
-                                             int z2 = 0) {
-  using V = typename VecT<ZV>::T;
-  const int p = lane & 3, a = lane >> 2;
-  const bool pin = (active >> p) & 1u;
-  const double x = (double)(c0 + (p & 1) - g.c), y = (double)(r0 + (p >> 1) - g.c);
-  const size_t nzs = (size_t)g.nz;
-  const size_t step_j = (size_t)g.na * nzs;
-  const uint32_t zb = 4u * (uint32_t)z, zb2 = 4u * (uint32_t)z2, row_b = (uint32_t)(4 * step_j);
-  const uint32_t rows_b = 3 * row_b + 4u * (uint32_t)g.nz;
-  float4* const bw0 = bp_lds_slot();   // [16] lower-row weights, then [16] upper-row weights
-  float4* const bw1 = bw0 + 16;
+// Slices of a lane in the back projection's wavefronts: CONTIG (ZV = 4) z ..
+// z + 3, else z + 64 q (dword loads: a 64-lane dword load takes the texture
+// path 5 cycles, an 8-byte one 16, a 16-byte one 16).  Slices past nz load a
+// copy of the last one and are not stored.
+template <int ZV, bool CONTIG>
+struct ZLane {
+  static_assert(!CONTIG || ZV == 4, "contiguous slices are 16-byte loads");
+  int z;
+  uint32_t zb[CONTIG ? 1 : ZV];   // byte offsets of the loads
+  __device__ __forceinline__ ZLane(int chunk, int lane, int nz) {
+    z = chunk * 64 * ZV + (CONTIG ? 4 * lane : lane);
+    if constexpr (CONTIG) {
+      zb[0] = 4u * (uint32_t)(z < nz - 4 ? z : nz - 4);
+    } else {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) acc[q] = vzero<ZV>();
-  // One loop over the angles (a nested per-batch loop makes the compiler
-  // copy the accumulators between two register sets on every angle); every
-  // 16th angle first evaluates the geometry of the next 16.
-  unsigned long long m = 0ull;   // valid pixels of the batch's angles (bit 4a + p)
-  int pk = 0;
-  for (int ia = 0; ia < g.na; ++ia) {
-    if ((ia & 15) == 0) {
-      const int i = ia + a;
-      int jr = 0;
-      float w0 = 0.f, w1 = 0.f;
-      bool valid = false;
-      if (pin && i < g.na) {
-        const double co = g.cs[2 * i], sn = g.cs[2 * i + 1];
-        const double t = x * co - y * sn;
-        int j, j1;
-        float w;
-        if (interp_node(g, t, j, j1, w)) {
-          const float aw = (g.mu != 0.0) ? abs_weight(g, t, x * sn + y * co) : 1.0f;
-          valid = aw != 0.0f;
-          if (j == g.n - 1) {        // exactly at the last node: fp[n-1]
-            jr = j - 1;
-            w1 = aw;
-          } else {
-            jr = j;
-            w0 = aw * (1.0f - w);
-            w1 = aw * w;
-          }
-        }
-      }
-      m = __ballot(valid);
-      // the quad's row range over its valid pixels (the four lanes of one angle
-      // are lanes 4a .. 4a+3), each pixel's row offset in it and the element
-      // offset of its first row, (bmin * na + i) * nz -- lane-parallel for 16
-      // angles at once, so the per-angle loop below only broadcasts them
-      int lo = valid ? jr : 0x7fffffff, hi = valid ? jr : -1;
-      lo = min(lo, __shfl_xor(lo, 1));
-      lo = min(lo, __shfl_xor(lo, 2));
-      hi = max(hi, __shfl_xor(hi, 1));
-      hi = max(hi, __shfl_xor(hi, 2));
-      // per angle: bits 0-7 the pixels' row offsets from bmin, 8-9 the span
-      // bmax - bmin, 10.. bmin (n < 16384)
-      int bits = valid ? (jr - lo) << (2 * p) : 0;
-      bits |= __shfl_xor(bits, 1);
-      bits |= __shfl_xor(bits, 2);
-      pk = hi >= 0 ? bits | ((hi - lo) << 8) | (lo << 10) : 0;
-      __builtin_amdgcn_wave_barrier();
-      reinterpret_cast<float*>(&bw0[a])[p] = w0;
-      reinterpret_cast<float*>(&bw1[a])[p] = w1;
-      __builtin_amdgcn_wave_barrier();
+      for (int q = 0; q < ZV; ++q) zb[q] = 4u * (uint32_t)(z + 64 * q < nz - 1 ? z + 64 * q : nz - 1);
     }
-    const int l0 = 4 * (ia & 15);   // lane of pixel 0 of this angle
-    const unsigned pm = (unsigned)(m >> l0) & 0xFu;
-    if (!pm) continue;              // no valid pixel at this angle
-    const int pkv = rl_i(pk, l0);
-    const float4 U0 = bw0[l0 >> 2], U1 = bw1[l0 >> 2];
-    const float u0[4] = {U0.x, U0.y, U0.z, U0.w}, u1[4] = {U1.x, U1.y, U1.z, U1.w};
-    // rows bmin .. bmax + 1 <= n - 1 (jr <= n - 2); span <= 2 by the bound above
-    // buffer loads from a descriptor at row bmin: lane byte offset 4z,
-    // scalar row offsets
-    const unsigned rowl = ((unsigned)(pkv >> 10) * (unsigned)g.na + (unsigned)ia) * (unsigned)g.nz;
-    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sino + (size_t)rowl, rows_b);
-    const int span = (pkv >> 8) & 3;
-    const V T0 = tload<ZV, SPLIT>(rs, zb, zb2, 0), T1 = tload<ZV, SPLIT>(rs, zb, zb2, row_b);
-    V T2 = vzero<ZV>(), T3 = vzero<ZV>();
-    if (span >= 1) T2 = tload<ZV, SPLIT>(rs, zb, zb2, 2 * row_b);
-    if (span >= 2) T3 = tload<ZV, SPLIT>(rs, zb, zb2, 3 * row_b);
-    // one branch per pixel and row offset (the offsets are wave-uniform);
-    // the empty asm markers keep the compiler from turning the branches
-    // into register selects
-#define VAMX_BP_PIXEL(Q)                                                        \
-  if ((pm >> (Q)) & 1u) {                                                      \
-    const int off = (pkv >> (2 * (Q))) & 3;                                    \
-    if (off == 0) {                                                            \
-      asm volatile("; vamx bp " #Q " 0");                                      \
-      acc[Q] = vfma(u1[Q], T1, vfma(u0[Q], T0, acc[Q]));                       \
-    } else if (off == 1) {                                                     \
-      asm volatile("; vamx bp " #Q " 1");                                      \
-      acc[Q] = vfma(u1[Q], T2, vfma(u0[Q], T1, acc[Q]));                       \
-    } else {                                                                   \
-      asm volatile("; vamx bp " #Q " 2");                                      \
-      acc[Q] = vfma(u1[Q], T3, vfma(u0[Q], T2, acc[Q]));                       \
-    }                                                                          \
   }
-    VAMX_BP_PIXEL(0)
-    VAMX_BP_PIXEL(1)
-    VAMX_BP_PIXEL(2)
-    VAMX_BP_PIXEL(3)
-#undef VAMX_BP_PIXEL
+  __device__ __forceinline__ int slice(int q) const { return CONTIG ? z + q : z + 64 * q; }
+};
+typedef float mf4 __attribute__((ext_vector_type(4)));
+
+// the lane's ZV slices of a row
+template <int ZV, bool CONTIG>
+__device__ __forceinline__ void zload(__amdgpu_buffer_rsrc_t r, const ZLane<ZV, CONTIG>& ln, uint32_t soff,
+                                      float (&t)[ZV]) {
+  if constexpr (CONTIG) {
+    const float4 v = bload<4>(r, ln.zb[0], soff);
+    t[0] = v.x; t[1] = v.y; t[2] = v.z; t[3] = v.w;
+  } else {
+#pragma unroll
+    for (int q = 0; q < ZV; ++q) t[q] = bload<1>(r, ln.zb[q], soff);
+  }
+}
+
+// Back projection of a patch of voxel columns on one wavefront, lanes = z: NQ 2 x
+// 2 quads, two side by side (2 x 4 columns) or four (4 x 4).  Pixel p (0..3) of quad h is at row r0 + 2 (h >> 1) + (p >> 1),
+// column c0 + 2 (h & 1) + (p & 1); bit 4 h + p of `active` says whether it is
+// computed (in range and not circle-clipped).  Within one angle the patch's
+// detector coordinates lie within 3 |cos| + |sin| <= 3.2 (4 x 4: 4.3) of each
+// other, so its lower np.interp nodes span at most 5 (6) rows and it reads at
+// most 6 (7).
+//
+// Each row loaded is multiplied into the four columns of a quad by one
+// v_mfma_f32_4x4x1_16b_f32: 16 independent 4 x 1 x 4 products, of which block
+// b holds the quad's four weights (one per lane of the block) and the row's
+// slices of lanes 4 b .. 4 b + 3, so lane l accumulates its slice for all four
+// columns.  It rounds like the four fused multiply-adds it replaces (checked
+// bitwise), takes 8 to 10 cycles against their 18, and needs neither the
+// weights in scalar registers nor a branch per column and row: a column that
+// does not use a row has weight 0 there.  Adding 0 * row changes nothing
+// unless the row holds an infinity or a NaN, which then makes a NaN:
+// bp_patch_store recomputes those.  Each column thus sums
+// fma(w1, b[j+1], fma(w0, b[j], acc)) in angle order.
+//
+// Lanes first evaluate the float64 geometry of 16 angles and leave each
+// pixel's weights for the patch's rows in a per-wavefront LDS table; the
+// per-angle loop reads its lanes' weights from there and takes the angle's
+// first row and row count from a lane.
+//
+// COMB (no absorption): the angles are the plan's units (an angle and its
+// opposite, or one angle), and the opposite angle's rows, mirrored, are added
+// to the primary's as they are loaded: a column at detector coordinate t of
+// angle a is at -t of angle a + 180 deg, where the mirrored bins (2c + 2
+// det_offset - k) have the same neighbours and fractions.  np.interp is
+// continuous inside the detector, so the primary's interval and fraction serve
+// both; at the detector's ends, where it drops to 0, a column that only one of
+// the two angles sees takes that angle's own rows in further passes.
+//
+// Bound by the row loads, the chain of an angle (weights, loads, products) and
+// the few wavefronts: a row hardly ever is in the L1 (32 KB; the patches in
+// flight on a CU read about 80 rows of 256 slices at a time), and a missed KiB
+// occupies the texture path twice, 16 cycles to fill and 16 to return.
+// Measured, four columns a wavefront with scalar weights and branches -> patches:
+//   256 x 256 x 256, 360 angles, mu = 0.01   0.83 -> 0.76 ms
+//   256 x 256 x 64, 360 angles               493 -> 368 us
+//   201 x 201 x 77, 240 angles, mu = 0       268 -> 193 us
+//   160 x 160 x 120, 180 angles              136 -> 113 us
+//   64 x 64 x 64, 180 angles                 67 -> 52 us
+// 4 x 4 columns where a lane holds four slices: 0.76 against 0.80 ms as 2 x 4;
+// with fewer slices 4 x 4 leaves too few wavefronts.  In the batch's kernel,
+// which holds every layout, 4 x 4 spills (574 us against 449 us all 2 x 4).
+// Two ways of sharing rows through LDS measured slower at 256^3: 8 x 8 tiles
+// with a barrier per two angles 1.22 ms, with these products and a barrier per
+// angle 0.87 ms -- the staging's own scalar and vector instructions outweigh the
+// loads saved.
+// Requires n >= 2, all 64 lanes and blocks of at most 4 wavefronts.
+__host__ __device__ constexpr int bp_max_rows(int nq) { return nq == 4 ? 7 : 6; }
+__device__ __forceinline__ int bp_bit_row(int bit) { return 2 * (bit >> 3) + ((bit >> 1) & 1); }
+__device__ __forceinline__ int bp_bit_col(int bit) { return 2 * ((bit >> 2) & 1) + (bit & 1); }
+
+template <int NQ> struct BpW;
+template <> struct BpW<2> { using T = float2; };
+template <> struct BpW<4> { using T = float4; };
+
+// [16 angles][4 pixels][8 rows] of the quads' weights
+template <int NQ>
+__device__ __forceinline__ typename BpW<NQ>::T* bp_slot() {
+  __shared__ typename BpW<NQ>::T w[4][16 * 4 * 8];
+  return w[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 3];
+}
+
+// rows first .. first + M - 1 of angle i (COMB, i2 >= 0: plus the mirrored
+// rows of i2), multiplied into the patch with the angle's weights
+template <int NQ, int ZV, bool CONTIG, bool COMB, int M>
+__device__ __forceinline__ void bp_rows(const ParDev& g, const float* __restrict__ sino, int first, int i, int i2,
+                                        const ZLane<ZV, CONTIG>& ln, const typename BpW<NQ>::T* wa,
+                                        mf4 (&acc)[NQ][ZV]) {
+  const uint32_t row_b = 4u * (uint32_t)g.na * (uint32_t)g.nz, rows_b = (M - 1) * row_b + 4u * (uint32_t)g.nz;
+  const uint32_t at = ((uint32_t)first * (uint32_t)g.na + (uint32_t)i) * (uint32_t)g.nz;
+  const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sino + (size_t)at, rows_b);
+  float T[M][ZV];
+#pragma unroll
+  for (int k = 0; k < M; ++k) zload<ZV, CONTIG>(rs, ln, k * row_b, T[k]);
+  if constexpr (COMB) {
+    if (i2 >= 0) {
+      const int last = 2 * g.c + g.pair_D - first - (M - 1);   // mirror of the last row
+      const uint32_t at2 = ((uint32_t)last * (uint32_t)g.na + (uint32_t)i2) * (uint32_t)g.nz;
+      const __amdgpu_buffer_rsrc_t rs2 = buf_rsrc(sino + (size_t)at2, rows_b);
+      float O[M][ZV];
+#pragma unroll
+      for (int k = 0; k < M; ++k) zload<ZV, CONTIG>(rs2, ln, (M - 1 - k) * row_b, O[k]);
+#pragma unroll
+      for (int k = 0; k < M; ++k)
+#pragma unroll
+        for (int q = 0; q < ZV; ++q) T[k][q] += O[k][q];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    const typename BpW<NQ>::T w = wa[k];
+#pragma unroll
+    for (int h = 0; h < NQ; ++h)
+#pragma unroll
+      for (int q = 0; q < ZV; ++q)
+        acc[h][q] = __builtin_amdgcn_mfma_f32_4x4x1f32(vget(w, h), T[k][q], acc[h][q], 0, 0, 0);
+  }
+}
+
+template <int NQ, int ZV, bool CONTIG, bool COMB>
+__device__ __forceinline__ void bp_rows_of(const ParDev& g, const float* __restrict__ sino, int rows, int first, int i,
+                                           int i2, const ZLane<ZV, CONTIG>& ln,
+                                           const typename BpW<NQ>::T* wa,
+                                           mf4 (&acc)[NQ][ZV]) {
+  switch (rows) {   // wave-uniform; 0: no pixel of the patch is seen
+    case 2: bp_rows<NQ, ZV, CONTIG, COMB, 2>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 3: bp_rows<NQ, ZV, CONTIG, COMB, 3>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 4: bp_rows<NQ, ZV, CONTIG, COMB, 4>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 5: bp_rows<NQ, ZV, CONTIG, COMB, 5>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 6: bp_rows<NQ, ZV, CONTIG, COMB, 6>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 7:
+      if constexpr (bp_max_rows(NQ) >= 7) bp_rows<NQ, ZV, CONTIG, COMB, 7>(g, sino, first, i, i2, ln, wa, acc);
+      break;
+    default: break;
+  }
+}
+
+// lower row and weights of a pixel for one angle (np.interp; exactly at the
+// last node fp[n - 1]); jr = -1: not seen
+struct BpNode {
+  int jr;
+  float w0, w1;
+};
+
+// mirrored nodes common to both angles of a pair
+__device__ __forceinline__ int bp_jlo(const ParDev& g) { return max(0, 2 * g.c + g.pair_D - (g.n - 1)); }
+__device__ __forceinline__ int bp_jhi(const ParDev& g) { return min(g.n - 1, 2 * g.c + g.pair_D); }
+
+// which nodes a pass over the angles takes: of every angle (COMB: of the pairs,
+// where both angles see the pixel), or of the pixels that the pair's first or
+// second angle alone sees
+enum BpPass { BP_ALL = 0, BP_ONE = 1, BP_TWO = 2 };
+
+// node of the pixel at (x, y) for angle i (COMB: unit (i, i2)) in pass PASS;
+// single: only one angle of the pair sees it
+template <bool COMB, int PASS>
+__device__ __forceinline__ BpNode bp_node(const ParDev& g, bool on, int i, int i2, double x, double y, bool& single) {
+  const BpNode none{-1, 0.f, 0.f};
+  if (!on) return none;
+  const int n = g.n;
+  const double co = g.cs[2 * i], sn = g.cs[2 * i + 1];
+  const double t = x * co - y * sn;
+  int j, j1;
+  float f;
+  bool in = interp_node(g, t, j, j1, f);
+  if constexpr (COMB) {
+    if (i2 >= 0) {
+      const double t2 = x * g.cs[2 * i2] - y * g.cs[2 * i2 + 1];
+      int k, k1;
+      float f2;
+      const bool in2 = interp_node(g, t2, k, k1, f2);
+      if (in != in2) {
+        single = true;
+        if (PASS != (in ? BP_ONE : BP_TWO)) return none;
+        if (in2) {
+          j = k;
+          f = f2;
+          in = true;
+        }
+      } else if (PASS != BP_ALL) {
+        return none;
+      } else if (in) {
+        if (j < bp_jlo(g)) { j = bp_jlo(g); f = 0.0f; }
+        if (j >= bp_jhi(g)) { j = bp_jhi(g) - 1; f = 1.0f; }
+      }
+    } else if (PASS != BP_ALL) {
+      return none;
+    }
+  }
+  if (!in) return none;
+  const float aw = (!COMB && g.mu != 0.0) ? abs_weight(g, t, x * sn + y * co) : 1.0f;
+  if (aw == 0.0f) return none;
+  const bool last = j == n - 1;
+  return BpNode{last ? j - 1 : j, last ? 0.0f : aw * (1.0f - f), last ? aw : aw * f};
+}
+
+// one pass over the angles; true: COMB, a pixel is seen by one angle of a pair
+template <int NQ, int ZV, bool CONTIG, bool COMB, int PASS>
+__device__ __forceinline__ bool bp_pass(const ParDev& g, const float* __restrict__ sino, int r0, int c0,
+                                        unsigned active, const ZLane<ZV, CONTIG>& ln, int lane,
+                                        mf4 (&acc)[NQ][ZV]) {
+  using W = typename BpW<NQ>::T;
+  const int p = lane & 3, pa = lane >> 2;
+  const double y = (double)(r0 + (p >> 1) - g.c), x = (double)(c0 + (p & 1) - g.c);
+  W* const tab = bp_slot<NQ>();
+  float* const put = reinterpret_cast<float*>(tab + (pa * 4 + p) * 8);
+  const W* const get = tab + p * 8;              // this lane's pixel, angle 0
+  const int steps = COMB ? g.n_units : g.na;
+  bool singles = false;
+#pragma unroll 1
+  for (int u0 = 0; u0 < steps; u0 += 16) {
+    const int u = u0 + pa;
+    int i = u, i2 = -1;
+    if constexpr (COMB)
+      if (u < steps) {
+        i = g.units[2 * u];
+        i2 = g.units[2 * u + 1];
+      }
+    // rows of the patch's pixels at this lane's angle: their weights go to the
+    // table, the first row and the row count to pk (first | rows << 16)
+    BpNode nd[NQ];
+    bool single = false;
+    int lo = 0x7fffffff, hi = -1;
+#pragma unroll
+    for (int h = 0; h < NQ; ++h) {
+      nd[h] = bp_node<COMB, PASS>(g, u < steps && ((active >> (4 * h + p)) & 1u), i, i2, x + (double)(2 * (h & 1)),
+                                  y + (double)(2 * (h >> 1)), single);
+      if (nd[h].jr >= 0) {
+        lo = min(lo, nd[h].jr);
+        hi = max(hi, nd[h].jr);
+      }
+    }
+    lo = min(lo, __shfl_xor(lo, 1));
+    lo = min(lo, __shfl_xor(lo, 2));
+    hi = max(hi, __shfl_xor(hi, 1));
+    hi = max(hi, __shfl_xor(hi, 2));
+    if constexpr (COMB) singles |= __ballot(single) != 0ull;
+    const int pk = hi >= 0 ? lo | ((hi + 2 - lo) << 16) : 0;
+    if (PASS != BP_ALL && __ballot(pk != 0) == 0ull) continue;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int h = 0; h < NQ; ++h) {
+      const int d = nd[h].jr >= 0 ? nd[h].jr - lo : 0;
+#pragma unroll
+      for (int k = 0; k < bp_max_rows(NQ); ++k) put[k * NQ + h] = d == k ? nd[h].w0 : (d == k - 1 ? nd[h].w1 : 0.0f);
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int m = steps - u0 < 16 ? steps - u0 : 16;
+#pragma unroll 1
+    for (int a = 0; a < m; ++a) {
+      const int pkv = rl_i(pk, 4 * a);
+      const int ia = COMB ? rl_i(PASS == BP_TWO ? i2 : i, 4 * a) : u0 + a;
+      const int ib = COMB && PASS == BP_ALL ? rl_i(i2, 4 * a) : -1;
+      bp_rows_of<NQ, ZV, CONTIG, COMB && PASS == BP_ALL>(g, sino, pkv >> 16, pkv & 0xffff, ia, ib, ln, get + a * 32, acc);
+    }
+  }
+  return singles;
+}
+
+// a patch's sums
+template <int NQ, int ZV, bool CONTIG, bool COMB>
+__device__ __forceinline__ void bp_patch(const ParDev& g, const float* __restrict__ sino, int r0, int c0,
+                                         unsigned active, const ZLane<ZV, CONTIG>& ln, int lane,
+                                         mf4 (&acc)[NQ][ZV]) {
+#pragma unroll
+  for (int h = 0; h < NQ; ++h)
+#pragma unroll
+    for (int q = 0; q < ZV; ++q) acc[h][q] = mf4{0.f, 0.f, 0.f, 0.f};
+  if (active) {
+    if (bp_pass<NQ, ZV, CONTIG, COMB, BP_ALL>(g, sino, r0, c0, active, ln, lane, acc)) {
+      bp_pass<NQ, ZV, CONTIG, true, BP_ONE>(g, sino, r0, c0, active, ln, lane, acc);
+      bp_pass<NQ, ZV, CONTIG, true, BP_TWO>(g, sino, r0, c0, active, ln, lane, acc);
+    }
   }
 }
 
@@ -1263,6 +1434,113 @@ __device__ __forceinline__ bool bp_tile_quad(long long q, const ParDev& g, int& 
   c0 = 2 * qc;
   return qr < bp_nquad(g) && qc < bp_nquad(g);
 }
+
+// back projection: patches (2 or 4 rows x 4 columns) in tiles of bp_tile quads'
+// edge
+__host__ __device__ inline int bp_patch_rows(const ParDev& g, int nq) {
+  return (g.n + nq - 1) / nq;
+}
+__host__ __device__ inline int bp_patch_cols(const ParDev& g) { return (g.n + 3) / 4; }
+__host__ __device__ inline int bp_patch_tr(const ParDev& g, int nq) {
+  const int t = 2 * g.bp_tile > nq ? 2 * g.bp_tile / nq : 1;
+  return t < bp_patch_rows(g, nq) ? t : bp_patch_rows(g, nq);
+}
+__host__ __device__ inline int bp_patch_tc(const ParDev& g) {
+  const int t = g.bp_tile > 1 ? g.bp_tile / 2 : 1;
+  return t < bp_patch_cols(g) ? t : bp_patch_cols(g);
+}
+__host__ __device__ inline long long bp_patches(const ParDev& g, int nq) {
+  const int tr = bp_patch_tr(g, nq), tc = bp_patch_tc(g);
+  return (long long)((bp_patch_rows(g, nq) + tr - 1) / tr) * ((bp_patch_cols(g) + tc - 1) / tc) * tr * tc;
+}
+// wave -> patch and z chunk (chunk slowest); false for padding
+template <int NQ>
+__device__ __forceinline__ bool bp_wave_patch(long long wave, int chunks, const ParDev& g, int& r0, int& c0,
+                                              int& chunk) {
+  const long long patches = bp_patches(g, NQ);
+  if (wave >= patches * chunks) return false;
+  chunk = (int)(wave / patches);
+  const long long q = wave % patches;
+  const int tr = bp_patch_tr(g, NQ), tc = bp_patch_tc(g), nc = (bp_patch_cols(g) + tc - 1) / tc;
+  const int tile = (int)(q / (tr * tc)), within = (int)(q % (tr * tc));
+  // four consecutive wavefronts (a block) take 2 x 2 patches: they read fewer
+  // distinct rows per angle than four in a row
+  int wr = within / tc, wc = within % tc;
+  if (tr % 2 == 0 && tc % 2 == 0) {
+    const int b = within >> 2, k = within & 3, bc = tc >> 1;
+    wr = 2 * (b / bc) + (k >> 1);
+    wc = 2 * (b % bc) + (k & 1);
+  }
+  const int pr = tile / nc * tr + wr, pc = tile % nc * tc + wc;
+  r0 = NQ * pr;
+  c0 = 4 * pc;
+  return pr < bp_patch_rows(g, NQ) && pc < bp_patch_cols(g);
+}
+// bit 4 h + p: pixel p of quad h is inside the grid and, of those, computed
+template <int NQ>
+__device__ __forceinline__ void bp_patch_masks(const ParDev& g, int r0, int c0, int clipc, unsigned& inrange,
+                                               unsigned& active) {
+  inrange = active = 0u;
+#pragma unroll
+  for (int b = 0; b < 4 * NQ; ++b) {
+    const int row = r0 + bp_bit_row(b), col = c0 + bp_bit_col(b);
+    if (row < g.n && col < g.n) {
+      inrange |= 1u << b;
+      if (!(clipc && g.outside[row * g.n + col])) active |= 1u << b;
+    }
+  }
+}
+// the patch's doses: zero outside the computed columns; an infinity or a NaN (a
+// row that another column of its quad skips may have held an infinity, two
+// opposite rows may add past the largest number) is summed again as bp_voxel
+// does it
+template <int NQ, int ZV, bool CONTIG>
+__device__ __forceinline__ void bp_patch_store(const ParDev& g, const float* __restrict__ sino, float* vol, int r0,
+                                               int c0, unsigned inrange, unsigned active,
+                                               const ZLane<ZV, CONTIG>& ln, const mf4 (&acc)[NQ][ZV]) {
+  bool bad = false;
+#pragma unroll
+  for (int h = 0; h < NQ; ++h)
+#pragma unroll
+    for (int q = 0; q < ZV; ++q)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) bad |= !(fabsf(acc[h][q][p]) <= 3.4028234664e38f);
+#pragma unroll
+  for (int b = 0; b < 4 * NQ; ++b) {
+    if (!((inrange >> b) & 1u)) continue;
+    const int h = b >> 2, p = b & 3;
+    float* outp = vol + ((size_t)(r0 + bp_bit_row(b)) * g.n + c0 + bp_bit_col(b)) * g.nz;
+    const bool on = (active >> b) & 1u;
+    if constexpr (CONTIG) {
+      if (ln.z < g.nz)
+        vstore<4>(outp + ln.z, on ? make_float4(acc[h][0][p], acc[h][1][p], acc[h][2][p], acc[h][3][p]) : vzero<4>());
+    } else {
+#pragma unroll
+      for (int q = 0; q < ZV; ++q)
+        if (ln.slice(q) < g.nz) outp[ln.slice(q)] = on ? acc[h][q][p] : 0.0f;
+    }
+  }
+  if (__ballot(bad) == 0ull) return;
+#pragma unroll 1
+  for (int b = 0; b < 4 * NQ; ++b) {
+    if (!((active >> b) & 1u)) continue;
+    const int pix = (r0 + bp_bit_row(b)) * g.n + c0 + bp_bit_col(b);
+#pragma unroll 1
+    for (int q = 0; q < ZV; ++q) {
+      const int z = ln.slice(q);
+      if (z >= g.nz) continue;
+      float* at = vol + (size_t)pix * g.nz + z;
+      if (!(fabsf(*at) <= 3.4028234664e38f)) *at = bp_voxel<1>(g, sino, pix, z);
+    }
+  }
+}
+// how a problem's back projection lays out its slices: slices per lane (0: not
+// on these kernels), 16-byte loads of four, opposite angles combined
+struct BpLayout {
+  int zv = 0, nq = 2;
+  bool contig = false, comb = false;
+  int chunks = 0;
+};
 
 // Global index of the calling wavefront for logical block lb.  The wave's
 // slot in its block is made wave-uniform explicitly (readfirstlane), so that
@@ -1489,10 +1767,26 @@ struct UpdateOut {
   }
 };
 
+// calls f(NQ, ZV, CONTIG, COMB) with the layout's compile-time constants
+template <class F>
+void bp_dispatch(const BpLayout& l, F&& f) {
+  using std::integral_constant;
+  auto with = [&](auto comb) {
+    if (l.contig) f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, std::true_type{}, comb);
+    else if (l.zv == 4) f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, std::false_type{}, comb);
+    else if (l.zv == 3) f(integral_constant<int, 2>{}, integral_constant<int, 3>{}, std::false_type{}, comb);
+    else if (l.zv == 2) f(integral_constant<int, 2>{}, integral_constant<int, 2>{}, std::false_type{}, comb);
+    else f(integral_constant<int, 2>{}, integral_constant<int, 1>{}, std::false_type{}, comb);
+  };
+  if (l.comb) with(std::true_type{});
+  else with(std::false_type{});
+}
+
 // host helpers implemented in parallel.hip
 int par_slice_minmax(vamx_plan* p, const float* vol, hipStream_t s);
 int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t s, bool warp_clip);
 int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t s, bool clipc);
+BpLayout bp_layout(const vamx_plan* p, uintptr_t align_bits);
 bool par_use_vec4(const vamx_plan* p, const void* a, const void* b);
 bool par_use_vec2(const vamx_plan* p, const void* a, const void* b);
 int par_wave_zv(const vamx_plan* p, const void* a, const void* b, int requested);

@@ -217,26 +217,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void p
   if (k2 >= 0) wave_zstore<ZV, SPLIT>(sino + ((size_t)k2 * g.na + i2) * g.nz, z, g.nz, acc2);
 }
 
-// wavefront-uniform back projection: one wavefront = one 2x2 quad of voxel
-// columns x 64*ZV z
-template <int ZV, bool SPLIT>
-__global__ __launch_bounds__(256) void par_bp_wave_kernel(ParDev g, const float* __restrict__ sino,
-                                                          float* __restrict__ vol, int clipc) {
+// back projection: one wavefront = one patch of voxel columns x 64 ZV z.
+// The minimum of wavefronts per SIMD holds the kernel under 256 registers,
+// which makes the compiler keep the products' accumulators in vector
+// registers; left in accumulation registers it copied all 8 ZV of them in and
+// out for every angle.
+template <int NQ, int ZV, bool CONTIG, bool COMB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void par_bp_patch_kernel(
+    ParDev g, const float* __restrict__ sino, float* vol, int clipc, int chunks) {
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  int r0, c0, z, zl, zl2;
-  if (!bp_wave_quad<ZV, SPLIT>(wave, g, lane, r0, c0, z)) return;
-  wave_zload<ZV, SPLIT>(z, g.nz, zl, zl2);
+  int r0, c0, chunk;
+  if (!bp_wave_patch<NQ>(wave, chunks, g, r0, c0, chunk)) return;
+  const ZLane<ZV, CONTIG> ln(chunk, lane, g.nz);
   unsigned inrange, active;
-  bp_quad_masks(g, r0, c0, clipc, inrange, active);
-  typename VecT<ZV>::T acc[4];
-  bp_quad_wave<ZV, SPLIT>(g, sino, r0, c0, active, zl, lane, acc, zl2);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if (!((inrange >> q) & 1u)) continue;
-    float* outp = vol + ((size_t)(r0 + (q >> 1)) * g.n + c0 + (q & 1)) * g.nz;
-    wave_zstore<ZV, SPLIT>(outp, z, g.nz, ((active >> q) & 1u) ? acc[q] : vzero<ZV>());
-  }
+  bp_patch_masks<NQ>(g, r0, c0, clipc, inrange, active);
+  mf4 acc[NQ][ZV];
+  bp_patch<NQ, ZV, CONTIG, COMB>(g, sino, r0, c0, active, ln, lane, acc);
+  bp_patch_store<NQ, ZV, CONTIG>(g, sino, vol, r0, c0, inrange, active, ln, acc);
 }
 
 __global__ __launch_bounds__(256) void par_fp_incl_kernel(ParDev g, const float* __restrict__ vol,
@@ -418,6 +416,27 @@ int vamx::par_wave_zv(const vamx_plan* p, const void* a, const void* b, int requ
   // the per-lane kernels) when even the best leaves half the lanes idle
   if ((p->flags & VAMX_PAR_PER_LANE_GEOMETRY) || p->par.incl || p->par.n < 2 || p->par.occ) return 0;
   return wave_zv_choice(p->par.nz, (uintptr_t)a | (uintptr_t)b, requested);
+}
+
+BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits) {
+  const ParDev& g = p->par;
+  BpLayout l;
+  if ((p->flags & VAMX_PAR_PER_LANE_GEOMETRY) || g.incl || g.n < 2 || g.occ || g.nz < 32) return l;
+  // slices per lane, at most the tuning's bp_zv: the fewest slice slots, then
+  // the fewest chunks (the geometry is evaluated per chunk)
+  int slots = 0;
+  for (int zv = 1; zv <= g.bp_zv; ++zv) {
+    const int c = wave_zchunks(g.nz, zv);
+    if (!slots || c * zv <= slots) {
+      l.zv = zv;
+      l.chunks = c;
+      slots = c * zv;
+    }
+  }
+  if (l.zv == 4) l.nq = 4;
+  l.contig = l.zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0;
+  l.comb = g.mu == 0.0 && g.pair_ok;
+  return l;
 }
 
 int vamx::wave_zv_choice(int nz, uintptr_t align_bits, int requested) {
@@ -763,21 +782,13 @@ int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t
     VAMX_HIP(hipGetLastError());
     return VAMX_OK;
   }
-  int wz = par_wave_zv(p, sino, vol, g.bp_zv);
-  const bool split = par_wave_split(p, wz);
-  if (split) wz = 2;
-  if (wz) {
-    const long long threads = bp_tiled_quads(g) * wave_zchunks(g.nz, wz) * 64;
-    const dim3 grid(blocks_for(threads, 256)), block(256);
-    const int cc = clipc ? 1 : 0;
-    if (split)
-      hipLaunchKernelGGL((par_bp_wave_kernel<2, true>), grid, block, 0, s, g, sino, vol, cc);
-    else if (wz == 4)
-      hipLaunchKernelGGL((par_bp_wave_kernel<4, false>), grid, block, 0, s, g, sino, vol, cc);
-    else if (wz == 2)
-      hipLaunchKernelGGL((par_bp_wave_kernel<2, false>), grid, block, 0, s, g, sino, vol, cc);
-    else
-      hipLaunchKernelGGL((par_bp_wave_kernel<1, false>), grid, block, 0, s, g, sino, vol, cc);
+  if (const BpLayout l = bp_layout(p, (uintptr_t)sino | (uintptr_t)vol); l.zv) {
+    const dim3 grid(blocks_for(bp_patches(g, l.nq) * l.chunks * 64, 256)), block(256);
+    bp_dispatch(l, [&](auto nq, auto zv, auto contig, auto comb) {
+      hipLaunchKernelGGL((par_bp_patch_kernel<decltype(nq)::value, decltype(zv)::value, decltype(contig)::value,
+                                              decltype(comb)::value>),
+                         grid, block, 0, s, g, sino, vol, clipc ? 1 : 0, l.chunks);
+    });
     VAMX_HIP(hipGetLastError());
     return VAMX_OK;
   }
