@@ -28,6 +28,8 @@
 // Interaction taps use floor and floor+1 with weights 1-d and d (standard
 // trilinear); the reference selects floor and ceil, which counts a tap twice
 // when a coordinate is exactly integral.
+#include <climits>
+
 #include "bclp_core.h"
 #include "vamx_internal.h"
 
@@ -40,6 +42,9 @@ __device__ __forceinline__ d3 mk(double x, double y, double z) { return {x, y, z
 __device__ __forceinline__ d3 add(d3 a, d3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
 __device__ __forceinline__ d3 sub(d3 a, d3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
 __device__ __forceinline__ d3 scl(double s, d3 a) { return {s * a.x, s * a.y, s * a.z}; }
+
+__device__ __forceinline__ float min3(float a, float b, float c) { return fminf(fminf(a, b), c); }
+__device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 // Trilinear interpolation in polynomial form: from the corner values
 // t[c] (c = x + 2 y + 4 z bits) of one cell,
@@ -68,6 +73,31 @@ __device__ __forceinline__ float tri_eval(const Tri& r, float x, float y, float 
   return fmaf(z, fmaf(y, d, c), fmaf(y, b, a));
 }
 
+// A position on the grid: the interaction cell (the floors of the float64 index
+// coordinates, as float: exact where a ray can be inside the grid) and the
+// fractions in it; z is 0, 0 in 2-D.  Taken once per step: the interaction at
+// the step's end and the next step's field samples use it.
+struct GridPos {
+  double ix, iy, iz;   // index coordinates
+  float x0, y0, z0, wx, wy, wz;
+  bool inside;         // the cell has a tap inside the grid
+};
+// moves p to x; false: x is in p's cell and only the fractions changed
+__device__ __forceinline__ bool grid_move(const RtDev& g, d3 x, GridPos& p) {
+  const double ix = p.ix = (x.x - g.xmin) * g.inv_dx, iy = p.iy = (x.y - g.ymin) * g.inv_dy;
+  const double iz = p.iz = g.nz > 1 ? (x.z - g.zmin) * g.inv_dz : 0.0;
+  p.wx = (float)(ix - (double)p.x0);
+  p.wy = (float)(iy - (double)p.y0);
+  p.wz = (float)(iz - (double)p.z0);
+  if (p.wx >= 0.0f && p.wy >= 0.0f && p.wz >= 0.0f && p.wx < 1.0f && p.wy < 1.0f && p.wz < 1.0f) return false;
+  const double fx = floor(ix), fy = floor(iy), fz = floor(iz);
+  p.x0 = (float)fx; p.y0 = (float)fy; p.z0 = (float)fz;
+  p.wx = (float)(ix - fx); p.wy = (float)(iy - fy); p.wz = (float)(iz - fz);
+  p.inside = p.x0 >= -1.0f && p.x0 <= g.last_x && p.y0 >= -1.0f && p.y0 <= g.last_y && p.z0 >= -1.0f &&
+             p.z0 <= g.last_z;
+  return true;
+}
+
 // One grid cell of the float4 medium, held in registers as the trilinear
 // coefficients of its four channels.  The samples of a ray lie a quarter or
 // half voxel apart (RK4 samples x, twice x + h/2 and x + h, and x + h starts
@@ -76,15 +106,25 @@ __device__ __forceinline__ float tri_eval(const Tri& r, float x, float y, float 
 // adjacent rays, so a wavefront's lanes mostly change cells at the same
 // sample.
 struct FieldCell {
-  int key;       // linear index of the cell's corner voxel; -1 = nothing held
-  Tri ch[4];     // n, dn/dx, dn/dy, dn/dz
+  float x0, y0, z0;      // the cell's corner voxel
+  float hx, hy, hz;      // the last voxel, counted from it
+  double bx, by, bz;     // the step's start, counted from it
+  Tri ch[4];             // n, dn/dx, dn/dy, dn/dz
 };
+// no cell held: a corner that puts every sample outside the cell
+__device__ __forceinline__ void field_reset(const RtDev& g, FieldCell& fc) {
+  fc.x0 = fc.y0 = fc.z0 = -4.0f;
+  fc.hx = g.last_x + 4.0f;
+  fc.hy = g.last_y + 4.0f;
+  fc.hz = g.last_z + 4.0f;
+}
+// the step's start, for the samples of the step
+__device__ __forceinline__ void field_base(const GridPos& p, FieldCell& fc) {
+  fc.bx = p.ix - (double)fc.x0;
+  fc.by = p.iy - (double)fc.y0;
+  fc.bz = p.iz - (double)fc.z0;
+}
 
-// trilinear sample of the float4 field, grid_sample(align_corners=True,
-// padding_mode="border"): index coordinates clamped to [0, size-1].  The
-// position and the cell choice are float64; the interpolation is float32
-// (the field is stored in float32).  A tap past the last voxel along an axis
-// (coordinate exactly size - 1, weight 0) reads the last voxel.
 // analytical Luneburg lens at physical position (x, y, z) (medium.py:486-549):
 // n = n_sur (2 - (r/R)^p)^(1/p) and grad n = -(n_sur/R)^p n^(1-p) r^(p-2) x
 // for r < R; n = n_sur and grad n = 0 outside
@@ -111,25 +151,30 @@ __device__ __forceinline__ void lune_sample(const RtDev& g, double x, double y, 
   }
 }
 
-template <bool LUNE>
-__device__ __forceinline__ void field_sample_idx(const RtDev& g, double ix, double iy, double iz, FieldCell& fc,
-                                                 float& n, float& gx, float& gy, float& gz) {
-  if constexpr (LUNE) {
-    lune_sample(g, g.xmin + ix * g.dx, g.ymin + iy * g.dy, g.nz > 1 ? g.zmin + iz * g.dz : g.zmin, n, gx, gy, gz);
-    return;
-  }
-  ix = fmin(fmax(ix, 0.0), g.ixmax);
-  iy = fmin(fmax(iy, 0.0), g.iymax);
-  iz = fmin(fmax(iz, 0.0), g.izmax);
-  const double fx = floor(ix), fy = floor(iy), fz = floor(iz);
-  const int x0 = (int)fx, y0 = (int)fy, z0 = (int)fz;
-  const int key = (x0 * g.ny + y0) * g.nz + z0;
-  if (key != fc.key) {
-    fc.key = key;
-    const int sx = x0 + 1 < g.nx ? g.ny * g.nz : 0;
-    const int sy = y0 + 1 < g.ny ? g.nz : 0;
-    const int sz = z0 + 1 < g.nz ? 1 : 0;
-    const float4* b = g.field + key;
+// trilinear sample of the float4 field at the step's start plus an offset in
+// voxels, grid_sample(align_corners=True, padding_mode="border"): index
+// coordinates clamped to [0, size - 1].  The position is float64, counted from
+// the held cell's corner, so that its conversion to float32 is the fraction in
+// that cell (the field is stored and interpolated in float32); a sample that
+// stays in the cell takes no floor and no cell index.  A tap past the last voxel
+// along an axis (coordinate exactly size - 1, weight 0) reads the last voxel.
+__device__ __forceinline__ void field_sample_at(const RtDev& g, float ox, float oy, float oz, FieldCell& fc, float& n,
+                                                float& gx, float& gy, float& gz) {
+  float wx = __builtin_amdgcn_fmed3f((float)(fc.bx + (double)ox), -fc.x0, fc.hx);
+  float wy = __builtin_amdgcn_fmed3f((float)(fc.by + (double)oy), -fc.y0, fc.hy);
+  float wz = __builtin_amdgcn_fmed3f((float)(fc.bz + (double)oz), -fc.z0, fc.hz);
+  if (!(min3(wx, wy, wz) >= 0.0f && max3(wx, wy, wz) < 1.0f)) {
+    const float fx = floorf(wx), fy = floorf(wy), fz = floorf(wz);
+    fc.x0 += fx; fc.y0 += fy; fc.z0 += fz;
+    fc.hx -= fx; fc.hy -= fy; fc.hz -= fz;
+    fc.bx -= (double)fx; fc.by -= (double)fy; fc.bz -= (double)fz;
+    wx = __builtin_amdgcn_fmed3f((float)(fc.bx + (double)ox), 0.0f, fc.hx);
+    wy = __builtin_amdgcn_fmed3f((float)(fc.by + (double)oy), 0.0f, fc.hy);
+    wz = __builtin_amdgcn_fmed3f((float)(fc.bz + (double)oz), 0.0f, fc.hz);
+    const int sx = fc.hx >= 1.0f ? g.ny * g.nz : 0, sy = fc.hy >= 1.0f ? g.nz : 0, sz = fc.hz >= 1.0f ? 1 : 0;
+    // inside the grid for every finite position; kept there for any other
+    const int key = ((int)fc.x0 * g.ny + (int)fc.y0) * g.nz + (int)fc.z0;
+    const float4* b = g.field + min(max(key, 0), g.nx * g.ny * g.nz - 1 - sx - sy - sz);
     float4 t[8];
     t[0] = b[0];
     t[1] = b[sx];
@@ -153,7 +198,6 @@ __device__ __forceinline__ void field_sample_idx(const RtDev& g, double ix, doub
     for (int c = 0; c < 8; ++c) q[c] = t[c].w;
     fc.ch[3] = tri_coef(q);
   }
-  const float wx = (float)(ix - fx), wy = (float)(iy - fy), wz = (float)(iz - fz);
   n = tri_eval(fc.ch[0], wx, wy, wz);
   gx = tri_eval(fc.ch[1], wx, wy, wz);
   gy = tri_eval(fc.ch[2], wx, wy, wz);
@@ -166,8 +210,7 @@ __device__ __forceinline__ void field_sample(const RtDev& g, d3 x, FieldCell& fc
   if constexpr (LUNE)
     lune_sample(g, x.x, x.y, x.z, nf, gx, gy, gz);
   else
-    field_sample_idx<false>(g, (x.x - g.xmin) * g.inv_dx, (x.y - g.ymin) * g.inv_dy,
-                     g.nz > 1 ? (x.z - g.zmin) * g.inv_dz : 0.0, fc, nf, gx, gy, gz);
+    field_sample_at(g, 0.0f, 0.0f, 0.0f, fc, nf, gx, gy, gz);
   n = (double)nf;
   gn = mk((double)gx, (double)gy, (double)gz);
 }
@@ -199,25 +242,8 @@ __device__ __forceinline__ double att_alpha(const RtDev& g, d3 x) {
   return 0.0;
 }
 
-// right-hand side of the ray equation in parametrisation PARAM
+// grad n part of the ray equation in parametrisation PARAM
 // (pyTorchRayTrace.py:695-735)
-template <int PARAM, bool LUNE>
-__device__ __forceinline__ void rhs(const RtDev& g, d3 x, d3 v, FieldCell& fc, d3& dx, d3& dv) {
-  double n;
-  d3 gn;
-  field_sample<LUNE>(g, x, fc, n, gn);
-  if (PARAM == VAMX_RT_CANONICAL) {
-    dx = v;
-    dv = scl(n, gn);
-  } else if (PARAM == VAMX_RT_PHYSICAL) {
-    dx = scl(1.0 / n, v);
-    dv = gn;
-  } else {
-    dx = scl(1.0 / (n * n), v);
-    dv = scl(1.0 / n, gn);
-  }
-}
-
 template <int PARAM>
 __device__ __forceinline__ d3 accel(double n, d3 gn) {
   if (PARAM == VAMX_RT_CANONICAL) return scl(n, gn);
@@ -225,55 +251,50 @@ __device__ __forceinline__ d3 accel(double n, d3 gn) {
   return scl(1.0 / n, gn);
 }
 
-__device__ __forceinline__ d3 fma3(double s, d3 a, d3 b) { return {fma(s, a.x, b.x), fma(s, a.y, b.y), fma(s, a.z, b.z)}; }
-
-// one step of solver SOLVER: (x, v) -> (x', v')
+// one step of solver SOLVER: (x, v) -> (x', v'), the step x' - x returned;
+// field_base has been called for x
 template <int SOLVER, int PARAM, bool LUNE>
-__device__ __forceinline__ void advance(const RtDev& g, d3& x, d3& v, FieldCell& fc) {
+__device__ __forceinline__ d3 advance(const RtDev& g, d3& x, d3& v, FieldCell& fc) {
   const double h = g.step;
   if (SOLVER == VAMX_RT_RK4) {
     // x' = x + h/6 (k1 + 2 k2 + 2 k3 + k4), likewise v.  x and v stay
     // float64; the stage derivatives k, their running sums and the stage
-    // offsets c k (at most h apart from x) are float32, and the stage
-    // sample positions are formed in grid-index units as the float64 index
-    // of x plus the float32 offset.  The four stages are one loop (not
-    // unrolled), so the field sample -- and the cell it holds in registers --
-    // exists once in the code and keeps one set of registers.
-    const float hf = (float)h;
-    const double bx = (x.x - g.xmin) * g.inv_dx, by = (x.y - g.ymin) * g.inv_dy;
-    const double bz = g.nz > 1 ? (x.z - g.zmin) * g.inv_dz : 0.0;
-    const float idx = (float)g.inv_dx, idy = (float)g.inv_dy, idz = g.nz > 1 ? (float)g.inv_dz : 0.0f;
-    float kx0 = 0.0f, kx1 = 0.0f, kx2 = 0.0f, kv0 = 0.0f, kv1 = 0.0f, kv2 = 0.0f;
+    // offsets (at most about h from x) are float32.  The four stages are one
+    // loop, not unrolled: the field sample, and the cell it holds in registers,
+    // exists once in the code (unrolled it spilled).
+    float ox = 0.0f, oy = 0.0f, oz = 0.0f;   // the stage's offset from x in voxels
+    float kv0 = 0.0f, kv1 = 0.0f, kv2 = 0.0f;
     float sx0 = 0.0f, sx1 = 0.0f, sx2 = 0.0f, sv0 = 0.0f, sv1 = 0.0f, sv2 = 0.0f;
 #pragma unroll 1
     for (int st = 0; st < 4; ++st) {
-      const float c = st == 0 ? 0.0f : (st == 3 ? hf : 0.5f * hf);  // stage offset along the previous k
-      const float wk = (st == 0 || st == 3) ? 1.0f : 2.0f;          // weight of this k in the sum
+      const RkStage& k = g.rk[st];   // scalar loads: no selects in the loop
       float n, gx, gy, gz;
-      field_sample_idx<LUNE>(g, bx + (double)((c * kx0) * idx), by + (double)((c * kx1) * idy),
-                       bz + (double)((c * kx2) * idz), fc, n, gx, gy, gz);
-      const float vs0 = (float)(v.x + (double)(c * kv0));
-      const float vs1 = (float)(v.y + (double)(c * kv1));
-      const float vs2 = (float)(v.z + (double)(c * kv2));
-      if (PARAM == VAMX_RT_CANONICAL) {
-        kx0 = vs0; kx1 = vs1; kx2 = vs2;
-        kv0 = n * gx; kv1 = n * gy; kv2 = n * gz;
-      } else if (PARAM == VAMX_RT_PHYSICAL) {
-        const float r = __builtin_amdgcn_rcpf(n);
-        kx0 = vs0 * r; kx1 = vs1 * r; kx2 = vs2 * r;
-        kv0 = gx; kv1 = gy; kv2 = gz;
+      if constexpr (LUNE) {
+        const double ix = (x.x - g.xmin) * g.inv_dx + (double)ox, iy = (x.y - g.ymin) * g.inv_dy + (double)oy;
+        const double iz = g.nz > 1 ? (x.z - g.zmin) * g.inv_dz + (double)oz : 0.0;
+        lune_sample(g, g.xmin + ix * g.dx, g.ymin + iy * g.dy, g.nz > 1 ? g.zmin + iz * g.dz : g.zmin, n, gx, gy, gz);
       } else {
-        const float r = __builtin_amdgcn_rcpf(n), r2 = r * r;
-        kx0 = vs0 * r2; kx1 = vs1 * r2; kx2 = vs2 * r2;
-        kv0 = gx * r; kv1 = gy * r; kv2 = gz * r;
+        field_sample_at(g, ox, oy, oz, fc, n, gx, gy, gz);
       }
-      sx0 = fmaf(wk, kx0, sx0); sx1 = fmaf(wk, kx1, sx1); sx2 = fmaf(wk, kx2, sx2);
-      sv0 = fmaf(wk, kv0, sv0); sv1 = fmaf(wk, kv1, sv1); sv2 = fmaf(wk, kv2, sv2);
+      float kx0 = (float)(v.x + (double)(k.c * kv0));
+      float kx1 = (float)(v.y + (double)(k.c * kv1));
+      float kx2 = (float)(v.z + (double)(k.c * kv2));
+      if (PARAM == VAMX_RT_CANONICAL) {
+        kv0 = n * gx; kv1 = n * gy; kv2 = n * gz;
+      } else {
+        const float r = __builtin_amdgcn_rcpf(n), rx = PARAM == VAMX_RT_PHYSICAL ? r : r * r;
+        kx0 *= rx; kx1 *= rx; kx2 *= rx;
+        if (PARAM == VAMX_RT_PHYSICAL) { kv0 = gx; kv1 = gy; kv2 = gz; }
+        else { kv0 = gx * r; kv1 = gy * r; kv2 = gz * r; }
+      }
+      ox = (k.next * kx0) * g.fx; oy = (k.next * kx1) * g.fy; oz = (k.next * kx2) * g.fz;
+      sx0 = fmaf(k.w, kx0, sx0); sx1 = fmaf(k.w, kx1, sx1); sx2 = fmaf(k.w, kx2, sx2);
+      sv0 = fmaf(k.w, kv0, sv0); sv1 = fmaf(k.w, kv1, sv1); sv2 = fmaf(k.w, kv2, sv2);
     }
-    const float h6 = hf / 6.0f;
-    x = add(x, mk((double)(h6 * sx0), (double)(h6 * sx1), (double)(h6 * sx2)));
-    v = add(v, mk((double)(h6 * sv0), (double)(h6 * sv1), (double)(h6 * sv2)));
-    return;
+    const d3 d = {(double)(g.h6 * sx0), (double)(g.h6 * sx1), (double)(g.h6 * sx2)};
+    x = add(x, d);
+    v = add(v, mk((double)(g.h6 * sv0), (double)(g.h6 * sv1), (double)(g.h6 * sv2)));
+    return d;
   }
   double n;
   d3 gn;
@@ -284,13 +305,16 @@ __device__ __forceinline__ void advance(const RtDev& g, d3& x, d3& v, FieldCell&
   if (PARAM == VAMX_RT_CANONICAL) dx = vx;
   else if (PARAM == VAMX_RT_PHYSICAL) dx = scl(1.0 / n, vx);
   else dx = scl(1.0 / (n * n), vx);
-  x = add(x, scl(h, dx));
+  const d3 d = scl(h, dx);
+  x = add(x, d);
   v = vnew;
+  return d;
 }
 
 // initial state of ray (t, a, zr) (setupRaysParallel, pyTorchRayTrace.py:1638-1666)
 template <int SOLVER, int PARAM, bool LUNE>
-__device__ __forceinline__ void ray_init(const RtDev& g, int t, int a, int zr, d3& x, d3& v, FieldCell& fc) {
+__device__ __forceinline__ void ray_init(const RtDev& g, int t, int a, int zr, d3& x, d3& v, GridPos& p,
+                                         FieldCell& fc) {
   const double ct = g.ray_cs[2 * a], st = g.ray_cs[2 * a + 1];
   const double ci = cos(g.incl), si = sin(g.incl);
   const double G0 = g.ray_t[t], G2 = g.ray_z[zr], D = g.radial_offset;
@@ -298,6 +322,14 @@ __device__ __forceinline__ void ray_init(const RtDev& g, int t, int a, int zr, d
   x.y = D * st * ci + (G0 * ct - G2 * st * si);
   x.z = D * si + G2 * ci;
   v = mk(-ct * ci, -st * ci, -si);
+  p.x0 = p.y0 = p.z0 = 0.0f;
+  p.inside = false;
+  grid_move(g, x, p);
+  field_reset(g, fc);
+  field_base(p, fc);
+  // the start is no interaction: no cell is held, and the first step enters one
+  p.inside = false;
+  p.x0 = __builtin_nanf("");
   if (SOLVER == VAMX_RT_LEAPFROG) {
     // _leapfrog_init: v -= dv(x, v) h / 2 (pyTorchRayTrace.py:817-828)
     double n;
@@ -314,34 +346,6 @@ __device__ __forceinline__ bool exited(const RtDev& g, d3 x, d3 v) {
   const bool neg = (x.x < g.exit_lo_x && v.x < 0.0) || (x.y < g.exit_lo_y && v.y < 0.0) ||
                    (x.z < g.exit_lo_z && v.z < 0.0);
   return pos || neg;
-}
-
-// interaction taps at position x: index coordinates and base weight
-struct Taps {
-  int x0, y0, z0;
-  double wx, wy, wz;
-  int nzt;  // 2 in 3-D, 1 in 2-D
-};
-__device__ __forceinline__ Taps taps_at(const RtDev& g, d3 x) {
-  Taps t;
-  const double ix = (x.x - g.xmin) * g.inv_dx, iy = (x.y - g.ymin) * g.inv_dy;
-  const double fx = floor(ix), fy = floor(iy);
-  t.x0 = (int)fmax(fmin(fx, 2.0e9), -2.0e9);
-  t.y0 = (int)fmax(fmin(fy, 2.0e9), -2.0e9);
-  t.wx = ix - fx;
-  t.wy = iy - fy;
-  if (g.nz > 1) {
-    const double iz = (x.z - g.zmin) * g.inv_dz;
-    const double fz = floor(iz);
-    t.z0 = (int)fmax(fmin(fz, 2.0e9), -2.0e9);
-    t.wz = iz - fz;
-    t.nzt = 2;
-  } else {
-    t.z0 = 0;
-    t.wz = 0.0;
-    t.nzt = 1;
-  }
-  return t;
 }
 
 // what a trace does at each interaction tap
@@ -364,66 +368,98 @@ struct RtIo {
   float upd_lr, upd_glb, upd_gub;
 };
 
-// Interaction taps of one cell (corner x0, y0, z0, possibly -1 on an axis):
+// Interaction taps of the ray's cell (its corner is possibly -1 on an axis):
 // integrate holds f_eff at its taps; deposit holds, per tap, the float32 sum
 // of the weights of the ray's consecutive steps in the cell, written out as
 // one fixed-point integer atomic per tap when the ray moves to another cell
 // and at the end of the ray (integer addition is associative, so the
 // accumulator does not depend on the order of the atomics).
 struct TapCell {
-  int key;           // cell key ((x0+1) (ny+1) + y0+1) (nz+1) + z0+1; -1 = nothing held
-  int x0, y0, z0;
   Tri f;             // integrate: f_eff at the taps (0 outside the grid), trilinear coefficients
   float q[8];        // deposit: summed tap weights
 };
 
-// writes out the taps of `mask` (bit c = tap c) and clears them
-__device__ __forceinline__ void tap_flush(const RtDev& g, const RtIo& io, TapCell& tc, double scale,
-                                          unsigned mask = 0xffu) {
+// the value of the next / previous lane; `none` where that lane is inactive
+__device__ __forceinline__ int lane_next(int none, int v) {
+  return __builtin_amdgcn_update_dpp(none, v, 0x130 /* wave_shl:1 */, 0xf, 0xf, false);
+}
+__device__ __forceinline__ int lane_prev(int none, int v) {
+  return __builtin_amdgcn_update_dpp(none, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+}
+
+// Moves the held taps of the cell at (x0, y0, z0) by one cell along axis AX
+// (bit AX of a tap index), up or down: the face the new cell shares with the
+// old one keeps its sums, the taps of the other face that lie inside the grid
+// are written out.
+template <int AX>
+__device__ __forceinline__ void tap_shift(const RtDev& g, const RtIo& io, TapCell& tc, double scale, int& x0, int& y0,
+                                          int& z0, bool up) {
+  constexpr int bit = 1 << AX;
+  const int fx = x0 + (AX == 0 && !up), fy = y0 + (AX == 1 && !up), fz = z0 + (AX == 2 && !up);   // corner of the face
+  const bool okx[2] = {(unsigned)fx < (unsigned)g.nx, (unsigned)(fx + 1) < (unsigned)g.nx};
+  const bool oky[2] = {(unsigned)fy < (unsigned)g.ny, (unsigned)(fy + 1) < (unsigned)g.ny};
+  const bool okz[2] = {(unsigned)fz < (unsigned)g.nz, (unsigned)(fz + 1) < (unsigned)g.nz};
+  const int key = (fx * g.ny + fy) * g.nz + fz;
+  unsigned long long* const at = io.acc + key;
+  // adjacent lanes trace adjacent z: where the next lane writes out the same
+  // face one voxel higher, it adds this lane's upper taps to its lower ones
+  // (integers: the same sums with half the atomics)
+  bool give = false, got = false;
+  if (AX != 2) {
+    const int next = lane_next(INT_MIN, okz[0] ? key : INT_MIN);
+    give = okz[1] && next == key + 1;
+    got = lane_prev(0, (int)give) != 0;
+  }
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
-    if (!((mask >> c) & 1u)) continue;
-    const long long q = llrint((double)tc.q[c] * scale);
-    tc.q[c] = 0.0f;
-    if (q == 0) continue;   // taps outside the grid carry weight 0
-    const int xi = tc.x0 + (c & 1), yi = tc.y0 + ((c >> 1) & 1), zi = tc.z0 + ((c >> 2) & 1);
-    atomicAdd(io.acc + ((size_t)xi * g.ny + yi) * g.nz + zi, (unsigned long long)q);
+    if (c & bit) continue;
+    if (AX != 2 && (c & 4)) continue;   // with its lower tap
+    const bool ok = okx[c & 1] && oky[(c >> 1) & 1];
+    unsigned long long* const ac = at + (((c & 1) * g.ny + ((c >> 1) & 1)) * g.nz + (c >> 2));
+    long long q = llrint((double)(up ? tc.q[c] : tc.q[c | bit]) * scale);
+    if (AX != 2) {
+      const long long qz = llrint((double)(up ? tc.q[c | 4] : tc.q[c | 4 | bit]) * scale);
+      const unsigned lo = (unsigned)lane_prev(0, (int)(unsigned)qz), hi = (unsigned)lane_prev(0, (int)(qz >> 32));
+      if (got) q += (long long)(((unsigned long long)hi << 32) | lo);
+      if (qz != 0 && !give && ok && okz[1]) atomicAdd(ac + 1, (unsigned long long)qz);
+    }
+    if (q != 0 && ok && okz[c >> 2]) atomicAdd(ac, (unsigned long long)q);
+  }
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    if (c & bit) continue;
+    const float keep = up ? tc.q[c | bit] : tc.q[c];
+    tc.q[c] = up ? keep : 0.0f;
+    tc.q[c | bit] = up ? 0.0f : keep;
+  }
+  (AX == 0 ? x0 : (AX == 1 ? y0 : z0)) += up ? 1 : -1;
+}
+
+// the taps of cell `from` follow the ray to cell `to`; what is not shared is
+// written out.  Farther than the next cell or outside the grid (to = null): two
+// moves along x write out everything.
+__device__ __forceinline__ void tap_move(const RtDev& g, const RtIo& io, TapCell& tc, double scale, const GridPos& from,
+                                         const GridPos* to) {
+  int x0 = (int)from.x0, y0 = (int)from.y0, z0 = (int)from.z0;
+  const float dx = to ? to->x0 - from.x0 : 2.0f, dy = to ? to->y0 - from.y0 : 0.0f, dz = to ? to->z0 - from.z0 : 0.0f;
+  const bool far = max3(fabsf(dx), fabsf(dy), fabsf(dz)) > 1.0f;
+#pragma unroll 1
+  for (int k = far ? 2 : (dx != 0.0f ? 1 : 0); k > 0; --k) tap_shift<0>(g, io, tc, scale, x0, y0, z0, far || dx > 0.0f);
+  if (!far) {
+    if (dy != 0.0f) tap_shift<1>(g, io, tc, scale, x0, y0, z0, dy > 0.0f);
+    if (dz != 0.0f) tap_shift<2>(g, io, tc, scale, x0, y0, z0, dz > 0.0f);
   }
 }
 
-// Moves the held cell by d (-1, 0 or +1) along axis AX (bit AX of a tap
-// index): the face the new cell shares with the old one keeps its sums, the
-// other face is written out.  |d| > 1: everything is written out.
-template <int AX>
-__device__ __forceinline__ void tap_shift(const RtDev& g, const RtIo& io, TapCell& tc, double scale, int d) {
-  constexpr unsigned lo = AX == 0 ? 0x55u : (AX == 1 ? 0x33u : 0x0fu);   // taps with bit AX = 0
-  constexpr int bit = 1 << AX;
-  if (d == 0) return;
-  if (d == 1) {
-    tap_flush(g, io, tc, scale, lo);
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      if (!(c & bit)) {
-        tc.q[c] = tc.q[c | bit];
-        tc.q[c | bit] = 0.0f;
-      }
-  } else if (d == -1) {
-    tap_flush(g, io, tc, scale, lo ^ 0xffu);
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      if (!(c & bit)) {
-        tc.q[c | bit] = tc.q[c];
-        tc.q[c] = 0.0f;
-      }
-  } else {
-    tap_flush(g, io, tc, scale);
-  }
-  if (AX == 0) tc.x0 += d;
-  else if (AX == 1) tc.y0 += d;
-  else tc.z0 += d;
-}
-
-// at most 128 VGPRs: 4 wavefronts per SIMD
+// at most 128 VGPRs: 4 wavefronts per SIMD (deposit at 5 spilled: 1285 us against
+// 997 at 64^3 x 90).  Bound by instructions: a step takes about 570 (wavefront
+// instructions, 4 to 4.5 cycles each on a SIMD), of them 74 for each of the four
+// stages and 100 for a field cell's change, of which a wavefront sees about one
+// per step; deposit, 440, waits besides for its atomics, which execute in memory
+// behind the L2s.  Measured, floors, cell indices and tap masks per sample and one
+// atomic per lane and tap -> cells held as corners and adjacent lanes' taps joined:
+//   64^3, 90 angles    integrate 1009 -> 984 us, deposit 1110 -> 997 us
+//   192^3, 360 angles  together 143.2 -> 124.3 ms
 template <int MODE, int SOLVER, int PARAM, bool LUNE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rt_trace_kernel(RtDev g, RtIo io) {
   const long long nrays = (long long)g.nt * g.na * g.nzr;
@@ -451,15 +487,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
   long long slot = (MODE == RT_RECORD && live) ? io.counts[r] : 0;   // record: this ray's first slot
   long long ntaps = 0;
   FieldCell fc;
-  fc.key = -1;
   TapCell tc;
-  tc.key = -1;
-  tc.x0 = tc.y0 = tc.z0 = 0;
   tc.f = Tri{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int c = 0; c < 8; ++c) tc.q[c] = 0.0f;
   d3 x, v;
-  ray_init<SOLVER, PARAM, LUNE>(g, t, a, zr, x, v, fc);
+  GridPos p;
+  ray_init<SOLVER, PARAM, LUNE>(g, t, a, zr, x, v, p, fc);
   const double hw = g.hw;
   const float e0f = (float)E0;
   double A = 0.0, integral = 0.0;
@@ -467,74 +501,65 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
   bool active = live;
   if (live) {
     for (; step < g.max_steps; ++step) {
-      const d3 xo = x;
-      advance<SOLVER, PARAM, LUNE>(g, x, v, fc);
-      const d3 d = sub(x, xo);
-      const double al = att_alpha(g, xo);
+      const double al = att_alpha(g, x);
+      const d3 d = advance<SOLVER, PARAM, LUNE>(g, x, v, fc);
       // attenuance (767-769) and ray energy (770-774); step length and
       // exponential in float32
       if (al != 0.0) A += al * (double)__builtin_amdgcn_sqrtf((float)(d.x * d.x + d.y * d.y + d.z * d.z));
       const double E = (double)(e0f * __expf(-(float)A));
-      const Taps tp = taps_at(g, x);
-      if (tp.x0 >= -1 && tp.x0 < g.nx && tp.y0 >= -1 && tp.y0 < g.ny && tp.z0 >= -1 && tp.z0 < g.nz) {
+      const GridPos from = p;
+      const bool moved = grid_move(g, x, p);
+      if (!LUNE) field_base(p, fc);
+      if (MODE == RT_DEPOSIT && moved && from.inside) tap_move(g, io, tc, scale, from, p.inside ? &p : nullptr);
+      if (p.inside) {
         const double base = hw * E;
-        // tap weights, 0 for taps outside the grid (and, in 2-D, above the plane)
-        const float wx = (float)tp.wx, wy = (float)tp.wy, wz = tp.nzt == 1 ? 0.0f : (float)tp.wz;
-        const float ux = 1.0f - wx, uy = 1.0f - wy, uz = 1.0f - wz;
-        const bool vx0 = tp.x0 >= 0, vx1 = tp.x0 + 1 < g.nx, vy0 = tp.y0 >= 0, vy1 = tp.y0 + 1 < g.ny;
-        const bool vz0 = tp.z0 >= 0, vz1 = tp.nzt == 2 && tp.z0 + 1 < g.nz;
-        float w[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const bool ok = ((c & 1) ? vx1 : vx0) && (((c >> 1) & 1) ? vy1 : vy0) && (((c >> 2) & 1) ? vz1 : vz0);
-          const float ww = (((c & 1) ? wx : ux) * (((c >> 1) & 1) ? wy : uy)) * (((c >> 2) & 1) ? wz : uz);
-          w[c] = ok ? ww : 0.0f;
-        }
-        const int key = ((tp.x0 + 1) * (g.ny + 1) + (tp.y0 + 1)) * (g.nz + 1) + (tp.z0 + 1);
         if (MODE == RT_INTEGRATE) {
-          if (key != tc.key) {
-            tc.key = key;
+          if (moved) {
+            const int x0 = (int)p.x0, y0 = (int)p.y0, z0 = (int)p.z0, plane = g.ny * g.nz;
             float fv[8];
+            // every lane's taps inside the grid: fixed strides; else taps outside
+            // read an in-grid voxel and hold 0
+            const bool in = x0 >= 0 && y0 >= 0 && z0 >= 0 && x0 + 1 < g.nx && y0 + 1 < g.ny && z0 + 1 < g.nz;
+            if (__ballot(!in) == 0ull) {
+              const float* b = io.feff + ((x0 * g.ny + y0) * g.nz + z0);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-              // taps outside the grid read an in-grid voxel and hold 0
-              const int xi = min(max(tp.x0 + (c & 1), 0), g.nx - 1);
-              const int yi = min(max(tp.y0 + ((c >> 1) & 1), 0), g.ny - 1);
-              const int zi = min(max(tp.z0 + ((c >> 2) & 1), 0), g.nz - 1);
-              const float f = io.feff[((size_t)xi * g.ny + yi) * g.nz + zi];
-              const bool ok = ((c & 1) ? vx1 : vx0) && (((c >> 1) & 1) ? vy1 : vy0) && (((c >> 2) & 1) ? vz1 : vz0);
-              fv[c] = ok ? f : 0.0f;
+              for (int c = 0; c < 8; ++c) fv[c] = b[(c & 1) * plane + ((c >> 1) & 1) * g.nz + (c >> 2)];
+            } else {
+              const bool vx[2] = {x0 >= 0, x0 + 1 < g.nx}, vy[2] = {y0 >= 0, y0 + 1 < g.ny};
+              const bool vz[2] = {z0 >= 0, z0 + 1 < g.nz};
+              const int ax[2] = {max(x0, 0) * plane, min(x0 + 1, g.nx - 1) * plane};
+              const int ay[2] = {max(y0, 0) * g.nz, min(y0 + 1, g.ny - 1) * g.nz};
+              const int az[2] = {max(z0, 0), min(z0 + 1, g.nz - 1)};
+#pragma unroll
+              for (int c = 0; c < 8; ++c) {
+                const float f = io.feff[ax[c & 1] + ay[(c >> 1) & 1] + az[c >> 2]];
+                fv[c] = vx[c & 1] && vy[(c >> 1) & 1] && vz[c >> 2] ? f : 0.0f;
+              }
             }
             tc.f = tri_coef(fv);
           }
-          integral += base * (double)tri_eval(tc.f, wx, wy, wz);
+          integral += base * (double)tri_eval(tc.f, p.wx, p.wy, p.wz);
         } else if (MODE == RT_DEPOSIT) {
-          if (key != tc.key) {
-            // the taps shared with the previous cell keep accumulating: about
-            // half of the atomics of a flush per cell change
-            if (tc.key >= 0) {
-              tap_shift<0>(g, io, tc, scale, tp.x0 - tc.x0);
-              tap_shift<1>(g, io, tc, scale, tp.y0 - tc.y0);
-              tap_shift<2>(g, io, tc, scale, tp.z0 - tc.z0);
-            }
-            tc.key = key;
-            tc.x0 = tp.x0;
-            tc.y0 = tp.y0;
-            tc.z0 = tp.z0;
-          }
+          // taps outside the grid are summed too and dropped when written out
           const float bf = (float)base;
+          const float ux = 1.0f - p.wx, uy = 1.0f - p.wy;
+          const float bz[2] = {bf * (1.0f - p.wz), bf * p.wz};
+          const float wxy[4] = {ux * uy, p.wx * uy, ux * p.wy, p.wx * p.wy};
 #pragma unroll
-          for (int c = 0; c < 8; ++c) tc.q[c] = fmaf(bf, w[c], tc.q[c]);
+          for (int c = 0; c < 8; ++c) tc.q[c] = fmaf(bz[c >> 2], wxy[c & 3], tc.q[c]);
         } else {
+          // taps inside the grid of weight > 0
+          const int x0 = (int)p.x0, y0 = (int)p.y0, z0 = (int)p.z0;
 #pragma unroll
           for (int c = 0; c < 8; ++c) {
-            if (w[c] == 0.0f) continue;
+            const int xi = x0 + (c & 1), yi = y0 + ((c >> 1) & 1), zi = z0 + (c >> 2);
+            const float ww = (((c & 1) ? p.wx : 1.0f - p.wx) * ((c & 2) ? p.wy : 1.0f - p.wy)) * ((c & 4) ? p.wz : 1.0f - p.wz);
+            if (ww == 0.0f || xi < 0 || xi >= g.nx || yi < 0 || yi >= g.ny || zi < 0 || zi >= g.nz) continue;
             if (MODE == RT_COUNT) {
               ++ntaps;
             } else {
-              const int xi = tp.x0 + (c & 1), yi = tp.y0 + ((c >> 1) & 1), zi = tp.z0 + ((c >> 2) & 1);
-              io.rec_vox[slot] = (int32_t)(((size_t)xi * g.ny + yi) * g.nz + zi);
-              io.rec_w[slot] = (float)(base * (double)w[c]);
+              io.rec_vox[slot] = (int32_t)((xi * g.ny + yi) * g.nz + zi);
+              io.rec_w[slot] = (float)(base * (double)ww);
               ++slot;
             }
           }
@@ -550,7 +575,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         }
       }
     }
-    if (MODE == RT_DEPOSIT && tc.key >= 0) tap_flush(g, io, tc, scale);
+    if (MODE == RT_DEPOSIT && p.inside) tap_move(g, io, tc, scale, p, nullptr);
   }
   if (MODE == RT_INTEGRATE && valid) {
     if (io.upd_g) {
@@ -752,7 +777,7 @@ extern "C" int vamx_rt_create(const vamx_rt_geom* geom, vamx_plan** out_plan) {
   g.ymax = g.ymin + (g.ny - 1) * g.dy;
   g.zmax = g.nz > 1 ? g.zmin + (g.nz - 1) * g.dz : g.zmin;
   g.span_x = g.xmax - g.xmin; g.span_y = g.ymax - g.ymin; g.span_z = g.zmax - g.zmin;
-  g.ixmax = g.nx - 1; g.iymax = g.ny - 1; g.izmax = g.nz - 1;
+  g.last_x = (float)(g.nx - 1); g.last_y = (float)(g.ny - 1); g.last_z = (float)(g.nz - 1);
   g.nt = geom->nt; g.na = geom->n_angles; g.nzr = geom->nzr;
   g.incl = geom->incl_deg * (M_PI / 180.0);
   g.step = geom->step;
@@ -772,6 +797,15 @@ extern "C" int vamx_rt_create(const vamx_rt_geom* geom, vamx_plan** out_plan) {
   g.att_alpha = geom->att_alpha;
   g.att_radius = geom->att_radius;
   g.att_r2 = g.att_radius * g.att_radius;
+  {
+    const float h = (float)g.step;
+    g.h6 = h / 6.0f;
+    g.rk[0] = {0.0f, 0.5f * h, 1.0f};
+    g.rk[1] = {0.5f * h, 0.5f * h, 2.0f};
+    g.rk[2] = {0.5f * h, h, 2.0f};
+    g.rk[3] = {h, 0.0f, 1.0f};
+  }
+  g.fx = (float)g.inv_dx; g.fy = (float)g.inv_dy; g.fz = g.nz > 1 ? (float)g.inv_dz : 0.0f;
   g.hw = g.step / g.dx;   // step_size_idx_unit (pyTorchRayTrace.py:840-842)
   {
     const double vz = g.nz > 1 ? g.dz : INFINITY;   // exitCheck (pyTorchRayTrace.py:1391-1420)

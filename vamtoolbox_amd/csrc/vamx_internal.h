@@ -47,13 +47,23 @@ struct ParDev {
 };
 
 // Geometry of the curved-ray tracer, passed by value.
+// one stage of the classical Runge-Kutta step: its and the next stage's offset
+// along the k of the stage before, and its k's weight in the sum
+struct RkStage {
+  float c, next, w;
+};
+
 struct RtDev {
   int nx, ny, nz;
   double xmin, ymin, zmin, dx, dy, dz;
   double inv_dx, inv_dy, inv_dz;
   double span_x, span_y, span_z;
   double xmax, ymax, zmax;
-  double ixmax, iymax, izmax;  // largest index coordinate: size - 1
+  // derived on the host: the last voxel's index, 1 / d in float32 (z: 0 in 2-D),
+  // the Runge-Kutta stages and step / 6
+  float last_x, last_y, last_z, fx, fy, fz;
+  RkStage rk[4];
+  float h6;
   int nt, na, nzr;
   double incl;               // radians
   double step;
