@@ -97,16 +97,16 @@ __device__ __forceinline__ void batch_fp_pair(const BatchItem& it, const float* 
 
 template <int ZV, bool CONTIG, bool COMB>
 __device__ __forceinline__ void batch_bp_patch(const BatchItem& it, const float* in, float* out, long long w,
-                                               int lane) {
+                                               int lane, float2* tab) {
   const ParDev& g = it.g;
   int r0, c0, chunk;
-  if (!bp_wave_patch<2>(w, it.chunks, g, r0, c0, chunk)) return;
+  if (!bp_wave_patch(w, it.chunks, g, it.clip, r0, c0, chunk)) return;
   const ZLane<ZV, CONTIG> ln(chunk, lane, g.nz);
   unsigned inrange, active;
-  bp_patch_masks<2>(g, r0, c0, it.clip, inrange, active);
-  mf4 acc[2][ZV];
-  bp_patch<2, ZV, CONTIG, COMB>(g, in, r0, c0, active, ln, lane, acc);
-  bp_patch_store<2, ZV, CONTIG>(g, in, out, r0, c0, inrange, active, ln, acc);
+  bp_patch_masks(g, r0, c0, it.clip, inrange, active);
+  mf4 acc[BP_QUADS][ZV];
+  bp_patch<ZV, CONTIG, COMB>(g, in, r0, c0, active, ln, lane, tab, acc);
+  bp_patch_store<ZV, CONTIG>(g, in, out, r0, c0, inrange, active, ln, acc);
 }
 
 template <bool FORWARD>
@@ -146,6 +146,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
                                                     long long ntiles, unsigned long long* counter,
                                                     BatchPtrs ptrs) {
   __shared__ long long tile_sh;
+  __shared__ float2 tabs[FORWARD ? 1 : 4][FORWARD ? 1 : BP_TABLE];
   const int lane = threadIdx.x & 63;
   const int slot = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (;;) {
@@ -184,18 +185,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
           else if (it.zv == 2) batch_fp_wave<2, false>(it, in, out, w, lane);
           else batch_fp_wave<1, false>(it, in, out, w, lane);
         } else {
+          float2* const tab = tabs[FORWARD ? 0 : slot];
           if (it.comb) {
-            if (it.contig) batch_bp_patch<4, true, true>(it, in, out, w, lane);
-            else if (it.zv == 4) batch_bp_patch<4, false, true>(it, in, out, w, lane);
-            else if (it.zv == 3) batch_bp_patch<3, false, true>(it, in, out, w, lane);
-            else if (it.zv == 2) batch_bp_patch<2, false, true>(it, in, out, w, lane);
-            else batch_bp_patch<1, false, true>(it, in, out, w, lane);
+            if (it.contig) batch_bp_patch<4, true, true>(it, in, out, w, lane, tab);
+            else if (it.zv == 4) batch_bp_patch<4, false, true>(it, in, out, w, lane, tab);
+            else if (it.zv == 3) batch_bp_patch<3, false, true>(it, in, out, w, lane, tab);
+            else if (it.zv == 2) batch_bp_patch<2, false, true>(it, in, out, w, lane, tab);
+            else batch_bp_patch<1, false, true>(it, in, out, w, lane, tab);
           } else {
-            if (it.contig) batch_bp_patch<4, true, false>(it, in, out, w, lane);
-            else if (it.zv == 4) batch_bp_patch<4, false, false>(it, in, out, w, lane);
-            else if (it.zv == 3) batch_bp_patch<3, false, false>(it, in, out, w, lane);
-            else if (it.zv == 2) batch_bp_patch<2, false, false>(it, in, out, w, lane);
-            else batch_bp_patch<1, false, false>(it, in, out, w, lane);
+            if (it.contig) batch_bp_patch<4, true, false>(it, in, out, w, lane, tab);
+            else if (it.zv == 4) batch_bp_patch<4, false, false>(it, in, out, w, lane, tab);
+            else if (it.zv == 3) batch_bp_patch<3, false, false>(it, in, out, w, lane, tab);
+            else if (it.zv == 2) batch_bp_patch<2, false, false>(it, in, out, w, lane, tab);
+            else batch_bp_patch<1, false, false>(it, in, out, w, lane, tab);
           }
         }
       }
@@ -350,7 +352,7 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
       it.contig = (path >> 3) & 1;
       it.comb = (path >> 4) & 1;
       it.chunks = wave_zchunks(it.g.nz, it.zv);
-      it.items = bp_patches(it.g, 2) * it.chunks;
+      it.items = (long long)it.g.bp_all * it.chunks;
     } else if (path > 0) {
       const int wz = path == 3 ? 2 : path;
       it.wave = 1;

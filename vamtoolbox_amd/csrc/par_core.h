@@ -1119,13 +1119,12 @@ __device__ __forceinline__ void zload(__amdgpu_buffer_rsrc_t r, const ZLane<ZV, 
   }
 }
 
-// Back projection of a patch of voxel columns on one wavefront, lanes = z: NQ 2 x
-// 2 quads, two side by side (2 x 4 columns) or four (4 x 4).  Pixel p (0..3) of quad h is at row r0 + 2 (h >> 1) + (p >> 1),
-// column c0 + 2 (h & 1) + (p & 1); bit 4 h + p of `active` says whether it is
-// computed (in range and not circle-clipped).  Within one angle the patch's
-// detector coordinates lie within 3 |cos| + |sin| <= 3.2 (4 x 4: 4.3) of each
-// other, so its lower np.interp nodes span at most 5 (6) rows and it reads at
-// most 6 (7).
+// Back projection of a patch of 2 x 4 voxel columns on one wavefront, lanes = z:
+// two 2 x 2 quads side by side.  Pixel p (0..3) of quad h is at row r0 + (p >> 1),
+// column c0 + 2 h + (p & 1); bit 4 h + p of `active` says whether it is computed
+// (in range and not circle-clipped).  Within one angle the patch's detector
+// coordinates lie within 3 |cos| + |sin| <= 3.2 of each other, so its lower
+// np.interp nodes span at most 5 rows and it reads at most 6.
 //
 // Each row loaded is multiplied into the four columns of a quad by one
 // v_mfma_f32_4x4x1_16b_f32: 16 independent 4 x 1 x 4 products, of which block
@@ -1153,45 +1152,37 @@ __device__ __forceinline__ void zload(__amdgpu_buffer_rsrc_t r, const ZLane<ZV, 
 // both; at the detector's ends, where it drops to 0, a column that only one of
 // the two angles sees takes that angle's own rows in further passes.
 //
-// Bound by the row loads, the chain of an angle (weights, loads, products) and
-// the few wavefronts: a row hardly ever is in the L1 (32 KB; the patches in
-// flight on a CU read about 80 rows of 256 slices at a time), and a missed KiB
-// occupies the texture path twice, 16 cycles to fill and 16 to return.
+// Bound by issuing: a 1 KiB row load takes a CU's texture path 17 to 20 cycles
+// (a 256-byte one 8.5), its products 4 * 2 * 8.5 cycles of one SIMD, and the two
+// overlap little: 256^3 x 360 angles takes 1.4 M cycles per CU, of them 0.83 M for
+// the loads, 0.87 M for products and vector instructions, 0.3 M for scalar ones.
+// With 16-byte loads the next angle's rows are loaded before this angle's products
+// (0.62 against 0.70 ms); with 4-byte loads the second set of rows costs more
+// wavefronts than it gains (256 x 256 x 128: 0.45 against 0.39 ms).
 // Measured, four columns a wavefront with scalar weights and branches -> patches:
-//   256 x 256 x 256, 360 angles, mu = 0.01   0.83 -> 0.76 ms
-//   256 x 256 x 64, 360 angles               493 -> 368 us
-//   201 x 201 x 77, 240 angles, mu = 0       268 -> 193 us
-//   160 x 160 x 120, 180 angles              136 -> 113 us
-//   64 x 64 x 64, 180 angles                 67 -> 52 us
-// 4 x 4 columns where a lane holds four slices: 0.76 against 0.80 ms as 2 x 4;
-// with fewer slices 4 x 4 leaves too few wavefronts.  In the batch's kernel,
-// which holds every layout, 4 x 4 spills (574 us against 449 us all 2 x 4).
-// Two ways of sharing rows through LDS measured slower at 256^3: 8 x 8 tiles
-// with a barrier per two angles 1.22 ms, with these products and a barrier per
-// angle 0.87 ms -- the staging's own scalar and vector instructions outweigh the
-// loads saved.
-// Requires n >= 2, all 64 lanes and blocks of at most 4 wavefronts.
-__host__ __device__ constexpr int bp_max_rows(int nq) { return nq == 4 ? 7 : 6; }
-__device__ __forceinline__ int bp_bit_row(int bit) { return 2 * (bit >> 3) + ((bit >> 1) & 1); }
-__device__ __forceinline__ int bp_bit_col(int bit) { return 2 * ((bit >> 2) & 1) + (bit & 1); }
+//   256 x 256 x 256, 360 angles, mu = 0.01   0.83 -> 0.64 ms
+//   256 x 256 x 64, 360 angles               493 -> 230 us
+//   201 x 201 x 77, 240 angles, mu = 0       284 -> 154 us
+//   200 x 200 x 180, 240 angles              608 -> 237 us
+//   160 x 160 x 120, 180 angles              136 -> 118 us
+//   64 x 64 x 64, 180 angles                 67 -> 48 us
+// Tried and slower at 256^3: 4 x 4 columns a wavefront (0.78 ms against 0.70: too
+// few wavefronts for their shares to be even), 8 x 8 tiles of columns with the rows
+// in LDS, a barrier per two angles (1.22) or per angle with these products (0.87).
+// Requires n >= 2 and all 64 lanes.
+constexpr int BP_QUADS = 2, BP_ROWS = 6;
+__device__ __forceinline__ int bp_bit_row(int bit) { return (bit >> 1) & 1; }
+__device__ __forceinline__ int bp_bit_col(int bit) { return 2 * (bit >> 2) + (bit & 1); }
 
-template <int NQ> struct BpW;
-template <> struct BpW<2> { using T = float2; };
-template <> struct BpW<4> { using T = float4; };
-
-// [16 angles][4 pixels][8 rows] of the quads' weights
-template <int NQ>
-__device__ __forceinline__ typename BpW<NQ>::T* bp_slot() {
-  __shared__ typename BpW<NQ>::T w[4][16 * 4 * 8];
-  return w[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) & 3];
-}
+// a wavefront's table, [16 angles][4 pixels][8 rows] of the quads' weights
+constexpr int BP_TABLE = 16 * 4 * 8;
 
 // rows first .. first + M - 1 of angle i (COMB, i2 >= 0: plus the mirrored
 // rows of i2), multiplied into the patch with the angle's weights
-template <int NQ, int ZV, bool CONTIG, bool COMB, int M>
+template <int ZV, bool CONTIG, bool COMB, int M>
 __device__ __forceinline__ void bp_rows(const ParDev& g, const float* __restrict__ sino, int first, int i, int i2,
-                                        const ZLane<ZV, CONTIG>& ln, const typename BpW<NQ>::T* wa,
-                                        mf4 (&acc)[NQ][ZV]) {
+                                        const ZLane<ZV, CONTIG>& ln, const float2* wa,
+                                        mf4 (&acc)[BP_QUADS][ZV]) {
   const uint32_t row_b = 4u * (uint32_t)g.na * (uint32_t)g.nz, rows_b = (M - 1) * row_b + 4u * (uint32_t)g.nz;
   const uint32_t at = ((uint32_t)first * (uint32_t)g.na + (uint32_t)i) * (uint32_t)g.nz;
   const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sino + (size_t)at, rows_b);
@@ -1214,31 +1205,61 @@ __device__ __forceinline__ void bp_rows(const ParDev& g, const float* __restrict
   }
 #pragma unroll
   for (int k = 0; k < M; ++k) {
-    const typename BpW<NQ>::T w = wa[k];
+    const float2 w = wa[k];
 #pragma unroll
-    for (int h = 0; h < NQ; ++h)
+    for (int h = 0; h < BP_QUADS; ++h)
 #pragma unroll
       for (int q = 0; q < ZV; ++q)
         acc[h][q] = __builtin_amdgcn_mfma_f32_4x4x1f32(vget(w, h), T[k][q], acc[h][q], 0, 0, 0);
   }
 }
 
-template <int NQ, int ZV, bool CONTIG, bool COMB>
+template <int ZV, bool CONTIG, bool COMB>
 __device__ __forceinline__ void bp_rows_of(const ParDev& g, const float* __restrict__ sino, int rows, int first, int i,
                                            int i2, const ZLane<ZV, CONTIG>& ln,
-                                           const typename BpW<NQ>::T* wa,
-                                           mf4 (&acc)[NQ][ZV]) {
+                                           const float2* wa,
+                                           mf4 (&acc)[BP_QUADS][ZV]) {
   switch (rows) {   // wave-uniform; 0: no pixel of the patch is seen
-    case 2: bp_rows<NQ, ZV, CONTIG, COMB, 2>(g, sino, first, i, i2, ln, wa, acc); break;
-    case 3: bp_rows<NQ, ZV, CONTIG, COMB, 3>(g, sino, first, i, i2, ln, wa, acc); break;
-    case 4: bp_rows<NQ, ZV, CONTIG, COMB, 4>(g, sino, first, i, i2, ln, wa, acc); break;
-    case 5: bp_rows<NQ, ZV, CONTIG, COMB, 5>(g, sino, first, i, i2, ln, wa, acc); break;
-    case 6: bp_rows<NQ, ZV, CONTIG, COMB, 6>(g, sino, first, i, i2, ln, wa, acc); break;
-    case 7:
-      if constexpr (bp_max_rows(NQ) >= 7) bp_rows<NQ, ZV, CONTIG, COMB, 7>(g, sino, first, i, i2, ln, wa, acc);
-      break;
+    case 2: bp_rows<ZV, CONTIG, COMB, 2>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 3: bp_rows<ZV, CONTIG, COMB, 3>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 4: bp_rows<ZV, CONTIG, COMB, 4>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 5: bp_rows<ZV, CONTIG, COMB, 5>(g, sino, first, i, i2, ln, wa, acc); break;
+    case 6: bp_rows<ZV, CONTIG, COMB, 6>(g, sino, first, i, i2, ln, wa, acc); break;
     default: break;
   }
+}
+
+// the rows of one angle, loaded (pk: first | count << 16; count 0: none)
+template <int ZV>
+struct BpRows {
+  int rows;
+  float t[BP_ROWS][ZV];
+};
+template <int ZV, bool CONTIG>
+__device__ __forceinline__ void bp_load(const ParDev& g, const float* __restrict__ sino, int pk, int i,
+                                        const ZLane<ZV, CONTIG>& ln, BpRows<ZV>& r) {
+  r.rows = pk >> 16;
+  if (r.rows == 0) return;   // wave-uniform, like the tests below
+  const uint32_t row_b = 4u * (uint32_t)g.na * (uint32_t)g.nz;
+  const uint32_t at = ((uint32_t)(pk & 0xffff) * (uint32_t)g.na + (uint32_t)i) * (uint32_t)g.nz;
+  const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sino + (size_t)at, (uint32_t)(r.rows - 1) * row_b + 4u * (uint32_t)g.nz);
+#pragma unroll
+  for (int k = 0; k < BP_ROWS; ++k)
+    if (k < 2 || r.rows > k) zload<ZV, CONTIG>(rs, ln, k * row_b, r.t[k]);
+}
+template <int ZV>
+__device__ __forceinline__ void bp_products(const BpRows<ZV>& r, const float2* wa, mf4 (&acc)[BP_QUADS][ZV]) {
+  if (r.rows == 0) return;
+#pragma unroll
+  for (int k = 0; k < BP_ROWS; ++k)
+    if (k < 2 || r.rows > k) {
+      const float2 w = wa[k];
+#pragma unroll
+      for (int h = 0; h < BP_QUADS; ++h)
+#pragma unroll
+        for (int q = 0; q < ZV; ++q)
+          acc[h][q] = __builtin_amdgcn_mfma_f32_4x4x1f32(vget(w, h), r.t[k][q], acc[h][q], 0, 0, 0);
+    }
 }
 
 // lower row and weights of a pixel for one angle (np.interp; exactly at the
@@ -1301,16 +1322,14 @@ __device__ __forceinline__ BpNode bp_node(const ParDev& g, bool on, int i, int i
 }
 
 // one pass over the angles; true: COMB, a pixel is seen by one angle of a pair
-template <int NQ, int ZV, bool CONTIG, bool COMB, int PASS>
+template <int ZV, bool CONTIG, bool COMB, int PASS>
 __device__ __forceinline__ bool bp_pass(const ParDev& g, const float* __restrict__ sino, int r0, int c0,
                                         unsigned active, const ZLane<ZV, CONTIG>& ln, int lane,
-                                        mf4 (&acc)[NQ][ZV]) {
-  using W = typename BpW<NQ>::T;
+                                        float2* tab, mf4 (&acc)[BP_QUADS][ZV]) {
   const int p = lane & 3, pa = lane >> 2;
   const double y = (double)(r0 + (p >> 1) - g.c), x = (double)(c0 + (p & 1) - g.c);
-  W* const tab = bp_slot<NQ>();
   float* const put = reinterpret_cast<float*>(tab + (pa * 4 + p) * 8);
-  const W* const get = tab + p * 8;              // this lane's pixel, angle 0
+  const float2* const get = tab + p * 8;              // this lane's pixel, angle 0
   const int steps = COMB ? g.n_units : g.na;
   bool singles = false;
 #pragma unroll 1
@@ -1324,13 +1343,12 @@ __device__ __forceinline__ bool bp_pass(const ParDev& g, const float* __restrict
       }
     // rows of the patch's pixels at this lane's angle: their weights go to the
     // table, the first row and the row count to pk (first | rows << 16)
-    BpNode nd[NQ];
+    BpNode nd[BP_QUADS];
     bool single = false;
     int lo = 0x7fffffff, hi = -1;
 #pragma unroll
-    for (int h = 0; h < NQ; ++h) {
-      nd[h] = bp_node<COMB, PASS>(g, u < steps && ((active >> (4 * h + p)) & 1u), i, i2, x + (double)(2 * (h & 1)),
-                                  y + (double)(2 * (h >> 1)), single);
+    for (int h = 0; h < BP_QUADS; ++h) {
+      nd[h] = bp_node<COMB, PASS>(g, u < steps && ((active >> (4 * h + p)) & 1u), i, i2, x + (double)(2 * h), y, single);
       if (nd[h].jr >= 0) {
         lo = min(lo, nd[h].jr);
         hi = max(hi, nd[h].jr);
@@ -1345,37 +1363,50 @@ __device__ __forceinline__ bool bp_pass(const ParDev& g, const float* __restrict
     if (PASS != BP_ALL && __ballot(pk != 0) == 0ull) continue;
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int h = 0; h < NQ; ++h) {
+    for (int h = 0; h < BP_QUADS; ++h) {
       const int d = nd[h].jr >= 0 ? nd[h].jr - lo : 0;
 #pragma unroll
-      for (int k = 0; k < bp_max_rows(NQ); ++k) put[k * NQ + h] = d == k ? nd[h].w0 : (d == k - 1 ? nd[h].w1 : 0.0f);
+      for (int k = 0; k < BP_ROWS; ++k) put[k * BP_QUADS + h] = d == k ? nd[h].w0 : (d == k - 1 ? nd[h].w1 : 0.0f);
     }
     __builtin_amdgcn_wave_barrier();
     const int m = steps - u0 < 16 ? steps - u0 : 16;
+    if constexpr (CONTIG && !COMB) {
+      // the next angle's rows are loaded before this angle's products
+      BpRows<ZV> even, odd;
+      bp_load<ZV, CONTIG>(g, sino, rl_i(pk, 0), u0, ln, even);
 #pragma unroll 1
-    for (int a = 0; a < m; ++a) {
-      const int pkv = rl_i(pk, 4 * a);
-      const int ia = COMB ? rl_i(PASS == BP_TWO ? i2 : i, 4 * a) : u0 + a;
-      const int ib = COMB && PASS == BP_ALL ? rl_i(i2, 4 * a) : -1;
-      bp_rows_of<NQ, ZV, CONTIG, COMB && PASS == BP_ALL>(g, sino, pkv >> 16, pkv & 0xffff, ia, ib, ln, get + a * 32, acc);
+      for (int a = 0; a < m; a += 2) {
+        bp_load<ZV, CONTIG>(g, sino, a + 1 < m ? rl_i(pk, 4 * a + 4) : 0, u0 + a + 1, ln, odd);
+        bp_products<ZV>(even, get + a * 32, acc);
+        bp_load<ZV, CONTIG>(g, sino, a + 2 < m ? rl_i(pk, (4 * a + 8) & 63) : 0, u0 + a + 2, ln, even);
+        bp_products<ZV>(odd, get + a * 32 + 32, acc);
+      }
+    } else {
+#pragma unroll 1
+      for (int a = 0; a < m; ++a) {
+        const int pkv = rl_i(pk, 4 * a);
+        const int ia = COMB ? rl_i(PASS == BP_TWO ? i2 : i, 4 * a) : u0 + a;
+        const int ib = COMB && PASS == BP_ALL ? rl_i(i2, 4 * a) : -1;
+        bp_rows_of<ZV, CONTIG, COMB && PASS == BP_ALL>(g, sino, pkv >> 16, pkv & 0xffff, ia, ib, ln, get + a * 32, acc);
+      }
     }
   }
   return singles;
 }
 
 // a patch's sums
-template <int NQ, int ZV, bool CONTIG, bool COMB>
+template <int ZV, bool CONTIG, bool COMB>
 __device__ __forceinline__ void bp_patch(const ParDev& g, const float* __restrict__ sino, int r0, int c0,
                                          unsigned active, const ZLane<ZV, CONTIG>& ln, int lane,
-                                         mf4 (&acc)[NQ][ZV]) {
+                                         float2* tab, mf4 (&acc)[BP_QUADS][ZV]) {
 #pragma unroll
-  for (int h = 0; h < NQ; ++h)
+  for (int h = 0; h < BP_QUADS; ++h)
 #pragma unroll
     for (int q = 0; q < ZV; ++q) acc[h][q] = mf4{0.f, 0.f, 0.f, 0.f};
   if (active) {
-    if (bp_pass<NQ, ZV, CONTIG, COMB, BP_ALL>(g, sino, r0, c0, active, ln, lane, acc)) {
-      bp_pass<NQ, ZV, CONTIG, true, BP_ONE>(g, sino, r0, c0, active, ln, lane, acc);
-      bp_pass<NQ, ZV, CONTIG, true, BP_TWO>(g, sino, r0, c0, active, ln, lane, acc);
+    if (bp_pass<ZV, CONTIG, COMB, BP_ALL>(g, sino, r0, c0, active, ln, lane, tab, acc)) {
+      bp_pass<ZV, CONTIG, true, BP_ONE>(g, sino, r0, c0, active, ln, lane, tab, acc);
+      bp_pass<ZV, CONTIG, true, BP_TWO>(g, sino, r0, c0, active, ln, lane, tab, acc);
     }
   }
 }
@@ -1435,54 +1466,55 @@ __device__ __forceinline__ bool bp_tile_quad(long long q, const ParDev& g, int& 
   return qr < bp_nquad(g) && qc < bp_nquad(g);
 }
 
-// back projection: patches (2 or 4 rows x 4 columns) in tiles of bp_tile quads'
-// edge
-__host__ __device__ inline int bp_patch_rows(const ParDev& g, int nq) {
-  return (g.n + nq - 1) / nq;
+// Back projection: the plan lists its patches of 2 rows x 4 columns (bp_list, row
+// << 16 | column) along a Z curve, those with a column inside the clip circle
+// first.  The wavefronts of a launch are the listed patches x z chunks, chunk
+// slowest, in two groups: the active ones in equal contiguous shares per XCD
+// (a compact part of the volume, whose rows its L2 holds), then the ones that
+// only store zeros.  In tiles row by row without regard to the circle, the XCDs
+// of the middle rows had a quarter more active patches than the mean (201 x 201 x
+// 77 x 240 angles: 202 us against 154).
+__host__ __device__ inline long long bp_active(const ParDev& g, int clipc) {
+  return clipc ? g.bp_act : g.bp_all;
 }
-__host__ __device__ inline int bp_patch_cols(const ParDev& g) { return (g.n + 3) / 4; }
-__host__ __device__ inline int bp_patch_tr(const ParDev& g, int nq) {
-  const int t = 2 * g.bp_tile > nq ? 2 * g.bp_tile / nq : 1;
-  return t < bp_patch_rows(g, nq) ? t : bp_patch_rows(g, nq);
+// blocks of BP_WAVES wavefronts: few, so that the compute units' shares differ
+// by little where all wavefronts are resident at once
+constexpr int BP_WAVES = 2;
+__host__ __device__ inline long long bp_blocks(const ParDev& g, int clipc, int chunks, bool active) {
+  const long long act = bp_active(g, clipc), w = (active ? act : g.bp_all - act) * chunks;
+  return (w + BP_WAVES - 1) / BP_WAVES;
 }
-__host__ __device__ inline int bp_patch_tc(const ParDev& g) {
-  const int t = g.bp_tile > 1 ? g.bp_tile / 2 : 1;
-  return t < bp_patch_cols(g) ? t : bp_patch_cols(g);
-}
-__host__ __device__ inline long long bp_patches(const ParDev& g, int nq) {
-  const int tr = bp_patch_tr(g, nq), tc = bp_patch_tc(g);
-  return (long long)((bp_patch_rows(g, nq) + tr - 1) / tr) * ((bp_patch_cols(g) + tc - 1) / tc) * tr * tc;
-}
-// wave -> patch and z chunk (chunk slowest); false for padding
-template <int NQ>
-__device__ __forceinline__ bool bp_wave_patch(long long wave, int chunks, const ParDev& g, int& r0, int& c0,
+// wavefront w of the list -> patch and z chunk; false past its end
+__device__ __forceinline__ bool bp_wave_patch(long long w, int chunks, const ParDev& g, int clipc, int& r0, int& c0,
                                               int& chunk) {
-  const long long patches = bp_patches(g, NQ);
-  if (wave >= patches * chunks) return false;
-  chunk = (int)(wave / patches);
-  const long long q = wave % patches;
-  const int tr = bp_patch_tr(g, NQ), tc = bp_patch_tc(g), nc = (bp_patch_cols(g) + tc - 1) / tc;
-  const int tile = (int)(q / (tr * tc)), within = (int)(q % (tr * tc));
-  // four consecutive wavefronts (a block) take 2 x 2 patches: they read fewer
-  // distinct rows per angle than four in a row
-  int wr = within / tc, wc = within % tc;
-  if (tr % 2 == 0 && tc % 2 == 0) {
-    const int b = within >> 2, k = within & 3, bc = tc >> 1;
-    wr = 2 * (b / bc) + (k >> 1);
-    wc = 2 * (b % bc) + (k & 1);
+  const long long all = g.bp_all, act = bp_active(g, clipc);
+  long long first = 0, count = act;
+  if (w >= act * chunks) {
+    if (w >= all * chunks) return false;
+    w -= act * chunks;
+    first = act;
+    count = all - act;
   }
-  const int pr = tile / nc * tr + wr, pc = tile % nc * tc + wc;
-  r0 = NQ * pr;
-  c0 = 4 * pc;
-  return pr < bp_patch_rows(g, NQ) && pc < bp_patch_cols(g);
+  chunk = (int)(w / count);
+  const int at = g.bp_list[first + w % count];
+  r0 = 2 * (at >> 16);
+  c0 = 4 * (at & 0xffff);
+  return true;
+}
+// the calling wavefront's place in the list; -1: none
+__device__ __forceinline__ long long bp_wave(const ParDev& g, int clipc, int chunks) {
+  const long long nb = bp_blocks(g, clipc, chunks, true), act = bp_active(g, clipc) * chunks;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (blockIdx.x >= nb) return act + (blockIdx.x - nb) * BP_WAVES + wv;
+  const long long w = (long long)xcd_remap(blockIdx.x, (unsigned)nb) * BP_WAVES + wv;
+  return w < act ? w : -1;
 }
 // bit 4 h + p: pixel p of quad h is inside the grid and, of those, computed
-template <int NQ>
 __device__ __forceinline__ void bp_patch_masks(const ParDev& g, int r0, int c0, int clipc, unsigned& inrange,
                                                unsigned& active) {
   inrange = active = 0u;
 #pragma unroll
-  for (int b = 0; b < 4 * NQ; ++b) {
+  for (int b = 0; b < 4 * BP_QUADS; ++b) {
     const int row = r0 + bp_bit_row(b), col = c0 + bp_bit_col(b);
     if (row < g.n && col < g.n) {
       inrange |= 1u << b;
@@ -1494,19 +1526,19 @@ __device__ __forceinline__ void bp_patch_masks(const ParDev& g, int r0, int c0, 
 // row that another column of its quad skips may have held an infinity, two
 // opposite rows may add past the largest number) is summed again as bp_voxel
 // does it
-template <int NQ, int ZV, bool CONTIG>
+template <int ZV, bool CONTIG>
 __device__ __forceinline__ void bp_patch_store(const ParDev& g, const float* __restrict__ sino, float* vol, int r0,
                                                int c0, unsigned inrange, unsigned active,
-                                               const ZLane<ZV, CONTIG>& ln, const mf4 (&acc)[NQ][ZV]) {
+                                               const ZLane<ZV, CONTIG>& ln, const mf4 (&acc)[BP_QUADS][ZV]) {
   bool bad = false;
 #pragma unroll
-  for (int h = 0; h < NQ; ++h)
+  for (int h = 0; h < BP_QUADS; ++h)
 #pragma unroll
     for (int q = 0; q < ZV; ++q)
 #pragma unroll
       for (int p = 0; p < 4; ++p) bad |= !(fabsf(acc[h][q][p]) <= 3.4028234664e38f);
 #pragma unroll
-  for (int b = 0; b < 4 * NQ; ++b) {
+  for (int b = 0; b < 4 * BP_QUADS; ++b) {
     if (!((inrange >> b) & 1u)) continue;
     const int h = b >> 2, p = b & 3;
     float* outp = vol + ((size_t)(r0 + bp_bit_row(b)) * g.n + c0 + bp_bit_col(b)) * g.nz;
@@ -1522,7 +1554,7 @@ __device__ __forceinline__ void bp_patch_store(const ParDev& g, const float* __r
   }
   if (__ballot(bad) == 0ull) return;
 #pragma unroll 1
-  for (int b = 0; b < 4 * NQ; ++b) {
+  for (int b = 0; b < 4 * BP_QUADS; ++b) {
     if (!((active >> b) & 1u)) continue;
     const int pix = (r0 + bp_bit_row(b)) * g.n + c0 + bp_bit_col(b);
 #pragma unroll 1
@@ -1537,7 +1569,7 @@ __device__ __forceinline__ void bp_patch_store(const ParDev& g, const float* __r
 // how a problem's back projection lays out its slices: slices per lane (0: not
 // on these kernels), 16-byte loads of four, opposite angles combined
 struct BpLayout {
-  int zv = 0, nq = 2;
+  int zv = 0;
   bool contig = false, comb = false;
   int chunks = 0;
 };
@@ -1767,16 +1799,16 @@ struct UpdateOut {
   }
 };
 
-// calls f(NQ, ZV, CONTIG, COMB) with the layout's compile-time constants
+// calls f(ZV, CONTIG, COMB) with the layout's compile-time constants
 template <class F>
 void bp_dispatch(const BpLayout& l, F&& f) {
   using std::integral_constant;
   auto with = [&](auto comb) {
-    if (l.contig) f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, std::true_type{}, comb);
-    else if (l.zv == 4) f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, std::false_type{}, comb);
-    else if (l.zv == 3) f(integral_constant<int, 2>{}, integral_constant<int, 3>{}, std::false_type{}, comb);
-    else if (l.zv == 2) f(integral_constant<int, 2>{}, integral_constant<int, 2>{}, std::false_type{}, comb);
-    else f(integral_constant<int, 2>{}, integral_constant<int, 1>{}, std::false_type{}, comb);
+    if (l.contig) f(integral_constant<int, 4>{}, std::true_type{}, comb);
+    else if (l.zv == 4) f(integral_constant<int, 4>{}, std::false_type{}, comb);
+    else if (l.zv == 3) f(integral_constant<int, 3>{}, std::false_type{}, comb);
+    else if (l.zv == 2) f(integral_constant<int, 2>{}, std::false_type{}, comb);
+    else f(integral_constant<int, 1>{}, std::false_type{}, comb);
   };
   if (l.comb) with(std::true_type{});
   else with(std::false_type{});

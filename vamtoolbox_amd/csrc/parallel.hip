@@ -5,6 +5,7 @@
 // consecutive z values; every output element is written by exactly one lane
 // after a fixed-order accumulation (no atomics, bitwise deterministic).
 #include <algorithm>
+#include <cstring>
 
 #include "par_core.h"
 
@@ -222,19 +223,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void p
 // which makes the compiler keep the products' accumulators in vector
 // registers; left in accumulation registers it copied all 8 ZV of them in and
 // out for every angle.
-template <int NQ, int ZV, bool CONTIG, bool COMB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void par_bp_patch_kernel(
+template <int ZV, bool CONTIG, bool COMB>
+__global__ __launch_bounds__(64 * BP_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void par_bp_patch_kernel(
     ParDev g, const float* __restrict__ sino, float* vol, int clipc, int chunks) {
+  __shared__ float2 tab[BP_WAVES][BP_TABLE];
   const int lane = threadIdx.x & 63;
-  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long wave = bp_wave(g, clipc, chunks);
   int r0, c0, chunk;
-  if (!bp_wave_patch<NQ>(wave, chunks, g, r0, c0, chunk)) return;
+  if (wave < 0 || !bp_wave_patch(wave, chunks, g, clipc, r0, c0, chunk)) return;
   const ZLane<ZV, CONTIG> ln(chunk, lane, g.nz);
   unsigned inrange, active;
-  bp_patch_masks<NQ>(g, r0, c0, clipc, inrange, active);
-  mf4 acc[NQ][ZV];
-  bp_patch<NQ, ZV, CONTIG, COMB>(g, sino, r0, c0, active, ln, lane, acc);
-  bp_patch_store<NQ, ZV, CONTIG>(g, sino, vol, r0, c0, inrange, active, ln, acc);
+  bp_patch_masks(g, r0, c0, clipc, inrange, active);
+  mf4 acc[BP_QUADS][ZV];
+  bp_patch<ZV, CONTIG, COMB>(g, sino, r0, c0, active, ln, lane,
+                                 tab[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))], acc);
+  bp_patch_store<ZV, CONTIG>(g, sino, vol, r0, c0, inrange, active, ln, acc);
 }
 
 __global__ __launch_bounds__(256) void par_fp_incl_kernel(ParDev g, const float* __restrict__ vol,
@@ -433,7 +436,6 @@ BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits) {
       slots = c * zv;
     }
   }
-  if (l.zv == 4) l.nq = 4;
   l.contig = l.zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0;
   l.comb = g.mu == 0.0 && g.pair_ok;
   return l;
@@ -540,6 +542,32 @@ void vamx::par_pair_units(const std::vector<double>& cs, int na, int n, int c, d
   }
 }
 
+// the patches of bp_wave_patch, and their counts
+static std::vector<int> bp_patch_list(ParDev& g, const uint8_t* outside) {
+  const int n = g.n, e = (n + 3) / 4;   // pairs of patches (4 x 4 columns) per edge
+  int side = 1;
+  while (side < e) side *= 2;
+  std::vector<int> list, clipped;
+  for (long long m = 0; m < (long long)side * side; ++m) {
+    int row = 0, col = 0;
+    for (int b = 0; (1ll << (2 * b)) < (long long)side * side; ++b) {
+      col |= (int)((m >> (2 * b)) & 1) << b;
+      row |= (int)((m >> (2 * b + 1)) & 1) << b;
+    }
+    if (row >= e || col >= e) continue;
+    for (int pr = 2 * row; pr < 2 * row + 2 && 2 * pr < n; ++pr) {
+      bool active = false;
+      for (int y = 2 * pr; y < std::min(n, 2 * pr + 2); ++y)
+        for (int x = 4 * col; x < std::min(n, 4 * col + 4); ++x) active |= !outside[(size_t)y * n + x];
+      (active ? list : clipped).push_back(pr << 16 | col);
+    }
+  }
+  g.bp_act = (int)list.size();
+  list.insert(list.end(), clipped.begin(), clipped.end());
+  g.bp_all = (int)list.size();
+  return list;
+}
+
 extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) {
   if (!geom || !out_plan) return set_error(VAMX_ERR_ARG, "vamx_par_create: null argument");
   *out_plan = nullptr;
@@ -621,15 +649,22 @@ extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) 
   g.bp_tile = 8;
   g.bp_zv = 4;
   p->minmax_parts = 256;
+  // the clip mask and, behind it, the back projection's patch list
+  std::vector<uint8_t> mask(((size_t)n * n + 3) / 4 * 4);
+  std::memcpy(mask.data(), geom->outside_mask, (size_t)n * n);
+  const std::vector<int> list = bp_patch_list(g, geom->outside_mask);
+  const size_t mask_bytes = mask.size(), list_bytes = list.size() * sizeof(int);
   hipError_t e = hipSuccess;
   e = hipMalloc((void**)&p->d_mats, mats.size() * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&p->d_cs, cs.size() * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&p->d_outside, (size_t)n * n);
+  if (e == hipSuccess) e = hipMalloc((void**)&p->d_outside, mask_bytes + list_bytes);
   if (e == hipSuccess) e = hipMalloc((void**)&p->d_minmax_part, (size_t)p->minmax_parts * 2 * nz * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&p->d_minmax, ((size_t)2 * nz + 4) * sizeof(float));
   if (e == hipSuccess) e = hipMemcpy(p->d_mats, mats.data(), mats.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(p->d_cs, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->d_outside, geom->outside_mask, (size_t)n * n, hipMemcpyHostToDevice);
+  mask.resize(mask_bytes + list_bytes);
+  std::memcpy(mask.data() + mask_bytes, list.data(), list_bytes);
+  if (e == hipSuccess) e = hipMemcpy(p->d_outside, mask.data(), mask.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess && !units.empty()) {
     e = hipMalloc((void**)&p->d_units, units.size() * sizeof(int));
     if (e == hipSuccess) e = hipMemcpy(p->d_units, units.data(), units.size() * sizeof(int), hipMemcpyHostToDevice);
@@ -642,6 +677,7 @@ extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) 
   g.cs = p->d_cs;
   g.units = p->d_units;
   g.outside = p->d_outside;
+  g.bp_list = reinterpret_cast<const int*>(p->d_outside + mask_bytes);
   g.occ = nullptr;
   g.occ_active = nullptr;
   if (geom->occlusion) {
@@ -783,11 +819,12 @@ int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t
     return VAMX_OK;
   }
   if (const BpLayout l = bp_layout(p, (uintptr_t)sino | (uintptr_t)vol); l.zv) {
-    const dim3 grid(blocks_for(bp_patches(g, l.nq) * l.chunks * 64, 256)), block(256);
-    bp_dispatch(l, [&](auto nq, auto zv, auto contig, auto comb) {
-      hipLaunchKernelGGL((par_bp_patch_kernel<decltype(nq)::value, decltype(zv)::value, decltype(contig)::value,
-                                              decltype(comb)::value>),
-                         grid, block, 0, s, g, sino, vol, clipc ? 1 : 0, l.chunks);
+    const int cc = clipc ? 1 : 0;
+    const dim3 block(64 * BP_WAVES);
+    const dim3 grid((unsigned)(bp_blocks(g, cc, l.chunks, true) + bp_blocks(g, cc, l.chunks, false)));
+    bp_dispatch(l, [&](auto zv, auto contig, auto comb) {
+      hipLaunchKernelGGL((par_bp_patch_kernel<decltype(zv)::value, decltype(contig)::value, decltype(comb)::value>),
+                         grid, block, 0, s, g, sino, vol, cc, l.chunks);
     });
     VAMX_HIP(hipGetLastError());
     return VAMX_OK;

@@ -33,7 +33,11 @@ struct ParDev {
   // work order of the wavefront-uniform kernels (set by vamx_par_set_tuning)
   int fp_ta, fp_tk, fp_zv;   // forward: tile of fp_ta angles x fp_tk rays, z values per lane
   int fp_reuse;              // forward: keep the previous sample's taps in registers
-  int bp_tile, bp_zv;        // back projection: bp_tile x bp_tile voxel columns, z values per lane
+  int bp_tile, bp_zv;        // A^T: tile of bp_tile x bp_tile quads of voxel columns; A, A^T: z values per lane
+  // A: the patches of 2 x 4 voxel columns, patch row << 16 | patch column, those
+  // inside the clip circle first, and their counts
+  const int* bp_list;
+  int bp_act, bp_all;
   int z_split;               // allow lanes holding z and z + 64 where one z per lane is the choice
   // Opposite-angle pairing of the forward projection.  Ray k at angle a and
   // ray 2c + D - k at angle a + 180 deg (D = 2 det_offset, an integer) sample
