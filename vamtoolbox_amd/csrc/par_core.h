@@ -941,27 +941,32 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
   }
   const size_t nzs = (size_t)g.nz;
   const size_t step_c = nzs, step_r = (size_t)n * nzs;
-  // taps are buffer loads from a per-sample descriptor at the cell's corner
-  // voxel column: lane byte offset 4z, scalar byte offsets of the other
-  // three corners; the descriptor spans the two rows of the cell
+  // taps are buffer loads: lane byte offset 4z, scalar byte offset of the voxel
+  // column from the first row that the 64 samples reach (their rows span at most
+  // 66; where 66 rows pass 32 bits, from the sample's own cell)
   const uint32_t zb = 4u * (uint32_t)z, zb2 = 4u * (uint32_t)z2;
-  const uint32_t oc = (uint32_t)(4 * step_c), orr = (uint32_t)(4 * step_r), orc = oc + orr;
-  const uint32_t span = orc + oc;
+  const uint32_t oc = (uint32_t)(4 * step_c), orr = (uint32_t)(4 * step_r);
+  const bool big = 66ull * orr + 4ull * nzs >= 0xffffffffull;
   V acc = vzero<ZV>(), accp = vzero<ZV>();
   // Tap registers by absolute parity: T<a><b> holds the tap of the current
   // cell whose volume row is even (a = 0) or odd (a = 1) and whose column is
   // even (b = 0) or odd (b = 1).  When the cell moves by one row or column
   // the taps it keeps stay where they are and the new ones replace exactly
   // the ones that left (same parity), so the window never shifts between
-  // registers; each lane delivers its weights in the same parity order.
+  // registers.  Each lane delivers, in that parity order, its sample's weights,
+  // the taps' byte offsets and which of the four the sample before it lacked:
+  // a sample tests four bits and moves one offset from its lane per new tap.
+  // (The scalar unit, one instruction per cycle for a CU's four SIMDs, was what
+  // bound the loop when it found the case of 36 by comparing cell numbers and
+  // built a descriptor per sample: 40 scalar instructions and branches.)
   V T00 = vzero<ZV>(), T01 = vzero<ZV>(), T10 = vzero<ZV>(), T11 = vzero<ZV>();
   const FpSlot sl = fp_lds_slot();
-  int prev = -2 * n - 2;   // no taps held
+  int last = -1;   // cell of the sample before the 64 (-1: none)
   const int r_end = PAIR ? (2 * g.c + 1 > n ? 2 * g.c + 1 : n) : n;
   const int r2_lo = 2 * g.c - n + 1;   // partner's first sample (PAIR)
   for (int r0 = 0; r0 < r_end; r0 += 64) {
     const int r = r0 + lane;
-    int base = 0;
+    int br = 0, bc = 0;
     float w00 = 0.f, w01 = 0.f, w10 = 0.f, w11 = 0.f, aw = 0.f;
     float aw2 = 0.f;
     bool valid = false, anyin = false;
@@ -970,11 +975,9 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
       const double col = (a0 + M01 * rr) + M02;
       const double row = (a1 + M11 * rr) + M12;
       if (row > -1.0 && row < (double)n && col > -1.0 && col < (double)n) {
-        int br, bc;
         double r0w, r1w, c0w, c1w;
         axis_slots(row, n, br, r0w, r1w);
         axis_slots(col, n, bc, c0w, c1w);
-        base = (br * n + bc) | ((br & 1) << 29) | ((bc & 1) << 28);   // cell and its row / column parity
         anyin = (r0w > 0.0 || r1w > 0.0) && (c0w > 0.0 || c1w > 0.0);
         if (!PAIR || r < n) aw = abs_weight(g, t, (double)(r - g.c));
         if constexpr (PAIR) {
@@ -997,6 +1000,25 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
       }
     }
     unsigned long long m = __ballot(valid);
+    if (!m) {
+      last = -1;
+      continue;
+    }
+    // taps that the sample before (in the lane before) does not hold
+    const int cell = valid ? (br << 14) | bc : -1;   // n < 2^14
+    const int up = __shfl_up(cell, 1), before = lane == 0 ? last : up;
+    last = rl_i(cell, 63);
+    const int dr = br - (before >> 14), dc = bc - (before & 0x3fff);
+    int lacks = 15;   // bit 2 a + b: the tap of row parity a, column parity b
+    if (REUSE && before >= 0 && dr >= -1 && dr <= 1 && dc >= -1 && dc <= 1)
+      lacks = (dr ? 3 << (2 * ((br + (dr > 0)) & 1)) : 0) | (dc ? 5 << ((bc + (dc > 0)) & 1) : 0);
+    const int row_lo = min(rl_i(br, __builtin_ctzll(m)), rl_i(br, 63 - __builtin_clzll(m)));
+    const uint32_t at = big ? 0u : (uint32_t)(br - row_lo) * orr + (uint32_t)bc * oc;
+    // the tap of parity (a, b) is the corner (a ^ row parity, b ^ column parity)
+    const uint32_t re = at + ((br & 1) ? orr : 0u), ro = at + ((br & 1) ? 0u : orr);
+    const uint32_t ce = (bc & 1) ? oc : 0u, co = (bc & 1) ? 0u : oc;
+    const int a00 = (int)(re + ce), a01 = (int)(re + co), a10 = (int)(ro + ce), a11 = (int)(ro + co);
+    __amdgpu_buffer_rsrc_t rs = buf_rsrc(vol + (size_t)row_lo * step_r, 0xffffffffu);
     // the wave's previous reads of the buffers precede these writes (LDS
     // operations of a wavefront complete in order)
     __builtin_amdgcn_wave_barrier();
@@ -1006,66 +1028,17 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
     while (m) {
       const int j = __builtin_ctzll(m);
       m &= m - 1;
-      const int bp = rl_i(base, j);
-      const int b = bp & 0x0fffffff, par = (bp >> 28) & 3;   // par: row parity << 1 | column parity
       const float4 Q = sl.w[j];
       const float q00 = Q.x, q01 = Q.y, q10 = Q.z, q11 = Q.w;
-      const __amdgpu_buffer_rsrc_t rs = buf_rsrc(vol + (size_t)b * nzs, span);
-      // C00..C11 name the registers of the cell's corners (0,0) .. (1,1) for
-      // this parity; each arm loads the corners the previous cell lacked
-#define VAMX_TAP_ARMS(C00, C01, C10, C11, P)                                       \
-  if (d == 1) {             /* one column right: the right column is new */      \
-    asm volatile("; vamx fp " #P " d1");                                        \
-    C01 = tload<ZV, SPLIT>(rs, zb, zb2, oc);                                                 \
-    C11 = tload<ZV, SPLIT>(rs, zb, zb2, orc);                                                \
-  } else if (d == n) {      /* one row down: the bottom row is new */           \
-    asm volatile("; vamx fp " #P " dn");                                        \
-    C10 = tload<ZV, SPLIT>(rs, zb, zb2, orr);                                                \
-    C11 = tload<ZV, SPLIT>(rs, zb, zb2, orc);                                                \
-  } else if (d == -1) {                                                         \
-    asm volatile("; vamx fp " #P " dm1");                                       \
-    C00 = tload<ZV, SPLIT>(rs, zb, zb2, 0);                                                  \
-    C10 = tload<ZV, SPLIT>(rs, zb, zb2, orr);                                                \
-  } else if (d == -n) {                                                         \
-    asm volatile("; vamx fp " #P " dmn");                                       \
-    C00 = tload<ZV, SPLIT>(rs, zb, zb2, 0);                                                  \
-    C01 = tload<ZV, SPLIT>(rs, zb, zb2, oc);                                                 \
-  } else if (d == n + 1) {  /* diagonal steps keep one tap */                   \
-    asm volatile("; vamx fp " #P " dnp1");                                      \
-    C01 = tload<ZV, SPLIT>(rs, zb, zb2, oc);                                                 \
-    C10 = tload<ZV, SPLIT>(rs, zb, zb2, orr);                                                \
-    C11 = tload<ZV, SPLIT>(rs, zb, zb2, orc);                                                \
-  } else if (d == n - 1) {                                                      \
-    asm volatile("; vamx fp " #P " dnm1");                                      \
-    C00 = tload<ZV, SPLIT>(rs, zb, zb2, 0);                                                  \
-    C10 = tload<ZV, SPLIT>(rs, zb, zb2, orr);                                                \
-    C11 = tload<ZV, SPLIT>(rs, zb, zb2, orc);                                                \
-  } else if (d == -n + 1) {                                                     \
-    asm volatile("; vamx fp " #P " dmnp1");                                     \
-    C00 = tload<ZV, SPLIT>(rs, zb, zb2, 0);                                                  \
-    C01 = tload<ZV, SPLIT>(rs, zb, zb2, oc);                                                 \
-    C11 = tload<ZV, SPLIT>(rs, zb, zb2, orc);                                                \
-  } else if (d == -n - 1) {                                                     \
-    asm volatile("; vamx fp " #P " dmnm1");                                     \
-    C00 = tload<ZV, SPLIT>(rs, zb, zb2, 0);                                                  \
-    C01 = tload<ZV, SPLIT>(rs, zb, zb2, oc);                                                 \
-    C10 = tload<ZV, SPLIT>(rs, zb, zb2, orr);                                                \
-  } else if (d != 0) {                                                          \
-    asm volatile("; vamx fp " #P " full");                                      \
-    C00 = tload<ZV, SPLIT>(rs, zb, zb2, 0);                                                  \
-    C01 = tload<ZV, SPLIT>(rs, zb, zb2, oc);                                                 \
-    C10 = tload<ZV, SPLIT>(rs, zb, zb2, orr);                                                \
-    C11 = tload<ZV, SPLIT>(rs, zb, zb2, orc);                                                \
-  }
-      const int d = REUSE ? b - prev : 2 * n + 2;   // without reuse every sample reloads
-      prev = b;
-      switch (par) {
-        case 0: { VAMX_TAP_ARMS(T00, T01, T10, T11, 0) break; }
-        case 1: { VAMX_TAP_ARMS(T01, T00, T11, T10, 1) break; }
-        case 2: { VAMX_TAP_ARMS(T10, T11, T00, T01, 2) break; }
-        default: { VAMX_TAP_ARMS(T11, T10, T01, T00, 3) break; }
+      const int load = rl_i(lacks, j);
+      if (big) {
+        const int at_j = rl_i(cell, j);
+        rs = buf_rsrc(vol + (size_t)(at_j >> 14) * step_r + (size_t)(at_j & 0x3fff) * step_c, 0xffffffffu);
       }
-#undef VAMX_TAP_ARMS
+      if (load & 1) T00 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a00, j));
+      if (load & 2) T01 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a01, j));
+      if (load & 4) T10 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a10, j));
+      if (load & 8) T11 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a11, j));
       if constexpr (CLIP) {
         V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
         v = vclamp(v, lo, hi);  // every enumerated sample has an in-range tap of positive weight
