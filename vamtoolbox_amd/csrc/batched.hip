@@ -35,7 +35,7 @@ struct BatchItem {
   int clip;              // forward: warp clip; backward: circle clip
   int wave;              // 1: wavefront-uniform kernels
   int pair;              // forward, wave mode: opposite-angle pairs (the plan's paired work order)
-  int split;             // forward, wave mode, zv 2: lanes hold z and z + 64
+  int split;             // forward, wave mode: lanes hold slices 64 apart
   int contig, comb, chunks;   // backward, wave mode: BpLayout
 };
 
@@ -54,14 +54,13 @@ template <int ZV, bool SPLIT>
 __device__ __forceinline__ void batch_fp_wave(const BatchItem& it, const float* in, float* out, long long w,
                                               int lane) {
   const ParDev& g = it.g;
-  int k, i, z, zl, zl2;
-  if (!fp_wave_item<ZV, SPLIT>(w, g, lane, k, i, z)) return;
-  wave_zload<ZV, SPLIT>(z, g.nz, zl, zl2);
-  const bool clip_on = it.clip && wave_clip_active<ZV, SPLIT>(it.minmax, g.nz, zl, zl2);
-  const typename VecT<ZV>::T acc =
-      clip_on ? fp_ray_wave<ZV, true, true, false, SPLIT>(g, in, it.minmax, k, i, zl, lane, nullptr, zl2)
-              : fp_ray_wave<ZV, false, true, false, SPLIT>(g, in, it.minmax, k, i, zl, lane, nullptr, zl2);
-  wave_zstore<ZV, SPLIT>(out + ((size_t)k * g.na + i) * g.nz, z, g.nz, acc);
+  int k, i, zc;
+  if (!fp_wave_item<ZV>(w, g, k, i, zc)) return;
+  const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
+  const typename VecT<ZV>::T acc = it.clip && wave_clip_active(it.minmax, g.nz, ln)
+                                       ? fp_ray_wave<true, true, false>(g, in, it.minmax, k, i, ln, lane)
+                                       : fp_ray_wave<false, true, false>(g, in, it.minmax, k, i, ln, lane);
+  ln.store(out + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
 }
 
 // paired forward: ray (k, i) and its opposite ray from one pass over the
@@ -72,27 +71,22 @@ __device__ __forceinline__ void batch_fp_pair(const BatchItem& it, const float* 
                                               int lane) {
   using V = typename VecT<ZV>::T;
   const ParDev& g = it.g;
-  const PairItem pi = fp_pair_item<ZV, SPLIT>(w, g, lane);
+  const PairItem pi = fp_pair_item<ZV>(w, g);
   if (!pi.ok) return;
-  const int z = pi.z;
-  int zl, zl2;
-  wave_zload<ZV, SPLIT>(z, g.nz, zl, zl2);
-  const bool clip_on = it.clip && wave_clip_active<ZV, SPLIT>(it.minmax, g.nz, zl, zl2);
-  if (clip_on) {
+  const FpLane<ZV, SPLIT> ln(pi.zc, lane, g.nz);
+  if (it.clip && wave_clip_active(it.minmax, g.nz, ln)) {
     for (int h = 0; h < (pi.k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? pi.k2 : pi.k, ih = h ? pi.i2 : pi.i;
-      const V acc = fp_ray_wave<ZV, true, true, false, SPLIT>(g, in, it.minmax, kh, ih, zl, lane, nullptr, zl2);
-      wave_zstore<ZV, SPLIT>(out + ((size_t)kh * g.na + ih) * g.nz, z, g.nz, acc);
+      ln.store(out + ((size_t)kh * g.na + ih) * g.nz, g.nz,
+               fp_ray_wave<true, true, false>(g, in, it.minmax, kh, ih, ln, lane));
     }
     return;
   }
   V acc, acc2 = vzero<ZV>();
-  if (pi.k2 >= 0)
-    acc = fp_ray_wave<ZV, false, true, true, SPLIT>(g, in, it.minmax, pi.k, pi.i, zl, lane, &acc2, zl2);
-  else
-    acc = fp_ray_wave<ZV, false, true, false, SPLIT>(g, in, it.minmax, pi.k, pi.i, zl, lane, nullptr, zl2);
-  wave_zstore<ZV, SPLIT>(out + ((size_t)pi.k * g.na + pi.i) * g.nz, z, g.nz, acc);
-  if (pi.k2 >= 0) wave_zstore<ZV, SPLIT>(out + ((size_t)pi.k2 * g.na + pi.i2) * g.nz, z, g.nz, acc2);
+  if (pi.k2 >= 0) acc = fp_ray_wave<false, true, true>(g, in, it.minmax, pi.k, pi.i, ln, lane, &acc2);
+  else acc = fp_ray_wave<false, true, false>(g, in, it.minmax, pi.k, pi.i, ln, lane);
+  ln.store(out + ((size_t)pi.k * g.na + pi.i) * g.nz, g.nz, acc);
+  if (pi.k2 >= 0) ln.store(out + ((size_t)pi.k2 * g.na + pi.i2) * g.nz, g.nz, acc2);
 }
 
 template <int ZV, bool CONTIG, bool COMB>
@@ -142,7 +136,7 @@ __device__ __forceinline__ void batch_lane_item(const BatchItem& it, const float
 }
 
 template <bool FORWARD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void batch_kernel(const BatchItem* __restrict__ items, int nitems,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORWARD ? 5 : 4))) void batch_kernel(const BatchItem* __restrict__ items, int nitems,
                                                     long long ntiles, unsigned long long* counter,
                                                     BatchPtrs ptrs) {
   __shared__ long long tile_sh;
@@ -175,12 +169,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
       const long long w = (tile - it.tile_begin) * 4 + slot;
       if (w < it.items) {
         if (FORWARD && it.pair) {
-          if (it.split) batch_fp_pair<2, true>(it, in, out, w, lane);
+          if (it.split && it.zv == 4) batch_fp_pair<4, true>(it, in, out, w, lane);
+          else if (it.split && it.zv == 3) batch_fp_pair<3, true>(it, in, out, w, lane);
+          else if (it.split) batch_fp_pair<2, true>(it, in, out, w, lane);
           else if (it.zv == 4) batch_fp_pair<4, false>(it, in, out, w, lane);
           else if (it.zv == 2) batch_fp_pair<2, false>(it, in, out, w, lane);
           else batch_fp_pair<1, false>(it, in, out, w, lane);
         } else if (FORWARD) {
-          if (it.split) batch_fp_wave<2, true>(it, in, out, w, lane);
+          if (it.split && it.zv == 4) batch_fp_wave<4, true>(it, in, out, w, lane);
+          else if (it.split && it.zv == 3) batch_fp_wave<3, true>(it, in, out, w, lane);
+          else if (it.split) batch_fp_wave<2, true>(it, in, out, w, lane);
           else if (it.zv == 4) batch_fp_wave<4, false>(it, in, out, w, lane);
           else if (it.zv == 2) batch_fp_wave<2, false>(it, in, out, w, lane);
           else batch_fp_wave<1, false>(it, in, out, w, lane);
@@ -299,17 +297,15 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
   return VAMX_OK;
 }
 
-// kernel path of problem i for these buffers: forward, wave z width (1, 2, 4;
-// 3 = z and z + 64); backward, slices per lane (+ 8: contiguous, + 16: opposite
-// angles combined); -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
+// kernel path of problem i for these buffers: slices per lane (forward + 8: 64
+// apart; backward + 8: contiguous, + 16: opposite angles combined); -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
 // kOwnLaunch for plans whose kernels the persistent launch does not hold
 constexpr int kOwnLaunch = 0;
 int problem_path(vamx_plan* p, const float* in, float* out, bool forward) {
   if (incl_wave_ok(p) || thin_ok(p)) return kOwnLaunch;
   if (forward) {
-    const int wz = par_fp_wave_zv(p, in, out);
-    if (par_wave_split(p, wz)) return 3;
-    if (wz) return wz;
+    const FpLayout l = fp_layout(p, (uintptr_t)in | (uintptr_t)out);
+    if (l.zv) return l.zv | (l.split ? 8 : 0);
   } else {
     const BpLayout l = bp_layout(p, (uintptr_t)in | (uintptr_t)out);
     if (l.zv) return l.zv | (l.contig ? 8 : 0) | (l.comb ? 16 : 0);
@@ -354,12 +350,11 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
       it.chunks = wave_zchunks(it.g.nz, it.zv);
       it.items = (long long)it.g.bp_all * it.chunks;
     } else if (path > 0) {
-      const int wz = path == 3 ? 2 : path;
       it.wave = 1;
-      it.zv = wz;
-      it.split = path == 3 ? 1 : 0;
+      it.zv = path & 7;
+      it.split = (path >> 3) & 1;
       it.pair = it.g.fp_pair && it.g.pair_ok ? 1 : 0;
-      it.items = (it.pair ? fp_pair_tiled(it.g) : fp_tiled_rays(it.g)) * wave_zchunks(it.g.nz, wz);
+      it.items = (it.pair ? fp_pair_tiled(it.g) : fp_tiled_rays(it.g)) * wave_zchunks(it.g.nz, it.zv);
       if (!it.g.incl && it.items >= 16ll * cus) {
         L.single.push_back(i);
         continue;

@@ -75,8 +75,28 @@ __global__ __launch_bounds__(256) void bclp_epilogue_kernel(RespDev r, BclpDev b
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
+// the lane's entries of a sinogram row: g <- clip(g - lr scale fp)
+template <int ZV, bool SPLIT>
+__device__ __forceinline__ void bclp_update_row(float* row, int nz, const FpLane<ZV, SPLIT>& ln,
+                                                const typename VecT<ZV>::T& fp, float scale, float lr, float glb,
+                                                float gub) {
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int q = 0; q < ZV; ++q) {
+      const int z = ln.z + 64 * q;
+      if (z < nz) row[z] = clampf(row[z] - lr * (scale * vget(fp, q)), glb, gub);
+    }
+  } else {
+    if (ln.z >= nz) return;
+    typename VecT<ZV>::T gv = vload<ZV>(row + ln.z);
+#pragma unroll
+    for (int q = 0; q < ZV; ++q) vset(gv, q, clampf(vget(gv, q) - lr * (scale * vget(fp, q)), glb, gub));
+    vstore<ZV>(row + ln.z, gv);
+  }
+}
+
 // C (wavefront-uniform variant)
-template <int ZV, bool REUSE>
+template <int ZV, bool REUSE, bool SPLIT>
 __global__ __launch_bounds__(256) void bclp_fp_update_wave(ParDev g, const float* __restrict__ operand,
                                                            float* __restrict__ gsino,
                                                            const float* __restrict__ minmax, int clip,
@@ -84,24 +104,18 @@ __global__ __launch_bounds__(256) void bclp_fp_update_wave(ParDev g, const float
                                                            float gub) {
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  int k, i, z;
-  if (!fp_wave_item<ZV>(wave, g, lane, k, i, z)) return;
-  const int zl = z < g.nz - ZV ? z : g.nz - ZV;
-  const bool clip_on = clip && wave_clip_active<ZV>(minmax, g.nz, zl);
-  const typename VecT<ZV>::T fp = clip_on ? fp_ray_wave<ZV, true, REUSE>(g, operand, minmax, k, i, zl, lane)
-                                          : fp_ray_wave<ZV, false, REUSE>(g, operand, minmax, k, i, zl, lane);
-  if (z >= g.nz) return;
-  const float scale = (float)(*scale_p);
-  float* gp = gsino + ((size_t)k * g.na + i) * g.nz + z;
-  typename VecT<ZV>::T gv = vload<ZV>(gp);
-#pragma unroll
-  for (int q = 0; q < ZV; ++q) vset(gv, q, clampf(vget(gv, q) - lr * (scale * vget(fp, q)), glb, gub));
-  vstore<ZV>(gp, gv);
+  int k, i, zc;
+  if (!fp_wave_item<ZV>(wave, g, k, i, zc)) return;
+  const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
+  const typename VecT<ZV>::T fp = clip && wave_clip_active(minmax, g.nz, ln)
+                                      ? fp_ray_wave<true, REUSE, false>(g, operand, minmax, k, i, ln, lane)
+                                      : fp_ray_wave<false, REUSE, false>(g, operand, minmax, k, i, ln, lane);
+  bclp_update_row(gsino + ((size_t)k * g.na + i) * g.nz, g.nz, ln, fp, (float)(*scale_p), lr, glb, gub);
 }
 
 // C, paired: the opposite ray (k2, i2) of a pair is projected from the same
 // taps and updated too
-template <int ZV, bool REUSE>
+template <int ZV, bool REUSE, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void bclp_fp_update_pair(ParDev g, const float* __restrict__ operand,
                                                            float* __restrict__ gsino,
                                                            const float* __restrict__ minmax, int clip,
@@ -110,35 +124,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void b
   using V = typename VecT<ZV>::T;
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  const PairItem it = fp_pair_item<ZV>(wave, g, lane);
+  const PairItem it = fp_pair_item<ZV>(wave, g);
   if (!it.ok) return;
-  const int k = it.k, i = it.i, k2 = it.k2, i2 = it.i2, z = it.z;
-  const int zl = z < g.nz - ZV ? z : g.nz - ZV;
-  const bool clip_on = clip && wave_clip_active<ZV>(minmax, g.nz, zl);
+  const int k = it.k, i = it.i, k2 = it.k2, i2 = it.i2;
+  const FpLane<ZV, SPLIT> ln(it.zc, lane, g.nz);
   const float scale = (float)(*scale_p);
   auto update = [&](int kh, int ih, const V& fp) {
-    float* gp = gsino + ((size_t)kh * g.na + ih) * g.nz + z;
-    V gv = vload<ZV>(gp);
-#pragma unroll
-    for (int q = 0; q < ZV; ++q) vset(gv, q, clampf(vget(gv, q) - lr * (scale * vget(fp, q)), glb, gub));
-    vstore<ZV>(gp, gv);
+    bclp_update_row(gsino + ((size_t)kh * g.na + ih) * g.nz, g.nz, ln, fp, scale, lr, glb, gub);
   };
-  if (clip_on) {
+  if (clip && wave_clip_active(minmax, g.nz, ln)) {
     // the clipped sample is not continuous in its position: the two rays are
     // projected one after the other
     for (int h = 0; h < (k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? k2 : k, ih = h ? i2 : i;
-      const V fp = fp_ray_wave<ZV, true, REUSE>(g, operand, minmax, kh, ih, zl, lane);
-      if (z < g.nz) update(kh, ih, fp);
+      update(kh, ih, fp_ray_wave<true, REUSE, false>(g, operand, minmax, kh, ih, ln, lane));
     }
     return;
   }
   V fp, fp2 = vzero<ZV>();
-  if (k2 >= 0)
-    fp = fp_ray_wave<ZV, false, REUSE, true>(g, operand, minmax, k, i, zl, lane, &fp2);
-  else
-    fp = fp_ray_wave<ZV, false, REUSE>(g, operand, minmax, k, i, zl, lane);
-  if (z >= g.nz) return;
+  if (k2 >= 0) fp = fp_ray_wave<false, REUSE, true>(g, operand, minmax, k, i, ln, lane, &fp2);
+  else fp = fp_ray_wave<false, REUSE, false>(g, operand, minmax, k, i, ln, lane);
   update(k, i, fp);
   if (k2 >= 0) update(k2, i2, fp2);
 }
@@ -216,13 +221,13 @@ __global__ __launch_bounds__(256) void bclp_bpT_update_wave(ParDev g, int clipc,
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
   int k, i, k2 = -1, i2 = -1, z;
   if constexpr (PAIR) {
-    const PairItem it = fp_pair_item<ZV, false>(wave, g, lane);
+    const PairItem it = fp_pair_item<ZV>(wave, g);
     if (!it.ok) return;
     k = it.k;
     i = it.i;
     k2 = it.k2;
     i2 = it.i2;
-    z = it.z;
+    z = (it.zc * 64 + lane) * ZV;
   } else {
     const int nch = wave_zchunks(g.nz, ZV);
     if (wave >= (long long)g.n * g.na * nch) return;   // whole wavefronts
@@ -231,8 +236,7 @@ __global__ __launch_bounds__(256) void bclp_bpT_update_wave(ParDev g, int clipc,
     i = (int)(bin / g.n);
     z = (int)(wave % nch) * 64 * ZV + lane * ZV;
   }
-  int zl, zl2;
-  wave_zload<ZV, false>(z, g.nz, zl, zl2);
+  const int zl = wave_zload<ZV>(z, g.nz);
   const float scale = (float)(*scale_p);
   if (k2 < 0) {
     const V gr = bpT_bin_wave<ZV>(g, operand, k, i, zl, lane, clipc);
@@ -422,44 +426,21 @@ int bclp_update_impl(vamx_plan* plan, const vamx_bclp_params* prm, float* g, con
     }
     if (incl_wave_ok(plan)) return incl_forward_update(plan, operand, UpdateOut{g, scale, lr, glb, gub}, s);
     if (thin_ok(plan)) return thin_forward_update(plan, operand, UpdateOut{g, scale, lr, glb, gub}, clip, s);
-    const int wz = par_fp_wave_zv(plan, operand, g);
-    if (wz && gd.fp_pair && gd.pair_ok) {
-      const long long threads = fp_pair_tiled(gd) * wave_zchunks(gd.nz, wz) * 64;
-      const dim3 grid(blocks_for(threads, 256)), block(256);
+    if (const FpLayout l = fp_layout(plan, (uintptr_t)operand | (uintptr_t)g); l.zv) {
+      const bool pair = gd.fp_pair && gd.pair_ok;
+      const long long waves = (pair ? fp_pair_tiled(gd) : fp_tiled_rays(gd)) * wave_zchunks(gd.nz, l.zv);
+      const dim3 grid(blocks_for(waves * 64, 256)), block(256);
       const int cl = clip ? 1 : 0;
-#define VAMX_FPP(Z, R)                                                                                 \
-  hipLaunchKernelGGL((bclp_fp_update_pair<Z, R>), grid, block, 0, s, gd, operand, g, plan->d_minmax, cl, scale, \
-                     lr, glb, gub)
-      if (gd.fp_reuse) {
-        if (wz == 4) VAMX_FPP(4, true);
-        else if (wz == 2) VAMX_FPP(2, true);
-        else VAMX_FPP(1, true);
-      } else {
-        if (wz == 4) VAMX_FPP(4, false);
-        else if (wz == 2) VAMX_FPP(2, false);
-        else VAMX_FPP(1, false);
-      }
-#undef VAMX_FPP
-      VAMX_HIP(hipGetLastError());
-      return VAMX_OK;
-    }
-    if (wz) {
-      const long long threads = fp_tiled_rays(gd) * wave_zchunks(gd.nz, wz) * 64;
-      const dim3 grid(blocks_for(threads, 256)), block(256);
-      const int cl = clip ? 1 : 0;
-#define VAMX_FPU(Z, R)                                                                                 \
-  hipLaunchKernelGGL((bclp_fp_update_wave<Z, R>), grid, block, 0, s, gd, operand, g, plan->d_minmax, cl, scale, \
-                     lr, glb, gub)
-      if (gd.fp_reuse) {
-        if (wz == 4) VAMX_FPU(4, true);
-        else if (wz == 2) VAMX_FPU(2, true);
-        else VAMX_FPU(1, true);
-      } else {
-        if (wz == 4) VAMX_FPU(4, false);
-        else if (wz == 2) VAMX_FPU(2, false);
-        else VAMX_FPU(1, false);
-      }
-#undef VAMX_FPU
+      fp_dispatch(l, gd.fp_reuse != 0, [&](auto zw, auto split, auto reuse) {
+        constexpr int ZV = decltype(zw)::value;
+        constexpr bool R = decltype(reuse)::value, S = decltype(split)::value;
+        if (pair)
+          hipLaunchKernelGGL((bclp_fp_update_pair<ZV, R, S>), grid, block, 0, s, gd, operand, g, plan->d_minmax, cl,
+                             scale, lr, glb, gub);
+        else
+          hipLaunchKernelGGL((bclp_fp_update_wave<ZV, R, S>), grid, block, 0, s, gd, operand, g, plan->d_minmax, cl,
+                             scale, lr, glb, gub);
+      });
       VAMX_HIP(hipGetLastError());
       return VAMX_OK;
     }

@@ -25,11 +25,13 @@ namespace vamx {
 template <int ZV> struct VecT;
 template <> struct VecT<1> { using T = float; };
 template <> struct VecT<2> { using T = float2; };
+template <> struct VecT<3> { using T = float3; };
 template <> struct VecT<4> { using T = float4; };
 
 template <int ZV> __device__ __forceinline__ typename VecT<ZV>::T vzero();
 template <> __device__ __forceinline__ float vzero<1>() { return 0.0f; }
 template <> __device__ __forceinline__ float2 vzero<2>() { return make_float2(0.f, 0.f); }
+template <> __device__ __forceinline__ float3 vzero<3>() { return make_float3(0.f, 0.f, 0.f); }
 template <> __device__ __forceinline__ float4 vzero<4>() { return make_float4(0.f, 0.f, 0.f, 0.f); }
 
 template <int ZV> __device__ __forceinline__ typename VecT<ZV>::T vload(const float* p);
@@ -62,22 +64,6 @@ __device__ __forceinline__ float4 bload<4>(__amdgpu_buffer_rsrc_t r, uint32_t vo
   return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
 }
 
-// Lane z layouts of the wavefront kernels: contiguous (a lane owns ZV
-// consecutive z) or split (SPLIT, ZV = 2: a lane owns z and z + 64, so one
-// wavefront covers 128 z with dword loads when nz is odd and no wider load
-// is aligned).  zb / zb2 are the byte offsets of the lane's (clamped) z.
-template <int ZV, bool SPLIT>
-__device__ __forceinline__ typename VecT<ZV>::T tload(__amdgpu_buffer_rsrc_t r, uint32_t zb, uint32_t zb2,
-                                                      uint32_t soff) {
-  if constexpr (SPLIT) {
-    static_assert(ZV == 2, "the split layout holds two z values per lane");
-    return make_float2(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)zb, (int)soff, 0)),
-                       __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)zb2, (int)soff, 0)));
-  } else {
-    return bload<ZV>(r, zb, soff);
-  }
-}
-
 template <int ZV> __device__ __forceinline__ void vstore(float* p, typename VecT<ZV>::T v);
 template <> __device__ __forceinline__ void vstore<1>(float* p, float v) { *p = v; }
 template <> __device__ __forceinline__ void vstore<2>(float* p, float2 v) { *reinterpret_cast<float2*>(p) = v; }
@@ -91,6 +77,10 @@ __device__ __forceinline__ float4 vfma(float a, float4 x, float4 y) {
 __device__ __forceinline__ float2 vfma(float a, float2 x, float2 y) {
   return make_float2(__builtin_fmaf(a, x.x, y.x), __builtin_fmaf(a, x.y, y.y));
 }
+__device__ __forceinline__ float3 vfma(float a, float3 x, float3 y) {
+  return make_float3(__builtin_fmaf(a, x.x, y.x), __builtin_fmaf(a, x.y, y.y), __builtin_fmaf(a, x.z, y.z));
+}
+__device__ __forceinline__ float3 vmul(float a, float3 x) { return make_float3(a * x.x, a * x.y, a * x.z); }
 __device__ __forceinline__ float vmul(float a, float x) { return a * x; }
 __device__ __forceinline__ float2 vmul(float a, float2 x) { return make_float2(a * x.x, a * x.y); }
 __device__ __forceinline__ float4 vmul(float a, float4 x) { return make_float4(a * x.x, a * x.y, a * x.z, a * x.w); }
@@ -112,6 +102,15 @@ __device__ __forceinline__ float2 vclamp(float2 v, float2 lo, float2 hi) {
 __device__ __forceinline__ float4 vclamp(float4 v, float4 lo, float4 hi) {
   return make_float4(clampf(v.x, lo.x, hi.x), clampf(v.y, lo.y, hi.y), clampf(v.z, lo.z, hi.z),
                      clampf(v.w, lo.w, hi.w));
+}
+__device__ __forceinline__ float3 vclamp(float3 v, float3 lo, float3 hi) {
+  return make_float3(clampf(v.x, lo.x, hi.x), clampf(v.y, lo.y, hi.y), clampf(v.z, lo.z, hi.z));
+}
+__device__ __forceinline__ float vget(float3 v, int q) { return q == 0 ? v.x : (q == 1 ? v.y : v.z); }
+__device__ __forceinline__ void vset(float3& v, int q, float x) {
+  if (q == 0) v.x = x;
+  else if (q == 1) v.y = x;
+  else v.z = x;
 }
 __device__ __forceinline__ float vget(float v, int) { return v; }
 __device__ __forceinline__ float vget(float2 v, int q) { return q == 0 ? v.x : v.y; }
@@ -831,42 +830,76 @@ __device__ __forceinline__ float rl_f(float v, int lane) {
 // The warp clip of a slice is a no-op when 0 lies in [min, max] of the slice:
 // bilinear samples are convex combinations of the slice's values and the zero
 // padding.  Wave-uniform test over the wave's 64*ZV slices.
-// z of the loads of a lane whose first z is z: lanes past nz load a copy of
-// the last valid z and store nothing
-template <int ZV, bool SPLIT>
-__device__ __forceinline__ void wave_zload(int z, int nz, int& zl, int& zl2) {
-  if constexpr (SPLIT) {
-    zl = z < nz - 1 ? z : nz - 1;
-    zl2 = z + 64 < nz - 1 ? z + 64 : nz - 1;
-  } else {
-    zl = z < nz - ZV ? z : nz - ZV;
-    zl2 = 0;
-  }
-}
-// store of a lane's z values into the z column at col
-template <int ZV, bool SPLIT>
+// the transposes' lanes own ZV consecutive slices: those past nz load a copy of
+// the last ones and store nothing
+template <int ZV>
+__device__ __forceinline__ int wave_zload(int z, int nz) { return z < nz - ZV ? z : nz - ZV; }
+template <int ZV>
 __device__ __forceinline__ void wave_zstore(float* col, int z, int nz, typename VecT<ZV>::T v) {
-  if constexpr (SPLIT) {
-    if (z < nz) col[z] = v.x;
-    if (z + 64 < nz) col[z + 64] = v.y;
-  } else {
-    if (z < nz) vstore<ZV>(col + z, v);
-  }
+  if (z < nz) vstore<ZV>(col + z, v);
 }
 
-// the slice range of the lane's z values (contiguous, or z and z2 split)
-template <int ZV, bool SPLIT = false>
-__device__ __forceinline__ typename VecT<ZV>::T zvals(const float* __restrict__ a, int z, int z2) {
-  if constexpr (SPLIT) return make_float2(a[z], a[z2]);
-  else return vload<ZV>(a + z);
-}
-template <int ZV, bool SPLIT = false>
-__device__ __forceinline__ bool wave_clip_active(const float* __restrict__ minmax, int nz, int z, int z2 = 0) {
-  const typename VecT<ZV>::T lo = zvals<ZV, SPLIT>(minmax, z, z2), hi = zvals<ZV, SPLIT>(minmax + nz, z, z2);
+// Slices of a lane in the forward's wavefronts: ZV consecutive ones, or (SPLIT)
+// z + 64 q, q < ZV, with a 4-byte load each.  Lanes past nz load a copy of the
+// last valid slices and store nothing.
+template <int ZV, bool SPLIT>
+struct FpLane {
+  using V = typename VecT<ZV>::T;
+  int z;
+  uint32_t zb[SPLIT ? ZV : 1];   // byte offsets of the loads
+  __device__ __forceinline__ FpLane(int chunk, int lane, int nz) {
+    z = chunk * 64 * ZV + (SPLIT ? lane : lane * ZV);
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int q = 0; q < ZV; ++q) zb[q] = 4u * (uint32_t)(z + 64 * q < nz - 1 ? z + 64 * q : nz - 1);
+    } else {
+      zb[0] = 4u * (uint32_t)(z < nz - ZV ? z : nz - ZV);
+    }
+  }
+  __device__ __forceinline__ V load(__amdgpu_buffer_rsrc_t r, uint32_t soff) const {
+    if constexpr (SPLIT) {
+      V v;
+#pragma unroll
+      for (int q = 0; q < ZV; ++q) vset(v, q, bload<1>(r, zb[q], soff));
+      return v;
+    } else {
+      return bload<ZV>(r, zb[0], soff);
+    }
+  }
+  // the lane's values of an array over z
+  __device__ __forceinline__ V values(const float* __restrict__ a) const {
+    if constexpr (SPLIT) {
+      V v;
+#pragma unroll
+      for (int q = 0; q < ZV; ++q) vset(v, q, a[zb[q] / 4]);
+      return v;
+    } else {
+      return vload<ZV>(a + zb[0] / 4);
+    }
+  }
+  __device__ __forceinline__ void store(float* col, int nz, V v) const {
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int q = 0; q < ZV; ++q)
+        if (z + 64 * q < nz) col[z + 64 * q] = vget(v, q);
+    } else {
+      if (z < nz) vstore<ZV>(col + z, v);
+    }
+  }
+};
+
+// the warp clip of the wavefront's slices is not a no-op, from their least and
+// largest values
+template <int ZV>
+__device__ __forceinline__ bool wave_clip_active(const typename VecT<ZV>::T& lo, const typename VecT<ZV>::T& hi) {
   bool need = false;
 #pragma unroll
   for (int q = 0; q < ZV; ++q) need |= !(vget(lo, q) <= 0.0f && 0.0f <= vget(hi, q));
   return __ballot(need) != 0ull;
+}
+template <int ZV, bool SPLIT>
+__device__ __forceinline__ bool wave_clip_active(const float* __restrict__ minmax, int nz, const FpLane<ZV, SPLIT>& ln) {
+  return wave_clip_active<ZV>(ln.values(minmax), ln.values(minmax + nz));
 }
 
 __device__ __forceinline__ void axis_slots(double coord, int n, int& b, double& s0, double& s1) {
@@ -921,11 +954,11 @@ __device__ __forceinline__ FpSlot fp_lds_slot() {
   return {w[wv], a[wv]};
 }
 
-template <int ZV, bool CLIP, bool REUSE, bool PAIR = false, bool SPLIT = false>
+template <bool CLIP, bool REUSE, bool PAIR, int ZV, bool SPLIT>
 __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, const float* __restrict__ vol,
-                                                             const float* __restrict__ minmax, int k, int i, int z,
-                                                             int lane, typename VecT<ZV>::T* acc2 = nullptr,
-                                                             int z2 = 0) {
+                                                             const float* __restrict__ minmax, int k, int i,
+                                                             const FpLane<ZV, SPLIT>& ln, int lane,
+                                                             typename VecT<ZV>::T* acc2 = nullptr) {
   using V = typename VecT<ZV>::T;
   static_assert(!(PAIR && CLIP), "the clipped sample is discontinuous at the border: no pairing");
   const int n = g.n;
@@ -936,15 +969,14 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
   const double t = (double)(k - g.c) - g.det_offset;
   V lo = vzero<ZV>(), hi = vzero<ZV>();
   if constexpr (CLIP) {
-    lo = zvals<ZV, SPLIT>(minmax, z, z2);
-    hi = zvals<ZV, SPLIT>(minmax + g.nz, z, z2);
+    lo = ln.values(minmax);
+    hi = ln.values(minmax + g.nz);
   }
   const size_t nzs = (size_t)g.nz;
   const size_t step_c = nzs, step_r = (size_t)n * nzs;
   // taps are buffer loads: lane byte offset 4z, scalar byte offset of the voxel
   // column from the first row that the 64 samples reach (their rows span at most
   // 66; where 66 rows pass 32 bits, from the sample's own cell)
-  const uint32_t zb = 4u * (uint32_t)z, zb2 = 4u * (uint32_t)z2;
   const uint32_t oc = (uint32_t)(4 * step_c), orr = (uint32_t)(4 * step_r);
   const bool big = 66ull * orr + 4ull * nzs >= 0xffffffffull;
   V acc = vzero<ZV>(), accp = vzero<ZV>();
@@ -1035,10 +1067,10 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
         const int at_j = rl_i(cell, j);
         rs = buf_rsrc(vol + (size_t)(at_j >> 14) * step_r + (size_t)(at_j & 0x3fff) * step_c, 0xffffffffu);
       }
-      if (load & 1) T00 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a00, j));
-      if (load & 2) T01 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a01, j));
-      if (load & 4) T10 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a10, j));
-      if (load & 8) T11 = tload<ZV, SPLIT>(rs, zb, zb2, (uint32_t)rl_i(a11, j));
+      if (load & 1) T00 = ln.load(rs, (uint32_t)rl_i(a00, j));
+      if (load & 2) T01 = ln.load(rs, (uint32_t)rl_i(a01, j));
+      if (load & 4) T10 = ln.load(rs, (uint32_t)rl_i(a10, j));
+      if (load & 8) T11 = ln.load(rs, (uint32_t)rl_i(a11, j));
       if constexpr (CLIP) {
         V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
         v = vclamp(v, lo, hi);  // every enumerated sample has an in-range tap of positive weight
@@ -1561,15 +1593,13 @@ __device__ __forceinline__ long long wave_index(unsigned lb) {
 // partial (lanes past nz load from a clamped z and store nothing)
 __host__ __device__ inline int wave_zchunks(int nz, int zv) { return (nz + 64 * zv - 1) / (64 * zv); }
 
-template <int ZV, bool SPLIT = false>
-__device__ __forceinline__ bool fp_wave_item(long long wave, const ParDev& g, int lane, int& k, int& i, int& z) {
+template <int ZV>
+__device__ __forceinline__ bool fp_wave_item(long long wave, const ParDev& g, int& k, int& i, int& zc) {
   const long long rays = fp_tiled_rays(g);
   const int nch = wave_zchunks(g.nz, ZV);
   if (wave >= rays * nch) return false;
-  const int zc = (int)(wave / rays);
-  if (!fp_tile_ray(wave % rays, g, k, i)) return false;
-  z = SPLIT ? zc * 64 * ZV + lane : zc * 64 * ZV + lane * ZV;
-  return true;
+  zc = (int)(wave / rays);
+  return fp_tile_ray(wave % rays, g, k, i);
 }
 
 // Paired forward work order: unit u (an angle pair, or a single angle) has
@@ -1588,16 +1618,16 @@ __host__ __device__ inline long long fp_pair_tiled(const ParDev& g) {
 // wave -> ray (k, i), partner ray (k2, i2) or k2 = -1, and z; ok = false for
 // padding waves
 struct PairItem {
-  int k, i, k2, i2, z;
+  int k, i, k2, i2, zc;
   bool ok;
 };
-template <int ZV, bool SPLIT = false>
-__host__ __device__ __forceinline__ PairItem fp_pair_item(long long wave, const ParDev& g, int lane) {
+template <int ZV>
+__host__ __device__ __forceinline__ PairItem fp_pair_item(long long wave, const ParDev& g) {
   PairItem it{0, 0, -1, -1, 0, false};
   const long long tiled = fp_pair_tiled(g);
   const int nch = wave_zchunks(g.nz, ZV);
   if (wave >= tiled * nch) return it;
-  const int zc = (int)(wave / tiled);
+  it.zc = (int)(wave / tiled);
   const long long q = wave % tiled;
   const int ta = fp_pair_ta(g), tk = fp_pair_tk(g), ne = fp_pair_next(g);
   const int ntk = (ne + tk - 1) / tk;
@@ -1615,20 +1645,19 @@ __host__ __device__ __forceinline__ PairItem fp_pair_item(long long wave, const 
   it.i = e < g.n ? u1 : u2;
   it.k2 = has2 ? kk : -1;
   it.i2 = has2 ? u2 : -1;
-  it.z = SPLIT ? zc * 64 * ZV + lane : zc * 64 * ZV + lane * ZV;   // split: z and z + 64
   it.ok = true;
   return it;
 }
 
 // wave -> (voxel quad, z) of the back-projection kernels; false for padding
-template <int ZV, bool SPLIT = false>
+template <int ZV>
 __device__ __forceinline__ bool bp_wave_quad(long long wave, const ParDev& g, int lane, int& r0, int& c0, int& z) {
   const long long quads = bp_tiled_quads(g);
   const int nch = wave_zchunks(g.nz, ZV);
   if (wave >= quads * nch) return false;
   const int zc = (int)(wave / quads);
   if (!bp_tile_quad(wave % quads, g, r0, c0)) return false;
-  z = SPLIT ? zc * 64 * ZV + lane : zc * 64 * ZV + lane * ZV;
+  z = zc * 64 * ZV + lane * ZV;
   return true;
 }
 
@@ -1772,6 +1801,32 @@ struct UpdateOut {
   }
 };
 
+// how a problem's forward projection lays out its slices: slices per lane (0:
+// not on the wavefront kernels), 64 apart or consecutive
+struct FpLayout {
+  int zv = 0;
+  bool split = false;
+};
+
+// calls f(ZV, SPLIT, REUSE) with the layout's compile-time constants
+template <class F>
+void fp_dispatch(const FpLayout& l, bool reuse, F&& f) {
+  using std::integral_constant;
+  auto with = [&](auto r) {
+    if (l.split) {
+      if (l.zv == 4) f(integral_constant<int, 4>{}, std::true_type{}, r);
+      else if (l.zv == 3) f(integral_constant<int, 3>{}, std::true_type{}, r);
+      else f(integral_constant<int, 2>{}, std::true_type{}, r);
+    } else {
+      if (l.zv == 4) f(integral_constant<int, 4>{}, std::false_type{}, r);
+      else if (l.zv == 2) f(integral_constant<int, 2>{}, std::false_type{}, r);
+      else f(integral_constant<int, 1>{}, std::false_type{}, r);
+    }
+  };
+  if (reuse) with(std::true_type{});
+  else with(std::false_type{});
+}
+
 // calls f(ZV, CONTIG, COMB) with the layout's compile-time constants
 template <class F>
 void bp_dispatch(const BpLayout& l, F&& f) {
@@ -1795,8 +1850,7 @@ BpLayout bp_layout(const vamx_plan* p, uintptr_t align_bits);
 bool par_use_vec4(const vamx_plan* p, const void* a, const void* b);
 bool par_use_vec2(const vamx_plan* p, const void* a, const void* b);
 int par_wave_zv(const vamx_plan* p, const void* a, const void* b, int requested);
-int par_fp_wave_zv(const vamx_plan* p, const void* vol, const void* sino);
-bool par_wave_split(const vamx_plan* p, int zv);
+FpLayout fp_layout(const vamx_plan* p, uintptr_t align_bits);
 int wave_zv_choice(int nz, uintptr_t align_bits, int requested);
 void par_pair_units(const std::vector<double>& cs, int na, int n, int c, double D, std::vector<int>& units,
                     int& npaired_rays, int& first2);

@@ -5,6 +5,7 @@
 // consecutive z values; every output element is written by exactly one lane
 // after a fixed-order accumulation (no atomics, bitwise deterministic).
 #include <algorithm>
+#include <climits>
 #include <cstring>
 
 #include "par_core.h"
@@ -165,26 +166,24 @@ __global__ __launch_bounds__(256) void par_fp_kernel(ParDev g, const float* __re
 }
 
 // wavefront-uniform forward projection: one wavefront = one ray x 64*ZV z
-// (SPLIT: ZV = 2 with lanes owning z and z + 64)
 template <int ZV, bool REUSE, bool SPLIT>
 __global__ __launch_bounds__(256) void par_fp_wave_kernel(ParDev g, const float* __restrict__ vol,
                                                           float* __restrict__ sino, const float* __restrict__ minmax,
                                                           int clip) {
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  int k, i, z, zl, zl2;
-  if (!fp_wave_item<ZV, SPLIT>(wave, g, lane, k, i, z)) return;
-  wave_zload<ZV, SPLIT>(z, g.nz, zl, zl2);
-  const bool clip_on = clip && wave_clip_active<ZV, SPLIT>(minmax, g.nz, zl, zl2);
-  typename VecT<ZV>::T acc =
-      clip_on ? fp_ray_wave<ZV, true, REUSE, false, SPLIT>(g, vol, minmax, k, i, zl, lane, nullptr, zl2)
-              : fp_ray_wave<ZV, false, REUSE, false, SPLIT>(g, vol, minmax, k, i, zl, lane, nullptr, zl2);
-  wave_zstore<ZV, SPLIT>(sino + ((size_t)k * g.na + i) * g.nz, z, g.nz, acc);
+  int k, i, zc;
+  if (!fp_wave_item<ZV>(wave, g, k, i, zc)) return;
+  const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
+  const typename VecT<ZV>::T acc = clip && wave_clip_active(minmax, g.nz, ln)
+                                       ? fp_ray_wave<true, REUSE, false>(g, vol, minmax, k, i, ln, lane)
+                                       : fp_ray_wave<false, REUSE, false>(g, vol, minmax, k, i, ln, lane);
+  ln.store(sino + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
 }
 
 // paired forward projection: one wavefront = ray (k, i) and, when it exists,
 // the opposite ray (k2, i2) x 64*ZV z, from one pass over the taps.  Held to
-// 64 VGPRs (8 waves per SIMD; a 12-byte spill) -- faster than 71 VGPRs at 7.
+// 64 VGPRs (8 waves per SIMD; a 28-byte spill outside the sample loop).
 template <int ZV, bool REUSE, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void par_fp_pair_kernel(ParDev g, const float* __restrict__ vol,
                                                           float* __restrict__ sino, const float* __restrict__ minmax,
@@ -192,30 +191,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void p
   using V = typename VecT<ZV>::T;
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  const PairItem it = fp_pair_item<ZV, SPLIT>(wave, g, lane);
+  const PairItem it = fp_pair_item<ZV>(wave, g);
   if (!it.ok) return;
-  const int k = it.k, i = it.i, k2 = it.k2, i2 = it.i2, z = it.z;
-  int zl, zl2;
-  wave_zload<ZV, SPLIT>(z, g.nz, zl, zl2);
-  const bool clip_on = clip && wave_clip_active<ZV, SPLIT>(minmax, g.nz, zl, zl2);
-  if (clip_on) {
+  const int k = it.k, i = it.i, k2 = it.k2, i2 = it.i2;
+  const FpLane<ZV, SPLIT> ln(it.zc, lane, g.nz);
+  if (clip && wave_clip_active(minmax, g.nz, ln)) {
     // the clipped sample is not continuous in its position: the two rays are
     // projected one after the other (one call site keeps the register count
     // of the unpaired kernel)
     for (int h = 0; h < (k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? k2 : k, ih = h ? i2 : i;
-      const V acc = fp_ray_wave<ZV, true, REUSE, false, SPLIT>(g, vol, minmax, kh, ih, zl, lane, nullptr, zl2);
-      wave_zstore<ZV, SPLIT>(sino + ((size_t)kh * g.na + ih) * g.nz, z, g.nz, acc);
+      const V acc = fp_ray_wave<true, REUSE, false>(g, vol, minmax, kh, ih, ln, lane);
+      ln.store(sino + ((size_t)kh * g.na + ih) * g.nz, g.nz, acc);
     }
     return;
   }
   V acc, acc2 = vzero<ZV>();
-  if (k2 >= 0)
-    acc = fp_ray_wave<ZV, false, REUSE, true, SPLIT>(g, vol, minmax, k, i, zl, lane, &acc2, zl2);
-  else
-    acc = fp_ray_wave<ZV, false, REUSE, false, SPLIT>(g, vol, minmax, k, i, zl, lane, nullptr, zl2);
-  wave_zstore<ZV, SPLIT>(sino + ((size_t)k * g.na + i) * g.nz, z, g.nz, acc);
-  if (k2 >= 0) wave_zstore<ZV, SPLIT>(sino + ((size_t)k2 * g.na + i2) * g.nz, z, g.nz, acc2);
+  if (k2 >= 0) acc = fp_ray_wave<false, REUSE, true>(g, vol, minmax, k, i, ln, lane, &acc2);
+  else acc = fp_ray_wave<false, REUSE, false>(g, vol, minmax, k, i, ln, lane);
+  ln.store(sino + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
+  if (k2 >= 0) ln.store(sino + ((size_t)k2 * g.na + i2) * g.nz, g.nz, acc2);
 }
 
 // back projection: one wavefront = one patch of voxel columns x 64 ZV z.
@@ -301,10 +296,9 @@ __global__ __launch_bounds__(256) void par_fpT_wave_kernel(ParDev g, const float
   if (w >= (long long)g.n * g.n * nch) return;   // whole wavefronts
   const int pix = (int)(w / nch);
   const int z = (int)(w % nch) * 64 * ZV + lane * ZV;
-  int zl, zl2;
-  wave_zload<ZV, false>(z, g.nz, zl, zl2);
+  const int zl = wave_zload<ZV>(z, g.nz);
   const typename VecT<ZV>::T acc = fpT_voxel_wave<ZV>(g, sino, pix, zl, lane);
-  wave_zstore<ZV, false>(vol + (size_t)pix * g.nz, z, g.nz, acc);
+  wave_zstore<ZV>(vol + (size_t)pix * g.nz, z, g.nz, acc);
 }
 
 template <int ZV>
@@ -318,10 +312,9 @@ __global__ __launch_bounds__(256) void par_bpT_wave_kernel(ParDev g, const float
   const long long bin = w / nch;
   const int k = (int)(bin % g.n), i = (int)(bin / g.n);
   const int z = (int)(w % nch) * 64 * ZV + lane * ZV;
-  int zl, zl2;
-  wave_zload<ZV, false>(z, g.nz, zl, zl2);
+  const int zl = wave_zload<ZV>(z, g.nz);
   const typename VecT<ZV>::T acc = bpT_bin_wave<ZV>(g, vol, k, i, zl, lane, clipc);
-  wave_zstore<ZV, false>(sino + ((size_t)k * g.na + i) * g.nz, z, g.nz, acc);
+  wave_zstore<ZV>(sino + ((size_t)k * g.na + i) * g.nz, z, g.nz, acc);
 }
 
 // A^T on voxel quads: one wavefront = one 2x2 quad of voxel columns x 64*ZV z
@@ -333,9 +326,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void p
                                                            float* __restrict__ vol) {
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  int r0, c0, z, zl, zl2;
-  if (!bp_wave_quad<ZV, false>(wave, g, lane, r0, c0, z)) return;
-  wave_zload<ZV, false>(z, g.nz, zl, zl2);
+  int r0, c0, z;
+  if (!bp_wave_quad<ZV>(wave, g, lane, r0, c0, z)) return;
+  const int zl = wave_zload<ZV>(z, g.nz);
   unsigned inrange, active;
   bp_quad_masks(g, r0, c0, 0, inrange, active);
   typename VecT<ZV>::T acc[4];
@@ -343,7 +336,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void p
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     if (!((inrange >> q) & 1u)) continue;
-    wave_zstore<ZV, false>(vol + ((size_t)(r0 + (q >> 1)) * g.n + c0 + (q & 1)) * g.nz, z, g.nz, acc[q]);
+    wave_zstore<ZV>(vol + ((size_t)(r0 + (q >> 1)) * g.n + c0 + (q & 1)) * g.nz, z, g.nz, acc[q]);
   }
 }
 
@@ -356,19 +349,19 @@ __global__ __launch_bounds__(256) void par_bpT_pair_kernel(ParDev g, const float
   using V = typename VecT<ZV>::T;
   const int lane = threadIdx.x & 63;
   const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
-  const PairItem it = fp_pair_item<ZV, false>(wave, g, lane);
+  const PairItem it = fp_pair_item<ZV>(wave, g);
   if (!it.ok) return;
-  int zl, zl2;
-  wave_zload<ZV, false>(it.z, g.nz, zl, zl2);
+  const int z = (it.zc * 64 + lane) * ZV;
+  const int zl = wave_zload<ZV>(z, g.nz);
   if (it.k2 < 0) {
     const V acc = bpT_bin_wave<ZV>(g, vol, it.k, it.i, zl, lane, clipc);
-    wave_zstore<ZV, false>(sino + ((size_t)it.k * g.na + it.i) * g.nz, it.z, g.nz, acc);
+    wave_zstore<ZV>(sino + ((size_t)it.k * g.na + it.i) * g.nz, z, g.nz, acc);
     return;
   }
   V acc, acc2;
   bpT_pair_wave<ZV>(g, vol, it.k, it.i, it.k2, it.i2, zl, lane, clipc, acc, acc2);
-  wave_zstore<ZV, false>(sino + ((size_t)it.k * g.na + it.i) * g.nz, it.z, g.nz, acc);
-  wave_zstore<ZV, false>(sino + ((size_t)it.k2 * g.na + it.i2) * g.nz, it.z, g.nz, acc2);
+  wave_zstore<ZV>(sino + ((size_t)it.k * g.na + it.i) * g.nz, z, g.nz, acc);
+  wave_zstore<ZV>(sino + ((size_t)it.k2 * g.na + it.i2) * g.nz, z, g.nz, acc2);
 }
 
 __global__ __launch_bounds__(256) void par_fpT_incl_kernel(ParDev g, const float* __restrict__ sino,
@@ -455,26 +448,36 @@ int vamx::wave_zv_choice(int nz, uintptr_t align_bits, int requested) {
   return best_util >= 0.5 ? best : 0;
 }
 
-int vamx::par_fp_wave_zv(const vamx_plan* p, const void* vol, const void* sino) {
-  // the forward's wavefront z width, 0 for the per-lane kernel.  At one z
-  // per lane a wavefront issues one 4-byte tap load per lane, and the forward
-  // is bound by load issue, not bytes; the per-lane kernel with four z per
-  // thread (several rays per wavefront, 16-byte tap loads) is then faster
-  // up to nz = 56.  At 256^2 x 360 with absorption, nz 32 / 40 / 48 measured
-  // 0.66 / 0.82 / 0.93 ms per-lane against 1.23 / 1.25 / 1.22 ms for the
-  // wavefront kernel, and they tie at nz = 64.
-  const int wz = par_wave_zv(p, vol, sino, p->par.fp_zv);
-  if (wz == 1 && p->par.nz <= 56 && par_use_vec4(p, vol, sino)) return 0;
-  return wz;
-}
-
-bool vamx::par_wave_split(const vamx_plan* p, int zv) {
-  // the split z layout (ZV = 2, lanes own z and z + 64) where the contiguous
-  // choice is one z per lane: half the wavefronts at the same lane
-  // utilisation when the 64-z chunk count is even
-  if (zv != 1 || !p->par.z_split) return false;
-  const int ch = wave_zchunks(p->par.nz, 1);
-  return ch % 2 == 0;
+FpLayout vamx::fp_layout(const vamx_plan* p, uintptr_t align_bits) {
+  const ParDev& g = p->par;
+  FpLayout l;
+  if ((p->flags & VAMX_PAR_PER_LANE_GEOMETRY) || g.incl || g.n < 2 || g.occ || g.nz < 32) return l;
+  if (!g.z_split) {
+    l.zv = wave_zv_choice(g.nz, align_bits, g.fp_zv);
+    return l;
+  }
+  // the least time, in 10 us of a pass over 256 x 256 x (64 to 256 slices: one
+  // chunk) and 360 angles, measured by slices per lane, 64 apart, and with
+  // 16-byte loads of four (0.77 ms at 192 slices, 0.83 at 256).  One slice per
+  // lane is already bound by latency and instructions, so wide chunks pay even
+  // where lanes idle: 180 slices took 1.56 ms as three chunks of 64, 0.78 as one;
+  // 255 slices 1.41 as two of 128, 1.32 as one; below 64 slices the per-lane
+  // kernels took 0.65 (32) to 1.01 ms (56) against 0.55 to 0.57.
+  constexpr int cost[5] = {0, 56, 70, 100, 132}, cost16 = 83;
+  int best = INT_MAX;
+  for (int zv = 1; zv <= g.fp_zv; ++zv) {
+    const int t = wave_zchunks(g.nz, zv) * cost[zv];
+    if (t < best) {
+      best = t;
+      l.zv = zv;
+      l.split = zv > 1;
+    }
+  }
+  if (g.fp_zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0 && wave_zchunks(g.nz, 4) * cost16 <= best) {
+    l.zv = 4;
+    l.split = false;
+  }
+  return l;
 }
 
 bool vamx::par_use_vec2(const vamx_plan* p, const void* a, const void* b) {
@@ -737,48 +740,17 @@ int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t 
     if (rc) return rc;
   }
   if (thin_ok(p)) return thin_forward_store(p, vol, sino, warp_clip, s);
-  int wz = par_fp_wave_zv(p, vol, sino);
-  const bool split = par_wave_split(p, wz);
-  if (split) wz = 2;
-  if (wz && g.fp_pair && g.pair_ok) {
-    const long long threads = fp_pair_tiled(g) * wave_zchunks(g.nz, wz) * 64;
-    const dim3 grid(blocks_for(threads, 256)), block(256);
+  if (const FpLayout l = fp_layout(p, (uintptr_t)vol | (uintptr_t)sino); l.zv) {
+    const bool pair = g.fp_pair && g.pair_ok;
+    const long long waves = (pair ? fp_pair_tiled(g) : fp_tiled_rays(g)) * wave_zchunks(g.nz, l.zv);
+    const dim3 grid(blocks_for(waves * 64, 256)), block(256);
     const int clip = warp_clip ? 1 : 0;
-#define VAMX_FPP(Z, R, S) \
-  hipLaunchKernelGGL((par_fp_pair_kernel<Z, R, S>), grid, block, 0, s, g, vol, sino, p->d_minmax, clip)
-    if (g.fp_reuse) {
-      if (split) VAMX_FPP(2, true, true);
-      else if (wz == 4) VAMX_FPP(4, true, false);
-      else if (wz == 2) VAMX_FPP(2, true, false);
-      else VAMX_FPP(1, true, false);
-    } else {
-      if (split) VAMX_FPP(2, false, true);
-      else if (wz == 4) VAMX_FPP(4, false, false);
-      else if (wz == 2) VAMX_FPP(2, false, false);
-      else VAMX_FPP(1, false, false);
-    }
-#undef VAMX_FPP
-    VAMX_HIP(hipGetLastError());
-    return VAMX_OK;
-  }
-  if (wz) {
-    const long long threads = fp_tiled_rays(g) * wave_zchunks(g.nz, wz) * 64;
-    const dim3 grid(blocks_for(threads, 256)), block(256);
-    const int clip = warp_clip ? 1 : 0;
-#define VAMX_FPW(Z, R, S) \
-  hipLaunchKernelGGL((par_fp_wave_kernel<Z, R, S>), grid, block, 0, s, g, vol, sino, p->d_minmax, clip)
-    if (g.fp_reuse) {
-      if (split) VAMX_FPW(2, true, true);
-      else if (wz == 4) VAMX_FPW(4, true, false);
-      else if (wz == 2) VAMX_FPW(2, true, false);
-      else VAMX_FPW(1, true, false);
-    } else {
-      if (split) VAMX_FPW(2, false, true);
-      else if (wz == 4) VAMX_FPW(4, false, false);
-      else if (wz == 2) VAMX_FPW(2, false, false);
-      else VAMX_FPW(1, false, false);
-    }
-#undef VAMX_FPW
+    fp_dispatch(l, g.fp_reuse != 0, [&](auto zv, auto split, auto reuse) {
+      constexpr int ZV = decltype(zv)::value;
+      constexpr bool R = decltype(reuse)::value, S = decltype(split)::value;
+      if (pair) hipLaunchKernelGGL((par_fp_pair_kernel<ZV, R, S>), grid, block, 0, s, g, vol, sino, p->d_minmax, clip);
+      else hipLaunchKernelGGL((par_fp_wave_kernel<ZV, R, S>), grid, block, 0, s, g, vol, sino, p->d_minmax, clip);
+    });
     VAMX_HIP(hipGetLastError());
     return VAMX_OK;
   }

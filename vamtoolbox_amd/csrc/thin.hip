@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __r
       k2 = !extra && u2 >= 0 && kk >= 0 && kk < g.n ? kk : -1;
       i2 = u2;
     }
-    const bool clip_on = clip && wave_clip_active<ZV>(minmax, g.nz, zl);
+    const bool clip_on = clip && wave_clip_active<ZV>(vload<ZV>(minmax + zl), vload<ZV>(minmax + g.nz + zl));
     const bool first = lane < R && store;
     V acc, acc2;
     if (clip_on) {
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __r
     return;
   }
   if (pair) {
-    const PairItem it = fp_pair_item<1>(wave, g, 0);
+    const PairItem it = fp_pair_item<1>(wave, g);
     if (!it.ok) return;
     k = it.k;
     i = it.i;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __r
   } else {
     if (wave >= fp_tiled_rays(g) || !fp_tile_ray(wave, g, k, i)) return;   // whole wavefronts
   }
-  const bool clip_on = clip && wave_clip_active<ZV>(minmax, g.nz, zl);
+  const bool clip_on = clip && wave_clip_active<ZV>(vload<ZV>(minmax + zl), vload<ZV>(minmax + g.nz + zl));
   auto put = [&](int kh, int ih, const V& v) {
     if (lane < L && z < g.nz) {
 #pragma unroll
