@@ -165,6 +165,19 @@ int vamx_bclp_eval(vamx_plan* plan, const vamx_response* resp, const vamx_bclp_p
                    const float* weight_arr, float* dose, float* operand, double* loss_out,
                    void* workspace, void* stream);
 
+/* Final evaluation of a device float dose of n voxels (BCLP.py:277-345, 396-437,
+ * 502-505): mapped (device float64 [n]) receives map(dose), and out[0 .. 8]
+ * (device) with e = mapped - target, b = |e| - eps, v = b > 0: sum v w |b|^p, the
+ * counts of v and of |e| > 0, sum v |b|, sum |e|, sum v b^2, sum e^2, max v |b|,
+ * max |e| (NaN if any element is), without dvol.  out holds
+ * VAMX_BCLP_METRICS * (1 + VAMX_BCLP_METRIC_BLOCKS) doubles; the ones past the
+ * first 9 are scratch. */
+#define VAMX_BCLP_METRICS 9
+#define VAMX_BCLP_METRIC_BLOCKS 2048
+int vamx_bclp_metrics(const vamx_response* resp, const vamx_bclp_params* prm, const float* dose,
+                      const float* target, const float* eps_arr, const float* weight_arr, int64_t n,
+                      double* mapped, double* out, void* stream);
+
 /* The update half of vamx_bclp_step: g <- clip(g - lr * s * A operand, glb, gub)
  * with the operand and the gradient scale s that the last vamx_bclp_step, or
  * vamx_bclp_eval called with operand == NULL, left in this workspace

@@ -82,6 +82,7 @@ class BclpParams(ctypes.Structure):
 
 
 IMGSEQ_MAX_COPIES = 64
+BCLP_METRICS, BCLP_METRIC_BLOCKS = 9, 2048
 
 
 class ImgSeqParams(ctypes.Structure):
@@ -154,6 +155,8 @@ SIGNATURES = {
     "vamx_bclp_eval": (c_int32, [_PLAN_P, ctypes.POINTER(Response), ctypes.POINTER(BclpParams),
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_void_p, c_void_p]),
+    "vamx_bclp_metrics": (c_int32, [ctypes.POINTER(Response), ctypes.POINTER(BclpParams), c_void_p, c_void_p, c_void_p,
+                                    c_void_p, ctypes.c_int64, c_void_p, c_void_p, c_void_p]),
     "vamx_bclp_update": (c_int32, [_PLAN_P, ctypes.POINTER(BclpParams), c_void_p, c_void_p, c_void_p]),
     "vamx_response_map": (c_int32, [ctypes.POINTER(Response), c_void_p, c_void_p, c_void_p, ctypes.c_int64,
                                     c_void_p]),

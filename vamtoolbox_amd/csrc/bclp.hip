@@ -75,6 +75,71 @@ __global__ __launch_bounds__(256) void bclp_epilogue_kernel(RespDev r, BclpDev b
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
+// Final evaluation of a dose: the mapped dose (float64) and, per block, the loss
+// integrand's sum and the L0, L1, L2 and Linf norms of the band error and of the
+// error (BCLP.py:277-345, 396-437), with the products of v = |e| > eps written
+// out as the reference multiplies them (so infinities and NaN reach the same
+// norms).  One pass, bound by the response's float64 exponential and division (68
+// us at 256^3 where the bytes take 55); element by element in float64 arrays the
+// same took 40 passes, 3.0 ms.
+constexpr int kMetrics = VAMX_BCLP_METRICS;
+__global__ __launch_bounds__(256) void bclp_metrics_kernel(RespDev r, BclpDev b, const float* __restrict__ dose,
+                                                           const float* __restrict__ target,
+                                                           double* __restrict__ mapped, double* __restrict__ partials,
+                                                           long long nv) {
+  __shared__ double sh[256];
+  double sum[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, top = 0.0, top0 = 0.0;
+  bool nan = false, nan0 = false;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += 256ll * gridDim.x) {
+    double m, dm;
+    response_eval(r, (double)dose[i], m, dm);
+    mapped[i] = m;
+    const double e = m - (double)target[i], ae = fabs(e);
+    const double eb = ae - (b.eps_arr ? (double)b.eps_arr[i] : b.eps), ab = fabs(eb);
+    const double v = eb > 0.0 ? 1.0 : 0.0, u = ae > 0.0 ? 1.0 : 0.0;
+    const double w = b.w_arr ? (double)b.w_arr[i] : b.weight;
+    sum[0] += v * w * (b.p == 2.0 ? ab * ab : pow(ab, b.p));
+    sum[1] += v;
+    sum[2] += u;
+    sum[3] += v * ab;
+    sum[4] += ae;
+    sum[5] += v * (eb * eb);
+    sum[6] += e * e;
+    const double f = v * ab, f0 = u * ae;
+    nan |= f != f;
+    nan0 |= f0 != f0;
+    top = fmax(top, f);
+    top0 = fmax(top0, f0);
+  }
+  if (nan) top = __longlong_as_double(0x7ff8000000000000ll);
+  if (nan0) top0 = __longlong_as_double(0x7ff8000000000000ll);
+  for (int q = 0; q < 7; ++q) {
+    const double s = block_sum_256(sum[q], sh);
+    if (threadIdx.x == 0) partials[(size_t)q * gridDim.x + blockIdx.x] = s;
+    __syncthreads();
+  }
+  for (int q = 7; q < kMetrics; ++q) {
+    const double s = block_max_256(q == 7 ? top : top0, sh);
+    if (threadIdx.x == 0) partials[(size_t)q * gridDim.x + blockIdx.x] = s;
+    __syncthreads();
+  }
+}
+// one block: the totals of the blocks' partials
+__global__ __launch_bounds__(256) void bclp_metrics_total(const double* __restrict__ partials, int nparts,
+                                                          double* __restrict__ out) {
+  __shared__ double sh[256];
+  for (int q = 0; q < kMetrics; ++q) {
+    double v = 0.0;
+    for (int i = threadIdx.x; i < nparts; i += 256) {
+      const double x = partials[(size_t)q * nparts + i];
+      v = q < 7 ? v + x : larger(v, x);
+    }
+    const double s = q < 7 ? block_sum_256(v, sh) : block_max_256(v, sh);
+    if (threadIdx.x == 0) out[q] = s;
+    __syncthreads();
+  }
+}
+
 // the lane's entries of a sinogram row: g <- clip(g - lr scale fp)
 template <int ZV, bool SPLIT>
 __device__ __forceinline__ void bclp_update_row(float* row, int nz, const FpLane<ZV, SPLIT>& ln,
@@ -599,6 +664,24 @@ extern "C" int vamx_response_map(const vamx_response* resp, const float* x, floa
   if (n == 0) return VAMX_OK;
   hipLaunchKernelGGL(response_map_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, (hipStream_t)stream, r, x, mapped,
                      dmap, (long long)n);
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+extern "C" int vamx_bclp_metrics(const vamx_response* resp, const vamx_bclp_params* prm, const float* dose,
+                                 const float* target, const float* eps_arr, const float* weight_arr, int64_t n,
+                                 double* mapped, double* out, void* stream) {
+  if (!prm || !dose || !target || !mapped || !out) return set_error(VAMX_ERR_ARG, "vamx_bclp_metrics: null argument");
+  if (n < 1) return set_error(VAMX_ERR_ARG, "vamx_bclp_metrics: empty volume");
+  RespDev r;
+  BclpDev b;
+  const int rc = bclp_fill_devs(resp, prm, eps_arr, weight_arr, r, b);
+  if (rc) return rc;
+  const int parts = (int)std::min<long long>(VAMX_BCLP_METRIC_BLOCKS, (n + 255) / 256);
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(bclp_metrics_kernel, dim3(parts), dim3(256), 0, s, r, b, dose, target, mapped,
+                     out + VAMX_BCLP_METRICS, (long long)n);
+  hipLaunchKernelGGL(bclp_metrics_total, dim3(1), dim3(256), 0, s, out + VAMX_BCLP_METRICS, parts, out);
   VAMX_HIP(hipGetLastError());
   return VAMX_OK;
 }

@@ -104,6 +104,18 @@ __device__ __forceinline__ double block_sum_256(double v, double* sh) {
   return sh[0];
 }
 
+// the larger of two values, NaN if either is
+__device__ __forceinline__ double larger(double a, double b) { return a != a || b != b ? a + b : fmax(a, b); }
+__device__ __forceinline__ double block_max_256(double v, double* sh) {
+  const int t = threadIdx.x;
+  sh[t] = v;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (t < s) sh[t] = larger(sh[t], sh[t + s]);
+    __syncthreads();
+  }
+  return sh[0];
+}
 
 // loss partials -> loss log / scalar and the gradient scale q L^((q-p)/q)
 // (one block, fixed order; defined in bclp.hip)

@@ -355,8 +355,28 @@ class BCLPNorm:
         torch.cuda.synchronize(dev)
         self.logs.loss[:k] = loss_log[:k].cpu().numpy()
         self.logs.recordIterTime()
-        self._finish(g.reshape(-1), k)
+        self._finish_fused(g, T, k)
         return g.reshape(-1)
+
+    def _finish_fused(self, g, T, k):
+        """_finish in one pass over the dose (vamx_bclp_metrics): the mapped dose, the loss and the norms."""
+        lib, lg = _lib.load(), self.logs
+        dose = self.P.backward(self._cyl(g)).reshape(self.T.shape).to(torch.float32).contiguous()
+        mapped = torch.empty(self.T.shape, device=self.device, dtype=torch.float64)
+        out = torch.empty(_lib.BCLP_METRICS * (1 + _lib.BCLP_METRIC_BLOCKS), device=self.device, dtype=torch.float64)
+        resp, prm = self._vamx_args()
+        _lib.check(lib.vamx_bclp_metrics(
+            ctypes.byref(resp), ctypes.byref(prm), dose.data_ptr(), T.data_ptr(),
+            0 if self.eps_t is None else self.eps_t.data_ptr(), 0 if self.w_t is None else self.w_t.data_ptr(),
+            dose.numel(), mapped.data_ptr(), out.data_ptr(), _lib.stream_ptr(self.device)), "vamx_bclp_metrics")
+        loss, l0, l0e, l1, l1e, l2, l2e, lf, lfe = out[:_lib.BCLP_METRICS].cpu().numpy()
+        self.dose, self.mapped_dose = dose, mapped
+        with np.errstate(all="ignore"):   # non-finite sums give non-finite norms, as torch's do
+            self.loss = lg.loss[k] = float((loss * self.dvol) ** (self.q / self.p))
+            lg.l0[k], lg.l0_eps0[k] = l0 * self.dvol, l0e * self.dvol
+            lg.l1[k], lg.l1_eps0[k] = l1 * self.dvol, l1e * self.dvol
+            lg.l2[k], lg.l2_eps0[k] = np.sqrt(l2 * self.dvol), np.sqrt(l2e * self.dvol)
+            lg.lf[k], lg.lf_eps0[k] = lf, lfe
 
     def _state_from_dose(self, dose):
         dd = dose.double()
