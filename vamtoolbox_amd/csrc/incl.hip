@@ -18,10 +18,12 @@
 // Below 64 rows (nz <= 31) the lanes form 64 / L groups of L; group g takes
 // every (64 / L)-th table entry, and the groups' sums are added at the end.
 //
-// Bound by vector instruction issue: per sample and 64 rows four dword loads
-// (5 cycles of the texture path each) and six multiply-adds.  The per-lane
+// Bound by the texture path (forward): per sample and 64 rows four dword loads of
+// 8.5 cycles each, and six multiply-adds; incl_fp_fixed_kernel loads fewer.  The per-lane
 // kernels this replaces evaluated the float64 geometry in every lane and
 // loaded eight taps per sample.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "par_core.h"
@@ -199,6 +201,181 @@ __global__ __launch_bounds__(256) void incl_fp_kernel(ParDev g, const float* __r
   }
 }
 
+// Forward of one ray where the shift over the whole ray is small against the
+// lanes: lanes own fixed slices, so that a sample finds the taps it shares with
+// the sample before (fp_ray_wave's scheme: two of four, as a rule) in registers,
+// and the rows' sums move past the lanes instead, one lane up (down) each time the
+// samples' shift grows (falls) by a slice.  A wavefront covers 64 NS slices from
+// slice j0 + shift.lo on and completes the `rows` detector rows from j0 on, whose
+// slices stay inside that range for every sample; slices outside the volume read 0.
+//
+// A tap of weight 0 is not read, and its register holds 0 then (it may lie outside,
+// or hold no number).
+//
+// Bound by latency and instructions (two slices per lane: 4.6 4-byte loads and 30
+// vector instructions per sample, against 8 loads and 24 with the rows' own lanes,
+// which the texture path bound): 128 x 128 x 96 x 180, 12 degrees 279 -> 207 us, x 256
+// x 90 398 -> 285, 100 x 100 x 300 x 60, 10 degrees 177 -> 122.
+struct InclShift {
+  int lo, rows;   // least shift of a ray's samples, detector rows of a wavefront
+};
+// values of the next / previous slice (lane, and across the NS registers); 0 past
+// the ends
+template <int NS>
+__device__ __forceinline__ float slice_next(const float (&v)[NS], int s) {
+  const int end = s + 1 < NS ? __builtin_amdgcn_readlane(__float_as_int(v[s + 1 < NS ? s + 1 : s]), 0) : 0;
+  return __int_as_float(__builtin_amdgcn_update_dpp(end, __float_as_int(v[s]), 0x130 /* wave_shl:1 */, 0xf, 0xf, false));
+}
+template <int NS>
+__device__ __forceinline__ float slice_prev(const float (&v)[NS], int s) {
+  const int end = s > 0 ? __builtin_amdgcn_readlane(__float_as_int(v[s > 0 ? s - 1 : s]), 63) : 0;
+  return __int_as_float(__builtin_amdgcn_update_dpp(end, __float_as_int(v[s]), 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+}
+
+template <int NS, class Out>
+__global__ __launch_bounds__(256) void incl_fp_fixed_kernel(ParDev g, const float* __restrict__ vol, InclShift shift,
+                                                            Out out) {
+  const int lane = threadIdx.x & 63;
+  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long rays = (long long)g.n * g.na;
+  const int nch = (g.nz + shift.rows - 1) / shift.rows;
+  if (wave >= rays * nch) return;   // whole wavefronts
+  const int j0 = (int)(wave / rays) * shift.rows;
+  const int i = (int)((wave % rays) / g.n), k = (int)((wave % rays) % g.n);
+  const int n = g.n, nz = g.nz;
+  const double* M = g.mats + 6 * i;
+  const double kp = (double)k - g.det_offset;
+  const double a0 = M[0] * kp, a1 = M[3] * kp;
+  const double t = (double)(k - g.c) - g.det_offset;
+  const uint32_t oc = 4u * (uint32_t)nz, orr = (uint32_t)n * oc;
+  // tap offsets count from the first row the 64 samples reach, or (big) from the
+  // sample's own cell; slices outside the volume lie past the descriptor's range
+  const bool big = 66ull * orr + 2ull * oc >= 0x7fffffffull;
+  const int z0 = j0 + shift.lo + lane;
+  uint32_t zo[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) zo[s] = slice_off(z0 + 64 * s, nz);
+  const InclSlot sl = incl_slot();
+  float acc[NS] = {}, T[4][NS] = {};   // T[2 a + b]: the tap of row parity a, column parity b
+  int at = 0;                          // shift of the last sample walked: lane z holds row z - at
+  bool any = false;
+  int last = -1, last_need = 15;       // cell and needed taps of the sample before the 64 (-1: none)
+  for (int r0 = 0; r0 < n; r0 += 64) {
+    const int r = r0 + lane;
+    float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+    float aw0 = 0.f, aw1 = 0.f;
+    int br = 0, bc = 0, q = 0, need = 0;
+    bool valid = false;
+    if (r < n) {
+      const double rr = (double)r;
+      const double col = (a0 + M[1] * rr) + M[2];
+      const double row = (a1 + M[4] * rr) + M[5];
+      if (row > -1.0 && row < (double)n && col > -1.0 && col < (double)n) {
+        double r0w, r1w, c0w, c1w;
+        axis_taps(row, n, br, r0w, r1w);
+        axis_taps(col, n, bc, c0w, c1w);
+        const double s = (double)(r - g.c), dz = s * g.tan_phi, fz = floor(dz);
+        const float aw = abs_weight(g, t, s);
+        q = (int)fz;
+        aw0 = aw * (float)(1.0 - (dz - fz));
+        aw1 = aw * (float)(dz - fz);
+        const float k00 = (float)(r0w * c0w), k01 = (float)(r0w * c1w), k10 = (float)(r1w * c0w), k11 = (float)(r1w * c1w);
+        const bool pr = br & 1, pc = bc & 1;
+        const float e0 = pc ? k01 : k00, e1 = pc ? k00 : k01, f0 = pc ? k11 : k10, f1 = pc ? k10 : k11;
+        w = pr ? make_float4(f0, f1, e0, e1) : make_float4(e0, e1, f0, f1);
+        need = (w.x != 0.0f) | (w.y != 0.0f) << 1 | (w.z != 0.0f) << 2 | (w.w != 0.0f) << 3;
+        valid = aw != 0.0f;
+      }
+    }
+    unsigned long long m = __ballot(valid);
+    if (!m) {
+      last = -1;
+      continue;
+    }
+    const int cell = valid ? (br << 14) | bc : -1;   // n < 2^14
+    const int upc = __shfl_up(cell, 1), upn = __shfl_up(need, 1);
+    const int before = lane == 0 ? last : upc, held = lane == 0 ? last_need : upn;
+    last = rl_i(cell, 63);
+    last_need = rl_i(need, 63);
+    const int dr = br - (before >> 14), dc = bc - (before & 0x3fff);
+    // taps to load, and (bits 4 to 7) registers to clear
+    int code = need | (15 & ~need) << 4;
+    if (before >= 0) {
+      int lacks = 15;
+      if (dr >= -1 && dr <= 1 && dc >= -1 && dc <= 1)
+        lacks = (dr ? 3 << (2 * ((br + (dr > 0)) & 1)) : 0) | (dc ? 5 << ((bc + (dc > 0)) & 1) : 0);
+      code = (need & (lacks | ~held)) | (held & ~need) << 4;
+    }
+    const int row_lo = min(rl_i(br, __builtin_ctzll(m)), rl_i(br, 63 - __builtin_clzll(m)));
+    const uint32_t from = big ? 0u : (uint32_t)(br - row_lo) * orr + (uint32_t)bc * oc;
+    const uint32_t re = from + ((br & 1) ? orr : 0u), ro = from + ((br & 1) ? 0u : orr);
+    const uint32_t ce = (bc & 1) ? oc : 0u, co = (bc & 1) ? 0u : oc;
+    const int o00 = (int)(re + ce), o01 = (int)(re + co), o10 = (int)(ro + ce), o11 = (int)(ro + co);
+    __amdgpu_buffer_rsrc_t rs = buf_rsrc(vol + (size_t)row_lo * n * nz, 0x7fffffffu);
+    __builtin_amdgcn_wave_barrier();
+    sl.w[lane] = w;
+    sl.a[lane] = make_float4(aw0, aw1, 0.f, 0.f);
+    __builtin_amdgcn_wave_barrier();
+    while (m) {
+      const int j = __builtin_ctzll(m);
+      m &= m - 1;
+      const float4 W = sl.w[j], A = sl.a[j];
+      const int c = rl_i(code, j), qj = rl_i(q, j);
+      if (big) {
+        const int b = rl_i(cell, j);
+        rs = buf_rsrc(vol + ((size_t)(b >> 14) * n + (b & 0x3fff)) * nz, 0x7fffffffu);
+      }
+      auto tap = [&](int a, int o) {
+        if (c >> a & 1) {
+          const uint32_t so = (uint32_t)rl_i(o, j);
+#pragma unroll
+          for (int s = 0; s < NS; ++s) T[a][s] = bload<1>(rs, zo[s], so);
+        }
+      };
+      tap(0, o00);
+      tap(1, o01);
+      tap(2, o10);
+      tap(3, o11);
+      if (c >> 4) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+          if (c >> (4 + a) & 1)
+#pragma unroll
+            for (int s = 0; s < NS; ++s) T[a][s] = 0.0f;
+      }
+      if (!any) at = qj;   // nothing summed yet
+      any = true;
+      while (at < qj) {
+        float moved[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) moved[s] = slice_prev<NS>(acc, s);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) acc[s] = moved[s];
+        ++at;
+      }
+      while (at > qj) {
+        float moved[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) moved[s] = slice_next<NS>(acc, s);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) acc[s] = moved[s];
+        --at;
+      }
+      float v[NS];
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        v[s] = vfma(W.w, T[3][s], vfma(W.z, T[2][s], vfma(W.y, T[1][s], W.x * T[0][s])));
+#pragma unroll
+      for (int s = 0; s < NS; ++s) acc[s] = vfma(A.y, slice_next<NS>(v, s), vfma(A.x, v[s], acc[s]));
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int j = z0 + 64 * s - at;
+    if (j >= j0 && j < j0 + shift.rows && j < nz) out.put(((size_t)k * g.na + i) * nz + j, acc[s]);
+  }
+}
+
 template <int NS, int L>
 __global__ __launch_bounds__(256) void incl_bp_kernel(ParDev g, const float* __restrict__ sino,
                                                       float* __restrict__ vol, int clipc) {
@@ -317,9 +494,47 @@ void incl_dispatch(int nz, F&& f) {
   else f(integral_constant<int, 3>{}, integral_constant<int, 64>{});
 }
 
+// whether the forward runs with fixed slices, and with how many slices per lane
+// (0: with its own lanes' rows): the least time, by microseconds of a pass over 128
+// x 128 columns, 180 angles, per chunk of rows -- 170, 200, 285, 370 with one to
+// four fixed slices, of which the shift over a ray takes some lanes, and 150, 275,
+// 400 with one to three rows (whose samples load all four taps and no shift is lost).
+// Where both take one chunk of one register, rows win: 19 against 22 us at 64 x 64 x
+// 48 x 60.
+int incl_fixed(const ParDev& g, InclShift& shift) {
+  if (g.nz < 32) return 0;
+  const double e0 = -(double)g.c * g.tan_phi, e1 = (double)(g.n - 1 - g.c) * g.tan_phi;
+  const double lo = std::floor(std::min(e0, e1)), span = std::floor(std::max(e0, e1)) - lo;
+  constexpr int fixed_us[5] = {0, 170, 200, 285, 370}, rows_us[4] = {0, 150, 275, 400};
+  const int slabs = incl_slabs(g.nz), own = 64 * slabs - 1;
+  long long best = (long long)((g.nz + own - 1) / own) * rows_us[slabs];
+  int ns = 0;
+  for (int k = 1; k <= 4; ++k) {
+    if (span > 64 * k - 2) continue;
+    const int rows = 64 * k - 1 - (int)span;
+    const long long t = (long long)((g.nz + rows - 1) / rows) * fixed_us[k];
+    if (t >= best) continue;
+    best = t;
+    ns = k;
+    shift = {(int)lo, rows};
+  }
+  return ns;
+}
+
 template <class Out>
 int incl_forward(vamx_plan* p, const float* vol, Out out, hipStream_t s) {
   const ParDev& g = p->par;
+  InclShift shift;
+  if (const int ns = incl_fixed(g, shift)) {
+    const long long waves = (long long)g.n * g.na * ((g.nz + shift.rows - 1) / shift.rows);
+    const dim3 grid(blocks_for(waves * 64, 256)), block(256);
+    if (ns == 4) hipLaunchKernelGGL((incl_fp_fixed_kernel<4, Out>), grid, block, 0, s, g, vol, shift, out);
+    else if (ns == 3) hipLaunchKernelGGL((incl_fp_fixed_kernel<3, Out>), grid, block, 0, s, g, vol, shift, out);
+    else if (ns == 2) hipLaunchKernelGGL((incl_fp_fixed_kernel<2, Out>), grid, block, 0, s, g, vol, shift, out);
+    else hipLaunchKernelGGL((incl_fp_fixed_kernel<1, Out>), grid, block, 0, s, g, vol, shift, out);
+    VAMX_HIP(hipGetLastError());
+    return VAMX_OK;
+  }
   incl_dispatch(g.nz, [&](auto ns, auto l) {
     constexpr int NS = decltype(ns)::value, L = decltype(l)::value, S = incl_rows<NS, L>();
     const long long waves = (long long)g.n * g.na * ((g.nz + S - 1) / S);
