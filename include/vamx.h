@@ -95,10 +95,10 @@ int vamx_par_backward_adjoint(vamx_plan* plan, const float* vol, float* sino, vo
 typedef struct vamx_par_tuning {
   int32_t fp_tile_angles;   /* forward: angles per tile of consecutive waves (default 10) */
   int32_t fp_tile_rays;     /* forward: rays per tile (default 4)                         */
-  int32_t fp_zv;            /* forward: z values per lane, 1, 2 or 4 (default 4)         */
+  int32_t fp_zv;            /* forward: at most this many z values per lane, 1, 2 or 4 (default 4) */
   int32_t fp_reuse;         /* forward: 1 = keep the previous sample's taps in registers (default 1) */
   int32_t bp_tile;          /* A^T: tile edge in 2x2 quads of voxel columns (default 8) */
-  int32_t bp_zv;            /* back projection: z values per lane (default 4)            */
+  int32_t bp_zv;            /* back projection: at most this many z values per lane (default 4) */
   int32_t fp_pair;          /* forward: 1 = project angles a and a + 180 deg in one pass over the
                                taps when 2 * det_offset is an integer and there is no inclination
                                or occlusion (default 1); fp_tile_angles then counts angle pairs */

@@ -381,6 +381,12 @@ __device__ __forceinline__ void os_min(unsigned long long m, OsWork* w) {
   if (__lane_id() == 0 && m != ~0ull) atomicMin(&w->min_gt, m);
 }
 
+// the bucket's count bounds the list; the test keeps calls that wrongly share a
+// workspace inside it
+__device__ __forceinline__ void os_put(OsWork* w, unsigned long long at, unsigned long long k) {
+  if (at < (unsigned long long)OS_LIST) w->list[at] = k;
+}
+
 // lists the elements that share the first two digits with the answer, through
 // LDS (one addition to the list's length per block), and takes the least key
 // above them
@@ -397,7 +403,7 @@ __global__ __launch_bounds__(OS_THREADS) void os_collect(const double* __restric
     if ((k >> 40) == (p.prefix >> 40)) {
       const unsigned at = atomicAdd(&held, 1u);
       if (at < 1024u) buf[at] = k;
-      else w->list[atomicAdd(&w->listed, 1ull)] = k;
+      else os_put(w, atomicAdd(&w->listed, 1ull), k);
     } else if (k > p.prefix && k < m) {
       m = k;
     }
@@ -407,7 +413,7 @@ __global__ __launch_bounds__(OS_THREADS) void os_collect(const double* __restric
   const unsigned c = held < 1024u ? held : 1024u;
   if (threadIdx.x == 0 && c) base = atomicAdd(&w->listed, (unsigned long long)c);
   __syncthreads();
-  if (threadIdx.x < c) w->list[base + threadIdx.x] = buf[threadIdx.x];
+  if (threadIdx.x < c) os_put(w, base + threadIdx.x, buf[threadIdx.x]);
 }
 
 // lists a whole array of at most OS_LIST elements
@@ -443,7 +449,7 @@ __global__ __launch_bounds__(OS_THREADS) void os_finish(long long n, long long r
   const int t = threadIdx.x;
   unsigned long long key = w->prefix[OS_PASSES], rem = w->rem[OS_PASSES], count = w->bucket[OS_PASSES];
   if (all || w->bucket[2] <= (unsigned long long)OS_LIST) {
-    const int listed = (int)w->listed;
+    const int listed = (int)(w->listed < (unsigned long long)OS_LIST ? w->listed : (unsigned long long)OS_LIST);
     key = all ? 0ull : w->prefix[2];
     rem = all ? (unsigned long long)rank : w->rem[2];
     for (int shift = all ? 56 : 32; shift >= 0; shift -= 8) {

@@ -655,7 +655,9 @@ extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) 
   // the clip mask and, behind it, the back projection's patch list
   std::vector<uint8_t> mask(((size_t)n * n + 3) / 4 * 4);
   std::memcpy(mask.data(), geom->outside_mask, (size_t)n * n);
-  const std::vector<int> list = bp_patch_list(g, geom->outside_mask);
+  std::vector<int> list;
+  g.bp_act = g.bp_all = 0;
+  if (nz >= 32 && !g.incl && !geom->occlusion) list = bp_patch_list(g, geom->outside_mask);   // as bp_layout asks
   const size_t mask_bytes = mask.size(), list_bytes = list.size() * sizeof(int);
   hipError_t e = hipSuccess;
   e = hipMalloc((void**)&p->d_mats, mats.size() * sizeof(double));
@@ -666,7 +668,7 @@ extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) 
   if (e == hipSuccess) e = hipMemcpy(p->d_mats, mats.data(), mats.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(p->d_cs, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice);
   mask.resize(mask_bytes + list_bytes);
-  std::memcpy(mask.data() + mask_bytes, list.data(), list_bytes);
+  if (list_bytes) std::memcpy(mask.data() + mask_bytes, list.data(), list_bytes);
   if (e == hipSuccess) e = hipMemcpy(p->d_outside, mask.data(), mask.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess && !units.empty()) {
     e = hipMalloc((void**)&p->d_units, units.size() * sizeof(int));

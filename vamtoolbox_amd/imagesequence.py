@@ -102,9 +102,6 @@ def _rotation(shape_uv, angle_deg):
     return (int(out_shape[0]), int(out_shape[1])), rot, in_center - out_center
 
 
-_OS_WORK = {}
-
-
 def _order_stats(flat, rank):
     """sorted(flat)[rank], sorted(flat)[rank + 1] of a float64 device vector
     (vamx_order_stats: an exact radix selection; NaN when it holds a NaN)."""
@@ -112,11 +109,10 @@ def _order_stats(flat, rank):
     from vamtoolbox_amd import _lib
     lib = _lib.load()
     dev = flat.device
-    ws = _OS_WORK.get(dev)
-    if ws is None:
-        nb = ctypes.c_int64()
-        _lib.check(lib.vamx_order_stats_workspace_bytes(ctypes.byref(nb)), "vamx_order_stats_workspace_bytes")
-        ws = _OS_WORK[dev] = torch.empty(int(nb.value), dtype=torch.uint8, device=dev)
+    # a workspace of this call: calls on several threads or streams may overlap
+    nb = ctypes.c_int64()
+    _lib.check(lib.vamx_order_stats_workspace_bytes(ctypes.byref(nb)), "vamx_order_stats_workspace_bytes")
+    ws = torch.empty(int(nb.value), dtype=torch.uint8, device=dev)
     out = torch.empty(2, dtype=torch.float64, device=dev)
     _lib.check(lib.vamx_order_stats(flat.data_ptr(), flat.numel(), int(rank), out.data_ptr(), ws.data_ptr(),
                                     _lib.stream_ptr(dev)), "vamx_order_stats")
