@@ -89,7 +89,7 @@ __device__ __forceinline__ bool grid_move(const RtDev& g, d3 x, GridPos& p) {
   p.wx = (float)(ix - (double)p.x0);
   p.wy = (float)(iy - (double)p.y0);
   p.wz = (float)(iz - (double)p.z0);
-  if (p.wx >= 0.0f && p.wy >= 0.0f && p.wz >= 0.0f && p.wx < 1.0f && p.wy < 1.0f && p.wz < 1.0f) return false;
+  if (p.wx >= 0.0f && p.wy >= 0.0f && p.wz >= 0.0f && p.wx <= 1.0f && p.wy <= 1.0f && p.wz <= 1.0f) return false;
   const double fx = floor(ix), fy = floor(iy), fz = floor(iz);
   p.x0 = (float)fx; p.y0 = (float)fy; p.z0 = (float)fz;
   p.wx = (float)(ix - fx); p.wy = (float)(iy - fy); p.wz = (float)(iz - fz);
@@ -156,15 +156,18 @@ __device__ __forceinline__ void lune_sample(const RtDev& g, double x, double y, 
 // coordinates clamped to [0, size - 1].  The position is float64, counted from
 // the held cell's corner, so that its conversion to float32 is the fraction in
 // that cell (the field is stored and interpolated in float32); a sample that
-// stays in the cell takes no floor and no cell index.  A tap past the last voxel
+// stays in the cell takes no floor and no cell index.  A fraction of 1 counts as
+// in the cell: rays start on voxels, and a position just below one, whose fraction
+// rounds to 1, would otherwise change cells at every sample.  A tap past the last voxel
 // along an axis (coordinate exactly size - 1, weight 0) reads the last voxel.
+__device__ __forceinline__ float cell_step(float w) { return w == 1.0f ? 0.0f : floorf(w); }
 __device__ __forceinline__ void field_sample_at(const RtDev& g, float ox, float oy, float oz, FieldCell& fc, float& n,
                                                 float& gx, float& gy, float& gz) {
   float wx = __builtin_amdgcn_fmed3f((float)(fc.bx + (double)ox), -fc.x0, fc.hx);
   float wy = __builtin_amdgcn_fmed3f((float)(fc.by + (double)oy), -fc.y0, fc.hy);
   float wz = __builtin_amdgcn_fmed3f((float)(fc.bz + (double)oz), -fc.z0, fc.hz);
-  if (!(min3(wx, wy, wz) >= 0.0f && max3(wx, wy, wz) < 1.0f)) {
-    const float fx = floorf(wx), fy = floorf(wy), fz = floorf(wz);
+  if (!(min3(wx, wy, wz) >= 0.0f && max3(wx, wy, wz) <= 1.0f)) {
+    const float fx = cell_step(wx), fy = cell_step(wy), fz = cell_step(wz);
     fc.x0 += fx; fc.y0 += fy; fc.z0 += fz;
     fc.hx -= fx; fc.hy -= fy; fc.hz -= fz;
     fc.bx -= (double)fx; fc.by -= (double)fy; fc.bz -= (double)fz;
@@ -458,8 +461,9 @@ __device__ __forceinline__ void tap_move(const RtDev& g, const RtIo& io, TapCell
 // per step; deposit, 440, waits besides for its atomics, which execute in memory
 // behind the L2s.  Measured, floors, cell indices and tap masks per sample and one
 // atomic per lane and tap -> cells held as corners and adjacent lanes' taps joined:
-//   64^3, 90 angles    integrate 1009 -> 984 us, deposit 1110 -> 997 us
-//   192^3, 360 angles  together 143.2 -> 124.3 ms
+//   64^3, 90 angles    both 1960 -> 1785 us
+//   192^3, 360 angles  both 145 -> 126 ms
+//   43^2 x 71, 71 angles (wavefronts across two rows of rays) 1040 -> 937 us
 template <int MODE, int SOLVER, int PARAM, bool LUNE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rt_trace_kernel(RtDev g, RtIo io) {
   const long long nrays = (long long)g.nt * g.na * g.nzr;
