@@ -481,7 +481,7 @@ def run_bclp(args):
     log("fused BCLP iteration with the exact gradient (grad_op 1): %.3f ms" % exact_ms)
 
     roof_c = roof("bclp_fp_update_pair", upd_ms, upd_alg)
-    roof_a = roof("bclp_bp_epilogue_wave", epi_ms, epi_alg)
+    roof_a = roof("par_bp_patch_kernel+bclp_epilogue_kernel", epi_ms, epi_alg)
     log("kernel C (FP + update) %.3f ms: %s GB/s measured traffic; kernel A (BP + epilogue) %.3f ms" % (
         upd_ms, "%.0f" % roof_c["achieved"] if roof_c["achieved"] else "n/a", epi_ms))
 
