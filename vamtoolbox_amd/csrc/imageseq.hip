@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void imgseq_compose(ComposeDev d, const double
 // passes run only where they are more than the list holds (many equal values);
 // arrays the list holds as a whole are listed at once.
 // Bound by reading the array: 23.6 M elements (189 MB) 39 us for a histogram pass
-// (4.9 TB/s) and 50 us for the listing one, all in all 172 us; the eight passes of
+// (4.9 TB/s) and 31 us for the listing one, all in all 152 us; the eight passes of
 // 8 bits, each with its own selection launch, and one for the key above took 362.
 // ---------------------------------------------------------------------------
 constexpr int OS_PASSES = 6, OS_BITS = 12, OS_BINS = 1 << OS_BITS;
@@ -372,13 +372,23 @@ __global__ __launch_bounds__(OS_THREADS) void os_hist(const double* __restrict__
     if (h[i]) atomicAdd(&w->counts[pass][i], (unsigned long long)h[i]);
 }
 
-// least key of the block's lanes into w->min_gt
+// least key of the block's lanes into w->min_gt; every thread of the block takes
+// part.  One atomic per block: with one per wavefront the 8192 minima at the one
+// address took longer than the array's reading where values above the rank are
+// spread over all wavefronts: os_collect over 23.6 M uniform values 121 -> 36 us, over
+// the projections of a part 50 -> 31 us (6.0 TB/s).
 __device__ __forceinline__ void os_min(unsigned long long m, OsWork* w) {
+  __shared__ unsigned long long sh[OS_THREADS / 64];
   for (int o = 32; o > 0; o >>= 1) {
     const unsigned long long q = __shfl_xor(m, o);
     m = q < m ? q : m;
   }
-  if (__lane_id() == 0 && m != ~0ull) atomicMin(&w->min_gt, m);
+  if (__lane_id() == 0) sh[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < OS_THREADS / 64; ++k) m = sh[k] < m ? sh[k] : m;
+    if (m != ~0ull) atomicMin(&w->min_gt, m);
+  }
 }
 
 // the bucket's count bounds the list; the test keeps calls that wrongly share a
