@@ -126,7 +126,7 @@ __device__ __forceinline__ void vset(float4& v, int q, float x) {
 // absorption weight of a sample at lateral coordinate t and along-ray s:
 // exp(-mu * max(0, sqrt(R^2 - t^2) - s) / cos(phi)) inside |t| < R, else 0
 // (per-ray form of astra3Dabsorption.getExpabs, astra3Dabsorption.py:129-145)
-__device__ __forceinline__ float abs_weight(const ParDev& g, double t, double s) {
+__host__ __device__ __forceinline__ float abs_weight(const ParDev& g, double t, double s) {
   if (g.mu == 0.0) return 1.0f;
   if (!(fabs(t) < g.radius)) return 0.0f;
   const double half = sqrt(g.radius * g.radius - t * t);
@@ -137,7 +137,7 @@ __device__ __forceinline__ float abs_weight(const ParDev& g, double t, double s)
 // np.interp(t, xp, fp, left=0, right=0) with xp[k] = (k - c) - det_offset:
 // value = fp[j] + w (fp[j1] - fp[j]); numpy compares t with the end nodes and
 // returns fp[-1] exactly at the last node.
-__device__ __forceinline__ bool interp_node(const ParDev& g, double t, int& j, int& j1, float& w) {
+__host__ __device__ __forceinline__ bool interp_node(const ParDev& g, double t, int& j, int& j1, float& w) {
   if (!(t >= g.xp0 && t <= g.xp_last)) return false;
   const double u = t - g.xp0;
   int jj = (int)floor(u);
@@ -1275,8 +1275,14 @@ struct BpNode {
 };
 
 // mirrored nodes common to both angles of a pair
-__device__ __forceinline__ int bp_jlo(const ParDev& g) { return max(0, 2 * g.c + g.pair_D - (g.n - 1)); }
-__device__ __forceinline__ int bp_jhi(const ParDev& g) { return min(g.n - 1, 2 * g.c + g.pair_D); }
+__host__ __device__ __forceinline__ int bp_jlo(const ParDev& g) { return max(0, 2 * g.c + g.pair_D - (g.n - 1)); }
+__host__ __device__ __forceinline__ int bp_jhi(const ParDev& g) { return min(g.n - 1, 2 * g.c + g.pair_D); }
+// whether opposite angles are combined: only where they share an interval, that is
+// two nodes.  Of a single common node (n = 2, or a detector shifted by half its
+// width) neither neighbour is a bin of both angles.
+__host__ __device__ inline bool bp_combines(const ParDev& g) {
+  return g.mu == 0.0 && g.pair_ok && bp_jhi(g) > bp_jlo(g);
+}
 
 // which nodes a pass over the angles takes: of every angle (COMB: of the pairs,
 // where both angles see the pixel), or of the pixels that the pair's first or
@@ -1286,7 +1292,7 @@ enum BpPass { BP_ALL = 0, BP_ONE = 1, BP_TWO = 2 };
 // node of the pixel at (x, y) for angle i (COMB: unit (i, i2)) in pass PASS;
 // single: only one angle of the pair sees it
 template <bool COMB, int PASS>
-__device__ __forceinline__ BpNode bp_node(const ParDev& g, bool on, int i, int i2, double x, double y, bool& single) {
+__host__ __device__ __forceinline__ BpNode bp_node(const ParDev& g, bool on, int i, int i2, double x, double y, bool& single) {
   const BpNode none{-1, 0.f, 0.f};
   if (!on) return none;
   const int n = g.n;

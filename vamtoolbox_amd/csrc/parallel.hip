@@ -430,7 +430,7 @@ BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits) {
     }
   }
   l.contig = l.zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0;
-  l.comb = g.mu == 0.0 && g.pair_ok;
+  l.comb = bp_combines(g);
   return l;
 }
 
