@@ -327,6 +327,9 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
     p0 = ((uint32_t)j * (uint32_t)g.na + (uint32_t)i) * bin_b;
     p1 = j < n - 1 ? p0 + row_b : kOut;
   };
+  // the angles of a step are summed from zero and added once: the sum so far,
+  // whose rounding is what the error is made of, is rounded once a step, not
+  // twice an angle
   int i = (int)((long long)g.na * wv / split);
   if constexpr (L == 1) {
     const uint32_t zb = 4u * (uint32_t)zl;
@@ -340,8 +343,10 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
         b0[u] = bload<ZV>(sr, p0 + zb, 0);
         b1[u] = bload<ZV>(sr, p1 + zb, 0);
       }
+      V part = vfma(w1[0], b1[0], vmul(w0[0], b0[0]));
 #pragma unroll
-      for (int u = 0; u < kAng; ++u) acc = vfma(w1[u], b1[u], vfma(w0[u], b0[u], acc));
+      for (int u = 1; u < kAng; ++u) part = vfma(w1[u], b1[u], vfma(w0[u], b0[u], part));
+      acc = vadd(acc, part);
     }
   } else {
     float4* const tb = thin_bp_lds + wv * 64;
@@ -365,8 +370,10 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
           b0[u] = bload<ZV>(sr, __float_as_uint(e[u].z) + zb, 0);
           b1[u] = bload<ZV>(sr, __float_as_uint(e[u].w) + zb, 0);
         }
+        V part = vfma(e[0].y, b1[0], vmul(e[0].x, b0[0]));
 #pragma unroll
-        for (int u = 0; u < K; ++u) acc = vfma(e[u].y, b1[u], vfma(e[u].x, b0[u], acc));
+        for (int u = 1; u < K; ++u) part = vfma(e[u].y, b1[u], vfma(e[u].x, b0[u], part));
+        acc = vadd(acc, part);
       }
     }
   }
