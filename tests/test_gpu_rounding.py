@@ -12,8 +12,10 @@ from tests.conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 
-# thin back projections with and without the angles split
-CASES = [(288, 28, 60, 0.0, 360.0, 0.0), (200, 24, 180, 0.0, 360.0, 0.0), (320, 1, 180, 0.01, 180.0, 0.0)]
+# thin back projections with and without the angles split, inclined projections with fixed slices and with rows
+# per lane
+CASES = [(288, 28, 60, 0.0, 360.0, 0.0), (200, 24, 180, 0.0, 360.0, 0.0), (320, 1, 180, 0.01, 180.0, 0.0),
+         (128, 96, 60, 0.005, 360.0, 12.0), (64, 128, 90, 0.01, 360.0, 20.0), (90, 40, 120, 0.0, 180.0, 4.0)]
 
 
 @pytest.mark.parametrize("n, nz, na, mu, span, incl", CASES)

@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256) void incl_fp_fixed_kernel(ParDev g, const floa
       for (int s = 0; s < NS; ++s)
         v[s] = vfma(W.w, T[3][s], vfma(W.z, T[2][s], vfma(W.y, T[1][s], W.x * T[0][s])));
 #pragma unroll
-      for (int s = 0; s < NS; ++s) acc[s] = vfma(A.y, slice_next<NS>(v, s), vfma(A.x, v[s], acc[s]));
+      for (int s = 0; s < NS; ++s) acc[s] += vfma(A.y, slice_next<NS>(v, s), A.x * v[s]);   // one rounding of the sum
     }
   }
 #pragma unroll
@@ -450,13 +450,19 @@ __global__ __launch_bounds__(256) void incl_bp_kernel(ParDev g, const float* __r
             v[u][0][1] = in_z ? x1 : 0.0f;
           }
         }
+        // summed from zero and added once: the sums so far are rounded once a step
 #pragma unroll
-        for (int u = 0; u < kU; ++u)
+        for (int s = 0; s < NS; ++s) {
+          float pl = vfma(ww[0].y, v[0][s][1], ww[0].x * v[0][s][0]);
+          float ph = vfma(ww[0].w, v[0][s][1], ww[0].z * v[0][s][0]);
 #pragma unroll
-          for (int s = 0; s < NS; ++s) {
-            lo[s] = vfma(ww[u].y, v[u][s][1], vfma(ww[u].x, v[u][s][0], lo[s]));
-            hi[s] = vfma(ww[u].w, v[u][s][1], vfma(ww[u].z, v[u][s][0], hi[s]));
+          for (int u = 1; u < kU; ++u) {
+            pl = vfma(ww[u].y, v[u][s][1], vfma(ww[u].x, v[u][s][0], pl));
+            ph = vfma(ww[u].w, v[u][s][1], vfma(ww[u].z, v[u][s][0], ph));
           }
+          lo[s] += pl;
+          hi[s] += ph;
+        }
       }
     }
     incl_combine<NS, L>(lo, hi, lane);
