@@ -12,10 +12,12 @@ from tests.conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 
-# thin back projections with and without the angles split, inclined projections with fixed slices and with rows
-# per lane
+# thin back projections with and without the angles split, inclined ones with fixed slices and with rows per
+# lane, unpaired forwards (angles over half a turn) of 32 slices and more (whose back projection multiplies
+# row by row into the sum, two roundings per angle)
 CASES = [(288, 28, 60, 0.0, 360.0, 0.0), (200, 24, 180, 0.0, 360.0, 0.0), (320, 1, 180, 0.01, 180.0, 0.0),
-         (128, 96, 60, 0.005, 360.0, 12.0), (64, 128, 90, 0.01, 360.0, 20.0), (90, 40, 120, 0.0, 180.0, 4.0)]
+         (128, 96, 60, 0.005, 360.0, 12.0), (64, 128, 90, 0.01, 360.0, 20.0), (90, 40, 120, 0.0, 180.0, 4.0),
+         (160, 48, 120, 0.01, 180.0, 0.0), (128, 32, 90, 0.02, 180.0, 0.0)]
 
 
 @pytest.mark.parametrize("n, nz, na, mu, span, incl", CASES)
@@ -29,6 +31,8 @@ def test_no_further_from_float64(gpu, n, nz, na, mu, span, incl):
     plan, lane = [ParallelPlan(n, nz, ang, warp_clip=False, per_lane_geometry=p, device=gpu, **kw) for p in (False, True)]
     at = np.unique(np.linspace(0, nz - 1, 6).astype(int))
     for name, shape in (("forward", (n, n, nz)), ("backward", (n, na, nz))):
+        if name == "backward" and nz >= 32 and not incl:
+            continue
         x = torch.tensor(rng.uniform(0.2, 1.0, shape), dtype=torch.float32, device=gpu)
         x64 = x.cpu().numpy().astype(np.float64)
         got, ref = [getattr(p, name)(x).cpu().numpy()[..., at] for p in (plan, lane)]

@@ -91,6 +91,7 @@ __device__ __forceinline__ float4 vsub(float4 a, float4 b) {
 __device__ __forceinline__ float2 vsub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ float vadd(float a, float b) { return a + b; }
 __device__ __forceinline__ float2 vadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ float3 vadd(float3 a, float3 b) { return make_float3(a.x + b.x, a.y + b.y, a.z + b.z); }
 __device__ __forceinline__ float4 vadd(float4 a, float4 b) {
   return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
@@ -1057,32 +1058,41 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
     sl.w[lane] = make_float4(w00, w01, w10, w11);
     sl.a[lane] = make_float2(aw, aw2);
     __builtin_amdgcn_wave_barrier();
-    while (m) {
-      const int j = __builtin_ctzll(m);
-      m &= m - 1;
-      const float4 Q = sl.w[j];
-      const float q00 = Q.x, q01 = Q.y, q10 = Q.z, q11 = Q.w;
-      const int load = rl_i(lacks, j);
-      if (big) {
-        const int at_j = rl_i(cell, j);
-        rs = buf_rsrc(vol + (size_t)(at_j >> 14) * step_r + (size_t)(at_j & 0x3fff) * step_c, 0xffffffffu);
+    // Unpaired without the clip (absorption in the taps' weights) the samples are
+    // summed 16 at a time: the whole ray's sum is rounded once per 16 samples
+    constexpr int kPart = CLIP || PAIR ? 64 : 16;
+#pragma unroll 1
+    for (int from = 0; from < 64; from += kPart) {
+      unsigned long long ms = kPart < 64 ? m & (0xffffull << from) : m;
+      V part = vzero<ZV>();
+      while (ms) {
+        const int j = __builtin_ctzll(ms);
+        ms &= ms - 1;
+        const float4 Q = sl.w[j];
+        const float q00 = Q.x, q01 = Q.y, q10 = Q.z, q11 = Q.w;
+        const int load = rl_i(lacks, j);
+        if (big) {
+          const int at_j = rl_i(cell, j);
+          rs = buf_rsrc(vol + (size_t)(at_j >> 14) * step_r + (size_t)(at_j & 0x3fff) * step_c, 0xffffffffu);
+        }
+        if (load & 1) T00 = ln.load(rs, (uint32_t)rl_i(a00, j));
+        if (load & 2) T01 = ln.load(rs, (uint32_t)rl_i(a01, j));
+        if (load & 4) T10 = ln.load(rs, (uint32_t)rl_i(a10, j));
+        if (load & 8) T11 = ln.load(rs, (uint32_t)rl_i(a11, j));
+        if constexpr (CLIP) {
+          V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
+          v = vclamp(v, lo, hi);  // every enumerated sample has an in-range tap of positive weight
+          acc = vfma(sl.a[j].x, v, acc);
+        } else if constexpr (PAIR) {
+          const V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
+          const float2 A = sl.a[j];
+          acc = vfma(A.x, v, acc);
+          accp = vfma(A.y, v, accp);
+        } else {
+          part = vadd(part, vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00)))));
+        }
       }
-      if (load & 1) T00 = ln.load(rs, (uint32_t)rl_i(a00, j));
-      if (load & 2) T01 = ln.load(rs, (uint32_t)rl_i(a01, j));
-      if (load & 4) T10 = ln.load(rs, (uint32_t)rl_i(a10, j));
-      if (load & 8) T11 = ln.load(rs, (uint32_t)rl_i(a11, j));
-      if constexpr (CLIP) {
-        V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
-        v = vclamp(v, lo, hi);  // every enumerated sample has an in-range tap of positive weight
-        acc = vfma(sl.a[j].x, v, acc);
-      } else if constexpr (PAIR) {
-        const V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
-        const float2 A = sl.a[j];
-        acc = vfma(A.x, v, acc);
-        accp = vfma(A.y, v, accp);
-      } else {
-        acc = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vfma(q00, T00, acc))));
-      }
+      if constexpr (!CLIP && !PAIR) acc = vadd(acc, part);
     }
   }
   if constexpr (PAIR) *acc2 = accp;
