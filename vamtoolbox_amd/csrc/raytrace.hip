@@ -28,8 +28,6 @@
 // Interaction taps use floor and floor+1 with weights 1-d and d (standard
 // trilinear); the reference selects floor and ceil, which counts a tap twice
 // when a coordinate is exactly integral.
-#include <climits>
-
 #include "bclp_core.h"
 #include "vamx_internal.h"
 
@@ -402,15 +400,15 @@ __device__ __forceinline__ void tap_shift(const RtDev& g, const RtIo& io, TapCel
   const bool okx[2] = {(unsigned)fx < (unsigned)g.nx, (unsigned)(fx + 1) < (unsigned)g.nx};
   const bool oky[2] = {(unsigned)fy < (unsigned)g.ny, (unsigned)(fy + 1) < (unsigned)g.ny};
   const bool okz[2] = {(unsigned)fz < (unsigned)g.nz, (unsigned)(fz + 1) < (unsigned)g.nz};
-  const int key = (fx * g.ny + fy) * g.nz + fz;
-  unsigned long long* const at = io.acc + key;
+  unsigned long long* const at = io.acc + ((fx * g.ny + fy) * g.nz + fz);
   // adjacent lanes trace adjacent z: where the next lane writes out the same
   // face one voxel higher, it adds this lane's upper taps to its lower ones
   // (integers: the same sums with half the atomics)
   bool give = false, got = false;
   if (AX != 2) {
-    const int next = lane_next(INT_MIN, okz[0] ? key : INT_MIN);
-    give = okz[1] && next == key + 1;
+    const unsigned key = rt_face_key(g, fx, fy, fz);
+    const unsigned next = (unsigned)lane_next(-1, okz[0] ? (int)key : -1);
+    give = okz[1] && next == key + 1u;
     got = lane_prev(0, (int)give) != 0;
   }
 #pragma unroll

@@ -50,13 +50,13 @@ struct ParDev {
   const int* units;          // [n_units][2]
 };
 
-// Geometry of the curved-ray tracer, passed by value.
 // one stage of the classical Runge-Kutta step: its and the next stage's offset
 // along the k of the stage before, and its k's weight in the sum
 struct RkStage {
   float c, next, w;
 };
 
+// Geometry of the curved-ray tracer, passed by value.
 struct RtDev {
   int nx, ny, nz;
   double xmin, ymin, zmin, dx, dy, dz;
@@ -91,6 +91,14 @@ struct RtDev {
   const double* ray_cs;      // [na][2] cos, sin of azimuth
   double radial_offset;      // proj_plane_radial_offset
 };
+
+// number of a face's corner, which may lie one voxel outside the grid on either
+// side: strides two wider than the grid, so that corners of different columns
+// differ by more than the slices of one (the voxel's linear index does not tell
+// the last row of one x from the row before the first of the next)
+__host__ __device__ inline unsigned rt_face_key(const RtDev& g, int fx, int fy, int fz) {
+  return ((unsigned)(fx + 1) * (unsigned)(g.ny + 2) + (unsigned)(fy + 1)) * (unsigned)(g.nz + 2) + (unsigned)(fz + 1);
+}
 
 // serial number of a new plan (unique for the process: a batch names its
 // plans by serial, so a new plan at a freed plan's address is another plan)
