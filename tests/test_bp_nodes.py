@@ -77,6 +77,7 @@ int main() {
         g.pair_D = D;
         const int lo2 = std::max(0, 2 * g.c + D - (n - 1)), hi2 = std::min(n - 1, 2 * g.c + D);
         g.pair_ok = hi2 >= lo2 && std::abs(D) < n;   // as the plan's units ask
+        g.fp_pair = 1;
         const bool comb = bp_combines(g);
         for (int pix = 0; pix < n * n; ++pix) {
           const double y = pix / n - g.c, x = pix % n - g.c;

@@ -35,3 +35,20 @@ def test_single_shared_bin(gpu, n, off, nz, na):
     assert e <= 5e-6, e
     flat = ParallelBatch([plan, other]).backward(torch.cat([s.reshape(-1), torch.zeros(5 * na * nz, device=gpu)]))
     assert torch.equal(flat[: n * n * nz].view(ref.shape), got)
+
+
+@pytest.mark.parametrize("n, nz", [(20, 40), (33, 128), (24, 256)])
+def test_unpaired_plan_sums_angle_by_angle(gpu, n, nz):
+    """fp_pair = 0 keeps the back projection unpaired too: without absorption the sums are bitwise those of a
+    plan with an absorption so small that every weight is 1, which never combines angles."""
+    import torch
+    from vamtoolbox_amd.parallel import ParallelPlan
+    ang = np.arange(0.0, 360.0, 15.0)
+    plain, weak = [ParallelPlan(n, nz, ang, mu=mu, radius=1e6, device=gpu) for mu in (0.0, 1e-300)]
+    s = torch.rand(plain.sino_shape, device=gpu)
+    paired = plain.backward(s)
+    plain.set_tuning(fp_pair=0)
+    assert torch.equal(plain.backward(s), weak.backward(s))
+    assert not torch.equal(paired, weak.backward(s))   # the two orders can be told apart here
+    plain.set_tuning(fp_pair=1)
+    assert torch.equal(plain.backward(s), paired)

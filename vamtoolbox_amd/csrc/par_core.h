@@ -1287,11 +1287,12 @@ struct BpNode {
 // mirrored nodes common to both angles of a pair
 __host__ __device__ __forceinline__ int bp_jlo(const ParDev& g) { return max(0, 2 * g.c + g.pair_D - (g.n - 1)); }
 __host__ __device__ __forceinline__ int bp_jhi(const ParDev& g) { return min(g.n - 1, 2 * g.c + g.pair_D); }
-// whether opposite angles are combined: only where they share an interval, that is
-// two nodes.  Of a single common node (n = 2, or a detector shifted by half its
-// width) neither neighbour is a bin of both angles.
+// whether opposite angles are combined (not where the tuning's fp_pair = 0 keeps the
+// plan unpaired): only where they share an interval, that is two nodes.  Of a
+// single common node (n = 2, or a detector shifted by half its width) neither
+// neighbour is a bin of both angles.
 __host__ __device__ inline bool bp_combines(const ParDev& g) {
-  return g.mu == 0.0 && g.pair_ok && bp_jhi(g) > bp_jlo(g);
+  return g.mu == 0.0 && g.pair_ok && g.fp_pair && bp_jhi(g) > bp_jlo(g);
 }
 
 // which nodes a pass over the angles takes: of every angle (COMB: of the pairs,
