@@ -551,3 +551,22 @@ def test_adjoint_wave_kernels_bitwise(gpu, case):
     e2 = rel_l2(bw[:, :, z].cpu().numpy(), d1.backward_adjoint(vol[:, :, z], ang, **kw))
     print("rel L2 F^T %.3e B^T %.3e" % (e1, e2))
     assert e1 <= TOL and e2 <= TOL
+
+
+@pytest.mark.parametrize("kind", ["plain", "occluded", "inclined", "thin"])
+def test_autotune_times_what_a_setting_changes(gpu, kind):
+    """One time per setting that changes the code or the order: z values per lane for the back projection, the
+    tile (the order of the forward's transpose) for that, none where it is not available."""
+    import torch
+    from vamtoolbox_amd.parallel import ParallelPlan
+    n, nz = {"plain": 24, "occluded": 26, "inclined": 28, "thin": 30}[kind], (3 if kind == "thin" else 40)
+    occ = np.zeros((n, n, nz))
+    occ[10:13, 10:13] = 1.0
+    plan = ParallelPlan(n, nz, np.arange(0.0, 360.0, 20.0), device=gpu, incl_deg=5.0 if kind == "inclined" else 0.0,
+                        occlusion=occ if kind == "occluded" else None)
+    rep = plan.autotune(reps=1)
+    zvs = [zv for _, zv in rep["backward"]]
+    tiles = [tile for tile, _ in rep["forward_adjoint"]]
+    assert sorted(zvs) == sorted({zv for _, zv in ParallelPlan.BP_CANDIDATES})
+    assert len(tiles) == len(set(tiles)) and bool(tiles) == (kind != "occluded")
+    assert rep["choice"]["bp_zv"] in zvs and rep["choice"]["bp_tile"] in (tiles or [8])

@@ -63,6 +63,7 @@ class ParallelPlan:
             det_offset=self.det_offset, incl_deg=self.incl_deg, mu=self.mu, radius=self.radius,
             outside_mask=mask.ctypes.data_as(ctypes.POINTER(ctypes.c_uint8)), flags=flags,
             occlusion=None if occ is None else occ.ctypes.data_as(ctypes.POINTER(ctypes.c_uint8)))
+        self.occluded = occ is not None
         handle = ctypes.c_void_p()
         with torch.cuda.device(self.device):
             _lib.check(self.lib.vamx_par_create(ctypes.byref(geom), ctypes.byref(handle)), "vamx_par_create")
@@ -143,9 +144,10 @@ class ParallelPlan:
     BP_CANDIDATES = [(8, 4), (16, 4), (4, 4), (32, 4), (8, 2), (16, 2)]
 
     def autotune(self, vol: torch.Tensor | None = None, sino: torch.Tensor | None = None, reps: int = 3) -> dict:
-        """Time the forward and back projection for each candidate work order
-        (tile shape x z values per lane) on this plan's shape and keep the
-        fastest of each; returns {setting: time_ms} plus the choice.  Results
+        """Time the forward (tile shape x z values per lane), the back
+        projection (z values per lane) and the forward's transpose (tile) for
+        each candidate work order on this plan's shape and keep the fastest of
+        each; returns {setting: time_ms} plus the choice.  Results
         are cached per (n, nz, angles, absorption on/off, inclination on/off,
         detector offset) -- the angles and the offset decide the pairing."""
         key = (self.n, self.nz, self.na, self.mu != 0.0, self.incl_deg != 0.0, self.det_offset,
@@ -171,17 +173,28 @@ class ParallelPlan:
             torch.cuda.synchronize(dev)
             return a.elapsed_time(b) / reps
 
-        report = {"forward": {}, "backward": {}}
+        report = {"forward": {}, "backward": {}, "forward_adjoint": {}}
         for ta, tk, zv, ru, pr in self.FP_CANDIDATES:
             self.set_tuning(fp_tile_angles=ta, fp_tile_rays=tk, fp_zv=zv, fp_reuse=ru, fp_pair=pr)
             report["forward"][(ta, tk, zv, ru, pr)] = timed(lambda: self.forward(vol, out=out_s))
-        for tile, zv in self.BP_CANDIDATES:
-            self.set_tuning(bp_tile=tile, bp_zv=zv)
-            report["backward"][(tile, zv)] = timed(lambda: self.backward(sino, out=out_v))
         fbest = min(report["forward"], key=report["forward"].get)
-        bbest = min(report["backward"], key=report["backward"].get)
+        self.set_tuning(fp_tile_angles=fbest[0], fp_tile_rays=fbest[1], fp_zv=fbest[2], fp_reuse=fbest[3],
+                        fp_pair=fbest[4])
+        # the back projection's time depends on the z values per lane only, the tile is
+        # the work order of the forward's transpose
+        tile0 = self.BP_CANDIDATES[0][0]
+        for zv in dict.fromkeys(zv for _, zv in self.BP_CANDIDATES):
+            self.set_tuning(bp_tile=tile0, bp_zv=zv)
+            report["backward"][(tile0, zv)] = timed(lambda: self.backward(sino, out=out_v))
+        zv = min(report["backward"], key=report["backward"].get)[1]
+        tile = tile0
+        if not self.occluded:   # (the transposes are not available with occlusion)
+            for tile in dict.fromkeys(t for t, z in self.BP_CANDIDATES if z == zv):
+                self.set_tuning(bp_tile=tile, bp_zv=zv)
+                report["forward_adjoint"][(tile, zv)] = timed(lambda: self.forward_adjoint(sino, out=out_v))
+            tile = min(report["forward_adjoint"], key=report["forward_adjoint"].get)[0]
         choice = dict(fp_tile_angles=fbest[0], fp_tile_rays=fbest[1], fp_zv=fbest[2], fp_reuse=fbest[3],
-                      fp_pair=fbest[4], bp_tile=bbest[0], bp_zv=bbest[1])
+                      fp_pair=fbest[4], bp_tile=tile, bp_zv=zv)
         self.set_tuning(**choice)
         report["choice"] = choice
         _TUNING_CACHE[key] = report
