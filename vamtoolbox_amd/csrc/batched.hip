@@ -301,13 +301,13 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
 // apart; backward + 8: contiguous, + 16: opposite angles combined); -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
 // kOwnLaunch for plans whose kernels the persistent launch does not hold
 constexpr int kOwnLaunch = 0;
-int problem_path(vamx_plan* p, const float* in, float* out, bool forward) {
+int problem_path(vamx_plan* p, const float* in, float* out, bool forward, int problems) {
   if (incl_wave_ok(p) || thin_ok(p)) return kOwnLaunch;
   if (forward) {
     const FpLayout l = fp_layout(p, (uintptr_t)in | (uintptr_t)out);
     if (l.zv) return l.zv | (l.split ? 8 : 0);
   } else {
-    const BpLayout l = bp_layout(p, (uintptr_t)in | (uintptr_t)out);
+    const BpLayout l = bp_layout(p, (uintptr_t)in | (uintptr_t)out, problems);
     if (l.zv) return l.zv | (l.contig ? 8 : 0) | (l.comb ? 16 : 0);
   }
   return par_use_vec4(p, in, out) ? -4 : -1;
@@ -430,7 +430,7 @@ int run_batch(vamx_batch* b, const float* const* ins, float* const* outs, hipStr
   for (int i = 0; i < n; ++i) {
     if (!ins[i] || !outs[i]) return set_error(VAMX_ERR_ARG, "batch: null buffer of problem " + std::to_string(i));
     vamx_plan* p = b->plans[(size_t)i];
-    sig[(size_t)i] = problem_path(p, ins[i], outs[i], forward);
+    sig[(size_t)i] = problem_path(p, ins[i], outs[i], forward, n);
     std::memcpy(devs.data() + (size_t)i * sizeof(ParDev), &p->par, sizeof(ParDev));
   }
   vamx_batch::Layout* L = nullptr;

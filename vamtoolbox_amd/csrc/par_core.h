@@ -1863,7 +1863,7 @@ void bp_dispatch(const BpLayout& l, F&& f) {
 int par_slice_minmax(vamx_plan* p, const float* vol, hipStream_t s);
 int par_forward_launch(vamx_plan* p, const float* vol, float* sino, hipStream_t s, bool warp_clip);
 int par_backward_launch(vamx_plan* p, const float* sino, float* vol, hipStream_t s, bool clipc);
-BpLayout bp_layout(const vamx_plan* p, uintptr_t align_bits);
+BpLayout bp_layout(const vamx_plan* p, uintptr_t align_bits, int problems = 1);   // problems: of one launch
 bool par_use_vec4(const vamx_plan* p, const void* a, const void* b);
 bool par_use_vec2(const vamx_plan* p, const void* a, const void* b);
 int par_wave_zv(const vamx_plan* p, const void* a, const void* b, int requested);

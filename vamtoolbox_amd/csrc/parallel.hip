@@ -414,23 +414,39 @@ int vamx::par_wave_zv(const vamx_plan* p, const void* a, const void* b, int requ
   return wave_zv_choice(p->par.nz, (uintptr_t)a | (uintptr_t)b, requested);
 }
 
-BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits) {
+BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits, int problems) {
   const ParDev& g = p->par;
   BpLayout l;
   if ((p->flags & VAMX_PAR_PER_LANE_GEOMETRY) || g.incl || g.n < 2 || g.occ || g.nz < 32) return l;
-  // slices per lane, at most the tuning's bp_zv: the fewest slice slots, then
-  // the fewest chunks (the geometry is evaluated per chunk)
-  int slots = 0;
+  l.comb = bp_combines(g);
+  // slices per lane, at most the tuning's bp_zv: the least time, in 10 us of a pass
+  // over 256 x 256 columns and 360 angles per chunk, measured by slices per lane 64
+  // apart and (cost16) with 16-byte loads of four, angle by angle and with opposite
+  // angles combined.  255 slices, angle by angle: 0.92 ms as one chunk of four, 0.68
+  // as two of two; 300, combined: 0.76 as five of one, 0.99 as two of three.
+  //
+  // Where the active patches are few, a lane's chain of slices is what takes the
+  // time, and fewer slices per lane and more wavefronts are faster: four need 1.5
+  // wavefronts per SIMD (96 x 96 x 256, 120 angles, 930 of them: 78 us, as 3700 of one
+  // slice 55; 128 x 128 x 256, 180 angles, 1650: 120 and 120), two need 2 per SIMD (128
+  // x 128 x 128, 1650: 101 us, as 3300 of one slice 90; 192 x 192 x 128, 240 angles,
+  // 3680: 168 and 228).  Problems of a batch fill the GPU together.
+  constexpr int costs[2][5] = {{0, 21, 33, 48, 92}, {0, 16, 29, 43, 57}}, costs16[2] = {56, 45};
+  constexpr int waves[5] = {0, 0, 2048, 1536, 1536};
+  const int* const cost = costs[l.comb ? 1 : 0];
+  const int cost16 = costs16[l.comb ? 1 : 0];
+  int best = INT_MAX;
   for (int zv = 1; zv <= g.bp_zv; ++zv) {
     const int c = wave_zchunks(g.nz, zv);
-    if (!slots || c * zv <= slots) {
-      l.zv = zv;
-      l.chunks = c;
-      slots = c * zv;
-    }
+    if ((long long)g.bp_act * c * problems < waves[zv]) continue;
+    const bool contig = zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0;
+    const int t = c * (contig ? cost16 : cost[zv]);
+    if (t >= best) continue;
+    best = t;
+    l.zv = zv;
+    l.chunks = c;
+    l.contig = contig;
   }
-  l.contig = l.zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0;
-  l.comb = bp_combines(g);
   return l;
 }
 
