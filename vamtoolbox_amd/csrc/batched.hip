@@ -42,7 +42,6 @@ struct BatchItem {
 // Buffers of the problems of one launch, passed by value as a kernel
 // argument (so a captured graph holds them and no device table changes from
 // call to call): entry r belongs to the problem at table position r.
-constexpr int kBatchChunk = 64;
 struct BatchPtrs {
   const float* in[kBatchChunk];
   float* out[kBatchChunk];
@@ -230,10 +229,19 @@ struct vamx_batch {
     std::vector<int> order;        // table position -> problem index
     std::vector<int> minmax;       // forward: problems whose per-slice min/max the warp clip needs
   };
+  struct Group {                   // thin or inclined problems of one class, in one launch
+    int key = 0;
+    LaneProblem* d_items = nullptr;
+    std::vector<int> order;        // table position -> problem index
+    std::vector<unsigned> begin;   // first block of each
+    unsigned blocks = 0;
+    bool minmax = false;           // the warp clip needs the slices' min/max
+  };
   struct Layout {
     std::vector<int> sig;          // per problem: kernel path chosen for the buffers' alignment
     std::vector<char> devs;        // the plans' ParDev bytes (work order set by vamx_par_set_tuning)
     std::vector<int> single;       // problems projected by their own single-problem launch
+    std::vector<Group> groups;
     std::vector<Chunk> chunks;
   };
   std::vector<Layout> layouts[2];  // [0] backward, [1] forward
@@ -250,14 +258,18 @@ constexpr size_t kMaxLayouts = 8;
 
 bool check_batch(const vamx_batch* b) { return b && b->magic == kBatchMagic; }
 
+void free_tables(vamx_batch::Layout& l) {
+  for (auto& c : l.chunks) (void)hipFree(c.d_items);
+  for (auto& g : l.groups) (void)hipFree(g.d_items);
+}
+
 void release_batch(vamx_batch* b) {
   int cur = 0;
   (void)hipGetDevice(&cur);
   if (cur != b->device) (void)hipSetDevice(b->device);
   (void)hipDeviceSynchronize();
   for (auto& ls : b->layouts)
-    for (auto& l : ls)
-      for (auto& c : l.chunks) (void)hipFree(c.d_items);
+    for (auto& l : ls) free_tables(l);
   if (b->d_counter) (void)hipFree(b->d_counter);
   for (int j = 0; j < kSideStreams; ++j) {
     if (b->join[j]) (void)hipEventDestroy(b->join[j]);
@@ -298,11 +310,24 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
 }
 
 // kernel path of problem i for these buffers: slices per lane (forward + 8: 64
-// apart; backward + 8: contiguous, + 16: opposite angles combined); -1 / -4 for the per-lane kernels with 1 / 4 z per thread, or
-// kOwnLaunch for plans whose kernels the persistent launch does not hold
+// apart; backward + 8: contiguous, + 16: opposite angles combined); -1 / -4 for
+// the per-lane kernels with 1 / 4 z per thread; the class of a thin or inclined
+// problem (1 << 16 and up), or kOwnLaunch where it has a launch of its own
 constexpr int kOwnLaunch = 0;
+// Thin and inclined problems run on kernels that the persistent launch does not
+// hold.  Below this many wavefronts (4 per SIMD) one cannot fill the GPU, and its
+// launch takes longer than its work: those of a class share a launch.
+constexpr long long kOwnWaves = 4096;
+LaneClass lane_class(const vamx_plan* p, const float* in, const float* out, bool forward) {
+  const bool clip = !(p->flags & (forward ? VAMX_PAR_NO_WARP_CLIP : VAMX_PAR_NO_CIRCLE_CLIP));
+  return incl_wave_ok(p) ? incl_class(p, forward, clip) : thin_class(p, in, out, forward, clip);
+}
 int problem_path(vamx_plan* p, const float* in, float* out, bool forward, int problems) {
-  if (incl_wave_ok(p) || thin_ok(p)) return kOwnLaunch;
+  if (incl_wave_ok(p) || thin_ok(p)) {
+    if (problems == 1) return kOwnLaunch;
+    const LaneClass c = lane_class(p, in, out, forward);
+    return c.waves < kOwnWaves ? c.key : kOwnLaunch;
+  }
   if (forward) {
     const FpLayout l = fp_layout(p, (uintptr_t)in | (uintptr_t)out);
     if (l.zv) return l.zv | (l.split ? 8 : 0);
@@ -313,8 +338,8 @@ int problem_path(vamx_plan* p, const float* in, float* out, bool forward, int pr
   return par_use_vec4(p, in, out) ? -4 : -1;
 }
 
-int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<char>& devs, bool forward,
-                 hipStream_t s, vamx_batch::Layout** out) {
+int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<char>& devs, const float* const* ins,
+                 float* const* outs, bool forward, hipStream_t s, vamx_batch::Layout** out) {
   std::vector<vamx_batch::Layout>& ls = b->layouts[forward ? 1 : 0];
   if (ls.size() >= kMaxLayouts)
     return set_error(VAMX_ERR_ARG, "batch: more than 8 distinct buffer alignments or work orders on one batch");
@@ -340,6 +365,15 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
     const int path = sig[(size_t)i];
     if (path == kOwnLaunch) {
       L.single.push_back(i);
+      continue;
+    }
+    if (path >= 1 << 16) {
+      // an open group of the class, or a new one
+      auto g = std::find_if(L.groups.begin(), L.groups.end(), [&](const vamx_batch::Group& q) {
+        return q.key == path && q.order.size() < (size_t)kBatchChunk;
+      });
+      if (g == L.groups.end()) g = L.groups.insert(g, vamx_batch::Group{path});
+      g->order.push_back(i);
       continue;
     }
     if (path > 0 && !forward) {
@@ -374,7 +408,7 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
     const ParDev& c = items[(size_t)y].g;
     return (double)a.n * a.n * a.na * a.nz > (double)c.n * c.n * c.na * c.nz;
   });
-  if (!shared.empty()) {
+  if (!shared.empty() || !L.groups.empty()) {
     // a new table: blocking upload (not allowed under graph capture, where
     // hipStreamSynchronize fails and the error is returned)
     VAMX_HIP(hipStreamSynchronize(s));
@@ -398,13 +432,45 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
     if (e != hipSuccess) rc = hip_check(e, "batch table upload");
     L.chunks.push_back(std::move(ch));
   }
+  for (auto& g : L.groups) {
+    if (rc != VAMX_OK) break;
+    std::vector<LaneProblem> tab;
+    for (const int i : g.order) {
+      const LaneClass c = lane_class(b->plans[(size_t)i], ins[i], outs[i], forward);
+      tab.push_back(c.problem);
+      g.begin.push_back(g.blocks);
+      g.blocks += (unsigned)c.blocks;
+      g.minmax |= forward && c.problem.clip && !c.problem.g.incl;
+    }
+    hipError_t e = hipMalloc((void**)&g.d_items, tab.size() * sizeof(LaneProblem));
+    if (e == hipSuccess) e = hipMemcpy(g.d_items, tab.data(), tab.size() * sizeof(LaneProblem), hipMemcpyHostToDevice);
+    if (e != hipSuccess) rc = hip_check(e, "batch table upload");
+  }
   if (rc != VAMX_OK) {
-    for (auto& c : L.chunks) (void)hipFree(c.d_items);
+    free_tables(L);
     return rc;
   }
   ls.push_back(std::move(L));
   *out = &ls.back();
   return VAMX_OK;
+}
+
+// the group's problems, in one launch (and their slices' ranges before it)
+int run_group(const vamx_batch* b, const vamx_batch::Group& g, const float* const* ins, float* const* outs,
+              hipStream_t s) {
+  LaneTable t;
+  std::memset(&t, 0, sizeof(t));
+  t.items = g.d_items;
+  t.m = (int)g.order.size();
+  for (int r = 0; r < t.m; ++r) {
+    const int i = g.order[(size_t)r];
+    if (vamx_plan* p = b->plans[(size_t)i]; g.minmax && !(p->flags & VAMX_PAR_NO_WARP_CLIP))
+      if (const int rc = par_slice_minmax(p, ins[i], s)) return rc;
+    t.begin[r] = g.begin[(size_t)r];
+    t.in[r] = ins[i];
+    t.out[r] = outs[i];
+  }
+  return g.key >> 16 == 1 ? thin_batch(g.key, t, g.blocks, s) : incl_batch(g.key, t, g.blocks, s);
 }
 
 int ensure_side_streams(vamx_batch* b) {
@@ -434,31 +500,47 @@ int run_batch(vamx_batch* b, const float* const* ins, float* const* outs, hipStr
     std::memcpy(devs.data() + (size_t)i * sizeof(ParDev), &p->par, sizeof(ParDev));
   }
   vamx_batch::Layout* L = nullptr;
-  for (auto& l : b->layouts[forward ? 1 : 0])
-    if (l.sig == sig && l.devs == devs) {
-      L = &l;
-      break;
+  auto find = [&]() {
+    for (auto& l : b->layouts[forward ? 1 : 0])
+      if (l.sig == sig && l.devs == devs) L = &l;
+  };
+  find();
+  if (!L && std::any_of(sig.begin(), sig.end(), [](int p) { return p >= 1 << 16; })) {
+    // a table cannot be uploaded while the stream is captured: thin and inclined
+    // problems then have launches of their own, which need none
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      for (int& p : sig)
+        if (p >= 1 << 16) p = kOwnLaunch;
+      find();
     }
+  }
   if (!L) {
-    int rc = build_layout(b, sig, devs, forward, s, &L);
+    int rc = build_layout(b, sig, devs, ins, outs, forward, s, &L);
     if (rc) return rc;
   }
-  // single-problem launches round-robin on the caller's stream and
+  // single-problem launches and those of the groups round-robin on the caller's stream and
   // two side streams forked from and joined back to it with events (so the
   // call stays graph-capturable): one launch's tail overlaps the next one's
   // start
-  if (!L->single.empty()) {
+  const size_t singles = L->single.size(), launches = singles + L->groups.size();
+  if (launches) {
     int ns = 1;
-    if (L->single.size() > 1 && ensure_side_streams(b) == VAMX_OK) ns = 1 + kSideStreams;
+    if (launches > 1 && ensure_side_streams(b) == VAMX_OK) ns = 1 + kSideStreams;
     if (ns > 1) {
       VAMX_HIP(hipEventRecord(b->fork, s));
       for (int j = 0; j < kSideStreams; ++j) VAMX_HIP(hipStreamWaitEvent(b->side[j], b->fork, 0));
     }
     int rc = VAMX_OK;
-    for (size_t k = 0; k < L->single.size() && rc == VAMX_OK; ++k) {
+    for (size_t k = 0; k < launches && rc == VAMX_OK; ++k) {
+      hipStream_t st = (k % ns == 0) ? s : b->side[k % ns - 1];
+      if (k >= singles) {
+        rc = run_group(b, L->groups[k - singles], ins, outs, st);
+        continue;
+      }
       const int i = L->single[k];
       vamx_plan* p = b->plans[(size_t)i];
-      hipStream_t st = (k % ns == 0) ? s : b->side[k % ns - 1];
       rc = forward ? par_forward_launch(p, ins[i], outs[i], st, !(p->flags & VAMX_PAR_NO_WARP_CLIP))
                    : par_backward_launch(p, ins[i], outs[i], st, !(p->flags & VAMX_PAR_NO_CIRCLE_CLIP));
     }

@@ -95,11 +95,13 @@ __device__ __forceinline__ void incl_combine(float (&lo)[NS], float (&hi)[NS], i
 // rows of one wavefront
 template <int NS, int L> constexpr int incl_rows() { return (L < 64 ? L : 64 * NS) - 1; }
 
+// (lb in the functions of a block: its number in the problem)
 template <int NS, int L, class Out>
-__global__ __launch_bounds__(256) void incl_fp_kernel(ParDev g, const float* __restrict__ vol, Out out) {
+__device__ __forceinline__ void incl_fp_block(const ParDev& g, const float* __restrict__ vol, const Out& out,
+                                              unsigned lb) {
   constexpr int G = 64 / L, S = incl_rows<NS, L>();
   const int lane = threadIdx.x & 63, l = lane & (L - 1), grp = lane / L;
-  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long wave = wave_index(lb);
   const long long rays = (long long)g.n * g.na;
   const int nch = (g.nz + S - 1) / S;
   if (wave >= rays * nch) return;   // whole wavefronts
@@ -200,6 +202,16 @@ __global__ __launch_bounds__(256) void incl_fp_kernel(ParDev g, const float* __r
     if (grp == 0 && so < S && j0 + so < nz) out.put(((size_t)k * g.na + i) * nz + j0 + so, lo[s]);
   }
 }
+template <int NS, int L, class Out>
+__global__ __launch_bounds__(256) void incl_fp_kernel(ParDev g, const float* __restrict__ vol, Out out) {
+  incl_fp_block<NS, L>(g, vol, out, xcd_remap(blockIdx.x, gridDim.x));
+}
+template <int NS, int L>
+__global__ __launch_bounds__(256) void incl_fp_batch_kernel(LaneTable t) {
+  unsigned lb;
+  const int p = lane_problem(t, lb);
+  incl_fp_block<NS, L>(t.items[p].g, t.in[p], StoreOut{t.out[p]}, lb);
+}
 
 // Forward of one ray where the shift over the whole ray is small against the
 // lanes: lanes own fixed slices, so that a sample finds the taps it shares with
@@ -216,9 +228,6 @@ __global__ __launch_bounds__(256) void incl_fp_kernel(ParDev g, const float* __r
 // vector instructions per sample, against 8 loads and 24 with the rows' own lanes,
 // which the texture path bound): 128 x 128 x 96 x 180, 12 degrees 279 -> 207 us, x 256
 // x 90 398 -> 285, 100 x 100 x 300 x 60, 10 degrees 177 -> 122.
-struct InclShift {
-  int lo, rows;   // least shift of a ray's samples, detector rows of a wavefront
-};
 // values of the next / previous slice (lane, and across the NS registers); 0 past
 // the ends
 template <int NS>
@@ -233,10 +242,10 @@ __device__ __forceinline__ float slice_prev(const float (&v)[NS], int s) {
 }
 
 template <int NS, class Out>
-__global__ __launch_bounds__(256) void incl_fp_fixed_kernel(ParDev g, const float* __restrict__ vol, InclShift shift,
-                                                            Out out) {
+__device__ __forceinline__ void incl_fp_fixed_block(const ParDev& g, const float* __restrict__ vol,
+                                                    const InclShift& shift, const Out& out, unsigned lb) {
   const int lane = threadIdx.x & 63;
-  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long wave = wave_index(lb);
   const long long rays = (long long)g.n * g.na;
   const int nch = (g.nz + shift.rows - 1) / shift.rows;
   if (wave >= rays * nch) return;   // whole wavefronts
@@ -375,13 +384,25 @@ __global__ __launch_bounds__(256) void incl_fp_fixed_kernel(ParDev g, const floa
     if (j >= j0 && j < j0 + shift.rows && j < nz) out.put(((size_t)k * g.na + i) * nz + j, acc[s]);
   }
 }
+template <int NS, class Out>
+__global__ __launch_bounds__(256) void incl_fp_fixed_kernel(ParDev g, const float* __restrict__ vol, InclShift shift,
+                                                            Out out) {
+  incl_fp_fixed_block<NS>(g, vol, shift, out, xcd_remap(blockIdx.x, gridDim.x));
+}
+template <int NS>
+__global__ __launch_bounds__(256) void incl_fp_fixed_batch_kernel(LaneTable t) {
+  unsigned lb;
+  const int p = lane_problem(t, lb);
+  const LaneProblem& q = t.items[p];
+  incl_fp_fixed_block<NS>(q.g, t.in[p], q.shift, StoreOut{t.out[p]}, lb);
+}
 
 template <int NS, int L>
-__global__ __launch_bounds__(256) void incl_bp_kernel(ParDev g, const float* __restrict__ sino,
-                                                      float* __restrict__ vol, int clipc) {
+__device__ __forceinline__ void incl_bp_block(const ParDev& g, const float* __restrict__ sino, float* __restrict__ vol,
+                                              int clipc, unsigned lb) {
   constexpr int G = 64 / L, S = incl_rows<NS, L>();
   const int lane = threadIdx.x & 63, l = lane & (L - 1), grp = lane / L;
-  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long wave = wave_index(lb);
   // consecutive wavefronts walk 8 x 8 patches of voxel columns (neighbouring
   // columns read the same detector rows)
   const int n = g.n, nz = g.nz, nt = (n + 7) / 8;
@@ -473,6 +494,18 @@ __global__ __launch_bounds__(256) void incl_bp_kernel(ParDev g, const float* __r
     if (grp == 0 && so < S && j0 + so < nz) vol[((size_t)row * n + col) * nz + j0 + so] = lo[s];
   }
 }
+template <int NS, int L>
+__global__ __launch_bounds__(256) void incl_bp_kernel(ParDev g, const float* __restrict__ sino,
+                                                      float* __restrict__ vol, int clipc) {
+  incl_bp_block<NS, L>(g, sino, vol, clipc, xcd_remap(blockIdx.x, gridDim.x));
+}
+template <int NS, int L>
+__global__ __launch_bounds__(256) void incl_bp_batch_kernel(LaneTable t) {
+  unsigned lb;
+  const int p = lane_problem(t, lb);
+  const LaneProblem& q = t.items[p];
+  incl_bp_block<NS, L>(q.g, t.in[p], t.out[p], q.clip, lb);
+}
 
 // slabs of 64 rows per wavefront: a wavefront's geometry costs about 0.7 of a
 // slab's walk, so NS minimises chunks (NS + 0.7)
@@ -489,15 +522,43 @@ int incl_slabs(int nz) {
   return best;
 }
 
+// slabs, and lanes of a row group, as slabs << 8 | lanes
+int incl_layout(int nz) {
+  if (nz <= 31) return 1 << 8 | (nz <= 7 ? 8 : nz <= 15 ? 16 : 32);
+  return incl_slabs(nz) << 8 | 64;
+}
 template <class F>
-void incl_dispatch(int nz, F&& f) {
+void incl_dispatch(int layout, F&& f) {
   using std::integral_constant;
-  if (nz <= 7) f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
-  else if (nz <= 15) f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
-  else if (nz <= 31) f(integral_constant<int, 1>{}, integral_constant<int, 32>{});
-  else if (incl_slabs(nz) == 1) f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
-  else if (incl_slabs(nz) == 2) f(integral_constant<int, 2>{}, integral_constant<int, 64>{});
+  if (layout == (1 << 8 | 8)) f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+  else if (layout == (1 << 8 | 16)) f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+  else if (layout == (1 << 8 | 32)) f(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+  else if (layout == (1 << 8 | 64)) f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
+  else if (layout == (2 << 8 | 64)) f(integral_constant<int, 2>{}, integral_constant<int, 64>{});
   else f(integral_constant<int, 3>{}, integral_constant<int, 64>{});
+}
+template <class F>
+void incl_fixed_dispatch(int ns, F&& f) {
+  using std::integral_constant;
+  if (ns == 4) f(integral_constant<int, 4>{});
+  else if (ns == 3) f(integral_constant<int, 3>{});
+  else if (ns == 2) f(integral_constant<int, 2>{});
+  else f(integral_constant<int, 1>{});
+}
+// wavefronts of a problem
+long long incl_fixed_waves(const ParDev& g, const InclShift& shift) {
+  return (long long)g.n * g.na * ((g.nz + shift.rows - 1) / shift.rows);
+}
+template <int NS, int L>
+long long incl_fp_waves(const ParDev& g) {
+  constexpr int S = incl_rows<NS, L>();
+  return (long long)g.n * g.na * ((g.nz + S - 1) / S);
+}
+template <int NS, int L>
+long long incl_bp_waves(const ParDev& g) {
+  constexpr int S = incl_rows<NS, L>();
+  const long long nt = (g.n + 7) / 8;
+  return 64 * nt * nt * ((g.nz + S - 1) / S);
 }
 
 // whether the forward runs with fixed slices, and with how many slices per lane
@@ -531,21 +592,18 @@ template <class Out>
 int incl_forward(vamx_plan* p, const float* vol, Out out, hipStream_t s) {
   const ParDev& g = p->par;
   InclShift shift;
-  if (const int ns = incl_fixed(g, shift)) {
-    const long long waves = (long long)g.n * g.na * ((g.nz + shift.rows - 1) / shift.rows);
-    const dim3 grid(blocks_for(waves * 64, 256)), block(256);
-    if (ns == 4) hipLaunchKernelGGL((incl_fp_fixed_kernel<4, Out>), grid, block, 0, s, g, vol, shift, out);
-    else if (ns == 3) hipLaunchKernelGGL((incl_fp_fixed_kernel<3, Out>), grid, block, 0, s, g, vol, shift, out);
-    else if (ns == 2) hipLaunchKernelGGL((incl_fp_fixed_kernel<2, Out>), grid, block, 0, s, g, vol, shift, out);
-    else hipLaunchKernelGGL((incl_fp_fixed_kernel<1, Out>), grid, block, 0, s, g, vol, shift, out);
-    VAMX_HIP(hipGetLastError());
-    return VAMX_OK;
+  if (const int fixed = incl_fixed(g, shift)) {
+    incl_fixed_dispatch(fixed, [&](auto ns) {
+      hipLaunchKernelGGL((incl_fp_fixed_kernel<decltype(ns)::value, Out>),
+                         dim3(blocks_for(incl_fixed_waves(g, shift) * 64, 256)), dim3(256), 0, s, g, vol, shift, out);
+    });
+  } else {
+    incl_dispatch(incl_layout(g.nz), [&](auto ns, auto l) {
+      constexpr int NS = decltype(ns)::value, L = decltype(l)::value;
+      const dim3 grid(blocks_for(incl_fp_waves<NS, L>(g) * 64, 256));
+      hipLaunchKernelGGL((incl_fp_kernel<NS, L, Out>), grid, dim3(256), 0, s, g, vol, out);
+    });
   }
-  incl_dispatch(g.nz, [&](auto ns, auto l) {
-    constexpr int NS = decltype(ns)::value, L = decltype(l)::value, S = incl_rows<NS, L>();
-    const long long waves = (long long)g.n * g.na * ((g.nz + S - 1) / S);
-    hipLaunchKernelGGL((incl_fp_kernel<NS, L, Out>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, vol, out);
-  });
   VAMX_HIP(hipGetLastError());
   return VAMX_OK;
 }
@@ -566,12 +624,50 @@ int incl_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, hi
 
 int incl_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s) {
   const ParDev& g = p->par;
-  incl_dispatch(g.nz, [&](auto ns, auto l) {
-    constexpr int NS = decltype(ns)::value, L = decltype(l)::value, S = incl_rows<NS, L>();
-    const long long nt = (g.n + 7) / 8, waves = 64 * nt * nt * ((g.nz + S - 1) / S);
-    hipLaunchKernelGGL((incl_bp_kernel<NS, L>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, sino, vol,
-                       clipc ? 1 : 0);
+  incl_dispatch(incl_layout(g.nz), [&](auto ns, auto l) {
+    constexpr int NS = decltype(ns)::value, L = decltype(l)::value;
+    const dim3 grid(blocks_for(incl_bp_waves<NS, L>(g) * 64, 256));
+    hipLaunchKernelGGL((incl_bp_kernel<NS, L>), grid, dim3(256), 0, s, g, sino, vol, clipc ? 1 : 0);
   });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+// class of a problem: 2 << 16, 1 << 15 forward, then fixed slices 1 << 14 | slices
+// per lane, or incl_layout
+LaneClass incl_class(const vamx_plan* p, bool forward, bool clip) {
+  const ParDev& g = p->par;
+  LaneClass c;
+  if (!incl_wave_ok(p)) return c;
+  c.problem.g = g;
+  c.problem.clip = clip;
+  const int fixed = forward ? incl_fixed(g, c.problem.shift) : 0, layout = incl_layout(g.nz);
+  if (fixed) {
+    c.waves = incl_fixed_waves(g, c.problem.shift);
+  } else {
+    incl_dispatch(layout, [&](auto ns, auto l) {
+      constexpr int NS = decltype(ns)::value, L = decltype(l)::value;
+      c.waves = forward ? incl_fp_waves<NS, L>(g) : incl_bp_waves<NS, L>(g);
+    });
+  }
+  c.blocks = (c.waves + 3) / 4;
+  c.key = 2 << 16 | (forward ? 1 << 15 : 0) | (fixed ? 1 << 14 | fixed : layout);
+  return c;
+}
+
+int incl_batch(int key, const LaneTable& t, unsigned blocks, hipStream_t s) {
+  const dim3 grid(blocks), block(256);
+  if (key >> 14 & 1) {
+    incl_fixed_dispatch(key & 7, [&](auto ns) {
+      hipLaunchKernelGGL((incl_fp_fixed_batch_kernel<decltype(ns)::value>), grid, block, 0, s, t);
+    });
+  } else {
+    incl_dispatch(key & 0x3fff, [&](auto ns, auto l) {
+      constexpr int NS = decltype(ns)::value, L = decltype(l)::value;
+      if (key >> 15 & 1) hipLaunchKernelGGL((incl_fp_batch_kernel<NS, L>), grid, block, 0, s, t);
+      else hipLaunchKernelGGL((incl_bp_batch_kernel<NS, L>), grid, block, 0, s, t);
+    });
+  }
   VAMX_HIP(hipGetLastError());
   return VAMX_OK;
 }

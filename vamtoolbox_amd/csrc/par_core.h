@@ -1871,16 +1871,59 @@ FpLayout fp_layout(const vamx_plan* p, uintptr_t align_bits);
 int wave_zv_choice(int nz, uintptr_t align_bits, int requested);
 void par_pair_units(const std::vector<double>& cs, int na, int n, int c, double D, std::vector<int>& units,
                     int& npaired_rays, int& first2);
+// Problems of a batch that share one launch of a thin or inclined kernel: those of
+// one class (kernel, lanes, slices per lane, wavefronts per block).  A block finds
+// its problem by its number; the table is on the device, the buffers come with the
+// launch.
+constexpr int kBatchChunk = 64;   // problems per launch
+struct InclShift {
+  int lo = 0, rows = 0;   // least shift of a ray's samples, detector rows of a wavefront
+};
+struct LaneProblem {
+  ParDev g;
+  const float* minmax;
+  int clip, pair;
+  InclShift shift;
+};
+struct LaneTable {
+  const LaneProblem* items;
+  int m;
+  unsigned begin[kBatchChunk];   // first block of each
+  const float* in[kBatchChunk];
+  float* out[kBatchChunk];
+};
+// the calling block's problem and its number there; each XCD takes a contiguous
+// share of the problems' blocks
+__device__ __forceinline__ int lane_problem(const LaneTable& t, unsigned& lb) {
+  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
+  int lo = 0, hi = t.m - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (t.begin[mid] <= b) lo = mid;
+    else hi = mid - 1;
+  }
+  lb = b - t.begin[lo];
+  return lo;
+}
+struct LaneClass {
+  int key = 0;                // 0: none
+  long long blocks = 0, waves = 0;
+  LaneProblem problem{};
+};
 // inclined projections on wavefronts (incl.hip)
 bool incl_wave_ok(const vamx_plan* p);
 int incl_forward_store(vamx_plan* p, const float* vol, float* sino, hipStream_t s);
 int incl_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, hipStream_t s);
 int incl_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s);
+LaneClass incl_class(const vamx_plan* p, bool forward, bool clip);
+int incl_batch(int key, const LaneTable& t, unsigned blocks, hipStream_t s);
 // thin problems at zero inclination (thin.hip); the forward reads the plan's
 // slice min / max when clip is set
 bool thin_ok(const vamx_plan* p);
 int thin_forward_store(vamx_plan* p, const float* vol, float* sino, bool clip, hipStream_t s);
 int thin_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, bool clip, hipStream_t s);
 int thin_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s);
+LaneClass thin_class(const vamx_plan* p, const void* in, const void* out, bool forward, bool clip);
+int thin_batch(int key, const LaneTable& t, unsigned blocks, hipStream_t s);
 
 }  // namespace vamx

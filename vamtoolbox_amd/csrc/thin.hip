@@ -200,14 +200,16 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
   }
 }
 
+// one block's rays, lb the block's number in the problem
 template <int ZV, int L, int R, class Out>
-__global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __restrict__ vol,
-                                                      const float* __restrict__ minmax, int clip, int pair, Out out) {
+__device__ __forceinline__ void thin_fp_block(const ParDev& g, const float* __restrict__ vol,
+                                              const float* __restrict__ minmax, int clip, int pair, const Out& out,
+                                              unsigned lb) {
   using V = typename VecT<ZV>::T;
   static_assert(R == 1 || L == 1, "several rays per wavefront: one lane per ray and sample");
   const int lane = threadIdx.x & 63, z = (lane & (L - 1)) * ZV;
   const int zl = z < g.nz ? z : g.nz - ZV;   // lanes past nz read a copy and store nothing
-  const long long wave = wave_index(xcd_remap(blockIdx.x, gridDim.x));
+  const long long wave = wave_index(lb);
   int k, i, k2 = -1, i2 = -1;
   if constexpr (R > 1) {
     // wavefronts in ray order; a lane without a ray of its own walks the last
@@ -281,9 +283,23 @@ __global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __r
   }
 }
 
+template <int ZV, int L, int R, class Out>
+__global__ __launch_bounds__(256) void thin_fp_kernel(ParDev g, const float* __restrict__ vol,
+                                                      const float* __restrict__ minmax, int clip, int pair, Out out) {
+  thin_fp_block<ZV, L, R>(g, vol, minmax, clip, pair, out, xcd_remap(blockIdx.x, gridDim.x));
+}
 template <int ZV, int L>
-__global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __restrict__ sino,
-                                                       float* __restrict__ vol, int clipc) {
+__global__ __launch_bounds__(256) void thin_fp_batch_kernel(LaneTable t) {
+  unsigned lb;
+  const int p = lane_problem(t, lb);
+  const LaneProblem& q = t.items[p];
+  thin_fp_block<ZV, L, 1>(q.g, t.in[p], q.minmax, q.clip, q.pair, StoreOut{t.out[p]}, lb);
+}
+
+// one block's columns, lb the block's number in the problem
+template <int ZV, int L>
+__device__ __forceinline__ void thin_bp_block(const ParDev& g, const float* __restrict__ sino, float* __restrict__ vol,
+                                              int clipc, unsigned lb) {
   using V = typename VecT<ZV>::T;
   constexpr int G = 64 / L, kAng = 4;
   // per wavefront: its table of 64 entries (L > 1) and its lanes' sums
@@ -293,7 +309,6 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
   const int n = g.n, nz = g.nz, nt = (n + 7) / 8;
   const int z = l * ZV, zl = z < nz ? z : nz - ZV;
   // block -> G columns of an 8 x 8 patch
-  const unsigned lb = xcd_remap(blockIdx.x, gridDim.x);
   const int patch = (int)(lb / (64 / G)), in = (int)(lb % (64 / G)) * G + grp;
   const int row = (patch / nt) * 8 + (in >> 3), col = (patch % nt) * 8 + (in & 7);
   const bool inside = row < n && col < n;
@@ -391,6 +406,19 @@ __global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __
   if (wv == 0 && inside && z < nz) vstore<ZV>(vol + ((size_t)row * n + col) * nz + z, acc);
 }
 
+template <int ZV, int L>
+__global__ __launch_bounds__(1024) void thin_bp_kernel(ParDev g, const float* __restrict__ sino,
+                                                       float* __restrict__ vol, int clipc) {
+  thin_bp_block<ZV, L>(g, sino, vol, clipc, xcd_remap(blockIdx.x, gridDim.x));
+}
+template <int ZV, int L>
+__global__ __launch_bounds__(1024) void thin_bp_batch_kernel(LaneTable t) {
+  unsigned lb;
+  const int p = lane_problem(t, lb);
+  const LaneProblem& q = t.items[p];
+  thin_bp_block<ZV, L>(q.g, t.in[p], t.out[p], q.clip, lb);
+}
+
 // z layout: four slices per lane where nz is a multiple of 4 and the buffers
 // are 16-byte aligned (a 16-byte load costs the texture path 16 cycles for 64
 // lanes, a dword load 5: 4 slices per 16 against 4 per 20), else one
@@ -398,41 +426,69 @@ bool thin_v4(int nz, const void* a, const void* b) {
   return nz % 4 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0;
 }
 
-template <class F>
-void thin_dispatch(int nz, bool v4, F&& f) {
-  using std::integral_constant;
+// lanes that hold a problem's slices
+int thin_lanes(int nz, bool v4) {
   const int lanes = v4 ? nz / 4 : nz;
+  int l = 1;
+  while (l < lanes) l *= 2;
+  return l;
+}
+
+template <class F>
+void thin_dispatch(int lanes, bool v4, F&& f) {
+  using std::integral_constant;
   auto with = [&](auto zv) {
-    if (lanes <= 1) f(zv, integral_constant<int, 1>{});
-    else if (lanes <= 2) f(zv, integral_constant<int, 2>{});
-    else if (lanes <= 4) f(zv, integral_constant<int, 4>{});
-    else if (lanes <= 8) f(zv, integral_constant<int, 8>{});
-    else if (lanes <= 16) f(zv, integral_constant<int, 16>{});
+    if (lanes == 1) f(zv, integral_constant<int, 1>{});
+    else if (lanes == 2) f(zv, integral_constant<int, 2>{});
+    else if (lanes == 4) f(zv, integral_constant<int, 4>{});
+    else if (lanes == 8) f(zv, integral_constant<int, 8>{});
+    else if (lanes == 16) f(zv, integral_constant<int, 16>{});
     else f(zv, integral_constant<int, 32>{});
   };
   if (v4) with(integral_constant<int, 4>{});
   else with(integral_constant<int, 1>{});
 }
 
+// opposite rays share their taps' loads, but below about 4 wavefronts per SIMD the
+// GPU has room to project them side by side instead
+int thin_pair(const ParDev& g) { return g.fp_pair && g.pair_ok && fp_pair_tiled(g) >= 4096; }
+
+// one slice: 8 neighbouring rays x 8 samples per wavefront, whose taps lie in a
+// patch of about 11 x 11 voxels (64 samples of one ray can touch 64 cache lines),
+// where that still leaves 4 wavefronts per SIMD; 0: not so
+long long thin_waves8(const ParDev& g) {
+  const int pair = thin_pair(g), nu = pair ? g.n_units : g.na, ne = pair ? fp_pair_next(g) : g.n;
+  const long long waves = (long long)nu * ((ne + 7) / 8);
+  return g.nz == 1 && waves >= 4096 ? waves : 0;
+}
+
+// back projection: blocks, and wavefronts per block -- the angles are split until
+// about 8 wavefronts per SIMD are in flight, at most 16 ways and into no fewer than
+// 8 angles
+long long thin_bp_blocks(const ParDev& g, int lanes) { return ((g.n + 7) / 8) * (long long)((g.n + 7) / 8) * lanes; }
+int thin_bp_split(const ParDev& g, long long blocks) {
+  int split = 1;
+  while (split < 16 && blocks * split < 8192 && g.na >= 16 * split) split *= 2;
+  return split;
+}
+template <int ZV, int L>
+size_t thin_bp_lds_bytes(int split) {
+  return (L == 1 ? 0 : 64 * split * sizeof(float4)) + (split > 1 ? 64 * split * ZV * sizeof(float) : 0);
+}
+
 template <class Out>
 int thin_forward(vamx_plan* p, const float* vol, const void* sino, Out out, bool clip, hipStream_t s) {
   const ParDev& g = p->par;
-  // opposite rays share their taps' loads, but below about 4 wavefronts per
-  // SIMD the GPU has room to project them side by side instead
-  const int pair = g.fp_pair && g.pair_ok && fp_pair_tiled(g) >= 4096;
-  const long long waves = pair ? fp_pair_tiled(g) : fp_tiled_rays(g);
-  // one slice: 8 neighbouring rays x 8 samples per wavefront, whose taps lie in
-  // a patch of about 11 x 11 voxels (64 samples of one ray can touch 64 cache
-  // lines), where that still leaves 4 wavefronts per SIMD
-  const int nu = pair ? g.n_units : g.na, ne = pair ? fp_pair_next(g) : g.n;
-  const long long waves8 = (long long)nu * ((ne + 7) / 8);
-  if (g.nz == 1 && waves8 >= 4096) {
+  const int pair = thin_pair(g);
+  if (const long long waves8 = thin_waves8(g)) {
     hipLaunchKernelGGL((thin_fp_kernel<1, 1, 8, Out>), dim3(blocks_for(waves8 * 64, 256)), dim3(256), 0, s, g, vol,
                        p->d_minmax, clip ? 1 : 0, pair, out);
     VAMX_HIP(hipGetLastError());
     return VAMX_OK;
   }
-  thin_dispatch(g.nz, thin_v4(g.nz, vol, sino), [&](auto zv, auto l) {
+  const long long waves = pair ? fp_pair_tiled(g) : fp_tiled_rays(g);
+  const bool v4 = thin_v4(g.nz, vol, sino);
+  thin_dispatch(thin_lanes(g.nz, v4), v4, [&](auto zv, auto l) {
     constexpr int ZV = decltype(zv)::value, L = decltype(l)::value;
     hipLaunchKernelGGL((thin_fp_kernel<ZV, L, 1, Out>), dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, g, vol,
                        p->d_minmax, clip ? 1 : 0, pair, out);
@@ -460,17 +516,52 @@ int thin_forward_update(vamx_plan* p, const float* vol, const UpdateOut& out, bo
 
 int thin_backward(vamx_plan* p, const float* sino, float* vol, bool clipc, hipStream_t s) {
   const ParDev& g = p->par;
-  const long long nt = (g.n + 7) / 8;
-  thin_dispatch(g.nz, thin_v4(g.nz, sino, vol), [&](auto zv, auto l) {
+  const bool v4 = thin_v4(g.nz, sino, vol);
+  thin_dispatch(thin_lanes(g.nz, v4), v4, [&](auto zv, auto l) {
     constexpr int ZV = decltype(zv)::value, L = decltype(l)::value;
-    const long long blocks = nt * nt * L;
-    // wavefronts per block: the angles are split until about 8 wavefronts per
-    // SIMD are in flight, at most 16 ways and into no fewer than 8 angles
-    int split = 1;
-    while (split < 16 && blocks * split < 8192 && g.na >= 16 * split) split *= 2;
+    const long long blocks = thin_bp_blocks(g, L);
+    const int split = thin_bp_split(g, blocks);
     hipLaunchKernelGGL((thin_bp_kernel<ZV, L>), dim3((unsigned)blocks), dim3(64 * split),
-                       (L == 1 ? 0 : 64 * split * sizeof(float4)) + (split > 1 ? 64 * split * ZV * sizeof(float) : 0), s, g,
-                       sino, vol, clipc ? 1 : 0);
+                       (thin_bp_lds_bytes<ZV, L>(split)), s, g, sino, vol, clipc ? 1 : 0);
+  });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+
+// class of a problem: 1 << 16, 1 << 15 forward, 1 << 14 four slices per lane,
+// wavefronts per block << 8, lanes
+LaneClass thin_class(const vamx_plan* p, const void* in, const void* out, bool forward, bool clip) {
+  const ParDev& g = p->par;
+  LaneClass c;
+  if (!thin_ok(p) || (forward && thin_waves8(g))) return c;
+  const bool v4 = thin_v4(g.nz, in, out);
+  const int lanes = thin_lanes(g.nz, v4);
+  c.problem.g = g;
+  c.problem.minmax = p->d_minmax;
+  c.problem.clip = clip;
+  int per_block = 4;
+  if (forward) {
+    c.problem.pair = thin_pair(g);
+    c.waves = c.problem.pair ? fp_pair_tiled(g) : fp_tiled_rays(g);
+    c.blocks = (c.waves + 3) / 4;
+  } else {
+    c.blocks = thin_bp_blocks(g, lanes);
+    per_block = thin_bp_split(g, c.blocks);
+    c.waves = c.blocks * per_block;
+  }
+  c.key = 1 << 16 | (forward ? 1 << 15 : 0) | (v4 ? 1 << 14 : 0) | per_block << 8 | lanes;
+  return c;
+}
+
+int thin_batch(int key, const LaneTable& t, unsigned blocks, hipStream_t s) {
+  const int per_block = key >> 8 & 31;
+  thin_dispatch(key & 63, key >> 14 & 1, [&](auto zv, auto l) {
+    constexpr int ZV = decltype(zv)::value, L = decltype(l)::value;
+    if (key >> 15 & 1)
+      hipLaunchKernelGGL((thin_fp_batch_kernel<ZV, L>), dim3(blocks), dim3(256), 0, s, t);
+    else
+      hipLaunchKernelGGL((thin_bp_batch_kernel<ZV, L>), dim3(blocks), dim3(64 * per_block),
+                         (thin_bp_lds_bytes<ZV, L>(per_block)), s, t);
   });
   VAMX_HIP(hipGetLastError());
   return VAMX_OK;
