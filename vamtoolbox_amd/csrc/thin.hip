@@ -200,6 +200,35 @@ __device__ __forceinline__ void thin_ray(const ParDev& g, const float* __restric
   }
 }
 
+template <int ZV>
+__device__ __forceinline__ bool thin_finite(const typename VecT<ZV>::T& v) {
+  bool ok = true;
+#pragma unroll
+  for (int q = 0; q < ZV; ++q) ok &= fabsf(vget(v, q)) <= 3.4028234664e38f;
+  return ok;
+}
+// A ray and its opposite ray (k2 < 0: none) from the same taps.  The two samples at
+// the ends of a pair that belong to one of the rays count for the other with weight
+// 0, which a voxel without a finite value turns into a NaN: where a sum is not
+// finite, the rays are walked one by one (all lanes take part) and replace such sums.
+template <int ZV, int L, int R>
+__device__ __forceinline__ void thin_pair_rays(const ParDev& g, const float* __restrict__ vol,
+                                               const float* __restrict__ minmax, int k, int i, int k2, int i2, int z,
+                                               int lane, typename VecT<ZV>::T& acc, typename VecT<ZV>::T& acc2) {
+  using V = typename VecT<ZV>::T;
+  thin_ray<ZV, L, R, false, true>(g, vol, minmax, k, i, z, lane, acc, acc2);
+  if (__ballot(!thin_finite<ZV>(acc) || !thin_finite<ZV>(acc2)) == 0ull) return;
+#pragma unroll 1
+  for (int h = 0; h < 2; ++h) {
+    V alone, none;
+    thin_ray<ZV, L, R, false, false>(g, vol, minmax, h && k2 >= 0 ? k2 : k, h && k2 >= 0 ? i2 : i, z, lane, alone, none);
+    V& sum = h ? acc2 : acc;
+#pragma unroll
+    for (int q = 0; q < ZV; ++q)
+      if (!(fabsf(vget(sum, q)) <= 3.4028234664e38f)) vset(sum, q, vget(alone, q));
+  }
+}
+
 // one block's rays, lb the block's number in the problem
 template <int ZV, int L, int R, class Out>
 __device__ __forceinline__ void thin_fp_block(const ParDev& g, const float* __restrict__ vol,
@@ -243,7 +272,7 @@ __device__ __forceinline__ void thin_fp_block(const ParDev& g, const float* __re
         if (first && k2 >= 0) out.put(((size_t)k2 * g.na + i2) * g.nz, vget(acc, 0));
       }
     } else {
-      thin_ray<ZV, L, R, false, true>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+      thin_pair_rays<ZV, L, R>(g, vol, minmax, k, i, k2, i2, zl, lane, acc, acc2);
       if (first) out.put(((size_t)k * g.na + i) * g.nz, vget(acc, 0));
       if (first && k2 >= 0) out.put(((size_t)k2 * g.na + i2) * g.nz, vget(acc2, 0));
     }
@@ -274,7 +303,7 @@ __device__ __forceinline__ void thin_fp_block(const ParDev& g, const float* __re
       put(kh, ih, acc);
     }
   } else if (k2 >= 0) {
-    thin_ray<ZV, L, 1, false, true>(g, vol, minmax, k, i, zl, lane, acc, acc2);
+    thin_pair_rays<ZV, L, 1>(g, vol, minmax, k, i, k2, i2, zl, lane, acc, acc2);
     put(k, i, acc);
     put(k2, i2, acc2);
   } else {
