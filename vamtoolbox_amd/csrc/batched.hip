@@ -56,9 +56,10 @@ __device__ __forceinline__ void batch_fp_wave(const BatchItem& it, const float* 
   int k, i, zc;
   if (!fp_wave_item<ZV>(w, g, k, i, zc)) return;
   const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
-  const typename VecT<ZV>::T acc = it.clip && wave_clip_active(it.minmax, g.nz, ln)
-                                       ? fp_ray_wave<true, true, false>(g, in, it.minmax, k, i, ln, lane)
-                                       : fp_ray_wave<false, true, false>(g, in, it.minmax, k, i, ln, lane);
+  const bool clip_on = it.clip && wave_clip_active(it.minmax, g.nz, ln);
+  typename VecT<ZV>::T acc = clip_on ? fp_ray_wave<true, true, false>(g, in, it.minmax, k, i, ln, lane)
+                                     : fp_ray_wave<false, true, false>(g, in, it.minmax, k, i, ln, lane);
+  fp_ray_finish(g, in, it.minmax, clip_on, k, i, ln, acc);
   ln.store(out + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
 }
 
@@ -76,14 +77,17 @@ __device__ __forceinline__ void batch_fp_pair(const BatchItem& it, const float* 
   if (it.clip && wave_clip_active(it.minmax, g.nz, ln)) {
     for (int h = 0; h < (pi.k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? pi.k2 : pi.k, ih = h ? pi.i2 : pi.i;
-      ln.store(out + ((size_t)kh * g.na + ih) * g.nz, g.nz,
-               fp_ray_wave<true, true, false>(g, in, it.minmax, kh, ih, ln, lane));
+      V acc = fp_ray_wave<true, true, false>(g, in, it.minmax, kh, ih, ln, lane);
+      fp_ray_finish(g, in, it.minmax, true, kh, ih, ln, acc);
+      ln.store(out + ((size_t)kh * g.na + ih) * g.nz, g.nz, acc);
     }
     return;
   }
   V acc, acc2 = vzero<ZV>();
   if (pi.k2 >= 0) acc = fp_ray_wave<false, true, true>(g, in, it.minmax, pi.k, pi.i, ln, lane, &acc2);
   else acc = fp_ray_wave<false, true, false>(g, in, it.minmax, pi.k, pi.i, ln, lane);
+  fp_ray_finish(g, in, it.minmax, false, pi.k, pi.i, ln, acc);
+  if (pi.k2 >= 0) fp_ray_finish(g, in, it.minmax, false, pi.k2, pi.i2, ln, acc2);
   ln.store(out + ((size_t)pi.k * g.na + pi.i) * g.nz, g.nz, acc);
   if (pi.k2 >= 0) ln.store(out + ((size_t)pi.k2 * g.na + pi.i2) * g.nz, g.nz, acc2);
 }

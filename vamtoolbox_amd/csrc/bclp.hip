@@ -172,9 +172,10 @@ __global__ __launch_bounds__(256) void bclp_fp_update_wave(ParDev g, const float
   int k, i, zc;
   if (!fp_wave_item<ZV>(wave, g, k, i, zc)) return;
   const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
-  const typename VecT<ZV>::T fp = clip && wave_clip_active(minmax, g.nz, ln)
-                                      ? fp_ray_wave<true, REUSE, false>(g, operand, minmax, k, i, ln, lane)
-                                      : fp_ray_wave<false, REUSE, false>(g, operand, minmax, k, i, ln, lane);
+  const bool clip_on = clip && wave_clip_active(minmax, g.nz, ln);
+  typename VecT<ZV>::T fp = clip_on ? fp_ray_wave<true, REUSE, false>(g, operand, minmax, k, i, ln, lane)
+                                    : fp_ray_wave<false, REUSE, false>(g, operand, minmax, k, i, ln, lane);
+  fp_ray_finish(g, operand, minmax, clip_on, k, i, ln, fp);
   bclp_update_row(gsino + ((size_t)k * g.na + i) * g.nz, g.nz, ln, fp, (float)(*scale_p), lr, glb, gub);
 }
 
@@ -202,13 +203,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void b
     // projected one after the other
     for (int h = 0; h < (k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? k2 : k, ih = h ? i2 : i;
-      update(kh, ih, fp_ray_wave<true, REUSE, false>(g, operand, minmax, kh, ih, ln, lane));
+      V fp = fp_ray_wave<true, REUSE, false>(g, operand, minmax, kh, ih, ln, lane);
+      fp_ray_finish(g, operand, minmax, true, kh, ih, ln, fp);
+      update(kh, ih, fp);
     }
     return;
   }
   V fp, fp2 = vzero<ZV>();
   if (k2 >= 0) fp = fp_ray_wave<false, REUSE, true>(g, operand, minmax, k, i, ln, lane, &fp2);
   else fp = fp_ray_wave<false, REUSE, false>(g, operand, minmax, k, i, ln, lane);
+  fp_ray_finish(g, operand, minmax, false, k, i, ln, fp);
+  if (k2 >= 0) fp_ray_finish(g, operand, minmax, false, k2, i2, ln, fp2);
   update(k, i, fp);
   if (k2 >= 0) update(k2, i2, fp2);
 }

@@ -994,6 +994,7 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
   // built a descriptor per sample: 40 scalar instructions and branches.)
   V T00 = vzero<ZV>(), T01 = vzero<ZV>(), T10 = vzero<ZV>(), T11 = vzero<ZV>();
   const FpSlot sl = fp_lds_slot();
+  bool number = true;   // one slice per lane: no sample was a NaN before the clip
   int last = -1;   // cell of the sample before the 64 (-1: none)
   const int r_end = PAIR ? (2 * g.c + 1 > n ? 2 * g.c + 1 : n) : n;
   const int r2_lo = 2 * g.c - n + 1;   // partner's first sample (PAIR)
@@ -1081,6 +1082,7 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
         if (load & 8) T11 = ln.load(rs, (uint32_t)rl_i(a11, j));
         if constexpr (CLIP) {
           V v = vfma(q11, T11, vfma(q10, T10, vfma(q01, T01, vmul(q00, T00))));
+          if constexpr (ZV == 1) number = number && v == v;
           v = vclamp(v, lo, hi);  // every enumerated sample has an in-range tap of positive weight
           acc = vfma(sl.a[j].x, v, acc);
         } else if constexpr (PAIR) {
@@ -1096,7 +1098,26 @@ __device__ __forceinline__ typename VecT<ZV>::T fp_ray_wave(const ParDev& g, con
     }
   }
   if constexpr (PAIR) *acc2 = accp;
+  if constexpr (ZV == 1 && CLIP)
+    if (!number) acc = __builtin_nanf("");   // for fp_ray_finish
   return acc;
+}
+
+// One slice per lane (up to 64 slices): a sum that is not finite is summed again as
+// fp_ray does it.  The core above weights whole cells, and both rays of a pair, with
+// weights that may be 0, and a voxel without a finite value would make NaNs of rays
+// that pass beside it.  Problems of 32 to 56 slices came from fp_ray, where it does
+// not; with more slices per lane, whose kernels never had this, it cost 1 us of a
+// small call and 1 % of a large one.
+template <int ZV, bool SPLIT>
+__device__ __forceinline__ void fp_ray_finish(const ParDev& g, const float* __restrict__ vol,
+                                              const float* __restrict__ minmax, bool clip, int k, int i,
+                                              const FpLane<ZV, SPLIT>& ln, typename VecT<ZV>::T& acc) {
+  if constexpr (ZV == 1) {
+    const bool bad = !(fabsf(acc) <= 3.4028234664e38f) && ln.z < g.nz;
+    if (__ballot(bad) == 0ull) return;
+    if (bad) acc = clip ? fp_ray<1, true>(g, vol, minmax, k, i, ln.z) : fp_ray<1, false>(g, vol, minmax, k, i, ln.z);
+  }
 }
 
 // Slices of a lane in the back projection's wavefronts: CONTIG (ZV = 4) z ..

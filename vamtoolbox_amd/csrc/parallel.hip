@@ -175,9 +175,10 @@ __global__ __launch_bounds__(256) void par_fp_wave_kernel(ParDev g, const float*
   int k, i, zc;
   if (!fp_wave_item<ZV>(wave, g, k, i, zc)) return;
   const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
-  const typename VecT<ZV>::T acc = clip && wave_clip_active(minmax, g.nz, ln)
-                                       ? fp_ray_wave<true, REUSE, false>(g, vol, minmax, k, i, ln, lane)
-                                       : fp_ray_wave<false, REUSE, false>(g, vol, minmax, k, i, ln, lane);
+  const bool clip_on = clip && wave_clip_active(minmax, g.nz, ln);
+  typename VecT<ZV>::T acc = clip_on ? fp_ray_wave<true, REUSE, false>(g, vol, minmax, k, i, ln, lane)
+                                     : fp_ray_wave<false, REUSE, false>(g, vol, minmax, k, i, ln, lane);
+  fp_ray_finish(g, vol, minmax, clip_on, k, i, ln, acc);
   ln.store(sino + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
 }
 
@@ -201,7 +202,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void p
     // of the unpaired kernel)
     for (int h = 0; h < (k2 >= 0 ? 2 : 1); ++h) {
       const int kh = h ? k2 : k, ih = h ? i2 : i;
-      const V acc = fp_ray_wave<true, REUSE, false>(g, vol, minmax, kh, ih, ln, lane);
+      V acc = fp_ray_wave<true, REUSE, false>(g, vol, minmax, kh, ih, ln, lane);
+      fp_ray_finish(g, vol, minmax, true, kh, ih, ln, acc);
       ln.store(sino + ((size_t)kh * g.na + ih) * g.nz, g.nz, acc);
     }
     return;
@@ -209,6 +211,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void p
   V acc, acc2 = vzero<ZV>();
   if (k2 >= 0) acc = fp_ray_wave<false, REUSE, true>(g, vol, minmax, k, i, ln, lane, &acc2);
   else acc = fp_ray_wave<false, REUSE, false>(g, vol, minmax, k, i, ln, lane);
+  fp_ray_finish(g, vol, minmax, false, k, i, ln, acc);
+  if (k2 >= 0) fp_ray_finish(g, vol, minmax, false, k2, i2, ln, acc2);
   ln.store(sino + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
   if (k2 >= 0) ln.store(sino + ((size_t)k2 * g.na + i2) * g.nz, g.nz, acc2);
 }
