@@ -430,19 +430,19 @@ BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits, int problems)
   // as two of two; 300, combined: 0.76 as five of one, 0.99 as two of three.
   //
   // Where the active patches are few, a lane's chain of slices is what takes the
-  // time, and fewer slices per lane and more wavefronts are faster: four need 1.5
-  // wavefronts per SIMD (96 x 96 x 256, 120 angles, 930 of them: 78 us, as 3700 of one
-  // slice 55; 128 x 128 x 256, 180 angles, 1650: 120 and 120), two need 2 per SIMD (128
-  // x 128 x 128, 1650: 101 us, as 3300 of one slice 90; 192 x 192 x 128, 240 angles,
-  // 3680: 168 and 228).  Problems of a batch fill the GPU together.
+  // time, and one slice per lane and more wavefronts are faster: more need 1.5
+  // wavefronts per SIMD (96 x 96 x 256, 120 angles, four slices in 930 of them: 78 us,
+  // one in 3700: 55; 128 x 128 x 256, 180 angles, 1650: 120 and 120; 96 x 96 x 128, two
+  // slices in 930: 52 us, one: 41; 128 x 128 x 77, 1650: 87 and 91).  Problems of a batch
+  // fill the GPU together.
   constexpr int costs[2][5] = {{0, 21, 33, 48, 92}, {0, 16, 29, 43, 57}}, costs16[2] = {56, 45};
-  constexpr int waves[5] = {0, 0, 2048, 1536, 1536};
+  constexpr int waves = 1536;
   const int* const cost = costs[l.comb ? 1 : 0];
   const int cost16 = costs16[l.comb ? 1 : 0];
   int best = INT_MAX;
   for (int zv = 1; zv <= g.bp_zv; ++zv) {
     const int c = wave_zchunks(g.nz, zv);
-    if ((long long)g.bp_act * c * problems < waves[zv]) continue;
+    if (zv > 1 && (long long)g.bp_act * c * problems < waves) continue;
     const bool contig = zv == 4 && g.nz % 4 == 0 && align_bits % 16 == 0;
     const int t = c * (contig ? cost16 : cost[zv]);
     if (t >= best) continue;
