@@ -97,16 +97,18 @@ typedef struct vamx_par_tuning {
   int32_t fp_tile_rays;     /* forward: rays per tile (default 4)                         */
   int32_t fp_zv;            /* forward: at most this many z values per lane, 1, 2 or 4 (default 4) */
   int32_t fp_reuse;         /* forward: 1 = keep the previous sample's taps in registers (default 1) */
-  int32_t bp_tile;          /* A^T: tile edge in 2x2 quads of voxel columns (default 8) */
-  int32_t bp_zv;            /* back projection: at most this many z values per lane (default 4) */
+  int32_t bp_tile;          /* forward's transpose: tile edge in 2x2 quads of voxel columns (default 8) */
+  int32_t bp_zv;            /* back projection, forward's transpose: at most this many z values per
+                               lane, 1, 2 or 4 (default 4) */
   int32_t fp_pair;          /* 1 = project angles a and a + 180 deg in one pass over the taps when
                                2 * det_offset is an integer and there is no inclination or
                                occlusion, and without absorption add their bins before they are
                                back projected (default 1); fp_tile_angles then counts angle pairs.
                                0 = every angle by itself, forward and back */
-  int32_t z_split;          /* both: 1 = where a lane would hold one z value (nz odd or buffers
-                               not 8-byte aligned) and the 64-z chunk count is even, lanes hold
-                               z and z + 64 instead: half the wavefronts (default 1) */
+  int32_t z_split;          /* forward, 32 z values and more: 1 = a lane holds one to four z values
+                               64 apart, or four consecutive ones, whichever takes the least time
+                               (default 1); 0 = 4, 2 or 1 consecutive ones, as nz and the buffers'
+                               alignment allow */
 } vamx_par_tuning;
 int vamx_par_set_tuning(vamx_plan* plan, const vamx_par_tuning* tuning);
 int vamx_par_get_tuning(vamx_plan* plan, vamx_par_tuning* tuning);

@@ -1,17 +1,18 @@
 // Batched parallel-beam projection of many independent problems of uneven
-// size in one persistent launch (gfx950); in the forward direction, problems
-// large enough to fill the GPU on their own get single-problem launches
-// instead (the same kernels and results as vamx_par_forward), spread over
-// three streams.
+// size (gfx950): one persistent launch for most; in the forward direction,
+// problems large enough to fill the GPU on their own get single-problem launches
+// instead; problems of fewer than 32 slices or at an inclination run on kernels of
+// their own, those that do not fill the GPU several to a launch.  The launches
+// outside the persistent one are spread over three streams, and every problem's
+// result is that of its single call.
 //
 // Each problem is a parallel plan (vamx_par_create) with its own volume and
 // sinogram.  A problem's work is cut into tiles of one 256-thread block:
 // four wavefronts of the wavefront-uniform kernels (one ray -- or a ray and
-// its opposite ray, when the plan pairs opposite angles -- or one 2x2 voxel
-// quad, and 64 x ZV z values per wavefront -- with ZV = 2 possibly split into
-// z and z + 64 -- in the plan's L2-aware order) or,
-// for shapes those do not take (inclination, very thin z), 256 items of the
-// per-lane kernels.  Tiles are ordered largest problem first and handed out
+// its opposite ray, when the plan pairs opposite angles -- or one patch of 2 x 4
+// voxel columns, and 64 x ZV z values per wavefront, in the plan's L2-aware order)
+// or, for what those do not take (occlusion, one column), 256 items of the per-lane
+// kernels.  Tiles are ordered largest problem first and handed out
 // by a device-side counter, so the resident blocks of the single launch drain
 // one queue until it is empty (every block exits when the counter passes the
 // tile count).  The counter is reset by a one-thread kernel on the same
@@ -31,7 +32,7 @@ struct BatchItem {
   const float* minmax;
   long long tile_begin;  // first tile of this problem
   long long items;       // wavefronts (wave mode) or threads (per-lane mode) of this problem
-  int zv;                // z values per lane: 1, 2, 4 (wave mode) or 1, 4 (per-lane mode)
+  int zv;                // z values per lane: 1 to 4 (wave mode) or 1, 4 (per-lane mode)
   int clip;              // forward: warp clip; backward: circle clip
   int wave;              // 1: wavefront-uniform kernels
   int pair;              // forward, wave mode: opposite-angle pairs (the plan's paired work order)

@@ -58,8 +58,9 @@ __global__ __launch_bounds__(256) void bclp_bp_epilogue(ParDev g, int clipc, Res
 }
 
 // A, second half, after a back projection into `dose` by the plain kernels:
-// response, band, Lp weighting and loss partials of a whole dose, grid-stride
-// (bound by its 12 bytes per voxel)
+// response, band, Lp weighting and loss partials of a whole dose, grid-stride.  64 to
+// 68 us at 256^3 where its 12 bytes per voxel take 41 at the rate of a copy: one voxel
+// per lane and turn, with a float64 exponential and division between load and store.
 __global__ __launch_bounds__(256) void bclp_epilogue_kernel(RespDev r, BclpDev b, const float* __restrict__ dose,
                                                             const float* __restrict__ target,
                                                             float* __restrict__ operand,
@@ -79,9 +80,9 @@ __global__ __launch_bounds__(256) void bclp_epilogue_kernel(RespDev r, BclpDev b
 // integrand's sum and the L0, L1, L2 and Linf norms of the band error and of the
 // error (BCLP.py:277-345, 396-437), with the products of v = |e| > eps written
 // out as the reference multiplies them (so infinities and NaN reach the same
-// norms).  One pass, bound by the response's float64 exponential and division (68
-// us at 256^3 where the bytes take 55); element by element in float64 arrays the
-// same took 40 passes, 3.0 ms.
+// norms).  One pass, bound by the response's float64 exponential and division: 114 us
+// at 256^3 (and 28 for the totals) where its 16 bytes per voxel take 55; element by
+// element in float64 arrays the same took 40 passes, 3.0 ms.
 constexpr int kMetrics = VAMX_BCLP_METRICS;
 __global__ __launch_bounds__(256) void bclp_metrics_kernel(RespDev r, BclpDev b, const float* __restrict__ dose,
                                                            const float* __restrict__ target,
@@ -439,8 +440,8 @@ int launch_epilogue(vamx_plan* p, const RespDev& r, const BclpDev& b, const floa
                                         std::to_string(max_parts) + " slots of the scratch");
   // the back projections on wavefronts and the element-wise epilogue as two
   // launches: with the epilogue in the patch kernel, whose accumulators fill
-  // its registers, 824 us at 256^3 x 360, apart 718 + 41; 160 x 120 x 180
-  // angles 155 and 138 + 14
+  // its registers, 824 us at 256^3 x 360, apart 718 + 65 (now 630 + 65); 160 x 160
+  // x 120, 180 angles 155, now 119 + 19
   if (incl_wave_ok(p) || thin_ok(p) || bp_layout(p, 0).zv)
     return split_epilogue(p, r, b, g, target, dose, operand, partials, clipc, nparts, s);
   const dim3 grid(nparts), block(256);

@@ -226,8 +226,9 @@ __global__ __launch_bounds__(256) void incl_fp_batch_kernel(LaneTable t) {
 //
 // Bound by latency and instructions (two slices per lane: 4.6 4-byte loads and 30
 // vector instructions per sample, against 8 loads and 24 with the rows' own lanes,
-// which the texture path bound): 128 x 128 x 96 x 180, 12 degrees 279 -> 207 us, x 256
-// x 90 398 -> 285, 100 x 100 x 300 x 60, 10 degrees 177 -> 122.
+// which the texture path bound): 128 x 128 x 96 x 180, 12 degrees 279 -> 212 us (206
+// with the sample's two slices multiplied into the sum one after the other, which
+// rounds it twice), x 256 x 90 398 -> 285, 100 x 100 x 300 x 60, 10 degrees 177 -> 121.
 // values of the next / previous slice (lane, and across the NS registers); 0 past
 // the ends
 template <int NS>
@@ -567,7 +568,8 @@ long long incl_bp_waves(const ParDev& g) {
 // four fixed slices, of which the shift over a ray takes some lanes, and 150, 275,
 // 400 with one to three rows (whose samples load all four taps and no shift is lost).
 // Where both take one chunk of one register, rows win: 19 against 22 us at 64 x 64 x
-// 48 x 60.
+// 48 x 60.  The figures are those of a GPU that is full; of 24 x 24 to 100 x 100 columns,
+// where it is not, no size was found slower than by one thread per row.
 int incl_fixed(const ParDev& g, InclShift& shift) {
   if (g.nz < 32) return 0;
   const double e0 = -(double)g.c * g.tan_phi, e1 = (double)(g.n - 1 - g.c) * g.tan_phi;

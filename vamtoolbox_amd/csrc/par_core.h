@@ -822,15 +822,7 @@ __device__ __forceinline__ typename VecT<ZV>::T fpT_voxel_wave(const ParDev& g, 
   }
   return acc;
 }
-__device__ __forceinline__ float rl_f(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
 
-// slot weights of one axis: the taps floor / floor+1 (skimage's floor / ceil
-// with weights 1-d / d) mapped onto the pair (b, b+1) with b in [0, n-2]
-// The warp clip of a slice is a no-op when 0 lies in [min, max] of the slice:
-// bilinear samples are convex combinations of the slice's values and the zero
-// padding.  Wave-uniform test over the wave's 64*ZV slices.
 // the transposes' lanes own ZV consecutive slices: those past nz load a copy of
 // the last ones and store nothing
 template <int ZV>
@@ -889,8 +881,10 @@ struct FpLane {
   }
 };
 
-// the warp clip of the wavefront's slices is not a no-op, from their least and
-// largest values
+// The warp clip of a slice is a no-op when 0 lies in [min, max] of the slice:
+// bilinear samples are convex combinations of the slice's values and the zero
+// padding.  Whether it is not one for any of the wavefront's slices (lo, hi: their
+// least and largest values).
 template <int ZV>
 __device__ __forceinline__ bool wave_clip_active(const typename VecT<ZV>::T& lo, const typename VecT<ZV>::T& hi) {
   bool need = false;
@@ -903,6 +897,8 @@ __device__ __forceinline__ bool wave_clip_active(const float* __restrict__ minma
   return wave_clip_active<ZV>(ln.values(minmax), ln.values(minmax + nz));
 }
 
+// slot weights of one axis: the taps floor / floor+1 (skimage's floor / ceil
+// with weights 1-d / d) mapped onto the pair (b, b+1) with b in [0, n-2]
 __device__ __forceinline__ void axis_slots(double coord, int n, int& b, double& s0, double& s1) {
   const double f = floor(coord);
   const double d = coord - f;
@@ -1121,9 +1117,9 @@ __device__ __forceinline__ void fp_ray_finish(const ParDev& g, const float* __re
 }
 
 // Slices of a lane in the back projection's wavefronts: CONTIG (ZV = 4) z ..
-// z + 3, else z + 64 q (dword loads: a 64-lane dword load takes the texture
-// path 5 cycles, an 8-byte one 16, a 16-byte one 16).  Slices past nz load a
-// copy of the last one and are not stored.
+// z + 3, else z + 64 q (4-byte loads: a wavefront's takes a CU's texture path 8.5
+// cycles, a 16-byte one, for four times the slices, 17 to 20, an 8-byte one as
+// long as that).  Slices past nz load a copy of the last one and are not stored.
 template <int ZV, bool CONTIG>
 struct ZLane {
   static_assert(!CONTIG || ZV == 4, "contiguous slices are 16-byte loads");
@@ -1459,8 +1455,9 @@ __device__ __forceinline__ void bp_patch(const ParDev& g, const float* __restric
 // run on the same XCD (xcd_remap), so consecutive waves should form a compact
 // tile whose data fits the XCD's 4 MB L2: forward = fp_ta consecutive angles x
 // fp_tk consecutive rays (their samples at one along-ray step lie within a few
-// tens of pixels), back projection = a bp_tile x bp_tile patch of 2x2 voxel
-// quads (detector footprint ~2.8 bp_tile bins per angle).  When a ray (or
+// tens of pixels), the forward's transpose = a bp_tile x bp_tile patch of 2x2
+// voxel quads (detector footprint ~2.8 bp_tile bins per angle; the back
+// projection's patches are listed by the plan, see bp_wave_patch).  When a ray (or
 // column) spans several z chunks, the chunk is the slowest index, so that all
 // resident waves share one z slab.  Padding waves exit.  Tiles never exceed
 // the problem: a tile edge beyond the angle / ray / quad count would only add
@@ -1481,7 +1478,7 @@ __device__ __forceinline__ bool fp_tile_ray(long long q, const ParDev& g, int& k
   k = (int)(tile % ntk) * tk + within % tk;
   return i < g.na && k < g.n;
 }
-// back projection: quads of 2x2 voxel columns, tiles of bp_tile x bp_tile quads
+// forward's transpose: quads of 2x2 voxel columns, tiles of bp_tile x bp_tile quads
 __host__ __device__ inline int bp_nquad(const ParDev& g) { return (g.n + 1) / 2; }
 __host__ __device__ inline int bp_tile_eff(const ParDev& g) {
   return g.bp_tile < bp_nquad(g) ? g.bp_tile : bp_nquad(g);
@@ -1626,11 +1623,11 @@ __device__ __forceinline__ long long wave_index(unsigned lb) {
   return (long long)lb * (blockDim.x >> 6) + slot;
 }
 
-// wave -> (ray, z) of the forward kernels; false for padding waves
 // z chunks of a wavefront: 64 lanes x ZV values; the last chunk may be
 // partial (lanes past nz load from a clamped z and store nothing)
 __host__ __device__ inline int wave_zchunks(int nz, int zv) { return (nz + 64 * zv - 1) / (64 * zv); }
 
+// wave -> (ray, z chunk) of the forward kernels; false for padding waves
 template <int ZV>
 __device__ __forceinline__ bool fp_wave_item(long long wave, const ParDev& g, int& k, int& i, int& zc) {
   const long long rays = fp_tiled_rays(g);
@@ -1687,7 +1684,7 @@ __host__ __device__ __forceinline__ PairItem fp_pair_item(long long wave, const 
   return it;
 }
 
-// wave -> (voxel quad, z) of the back-projection kernels; false for padding
+// wave -> (voxel quad, z) of the forward's transpose; false for padding
 template <int ZV>
 __device__ __forceinline__ bool bp_wave_quad(long long wave, const ParDev& g, int lane, int& r0, int& c0, int& z) {
   const long long quads = bp_tiled_quads(g);

@@ -184,7 +184,8 @@ __global__ __launch_bounds__(256) void par_fp_wave_kernel(ParDev g, const float*
 
 // paired forward projection: one wavefront = ray (k, i) and, when it exists,
 // the opposite ray (k2, i2) x 64*ZV z, from one pass over the taps.  Held to
-// 64 VGPRs (8 waves per SIMD; a 28-byte spill outside the sample loop).
+// 64 VGPRs (8 waves per SIMD); with four slices per lane that spills 28 bytes (40 with
+// the slices 64 apart, 8 or none without the reuse), outside the sample loop.
 template <int ZV, bool REUSE, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void par_fp_pair_kernel(ParDev g, const float* __restrict__ vol,
                                                           float* __restrict__ sino, const float* __restrict__ minmax,
@@ -482,7 +483,10 @@ FpLayout vamx::fp_layout(const vamx_plan* p, uintptr_t align_bits) {
   // lane is already bound by latency and instructions, so wide chunks pay even
   // where lanes idle: 180 slices took 1.56 ms as three chunks of 64, 0.78 as one;
   // 255 slices 1.41 as two of 128, 1.32 as one; below 64 slices the per-lane
-  // kernels took 0.65 (32) to 1.01 ms (56) against 0.55 to 0.57.
+  // kernels took 0.65 (32) to 1.01 ms (56) against 0.55 to 0.57.  The figures are
+  // those of a GPU that is full; from 24 x 24 columns x 24 angles to 128 x 128 x 180,
+  // where it is not, no size was found more than 4 % slower than with one or two
+  // slices per lane.
   constexpr int cost[5] = {0, 56, 70, 100, 132}, cost16 = 83;
   int best = INT_MAX;
   for (int zv = 1; zv <= g.fp_zv; ++zv) {
@@ -603,8 +607,9 @@ extern "C" int vamx_par_create(const vamx_par_geom* geom, vamx_plan** out_plan) 
   if (geom->mu < 0.0) return set_error(VAMX_ERR_ARG, "vamx_par_create: mu must be >= 0");
   if (geom->occlusion && geom->incl_deg != 0.0)
     return set_error(VAMX_ERR_ARG, "vamx_par_create: occlusion shadowing needs zero inclination");
-  // the wavefront kernels address a cell's two volume rows, and a voxel
-  // quad's four sinogram rows, through 32-bit buffer offsets
+  // the wavefront kernels address a cell's two volume rows, and a patch's six
+  // sinogram rows, through 32-bit buffer offsets: unsigned ones, five strides of a
+  // row and a row's slices are below 5/3 of 2^31
   if (4.0 * geom->nz * ((double)geom->n + 2) >= 2147483648.0 ||
       4.0 * geom->nz * (3.0 * geom->n_angles + 1) >= 2147483648.0)
     return set_error(VAMX_ERR_ARG, "vamx_par_create: n * nz or n_angles * nz too large for 32-bit row offsets");

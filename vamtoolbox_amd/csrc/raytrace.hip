@@ -778,7 +778,6 @@ extern "C" int vamx_rt_create(const vamx_rt_geom* geom, vamx_plan** out_plan) {
   g.xmax = g.xmin + (g.nx - 1) * g.dx;
   g.ymax = g.ymin + (g.ny - 1) * g.dy;
   g.zmax = g.nz > 1 ? g.zmin + (g.nz - 1) * g.dz : g.zmin;
-  g.span_x = g.xmax - g.xmin; g.span_y = g.ymax - g.ymin; g.span_z = g.zmax - g.zmin;
   g.last_x = (float)(g.nx - 1); g.last_y = (float)(g.ny - 1); g.last_z = (float)(g.nz - 1);
   g.nt = geom->nt; g.na = geom->n_angles; g.nzr = geom->nzr;
   g.incl = geom->incl_deg * (M_PI / 180.0);

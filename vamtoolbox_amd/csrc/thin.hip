@@ -448,9 +448,10 @@ __global__ __launch_bounds__(1024) void thin_bp_batch_kernel(LaneTable t) {
   thin_bp_block<ZV, L>(q.g, t.in[p], t.out[p], q.clip, lb);
 }
 
-// z layout: four slices per lane where nz is a multiple of 4 and the buffers
-// are 16-byte aligned (a 16-byte load costs the texture path 16 cycles for 64
-// lanes, a dword load 5: 4 slices per 16 against 4 per 20), else one
+// z layout: four slices per lane where nz is a multiple of 4 and the buffers are
+// 16-byte aligned, else one.  Forward and back with four, and with one: 200 x 200 x
+// 24, 180 angles 86 + 59 and 106 + 67 us, x 4 32 + 23 and 42 + 25, 512 x 512 x 4, 360
+// angles 277 + 240 and 360 + 277; 200 x 200 x 8 49 + 35 and 48 + 33.
 bool thin_v4(int nz, const void* a, const void* b) {
   return nz % 4 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0;
 }

@@ -33,18 +33,19 @@ struct ParDev {
   // work order of the wavefront-uniform kernels (set by vamx_par_set_tuning)
   int fp_ta, fp_tk, fp_zv;   // forward: tile of fp_ta angles x fp_tk rays, z values per lane
   int fp_reuse;              // forward: keep the previous sample's taps in registers
-  int bp_tile, bp_zv;        // A^T: tile of bp_tile x bp_tile quads of voxel columns; A, A^T: z values per lane
-  // A: the patches of 2 x 4 voxel columns, patch row << 16 | patch column, those
-  // inside the clip circle first, and their counts
+  int bp_tile;               // the forward's transpose: tile of bp_tile x bp_tile quads of voxel columns
+  int bp_zv;                 // back projection, the forward's transpose: at most this many z values per lane
+  // back projection: the patches of 2 x 4 voxel columns, patch row << 16 | patch
+  // column, those inside the clip circle first, and their counts
   const int* bp_list;
   int bp_act, bp_all;
-  int z_split;               // allow lanes holding z and z + 64 where one z per lane is the choice
-  // Opposite-angle pairing of the forward projection.  Ray k at angle a and
+  int z_split;               // forward: lanes may hold slices 64 apart
+  // Opposite-angle pairing.  Ray k at angle a and
   // ray 2c + D - k at angle a + 180 deg (D = 2 det_offset, an integer) sample
   // the same points in reverse order, so one pass over the taps serves both.
   // Work units are angles: (primary, partner) or (angle, -1).  Of the partner
   // angle's rays, pair_u have no primary ray; they start at pair_first2.
-  int fp_pair;               // tuning: pair opposite angles when pair_ok
+  int fp_pair;               // tuning: pair opposite angles when pair_ok, forward and back
   int pair_ok;               // the geometry has opposite angles and D is an integer
   int n_units, pair_D, pair_u, pair_first2;
   const int* units;          // [n_units][2]
@@ -61,7 +62,6 @@ struct RtDev {
   int nx, ny, nz;
   double xmin, ymin, zmin, dx, dy, dz;
   double inv_dx, inv_dy, inv_dz;
-  double span_x, span_y, span_z;
   double xmax, ymax, zmax;
   // derived on the host: the last voxel's index, 1 / d in float32 (z: 0 in 2-D),
   // the Runge-Kutta stages and step / 6
