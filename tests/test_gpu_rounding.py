@@ -42,3 +42,26 @@ def test_no_further_from_float64(gpu, n, nz, na, mu, span, incl):
         e, e_lane = rel_l2(got, exact), rel_l2(ref, exact)
         print("%s: %.3e, per lane %.3e, ratio %.2f" % (name, e, e_lane, e / e_lane), flush=True)
         assert e <= 1.05 * e_lane
+
+
+@pytest.mark.parametrize("n, nz, na, span, incl", [(128, 96, 60, 360.0, 12.0), (96, 150, 48, 360.0, 5.0),
+                                                   (128, 64, 75, 180.0, 0.0), (160, 40, 60, 180.0, 0.0)])
+def test_equal_samples(gpu, n, nz, na, span, incl):
+    """Equal samples round a running sum the same way every time, so the per-lane kernels' error grows with the
+    ray.  Sums of at most 16 samples round at most at 16 / n of the ray's size, and the n / 16 additions of those
+    sums at its size but not all alike: below 0.7 of the per-lane error for n >= 96."""
+    import torch
+    import oracle.d1 as d1
+    from vamtoolbox_amd.parallel import ParallelPlan
+    ang = np.linspace(0.0, span, na, endpoint=False) + 0.5
+    plan, lane = [ParallelPlan(n, nz, ang, incl_deg=incl, warp_clip=False, per_lane_geometry=p, device=gpu)
+                  for p in (False, True)]
+    x = torch.full((n, n, nz), 0.7, device=gpu)
+    at = np.linspace(nz // 3, 2 * nz // 3, 5).astype(int)
+    x64 = x.cpu().numpy().astype(np.float64)
+    exact = d1.forward(x64 if incl else x64[..., at], ang, incl_deg=incl, clip_output=False)
+    if incl:
+        exact = exact[..., at]
+    e, e_lane = [rel_l2(p.forward(x).cpu().numpy()[..., at], exact) for p in (plan, lane)]
+    print("%.3e, per lane %.3e, ratio %.2f" % (e, e_lane, e / e_lane), flush=True)
+    assert e <= 0.7 * e_lane

@@ -226,8 +226,8 @@ __global__ __launch_bounds__(256) void incl_fp_batch_kernel(LaneTable t) {
 //
 // Bound by latency and instructions (two slices per lane: 4.6 4-byte loads and 30
 // vector instructions per sample, against 8 loads and 24 with the rows' own lanes,
-// which the texture path bound): 128 x 128 x 96 x 180, 12 degrees 279 -> 212 us (206
-// with the sample's two slices multiplied into the sum one after the other, which
+// which the texture path bound): 128 x 128 x 96 x 180, 12 degrees 279 -> 211 us (206
+// with the sample's two slices multiplied into the ray's sum one after the other, which
 // rounds it twice), x 256 x 90 398 -> 285, 100 x 100 x 300 x 60, 10 degrees 177 -> 121.
 // values of the next / previous slice (lane, and across the NS registers); 0 past
 // the ends
@@ -266,7 +266,14 @@ __device__ __forceinline__ void incl_fp_fixed_block(const ParDev& g, const float
 #pragma unroll
   for (int s = 0; s < NS; ++s) zo[s] = slice_off(z0 + 64 * s, nz);
   const InclSlot sl = incl_slot();
-  float acc[NS] = {}, T[4][NS] = {};   // T[2 a + b]: the tap of row parity a, column parity b
+  float acc[NS] = {}, part[NS] = {}, T[4][NS] = {};   // T[2 a + b]: the tap of row parity a, column parity b
+  auto add_part = [&]() {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      acc[s] += part[s];
+      part[s] = 0.0f;
+    }
+  };
   int at = 0;                          // shift of the last sample walked: lane z holds row z - at
   bool any = false;
   int last = -1, last_need = 15;       // cell and needed taps of the sample before the 64 (-1: none)
@@ -326,57 +333,65 @@ __device__ __forceinline__ void incl_fp_fixed_block(const ParDev& g, const float
     sl.w[lane] = w;
     sl.a[lane] = make_float4(aw0, aw1, 0.f, 0.f);
     __builtin_amdgcn_wave_barrier();
-    while (m) {
-      const int j = __builtin_ctzll(m);
-      m &= m - 1;
-      const float4 W = sl.w[j], A = sl.a[j];
-      const int c = rl_i(code, j), qj = rl_i(q, j);
-      if (big) {
-        const int b = rl_i(cell, j);
-        rs = buf_rsrc(vol + ((size_t)(b >> 14) * n + (b & 0x3fff)) * nz, 0x7fffffffu);
-      }
-      auto tap = [&](int a, int o) {
-        if (c >> a & 1) {
-          const uint32_t so = (uint32_t)rl_i(o, j);
-#pragma unroll
-          for (int s = 0; s < NS; ++s) T[a][s] = bload<1>(rs, zo[s], so);
+    // the samples are summed up to 16 at a time, as long as the shift stays: the
+    // ray's sums are rounded once per part, not twice per sample
+#pragma unroll 1
+    for (int from = 0; from < 64; from += 16) {
+      unsigned long long ms = m & (0xffffull << from);
+      while (ms) {
+        const int j = __builtin_ctzll(ms);
+        ms &= ms - 1;
+        const float4 W = sl.w[j], A = sl.a[j];
+        const int c = rl_i(code, j), qj = rl_i(q, j);
+        if (big) {
+          const int b = rl_i(cell, j);
+          rs = buf_rsrc(vol + ((size_t)(b >> 14) * n + (b & 0x3fff)) * nz, 0x7fffffffu);
         }
-      };
-      tap(0, o00);
-      tap(1, o01);
-      tap(2, o10);
-      tap(3, o11);
-      if (c >> 4) {
+        auto tap = [&](int a, int o) {
+          if (c >> a & 1) {
+            const uint32_t so = (uint32_t)rl_i(o, j);
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-          if (c >> (4 + a) & 1)
+            for (int s = 0; s < NS; ++s) T[a][s] = bload<1>(rs, zo[s], so);
+          }
+        };
+        tap(0, o00);
+        tap(1, o01);
+        tap(2, o10);
+        tap(3, o11);
+        if (c >> 4) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) T[a][s] = 0.0f;
+          for (int a = 0; a < 4; ++a)
+            if (c >> (4 + a) & 1)
+#pragma unroll
+              for (int s = 0; s < NS; ++s) T[a][s] = 0.0f;
+        }
+        if (!any) at = qj;   // nothing summed yet
+        any = true;
+        if (at != qj) add_part();
+        while (at < qj) {
+          float moved[NS];
+#pragma unroll
+          for (int s = 0; s < NS; ++s) moved[s] = slice_prev<NS>(acc, s);
+#pragma unroll
+          for (int s = 0; s < NS; ++s) acc[s] = moved[s];
+          ++at;
+        }
+        while (at > qj) {
+          float moved[NS];
+#pragma unroll
+          for (int s = 0; s < NS; ++s) moved[s] = slice_next<NS>(acc, s);
+#pragma unroll
+          for (int s = 0; s < NS; ++s) acc[s] = moved[s];
+          --at;
+        }
+        float v[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          v[s] = vfma(W.w, T[3][s], vfma(W.z, T[2][s], vfma(W.y, T[1][s], W.x * T[0][s])));
+#pragma unroll
+        for (int s = 0; s < NS; ++s) part[s] = vfma(A.y, slice_next<NS>(v, s), vfma(A.x, v[s], part[s]));
       }
-      if (!any) at = qj;   // nothing summed yet
-      any = true;
-      while (at < qj) {
-        float moved[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) moved[s] = slice_prev<NS>(acc, s);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) acc[s] = moved[s];
-        ++at;
-      }
-      while (at > qj) {
-        float moved[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) moved[s] = slice_next<NS>(acc, s);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) acc[s] = moved[s];
-        --at;
-      }
-      float v[NS];
-#pragma unroll
-      for (int s = 0; s < NS; ++s)
-        v[s] = vfma(W.w, T[3][s], vfma(W.z, T[2][s], vfma(W.y, T[1][s], W.x * T[0][s])));
-#pragma unroll
-      for (int s = 0; s < NS; ++s) acc[s] += vfma(A.y, slice_next<NS>(v, s), A.x * v[s]);   // one rounding of the sum
+      add_part();
     }
   }
 #pragma unroll
