@@ -1,4 +1,4 @@
-"""Thin and inclined problems of a batch that share launches, by class of kernel and lanes: bitwise the single
+"""Problems of a batch that share launches, by class of kernel and lanes (thin, inclined, and forward ones): bitwise the single
 calls, over sizes on both sides of an own launch, uneven mixtures, misaligned buffers, more problems than a launch
 holds, the warp clip on and off, and with the first call under capture (where no table can be built)."""
 
@@ -20,6 +20,9 @@ def _plans(gpu, mix, warp_clip):
     elif mix == "inclined":
         sizes = [(20, 5, 20, 4.0), (18, 12, 30, -8.0), (22, 31, 18, 15.0), (16, 40, 20, 10.0), (16, 100, 12, -20.0),
                  (24, 260, 12, 6.0), (12, 5, 20, 40.0), (60, 96, 60, 12.0)]
+    elif mix == "slabs":
+        sizes = [(24, 40, 24, 0.0), (20, 33, 16, 0.0), (33, 100, 9, 0.0), (17, 200, 20, 0.0), (18, 257, 12, 0.0),
+                 (24, 40, 24, 0.0), (21, 64, 30, 0.0), (16, 150, 16, 0.0), (22, 128, 40, 0.0), (80, 64, 120, 0.0)]
     else:
         sizes = [(20, 1, 20, 0.0), (24, 40, 20, 0.0), (18, 9, 16, 7.0), (33, 77, 24, 0.0), (16, 20, 30, 0.0), (20, 50, 16, -5.0)]
     return [ParallelPlan(n, nz, np.linspace(0.0, 360.0, na, endpoint=False), mu=0.01 * (i % 2), incl_deg=inc,
@@ -40,7 +43,7 @@ def _check(plans, B, v, s, f, b):
         assert torch.equal(p.forward(vi, out=_alike(fi)), fi) and torch.equal(p.backward(si, out=_alike(bi)), bi)
 
 
-@pytest.mark.parametrize("mix", ["slices", "one", "thin", "inclined", "mixed"])
+@pytest.mark.parametrize("mix", ["slices", "one", "thin", "inclined", "mixed", "slabs"])
 @pytest.mark.parametrize("warp_clip", [True, False])
 @pytest.mark.parametrize("positive", [True, False])
 def test_shared_launches(gpu, mix, warp_clip, positive):

@@ -1,18 +1,16 @@
 // Batched parallel-beam projection of many independent problems of uneven
-// size (gfx950): one persistent launch for most; in the forward direction,
-// problems large enough to fill the GPU on their own get single-problem launches
-// instead; problems of fewer than 32 slices or at an inclination run on kernels of
-// their own, those that do not fill the GPU several to a launch.  The launches
-// outside the persistent one are spread over three streams, and every problem's
-// result is that of its single call.
+// size (gfx950).  The back projections of 32 slices and more, and what takes the
+// per-lane kernels, share one persistent launch.  Forward projections, and problems of
+// fewer than 32 slices or at an inclination, run on the single-problem kernels: those
+// that fill the GPU by launches of their own, smaller ones several to a launch.  The
+// launches outside the persistent one are spread over three streams, and every
+// problem's result is that of its single call.
 //
 // Each problem is a parallel plan (vamx_par_create) with its own volume and
 // sinogram.  A problem's work is cut into tiles of one 256-thread block:
-// four wavefronts of the wavefront-uniform kernels (one ray -- or a ray and
-// its opposite ray, when the plan pairs opposite angles -- or one patch of 2 x 4
-// voxel columns, and 64 x ZV z values per wavefront, in the plan's L2-aware order)
-// or, for what those do not take (occlusion, one column), 256 items of the per-lane
-// kernels.  Tiles are ordered largest problem first and handed out
+// four wavefronts of the back projection (one patch of 2 x 4 voxel columns and 64 x
+// ZV z values per wavefront, in the plan's L2-aware order) or, for occlusion and a
+// single column, 256 items of the per-lane kernels.  Tiles are ordered largest problem first and handed out
 // by a device-side counter, so the resident blocks of the single launch drain
 // one queue until it is empty (every block exits when the counter passes the
 // tile count).  The counter is reset by a one-thread kernel on the same
@@ -34,10 +32,8 @@ struct BatchItem {
   long long items;       // wavefronts (wave mode) or threads (per-lane mode) of this problem
   int zv;                // z values per lane: 1 to 4 (wave mode) or 1, 4 (per-lane mode)
   int clip;              // forward: warp clip; backward: circle clip
-  int wave;              // 1: wavefront-uniform kernels
-  int pair;              // forward, wave mode: opposite-angle pairs (the plan's paired work order)
-  int split;             // forward, wave mode: lanes hold slices 64 apart
-  int contig, comb, chunks;   // backward, wave mode: BpLayout
+  int wave;              // backward, 1: the patches' wavefronts
+  int contig, comb, chunks;   // wave mode: BpLayout
 };
 
 // Buffers of the problems of one launch, passed by value as a kernel
@@ -50,29 +46,36 @@ struct BatchPtrs {
 
 __global__ void batch_reset(unsigned long long* counter) { *counter = 0ull; }
 
+// Forward of problems that do not fill the GPU alone, several to a launch: the
+// single-problem kernels' work (par_fp_wave_kernel, par_fp_pair_kernel), a block's
+// problem from the table
 template <int ZV, bool SPLIT>
-__device__ __forceinline__ void batch_fp_wave(const BatchItem& it, const float* in, float* out, long long w,
-                                              int lane) {
+__global__ __launch_bounds__(256) void fp_wave_batch_kernel(LaneTable t) {
+  unsigned lb;
+  const int p = lane_problem(t, lb), lane = threadIdx.x & 63;
+  const LaneProblem& it = t.items[p];
   const ParDev& g = it.g;
+  const float* in = t.in[p];
   int k, i, zc;
-  if (!fp_wave_item<ZV>(w, g, k, i, zc)) return;
+  if (!fp_wave_item<ZV>(wave_index(lb), g, k, i, zc)) return;
   const FpLane<ZV, SPLIT> ln(zc, lane, g.nz);
   const bool clip_on = it.clip && wave_clip_active(it.minmax, g.nz, ln);
   typename VecT<ZV>::T acc = clip_on ? fp_ray_wave<true, true, false>(g, in, it.minmax, k, i, ln, lane)
                                      : fp_ray_wave<false, true, false>(g, in, it.minmax, k, i, ln, lane);
   fp_ray_finish(g, in, it.minmax, clip_on, k, i, ln, acc);
-  ln.store(out + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
+  ln.store(t.out[p] + ((size_t)k * g.na + i) * g.nz, g.nz, acc);
 }
 
-// paired forward: ray (k, i) and its opposite ray from one pass over the
-// taps, as the single-problem paired kernel (clipped waves project the two
-// rays one after the other)
 template <int ZV, bool SPLIT>
-__device__ __forceinline__ void batch_fp_pair(const BatchItem& it, const float* in, float* out, long long w,
-                                              int lane) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void fp_pair_batch_kernel(LaneTable t) {
   using V = typename VecT<ZV>::T;
+  unsigned lb;
+  const int p = lane_problem(t, lb), lane = threadIdx.x & 63;
+  const LaneProblem& it = t.items[p];
   const ParDev& g = it.g;
-  const PairItem pi = fp_pair_item<ZV>(w, g);
+  const float* in = t.in[p];
+  float* out = t.out[p];
+  const PairItem pi = fp_pair_item<ZV>(wave_index(lb), g);
   if (!pi.ok) return;
   const FpLane<ZV, SPLIT> ln(pi.zc, lane, g.nz);
   if (it.clip && wave_clip_active(it.minmax, g.nz, ln)) {
@@ -169,38 +172,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORWARD ? 5
     // No `continue` below: a per-thread continue makes the loop header (and
     // its barriers) run for a subset of lanes, so waves of the block would
     // disagree on the barrier count.  Every thread reaches the loop end.
-    if (it.wave) {
+    if (!FORWARD && it.wave) {
       const long long w = (tile - it.tile_begin) * 4 + slot;
       if (w < it.items) {
-        if (FORWARD && it.pair) {
-          if (it.split && it.zv == 4) batch_fp_pair<4, true>(it, in, out, w, lane);
-          else if (it.split && it.zv == 3) batch_fp_pair<3, true>(it, in, out, w, lane);
-          else if (it.split) batch_fp_pair<2, true>(it, in, out, w, lane);
-          else if (it.zv == 4) batch_fp_pair<4, false>(it, in, out, w, lane);
-          else if (it.zv == 2) batch_fp_pair<2, false>(it, in, out, w, lane);
-          else batch_fp_pair<1, false>(it, in, out, w, lane);
-        } else if (FORWARD) {
-          if (it.split && it.zv == 4) batch_fp_wave<4, true>(it, in, out, w, lane);
-          else if (it.split && it.zv == 3) batch_fp_wave<3, true>(it, in, out, w, lane);
-          else if (it.split) batch_fp_wave<2, true>(it, in, out, w, lane);
-          else if (it.zv == 4) batch_fp_wave<4, false>(it, in, out, w, lane);
-          else if (it.zv == 2) batch_fp_wave<2, false>(it, in, out, w, lane);
-          else batch_fp_wave<1, false>(it, in, out, w, lane);
+        float2* const tab = tabs[FORWARD ? 0 : slot];
+        if (it.comb) {
+          if (it.contig) batch_bp_patch<4, true, true>(it, in, out, w, lane, tab);
+          else if (it.zv == 4) batch_bp_patch<4, false, true>(it, in, out, w, lane, tab);
+          else if (it.zv == 3) batch_bp_patch<3, false, true>(it, in, out, w, lane, tab);
+          else if (it.zv == 2) batch_bp_patch<2, false, true>(it, in, out, w, lane, tab);
+          else batch_bp_patch<1, false, true>(it, in, out, w, lane, tab);
         } else {
-          float2* const tab = tabs[FORWARD ? 0 : slot];
-          if (it.comb) {
-            if (it.contig) batch_bp_patch<4, true, true>(it, in, out, w, lane, tab);
-            else if (it.zv == 4) batch_bp_patch<4, false, true>(it, in, out, w, lane, tab);
-            else if (it.zv == 3) batch_bp_patch<3, false, true>(it, in, out, w, lane, tab);
-            else if (it.zv == 2) batch_bp_patch<2, false, true>(it, in, out, w, lane, tab);
-            else batch_bp_patch<1, false, true>(it, in, out, w, lane, tab);
-          } else {
-            if (it.contig) batch_bp_patch<4, true, false>(it, in, out, w, lane, tab);
-            else if (it.zv == 4) batch_bp_patch<4, false, false>(it, in, out, w, lane, tab);
-            else if (it.zv == 3) batch_bp_patch<3, false, false>(it, in, out, w, lane, tab);
-            else if (it.zv == 2) batch_bp_patch<2, false, false>(it, in, out, w, lane, tab);
-            else batch_bp_patch<1, false, false>(it, in, out, w, lane, tab);
-          }
+          if (it.contig) batch_bp_patch<4, true, false>(it, in, out, w, lane, tab);
+          else if (it.zv == 4) batch_bp_patch<4, false, false>(it, in, out, w, lane, tab);
+          else if (it.zv == 3) batch_bp_patch<3, false, false>(it, in, out, w, lane, tab);
+          else if (it.zv == 2) batch_bp_patch<2, false, false>(it, in, out, w, lane, tab);
+          else batch_bp_patch<1, false, false>(it, in, out, w, lane, tab);
         }
       }
     } else {
@@ -234,7 +221,7 @@ struct vamx_batch {
     std::vector<int> order;        // table position -> problem index
     std::vector<int> minmax;       // forward: problems whose per-slice min/max the warp clip needs
   };
-  struct Group {                   // thin or inclined problems of one class, in one launch
+  struct Group {                   // problems of one class, in one launch
     int key = 0;
     LaneProblem* d_items = nullptr;
     std::vector<int> order;        // table position -> problem index
@@ -314,32 +301,63 @@ int create_batch(vamx_plan* const* plans, int n, vamx_batch** out) {
   return VAMX_OK;
 }
 
-// kernel path of problem i for these buffers: slices per lane (forward + 8: 64
-// apart; backward + 8: contiguous, + 16: opposite angles combined); -1 / -4 for
-// the per-lane kernels with 1 / 4 z per thread; the class of a thin or inclined
-// problem (1 << 16 and up), or kOwnLaunch where it has a launch of its own
+// Kernel path of problem i for these buffers: the class of one that shares a launch
+// (1 << 16 and up), kOwnLaunch where it has one of its own, and in the persistent
+// launch slices per lane (back projection; + 8: contiguous, + 16: opposite angles
+// combined) or -1 / -4 for the per-lane kernels with 1 / 4 z per thread.
+//
+// The forward's wavefront kernels, and the thin and inclined ones, are not in the
+// persistent launch.  Its registers cover every layout, and each tile of four
+// wavefronts costs it an atomic, two barriers and a search: 64 forwards of 24 x 24 x
+// 32, 24 angles took 144 us there, those of 32 x 32 x 40, 40 angles 180, those of 48 x 48 x
+// 128, 60 angles 452; in shared launches 48, 90 and 318.  Below
+// kOwnWaves wavefronts (4 per SIMD) a problem cannot fill the GPU, and its launch takes
+// longer than its work: those of a class share a launch.
 constexpr int kOwnLaunch = 0;
-// Thin and inclined problems run on kernels that the persistent launch does not
-// hold.  Below this many wavefronts (4 per SIMD) one cannot fill the GPU, and its
-// launch takes longer than its work: those of a class share a launch.
 constexpr long long kOwnWaves = 4096;
+// class of a forward problem on the wavefront kernels: 3 << 16, opposite angles in
+// pairs << 8, slices 64 apart << 4, slices per lane
+LaneClass fp_class(const vamx_plan* p, const FpLayout& l, bool clip) {
+  const ParDev& g = p->par;
+  LaneClass c;
+  c.problem.g = g;
+  c.problem.minmax = p->d_minmax;
+  c.problem.clip = clip;
+  const int pair = g.fp_pair && g.pair_ok ? 1 : 0;
+  c.waves = (pair ? fp_pair_tiled(g) : fp_tiled_rays(g)) * wave_zchunks(g.nz, l.zv);
+  c.blocks = (c.waves + 3) / 4;
+  c.key = 3 << 16 | pair << 8 | (l.split ? 1 : 0) << 4 | l.zv;
+  return c;
+}
+int fp_batch(int key, const LaneTable& t, unsigned blocks, hipStream_t s) {
+  FpLayout l;
+  l.zv = key & 15;
+  l.split = key >> 4 & 1;
+  const bool pair = key >> 8 & 1;
+  fp_dispatch(l, true, [&](auto zv, auto split, auto) {
+    constexpr int ZV = decltype(zv)::value;
+    constexpr bool S = decltype(split)::value;
+    if (pair) hipLaunchKernelGGL((fp_pair_batch_kernel<ZV, S>), dim3(blocks), dim3(256), 0, s, t);
+    else hipLaunchKernelGGL((fp_wave_batch_kernel<ZV, S>), dim3(blocks), dim3(256), 0, s, t);
+  });
+  VAMX_HIP(hipGetLastError());
+  return VAMX_OK;
+}
+// key 0: a problem of the persistent launch
 LaneClass lane_class(const vamx_plan* p, const float* in, const float* out, bool forward) {
   const bool clip = !(p->flags & (forward ? VAMX_PAR_NO_WARP_CLIP : VAMX_PAR_NO_CIRCLE_CLIP));
-  return incl_wave_ok(p) ? incl_class(p, forward, clip) : thin_class(p, in, out, forward, clip);
+  if (incl_wave_ok(p)) return incl_class(p, forward, clip);
+  if (thin_ok(p)) return thin_class(p, in, out, forward, clip);
+  if (forward)
+    if (const FpLayout l = fp_layout(p, (uintptr_t)in | (uintptr_t)out); l.zv) return fp_class(p, l, clip);
+  return {};
 }
 int problem_path(vamx_plan* p, const float* in, float* out, bool forward, int problems) {
-  if (incl_wave_ok(p) || thin_ok(p)) {
-    if (problems == 1) return kOwnLaunch;
-    const LaneClass c = lane_class(p, in, out, forward);
-    return c.waves < kOwnWaves ? c.key : kOwnLaunch;
-  }
-  if (forward) {
-    const FpLayout l = fp_layout(p, (uintptr_t)in | (uintptr_t)out);
-    if (l.zv) return l.zv | (l.split ? 8 : 0);
-  } else {
-    const BpLayout l = bp_layout(p, (uintptr_t)in | (uintptr_t)out, problems);
-    if (l.zv) return l.zv | (l.contig ? 8 : 0) | (l.comb ? 16 : 0);
-  }
+  const LaneClass c = lane_class(p, in, out, forward);
+  if (c.key || thin_ok(p)) return problems > 1 && c.waves < kOwnWaves ? c.key : kOwnLaunch;
+  if (!forward)
+    if (const BpLayout l = bp_layout(p, (uintptr_t)in | (uintptr_t)out, problems); l.zv)
+      return l.zv | (l.contig ? 8 : 0) | (l.comb ? 16 : 0);
   return par_use_vec4(p, in, out) ? -4 : -1;
 }
 
@@ -348,16 +366,10 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
   std::vector<vamx_batch::Layout>& ls = b->layouts[forward ? 1 : 0];
   if (ls.size() >= kMaxLayouts)
     return set_error(VAMX_ERR_ARG, "batch: more than 8 distinct buffer alignments or work orders on one batch");
-  int cus = 0;
-  VAMX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
   const int n = (int)b->plans.size();
   vamx_batch::Layout L;
   L.sig = sig;
   L.devs = devs;
-  // Forward: a problem whose wavefront work alone fills the GPU (16 waves
-  // per CU) runs as its own single-problem launch: the persistent kernel,
-  // whose registers cover every z width and the per-lane fallback, reaches a
-  // lower occupancy than the single-problem forward kernels.
   std::vector<int> shared;
   std::vector<BatchItem> items((size_t)n);
   for (int i = 0; i < n; ++i) {
@@ -381,23 +393,13 @@ int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<c
       g->order.push_back(i);
       continue;
     }
-    if (path > 0 && !forward) {
+    if (path > 0) {
       it.wave = 1;
       it.zv = path & 7;
       it.contig = (path >> 3) & 1;
       it.comb = (path >> 4) & 1;
       it.chunks = wave_zchunks(it.g.nz, it.zv);
       it.items = (long long)it.g.bp_all * it.chunks;
-    } else if (path > 0) {
-      it.wave = 1;
-      it.zv = path & 7;
-      it.split = (path >> 3) & 1;
-      it.pair = it.g.fp_pair && it.g.pair_ok ? 1 : 0;
-      it.items = (it.pair ? fp_pair_tiled(it.g) : fp_tiled_rays(it.g)) * wave_zchunks(it.g.nz, it.zv);
-      if (!it.g.incl && it.items >= 16ll * cus) {
-        L.single.push_back(i);
-        continue;
-      }
     } else {
       it.wave = 0;
       it.zv = -path;
@@ -475,7 +477,8 @@ int run_group(const vamx_batch* b, const vamx_batch::Group& g, const float* cons
     t.in[r] = ins[i];
     t.out[r] = outs[i];
   }
-  return g.key >> 16 == 1 ? thin_batch(g.key, t, g.blocks, s) : incl_batch(g.key, t, g.blocks, s);
+  if (g.key >> 16 == 1) return thin_batch(g.key, t, g.blocks, s);
+  return g.key >> 16 == 2 ? incl_batch(g.key, t, g.blocks, s) : fp_batch(g.key, t, g.blocks, s);
 }
 
 int ensure_side_streams(vamx_batch* b) {
@@ -511,8 +514,8 @@ int run_batch(vamx_batch* b, const float* const* ins, float* const* outs, hipStr
   };
   find();
   if (!L && std::any_of(sig.begin(), sig.end(), [](int p) { return p >= 1 << 16; })) {
-    // a table cannot be uploaded while the stream is captured: thin and inclined
-    // problems then have launches of their own, which need none
+    // a table cannot be uploaded while the stream is captured: problems that share
+    // launches then have their own, which need none
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
       (void)hipGetLastError();

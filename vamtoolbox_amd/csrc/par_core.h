@@ -1889,8 +1889,8 @@ FpLayout fp_layout(const vamx_plan* p, uintptr_t align_bits);
 int wave_zv_choice(int nz, uintptr_t align_bits, int requested);
 void par_pair_units(const std::vector<double>& cs, int na, int n, int c, double D, std::vector<int>& units,
                     int& npaired_rays, int& first2);
-// Problems of a batch that share one launch of a thin or inclined kernel: those of
-// one class (kernel, lanes, slices per lane, wavefronts per block).  A block finds
+// Problems of a batch that share one launch of a forward, thin or inclined kernel:
+// those of one class (kernel, lanes, slices per lane, wavefronts per block).  A block finds
 // its problem by its number; the table is on the device, the buffers come with the
 // launch.
 constexpr int kBatchChunk = 64;   // problems per launch
