@@ -435,11 +435,16 @@ BpLayout vamx::bp_layout(const vamx_plan* p, uintptr_t align_bits, int problems)
   // wavefronts per SIMD (96 x 96 x 256, 120 angles, four slices in 930 of them: 78 us,
   // one in 3700: 55; 128 x 128 x 256, 180 angles, 1650: 120 and 120; 96 x 96 x 128, two
   // slices in 930: 52 us, one: 41; 128 x 128 x 77, 1650: 87 and 91).  Problems of a batch
-  // fill the GPU together.
-  constexpr int costs[2][5] = {{0, 21, 33, 48, 92}, {0, 16, 29, 43, 57}}, costs16[2] = {56, 45};
+  // fill the GPU together, in the persistent launch, whose registers leave one slice
+  // per lane no more wavefronts than four: 4 x 200 x 200, 240 angles took 1.02, 0.75, 0.90
+  // and 1.30 ms with one to four slices per lane (chunks of 128, 128, 192 and 256 slices)
+  // and 0.97 with 16-byte loads.
+  constexpr int costs[4][5] = {{0, 21, 33, 48, 92}, {0, 16, 29, 43, 57}, {0, 51, 75, 90, 130}, {0, 35, 53, 79, 105}};
+  constexpr int costs16[4] = {56, 45, 97, 80};
   constexpr int waves = 1536;
-  const int* const cost = costs[l.comb ? 1 : 0];
-  const int cost16 = costs16[l.comb ? 1 : 0];
+  const int mode = (l.comb ? 1 : 0) + (problems > 1 ? 2 : 0);
+  const int* const cost = costs[mode];
+  const int cost16 = costs16[mode];
   int best = INT_MAX;
   for (int zv = 1; zv <= g.bp_zv; ++zv) {
     const int c = wave_zchunks(g.nz, zv);
