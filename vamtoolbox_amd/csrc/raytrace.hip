@@ -87,7 +87,8 @@ __device__ __forceinline__ bool grid_move(const RtDev& g, d3 x, GridPos& p) {
   p.wx = (float)(ix - (double)p.x0);
   p.wy = (float)(iy - (double)p.y0);
   p.wz = (float)(iz - (double)p.z0);
-  if (p.wx >= 0.0f && p.wy >= 0.0f && p.wz >= 0.0f && p.wx <= 1.0f && p.wy <= 1.0f && p.wz <= 1.0f) return false;
+  // (the sum: min3 and max3 pass over a NaN)
+  if (min3(p.wx, p.wy, p.wz) >= 0.0f && max3(p.wx, p.wy, p.wz) <= 1.0f && p.wx + p.wy + p.wz >= 0.0f) return false;
   const double fx = floor(ix), fy = floor(iy), fz = floor(iz);
   p.x0 = (float)fx; p.y0 = (float)fy; p.z0 = (float)fz;
   p.wx = (float)(ix - fx); p.wy = (float)(iy - fy); p.wz = (float)(iz - fz);
@@ -159,19 +160,20 @@ __device__ __forceinline__ void lune_sample(const RtDev& g, double x, double y, 
 // rounds to 1, would otherwise change cells at every sample.  A tap past the last voxel
 // along an axis (coordinate exactly size - 1, weight 0) reads the last voxel.
 __device__ __forceinline__ float cell_step(float w) { return w == 1.0f ? 0.0f : floorf(w); }
+template <bool OFF>
 __device__ __forceinline__ void field_sample_at(const RtDev& g, float ox, float oy, float oz, FieldCell& fc, float& n,
                                                 float& gx, float& gy, float& gz) {
-  float wx = __builtin_amdgcn_fmed3f((float)(fc.bx + (double)ox), -fc.x0, fc.hx);
-  float wy = __builtin_amdgcn_fmed3f((float)(fc.by + (double)oy), -fc.y0, fc.hy);
-  float wz = __builtin_amdgcn_fmed3f((float)(fc.bz + (double)oz), -fc.z0, fc.hz);
+  float wx = __builtin_amdgcn_fmed3f((float)(OFF ? fc.bx + (double)ox : fc.bx), -fc.x0, fc.hx);
+  float wy = __builtin_amdgcn_fmed3f((float)(OFF ? fc.by + (double)oy : fc.by), -fc.y0, fc.hy);
+  float wz = __builtin_amdgcn_fmed3f((float)(OFF ? fc.bz + (double)oz : fc.bz), -fc.z0, fc.hz);
   if (!(min3(wx, wy, wz) >= 0.0f && max3(wx, wy, wz) <= 1.0f)) {
     const float fx = cell_step(wx), fy = cell_step(wy), fz = cell_step(wz);
     fc.x0 += fx; fc.y0 += fy; fc.z0 += fz;
     fc.hx -= fx; fc.hy -= fy; fc.hz -= fz;
     fc.bx -= (double)fx; fc.by -= (double)fy; fc.bz -= (double)fz;
-    wx = __builtin_amdgcn_fmed3f((float)(fc.bx + (double)ox), 0.0f, fc.hx);
-    wy = __builtin_amdgcn_fmed3f((float)(fc.by + (double)oy), 0.0f, fc.hy);
-    wz = __builtin_amdgcn_fmed3f((float)(fc.bz + (double)oz), 0.0f, fc.hz);
+    wx = __builtin_amdgcn_fmed3f((float)(OFF ? fc.bx + (double)ox : fc.bx), 0.0f, fc.hx);
+    wy = __builtin_amdgcn_fmed3f((float)(OFF ? fc.by + (double)oy : fc.by), 0.0f, fc.hy);
+    wz = __builtin_amdgcn_fmed3f((float)(OFF ? fc.bz + (double)oz : fc.bz), 0.0f, fc.hz);
     const int sx = fc.hx >= 1.0f ? g.ny * g.nz : 0, sy = fc.hy >= 1.0f ? g.nz : 0, sz = fc.hz >= 1.0f ? 1 : 0;
     // inside the grid for every finite position; kept there for any other
     const int key = ((int)fc.x0 * g.ny + (int)fc.y0) * g.nz + (int)fc.z0;
@@ -211,7 +213,7 @@ __device__ __forceinline__ void field_sample(const RtDev& g, d3 x, FieldCell& fc
   if constexpr (LUNE)
     lune_sample(g, x.x, x.y, x.z, nf, gx, gy, gz);
   else
-    field_sample_at(g, 0.0f, 0.0f, 0.0f, fc, nf, gx, gy, gz);
+    field_sample_at<false>(g, 0.0f, 0.0f, 0.0f, fc, nf, gx, gy, gz);
   n = (double)nf;
   gn = mk((double)gx, (double)gy, (double)gz);
 }
@@ -275,7 +277,7 @@ __device__ __forceinline__ d3 advance(const RtDev& g, d3& x, d3& v, FieldCell& f
         const double iz = g.nz > 1 ? (x.z - g.zmin) * g.inv_dz + (double)oz : 0.0;
         lune_sample(g, g.xmin + ix * g.dx, g.ymin + iy * g.dy, g.nz > 1 ? g.zmin + iz * g.dz : g.zmin, n, gx, gy, gz);
       } else {
-        field_sample_at(g, ox, oy, oz, fc, n, gx, gy, gz);
+        field_sample_at<true>(g, ox, oy, oz, fc, n, gx, gy, gz);
       }
       float kx0 = (float)(v.x + (double)(k.c * kv0));
       float kx1 = (float)(v.y + (double)(k.c * kv1));
@@ -462,6 +464,10 @@ __device__ __forceinline__ void tap_move(const RtDev& g, const RtIo& io, TapCell
 //   64^3, 90 angles    both 1960 -> 1785 us
 //   192^3, 360 angles  both 145 -> 126 ms
 //   43^2 x 71, 71 angles (wavefronts across two rows of rays) 1040 -> 937 us
+// Integrate alone, taps outside the grid masked -> f_eff in a border of zeros (the masks
+// and clamps were a third of a cell's change, and a second set of loads for cells
+// inside): 300^2, 180 angles, leapfrog 950 -> 810 us, Euler 949 -> 816, RK4 1648 -> 1529;
+// 64^3, 90 angles 528 -> 477, 527 -> 476, 944 -> 873.
 template <int MODE, int SOLVER, int PARAM, bool LUNE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rt_trace_kernel(RtDev g, RtIo io) {
   const long long nrays = (long long)g.nt * g.na * g.nzr;
@@ -497,7 +503,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
   GridPos p;
   ray_init<SOLVER, PARAM, LUNE>(g, t, a, zr, x, v, p, fc);
   const double hw = g.hw;
-  const float e0f = (float)E0;
+  // in a vector register: the scalar ones are full, and a ray's energy that is the
+  // same for all was a scalar load, and a wait for it, in every step
+  float e0f = (float)E0;
+  asm("" : "+v"(e0f));
   double A = 0.0, integral = 0.0;
   int step = 0, until_exit = 1;
   bool active = live;
@@ -517,27 +526,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         const double base = hw * E;
         if (MODE == RT_INTEGRATE) {
           if (moved) {
-            const int x0 = (int)p.x0, y0 = (int)p.y0, z0 = (int)p.z0, plane = g.ny * g.nz;
+            // (the corner is -1 at the least: inside f_eff's border)
+            const int x0 = (int)p.x0, y0 = (int)p.y0, z0 = (int)p.z0;
             float fv[8];
-            // every lane's taps inside the grid: fixed strides; else taps outside
-            // read an in-grid voxel and hold 0
-            const bool in = x0 >= 0 && y0 >= 0 && z0 >= 0 && x0 + 1 < g.nx && y0 + 1 < g.ny && z0 + 1 < g.nz;
-            if (__ballot(!in) == 0ull) {
-              const float* b = io.feff + ((x0 * g.ny + y0) * g.nz + z0);
+            const float* b = io.feff + ((unsigned)x0 * (unsigned)g.eff_plane + (unsigned)y0 * (unsigned)g.eff_row +
+                                        (unsigned)z0 + g.eff_origin);
 #pragma unroll
-              for (int c = 0; c < 8; ++c) fv[c] = b[(c & 1) * plane + ((c >> 1) & 1) * g.nz + (c >> 2)];
-            } else {
-              const bool vx[2] = {x0 >= 0, x0 + 1 < g.nx}, vy[2] = {y0 >= 0, y0 + 1 < g.ny};
-              const bool vz[2] = {z0 >= 0, z0 + 1 < g.nz};
-              const int ax[2] = {max(x0, 0) * plane, min(x0 + 1, g.nx - 1) * plane};
-              const int ay[2] = {max(y0, 0) * g.nz, min(y0 + 1, g.ny - 1) * g.nz};
-              const int az[2] = {max(z0, 0), min(z0 + 1, g.nz - 1)};
-#pragma unroll
-              for (int c = 0; c < 8; ++c) {
-                const float f = io.feff[ax[c & 1] + ay[(c >> 1) & 1] + az[c >> 2]];
-                fv[c] = vx[c & 1] && vy[(c >> 1) & 1] && vz[c >> 2] ? f : 0.0f;
-              }
-            }
+            for (int c = 0; c < 8; ++c) fv[c] = b[(c & 1) * g.eff_plane + ((c >> 1) & 1) * g.eff_row + (c >> 2)];
             tc.f = tri_coef(fv);
           }
           integral += base * (double)tri_eval(tc.f, p.wx, p.wy, p.wz);
@@ -603,11 +598,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
   }
 }
 
+// f_eff is held in a border of zeros one voxel wide (in 2-D the border on z is the
+// one voxel above), so that the taps of every cell a ray can be in are loads at
+// fixed strides.  eff_voxel: place of voxel i; eff_border: place of the border's
+// voxel b.
+__device__ __forceinline__ size_t eff_voxel(const RtDev& g, long long i) {
+  const unsigned v = (unsigned)i, nz = (unsigned)g.nz, ny = (unsigned)g.ny;   // (fewer than 2^31 voxels)
+  const unsigned q = v / nz, x = q / ny;
+  return (size_t)x * g.eff_plane + (size_t)(q - x * ny) * g.eff_row + (v - q * nz) + g.eff_origin;
+}
+__device__ __forceinline__ size_t eff_border(const RtDev& g, long long b) {
+  const long long plane = g.eff_plane, row = g.eff_row;
+  if (b < 2 * plane) return (size_t)(b < plane ? b : b + (long long)g.nx * plane);   // the planes of x
+  b -= 2 * plane;
+  if (b < 2 * row * g.nx) {   // the rows of y in each other plane
+    const long long x = 1 + b / (2 * row), r = b % (2 * row);
+    return (size_t)(x * plane + (r < row ? r : r + (long long)g.ny * row));
+  }
+  b -= 2 * row * g.nx;        // the voxels of z in each other row
+  const int per = g.eff_row - g.nz;
+  const long long col = b / per;
+  const int e = (int)(b % per);
+  const int z = per == 2 && e == 0 ? 0 : g.eff_row - 1;
+  return (size_t)((1 + col / g.ny) * plane + (1 + col % g.ny) * row + z);
+}
+inline long long eff_size(const RtDev& g) { return (long long)(g.nx + 2) * g.eff_plane; }
+
 // f_eff = alpha_abs * f  (pyTorchRayTrace.py:515-519)
-__global__ __launch_bounds__(256) void rt_feff_kernel(const float* __restrict__ f, const float* __restrict__ ab,
-                                                      float* __restrict__ out, long long nv) {
+__global__ __launch_bounds__(256) void rt_feff_kernel(RtDev g, const float* __restrict__ f,
+                                                      const float* __restrict__ ab, float* __restrict__ out,
+                                                      long long nv, long long total) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nv) out[i] = ab ? f[i] * ab[i] : f[i];
+  if (i < nv)
+    out[eff_voxel(g, i)] = ab ? f[i] * ab[i] : f[i];
+  else if (i < total)
+    out[eff_border(g, i - nv)] = 0.0f;
 }
 
 // max |g| for the fixed-point scale, pass 1: block b reduces a contiguous
@@ -682,16 +707,25 @@ __global__ __launch_bounds__(256) void rt_finalize_kernel(const unsigned long lo
 // dose = alpha_abs acc / scale, the response, band and Lp weighting per
 // voxel, the operand (times ab_op when given: alpha_abs makes it the f_eff
 // that the gradient's integrate pass reads) and per-block loss partials.
-__global__ __launch_bounds__(256) void rt_bclp_finalize_kernel(const unsigned long long* __restrict__ acc,
+// EFF: the operand goes into f_eff's border of zeros, which the blocks from nparts on
+// write; else into an array like the dose.
+template <bool EFF>
+__global__ __launch_bounds__(256) void rt_bclp_finalize_kernel(RtDev g, const unsigned long long* __restrict__ acc,
                                                                const float* __restrict__ ab,
                                                                const float* __restrict__ ab_op,
                                                                const double* __restrict__ fx_scale, RespDev r,
                                                                BclpDev b, const float* __restrict__ target,
                                                                float* __restrict__ dose,
                                                                float* __restrict__ operand_eff,
-                                                               double* __restrict__ partials, long long nv) {
+                                                               double* __restrict__ partials, long long nv,
+                                                               int nparts, long long nborder) {
   __shared__ double sh[256];
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (EFF && (int)blockIdx.x >= nparts) {
+    const long long e = i - (long long)nparts * 256;
+    if (e < nborder) operand_eff[eff_border(g, e)] = 0.0f;
+    return;
+  }
   double part = 0.0;
   if (i < nv) {
     const double v = (double)(long long)acc[i] / *fx_scale;
@@ -699,7 +733,7 @@ __global__ __launch_bounds__(256) void rt_bclp_finalize_kernel(const unsigned lo
     dose[i] = d;
     float o;
     part = bclp_voxel(r, b, d, target[i], (size_t)i, o);
-    operand_eff[i] = ab_op ? o * ab_op[i] : o;
+    operand_eff[EFF ? eff_voxel(g, i) : (size_t)i] = ab_op ? o * ab_op[i] : o;
   }
   const double sum = block_sum_256(part, sh);
   if (threadIdx.x == 0) partials[blockIdx.x] = sum;
@@ -778,6 +812,9 @@ extern "C" int vamx_rt_create(const vamx_rt_geom* geom, vamx_plan** out_plan) {
   g.xmax = g.xmin + (g.nx - 1) * g.dx;
   g.ymax = g.ymin + (g.ny - 1) * g.dy;
   g.zmax = g.nz > 1 ? g.zmin + (g.nz - 1) * g.dz : g.zmin;
+  g.eff_row = g.nz > 1 ? g.nz + 2 : 2;
+  g.eff_plane = (g.ny + 2) * g.eff_row;
+  g.eff_origin = (unsigned)(g.eff_plane + g.eff_row + (g.nz > 1));
   g.last_x = (float)(g.nx - 1); g.last_y = (float)(g.ny - 1); g.last_z = (float)(g.nz - 1);
   g.nt = geom->nt; g.na = geom->n_angles; g.nzr = geom->nzr;
   g.incl = geom->incl_deg * (M_PI / 180.0);
@@ -837,7 +874,9 @@ extern "C" int vamx_rt_create(const vamx_rt_geom* geom, vamx_plan** out_plan) {
   const size_t nv = (size_t)g.nx * g.ny * g.nz;
   hipError_t e = hipMalloc((void**)&p->d_rt_tables, tab.size() * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(p->d_rt_tables, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc((void**)&p->d_accum, nv * sizeof(unsigned long long));
+  // the deposit's accumulator, or f_eff and its border
+  const size_t acc_bytes = std::max(nv * sizeof(unsigned long long), (size_t)eff_size(g) * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc((void**)&p->d_accum, acc_bytes);
   // [0]: scale (double); from byte 64: kGmaxParts per-block maxima (float)
   if (e == hipSuccess) e = hipMalloc((void**)&p->d_gmax, 64 + kGmaxParts * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&p->d_stats, 2 * sizeof(unsigned long long));
@@ -859,7 +898,8 @@ extern "C" int vamx_rt_integrate(vamx_plan* plan, const float* f, float* gout, v
   const RtDev& g = plan->rt;
   const long long nv = (long long)g.nx * g.ny * g.nz;
   float* feff = (float*)plan->d_accum;  // the accumulator doubles as f_eff storage
-  hipLaunchKernelGGL(rt_feff_kernel, dim3(blocks_for(nv, 256)), dim3(256), 0, s, f, g.abs_grid, feff, nv);
+  const long long ne = eff_size(g);
+  hipLaunchKernelGGL(rt_feff_kernel, dim3(blocks_for(ne, 256)), dim3(256), 0, s, g, f, g.abs_grid, feff, nv, ne);
   hipLaunchKernelGGL(rt_zero_stats, dim3(1), dim3(1), 0, s, plan->d_stats);
   const long long nrays = (long long)g.nt * g.na * g.nzr;
   RtIo io{};
@@ -963,7 +1003,7 @@ RtBclpWs rt_bclp_ws(const vamx_plan* p) {
   w.partials_off = 0;
   w.scale_off = ((size_t)w.nparts * sizeof(double) + 255) / 256 * 256;
   w.operand_off = w.scale_off + 256;
-  w.total = w.operand_off + (size_t)nv * sizeof(float);
+  w.total = w.operand_off + (size_t)eff_size(g) * sizeof(float);
   return w;
 }
 
@@ -1013,8 +1053,10 @@ extern "C" int vamx_rt_bclp_step(vamx_plan* plan, const vamx_response* resp, con
   rc = launch_trace<RT_DEPOSIT>(gd, dim3(blocks_for(nrays, 256)), s, io);
   if (rc) return rc;
   // response, band, Lp weighting, operand and loss partials; loss and scale
-  hipLaunchKernelGGL(rt_bclp_finalize_kernel, dim3(w.nparts), dim3(256), 0, s, plan->d_accum, gd.abs_grid,
-                     gd.abs_grid, (const double*)fx_scale, r, b, target, dose, operand_eff, partials, nv);
+  const long long nborder = eff_size(gd) - nv;
+  hipLaunchKernelGGL((rt_bclp_finalize_kernel<true>), dim3(w.nparts + blocks_for(nborder, 256)), dim3(256), 0, s, gd,
+                     plan->d_accum, gd.abs_grid, gd.abs_grid, (const double*)fx_scale, r, b, target, dose, operand_eff,
+                     partials, nv, w.nparts, nborder);
   VAMX_HIP(hipGetLastError());
   rc = bclp_reduce_launch(partials, w.nparts, b, nullptr, iter_counter, loss_log, scale, s);
   if (rc) return rc;
@@ -1068,8 +1110,9 @@ extern "C" int vamx_rt_bclp_eval(vamx_plan* plan, const vamx_response* resp, con
   io.stats = plan->d_stats;
   rc = launch_trace<RT_DEPOSIT>(gd, dim3(blocks_for(nrays, 256)), s, io);
   if (rc) return rc;
-  hipLaunchKernelGGL(rt_bclp_finalize_kernel, dim3(w.nparts), dim3(256), 0, s, plan->d_accum, gd.abs_grid,
-                     (const float*)nullptr, (const double*)fx_scale, r, b, target, dose, op, partials, nv);
+  hipLaunchKernelGGL((rt_bclp_finalize_kernel<false>), dim3(w.nparts), dim3(256), 0, s, gd, plan->d_accum, gd.abs_grid,
+                     (const float*)nullptr, (const double*)fx_scale, r, b, target, dose, op, partials, nv, w.nparts,
+                     0ll);
   VAMX_HIP(hipGetLastError());
   rc = bclp_reduce_launch(partials, w.nparts, b, loss_out, nullptr, nullptr, scale, s);
   if (rc) return rc;

@@ -60,6 +60,8 @@ struct RkStage {
 // Geometry of the curved-ray tracer, passed by value.
 struct RtDev {
   int nx, ny, nz;
+  int eff_row, eff_plane;     // strides of f_eff in its border of zeros (rows of z, planes of y)
+  unsigned eff_origin;        // place of voxel (0, 0, 0) in it
   double xmin, ymin, zmin, dx, dy, dz;
   double inv_dx, inv_dy, inv_dz;
   double xmax, ymax, zmax;
