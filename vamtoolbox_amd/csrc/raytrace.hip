@@ -455,7 +455,7 @@ __device__ __forceinline__ void tap_move(const RtDev& g, const RtIo& io, TapCell
 }
 
 // at most 128 VGPRs: 4 wavefronts per SIMD (deposit at 5 spilled: 1285 us against
-// 997 at 64^3 x 90).  Bound by instructions: a step takes about 570 (wavefront
+// 997 at 64^3 x 90).  Bound by instructions: a step takes about 560 (wavefront
 // instructions, 4 to 4.5 cycles each on a SIMD), of them 74 for each of the four
 // stages and 100 for a field cell's change, of which a wavefront sees about one
 // per step; deposit, 440, waits besides for its atomics, which execute in memory
