@@ -83,3 +83,38 @@ def test_capture(gpu, mix, warm):
         torch.cuda.synchronize()
         _check(plans, B, v, s, f, b)
         f.zero_(), b.zero_()
+
+
+def test_many_alignments(gpu):
+    """Each problem's buffers aligned and not: more combinations than a batch keeps tables of."""
+    import ctypes
+    import torch
+    from vamtoolbox_amd import _lib
+    from vamtoolbox_amd.parallel import ParallelPlan
+    lib = _lib.load()
+    plans = [ParallelPlan(n, 4, np.linspace(0.0, 360.0, na, endpoint=False), mu=0.01, device=gpu)
+             for n, na in [(12, 9), (16, 12), (18, 20), (21, 16)]]
+    handle = ctypes.c_void_p()
+    arr = (ctypes.c_void_p * 4)(*[p.handle for p in plans])
+    _lib.check(lib.vamx_batch_create(arr, 4, ctypes.byref(handle)), "vamx_batch_create")
+
+    def buffers(shapes, bits):
+        out = []
+        for j, sh in enumerate(shapes):
+            m = int(np.prod(sh))
+            out.append(torch.rand(m + 4, device=gpu)[bits >> j & 1:][:m].view(sh))
+        return out
+
+    try:
+        for bits in list(range(12)) + [0, 11]:
+            v = buffers([p.vol_shape for p in plans], bits)
+            s, f, b = (buffers([x.shape for x in y], bits) for y in ([torch.empty(p.sino_shape) for p in plans],
+                                                                     [torch.empty(p.sino_shape) for p in plans], v))
+            pv, ps, pf, pb = ((ctypes.c_void_p * 4)(*[x.data_ptr() for x in y]) for y in (v, s, f, b))
+            _lib.check(lib.vamx_batch_forward(handle, pv, pf, _lib.stream_ptr(gpu)), "vamx_batch_forward")
+            _lib.check(lib.vamx_batch_backward(handle, ps, pb, _lib.stream_ptr(gpu)), "vamx_batch_backward")
+            for p, vi, si, fi, bi in zip(plans, v, s, f, b):
+                assert torch.equal(p.forward(vi, out=_alike(fi)), fi) and torch.equal(p.backward(si, out=_alike(bi)), bi)
+    finally:
+        torch.cuda.synchronize()
+        lib.vamx_batch_destroy(handle)

@@ -361,10 +361,16 @@ int problem_path(vamx_plan* p, const float* in, float* out, bool forward, int pr
   return par_use_vec4(p, in, out) ? -4 : -1;
 }
 
+// layouts that have shared launches, or those that don't: each kind up to kMaxLayouts
+size_t layouts_with(const std::vector<vamx_batch::Layout>& ls, bool groups) {
+  return (size_t)std::count_if(ls.begin(), ls.end(), [&](const vamx_batch::Layout& l) { return groups != l.groups.empty(); });
+}
+
 int build_layout(vamx_batch* b, const std::vector<int>& sig, const std::vector<char>& devs, const float* const* ins,
                  float* const* outs, bool forward, hipStream_t s, vamx_batch::Layout** out) {
   std::vector<vamx_batch::Layout>& ls = b->layouts[forward ? 1 : 0];
-  if (ls.size() >= kMaxLayouts)
+  const bool groups = std::any_of(sig.begin(), sig.end(), [](int p) { return p >= 1 << 16; });
+  if (layouts_with(ls, groups) >= kMaxLayouts)
     return set_error(VAMX_ERR_ARG, "batch: more than 8 distinct buffer alignments or work orders on one batch");
   const int n = (int)b->plans.size();
   vamx_batch::Layout L;
@@ -514,11 +520,13 @@ int run_batch(vamx_batch* b, const float* const* ins, float* const* outs, hipStr
   };
   find();
   if (!L && std::any_of(sig.begin(), sig.end(), [](int p) { return p >= 1 << 16; })) {
-    // a table cannot be uploaded while the stream is captured: problems that share
-    // launches then have their own, which need none
+    // a table cannot be uploaded while the stream is captured, and a batch keeps
+    // kMaxLayouts of them: problems that share launches then have their own, which
+    // need none
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
+    const bool capturing = hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+    if (capturing || layouts_with(b->layouts[forward ? 1 : 0], true) >= kMaxLayouts) {
+      if (capturing) (void)hipGetLastError();
       for (int& p : sig)
         if (p >= 1 << 16) p = kOwnLaunch;
       find();
